@@ -78,7 +78,6 @@ struct pikgpu_ctx {
   int out_flags = kOutLinear;
   int downsample = 1;
   int ran_flags = 0;
-  int spitch = 0;
   int out_xsize = 0, out_ysize = 0;  // output size of the last run
   bool ran_downsampled = false;
   bool timed = false;   // the last run recorded timing events
@@ -154,6 +153,9 @@ void FreeAll(pikgpu_ctx* ctx) {
 // the host plane is strided; longer ones go row by row (per-row copy cost
 // is then small against the row's own transfer).
 constexpr size_t kStageRowMax = 32 << 10;
+// Dense planes of at most this many bytes together are downloaded as one
+// staged copy instead of one copy each.
+constexpr size_t kStageSmall = 128 << 10;
 // Most bytes staged at once (larger planes go in chunks of rows).
 constexpr size_t kStageChunk = 16 << 20;
 
@@ -668,7 +670,8 @@ int pikgpu_frame_upload(pikgpu_ctx* ctx, const pikgpu_frame* f) {
   const size_t nblk = bx * by;
   const size_t ngroups = size_t(P.gx) * P.gy;
   const size_t ipitch = DivCeil(bx * 8, 32) * 32;
-  const size_t opitch = DivCeil(f->xsize, 32) * 32;
+  // dense output rows: a download is one linear copy per plane
+  const size_t opitch = f->xsize;
   int rc;
 #define GROW(buf, bytes) \
   if ((rc = Grow(ctx, &ctx->buf, (bytes))) != PIKGPU_OK) return rc
@@ -1069,8 +1072,9 @@ static int Enqueue(pikgpu_ctx* ctx, hipStream_t st, bool keep_stages,
   }
   // output size (ShrinkTo of the reference's final stage)
   const int out_xs = int(DivCeil(P.xsize, ds)), out_ys = int(DivCeil(P.ysize, ds));
+  B.opitch = out_xs;
   if (P.out_flags & kOutSrgb8) {
-    B.spitch = int(DivCeil(size_t(out_xs) * 3, 64) * 64);
+    B.spitch = 3 * out_xs;
     if ((rc = Grow(ctx, &ctx->srgb8, size_t(B.spitch) * out_ys))) return rc;
     B.srgb8 = static_cast<uint8_t*>(ctx->srgb8.p);
   }
@@ -1104,11 +1108,52 @@ static int Enqueue(pikgpu_ctx* ctx, hipStream_t st, bool keep_stages,
   ctx->ran = true;
   ctx->kept = B.keep;
   ctx->ran_flags = P.out_flags;
-  ctx->spitch = B.spitch;
   ctx->out_xsize = out_xs;
   ctx->out_ysize = out_ys;
   ctx->ran_downsampled = ds != 1;
   return PIKGPU_OK;
+}
+
+// Copies `planes` dense device planes (rows rows of row_b bytes each, one
+// after the other from src) to host planes with the given row stride, and
+// waits. A dense host plane takes one linear copy. Short strided rows, and
+// planes so small that a copy each would cost more than the bytes (the
+// runtime's own cost per copy is about 10 us, a host memcpy of 128 KB about
+// the same), come through pinned staging in chunks and are placed by the
+// host. A 2-D copy is one DMA per row (13 us each, 4.4 ms for 533 rows), so
+// only long rows use it.
+static int DownloadRows(pikgpu_ctx* ctx, uint8_t* const* dst, int planes,
+                        size_t stride_b, const void* src, size_t row_b,
+                        size_t rows) {
+  const uint8_t* from = static_cast<const uint8_t*>(src);
+  const size_t plane_b = row_b * rows;
+  const bool dense = rows <= 1 || stride_b == row_b;
+  if (dense ? planes > 1 && planes * plane_b <= kStageSmall
+            : row_b < kStageRowMax) {
+    const size_t all = size_t(planes) * rows;
+    const size_t per = std::max<size_t>(1, kStageChunk / row_b);
+    int rc = StageReserve(ctx, std::min(per, all) * row_b);
+    if (rc != PIKGPU_OK) return rc;
+    const uint8_t* p = static_cast<const uint8_t*>(ctx->stage);
+    for (size_t r0 = 0; r0 < all; r0 += per) {
+      const size_t n = std::min(per, all - r0);
+      HIP_TRY(ctx, hipMemcpyAsync(ctx->stage, from + r0 * row_b, n * row_b,
+                                  hipMemcpyDeviceToHost, ctx->stream));
+      if ((rc = pikgpu_sync(ctx)) != PIKGPU_OK) return rc;
+      for (size_t r = r0; r < r0 + n;) {
+        const size_t c = r / rows, y = r - c * rows;
+        const size_t m = dense ? std::min(rows - y, r0 + n - r) : 1;
+        memcpy(dst[c] + y * stride_b, p + (r - r0) * row_b, m * row_b);
+        r += m;
+      }
+    }
+    return PIKGPU_OK;
+  }
+  for (int c = 0; c < planes; ++c) {
+    HIP_TRY(ctx, Copy2D(dst[c], stride_b, from + c * plane_b, row_b, row_b,
+                        rows, hipMemcpyDeviceToHost, ctx->stream));
+  }
+  return pikgpu_sync(ctx);
 }
 
 extern "C" {
@@ -1162,38 +1207,10 @@ int pikgpu_download(pikgpu_ctx* ctx, float* out_planes[3],
     return Fail(ctx, PIKGPU_EINVAL, "output stride smaller than a row");
   }
   HIP_TRY(ctx, hipSetDevice(ctx->device));
-  const size_t oplane = size_t(ctx->B.opitch) * ys;
-  const size_t dpitch_b = size_t(ctx->B.opitch) * 4, row_b = xs * 4;
-  if (ys > 1 && (dpitch_b != row_b || out_stride_bytes != row_b) &&
-      row_b < kStageRowMax) {
-    // Short strided rows: chunks of whole device rows (contiguous) to
-    // pinned staging, then row by row on the host.
-    const size_t per = std::max<size_t>(1, kStageChunk / dpitch_b);
-    int rc = StageReserve(ctx, std::min(per, ys) * dpitch_b);
-    if (rc != PIKGPU_OK) return rc;
-    const uint8_t* p = static_cast<const uint8_t*>(ctx->stage);
-    for (int c = 0; c < 3; ++c) {
-      uint8_t* q = reinterpret_cast<uint8_t*>(out_planes[c]);
-      const float* plane = ctx->B.out + c * oplane;
-      for (size_t y0 = 0; y0 < ys; y0 += per) {
-        const size_t ny = std::min(per, ys - y0);
-        HIP_TRY(ctx, hipMemcpyAsync(ctx->stage, plane + y0 * (dpitch_b / 4),
-                                    ny * dpitch_b, hipMemcpyDeviceToHost,
-                                    ctx->stream));
-        if ((rc = pikgpu_sync(ctx)) != PIKGPU_OK) return rc;
-        for (size_t y = 0; y < ny; ++y) {
-          memcpy(q + (y0 + y) * out_stride_bytes, p + y * dpitch_b, row_b);
-        }
-      }
-    }
-    return PIKGPU_OK;
-  }
-  for (int c = 0; c < 3; ++c) {
-    HIP_TRY(ctx, Copy2D(out_planes[c], out_stride_bytes,
-                        ctx->B.out + c * oplane, dpitch_b, row_b, ys,
-                        hipMemcpyDeviceToHost, ctx->stream));
-  }
-  return pikgpu_sync(ctx);
+  uint8_t* const dst[3] = {reinterpret_cast<uint8_t*>(out_planes[0]),
+                           reinterpret_cast<uint8_t*>(out_planes[1]),
+                           reinterpret_cast<uint8_t*>(out_planes[2])};
+  return DownloadRows(ctx, dst, 3, out_stride_bytes, ctx->B.out, xs * 4, ys);
 }
 
 int pikgpu_frame_add_pass(pikgpu_ctx* ctx, const int16_t* const ac[3],
@@ -1435,10 +1452,7 @@ int pikgpu_download_srgb8(pikgpu_ctx* ctx, uint8_t* rgb, size_t stride_bytes) {
     return Fail(ctx, PIKGPU_EINVAL, "bad output buffer or stride");
   }
   HIP_TRY(ctx, hipSetDevice(ctx->device));
-  HIP_TRY(ctx, Copy2D(rgb, stride_bytes, ctx->srgb8.p,
-                                size_t(ctx->spitch), xs * 3, ys,
-                                hipMemcpyDeviceToHost, ctx->stream));
-  return pikgpu_sync(ctx);
+  return DownloadRows(ctx, &rgb, 1, stride_bytes, ctx->srgb8.p, xs * 3, ys);
 }
 
 int pikgpu_reconstruct(pikgpu_ctx* ctx, const pikgpu_frame* frame,

@@ -79,8 +79,8 @@ struct FrameBuffers {
   float* mm_partial;      // [num_wg][6]
   float* mm;              // [8]: min[3], max[3], stretch/mul, all_min
   int ipitch;             // floats per row of idct/ar
-  int opitch;             // floats per row of out
-  int spitch;             // bytes per row of srgb8
+  int opitch;             // floats per row of out (dense: its width)
+  int spitch;             // bytes per row of srgb8 (dense: 3 x its width)
   int keep;               // write stage dumps
 };
 

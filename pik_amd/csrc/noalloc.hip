@@ -113,7 +113,7 @@ size_t NoAllocLayout(const pikgpu_frame* f, const FrameParams& P,
   B->gpitch = int(gpitch);
   B->grows = int(grows);
   B->ipitch = int(ipitch);
-  B->opitch = int(DivCeil(size_t(f->xsize), 32) * 32);
+  B->opitch = int(f->xsize);
   return c.off;
 }
 
