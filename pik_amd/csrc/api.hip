@@ -1399,8 +1399,7 @@ int pikgpu_quantize(pikgpu_ctx* ctx, const float* const opsin[3],
       KEncHfResidual<<<XcdGrid(tiles), 256, 0, st>>>(P, B, coef);
     }
   }
-  KEncQuant<<<DivCeil(nb, kEncQuantThreads), kEncQuantThreads, 0, st>>>(
-      P, B, coef, itable, gsf, ac16);
+  KEncQuant<<<XcdGrid(tiles), 256, 0, st>>>(P, B, coef, itable, gsf, ac16);
   HIP_TRY(ctx, hipGetLastError());
   HIP_TRY(ctx, hipEventRecord(ctx->enc_ev[1], st));
   for (int c = 0; c < 3; ++c) {
@@ -1898,8 +1897,7 @@ int pikgpu_search_quant_field(pikgpu_ctx* ctx,
     KSearchRound<<<round_groups, 256, 0, st>>>(P, B, st_u, qmax, qf, qfr,
                                                st_rate);
     KAdjLoss<<<1, 256, 0, st>>>(st_rate, round_groups, h_rate + t);
-    KEncQuant<<<DivCeil(nb, kEncQuantThreads), kEncQuantThreads, 0, st>>>(
-        P, B, coef, itable, gsf, ac16);
+    KEncQuant<<<grid, 256, 0, st>>>(P, B, coef, itable, gsf, ac16);
     KAdjForward<<<grid, 256, 0, st>>>(P, B, K, A);
     KAdjBackward<<<grid, 256, 0, st>>>(P, B, K, A);
     KAdjLoss<<<1, 256, 0, st>>>(A.loss_part, tiles, h_loss + t);

@@ -18,11 +18,11 @@
 //                (PredictLfForEncoder), whose 2x DC image KPred2x2Interior
 //                forms; KEncHfResidual per tile: the HF residuals
 //                (ComputePredictionResiduals);
-//   KEncQuant    per block: one 8x8 dither sub-block of its transform, Y
-//                quantized and dequantised (QuantizeRoundtripBlockAC), X and
-//                B with Y's colour correlation removed
-//                (UnapplyColorCorrelationAC), every channel quantized with
-//                QuantizeBlockAC's carried rounding error.
+//   KEncQuant    per 32x32 tile: Y quantized and dequantised
+//                (QuantizeRoundtripBlockAC), X and B with Y's colour
+//                correlation removed (UnapplyColorCorrelationAC), every
+//                channel quantized with QuantizeBlockAC's carried rounding
+//                error, each block one 8x8 dither sub-block of its transform.
 #include "device.h"
 #include "kernels.h"
 
@@ -133,17 +133,14 @@ __device__ inline float AdjustQuantBiasInt(int c, int q) {
   return q - 0.145f / q;
 }
 
-// One step k = 8 * row + j of QuantizeBlockAC's sub-block loop
-// (pik/quantizer.h:233-283): the rounding error carried in double along the
-// row (err) and from the row above (prev[j]).
-template <int j>
-__device__ inline int16_t DitherStep(float val, float thres, bool k0,
-                                     double& err, double (&prev)[8]) {
-  if (j == 0) {
-    err = prev[0];
-  } else {
-    err += prev[j];
-  }
+// Step j of a row of QuantizeBlockAC's sub-block loop (pik/quantizer.h:
+// 233-283): err is the rounding error carried in double along the row,
+// `above` the one step j of the row above left, `below` (out) what this
+// step leaves for the row below.
+__device__ inline int16_t DitherStep(int j, float val, float thres, bool k0,
+                                     double& err, double above,
+                                     double& below) {
+  err = j == 0 ? above : err + above;
   if (err > 0) {
     if (val > 0) {
       val += 0.5 * err;
@@ -161,106 +158,173 @@ __device__ inline int16_t DitherStep(float val, float thres, bool k0,
   }
   if (k0) err = 0;
   if (j == 7) {
-    prev[j] = 1.0 * err;
+    below = 1.0 * err;
     err = 0;
   } else {
     err *= 0.5;
-    prev[j] = err;
+    below = err;
   }
   if (v > 32767) v = 32767;
   if (v < -32767) v = -32767;
   return int16_t(v);
 }
 
-// Position k of dither sub-block (ix, iy) of an s x s transform whose first
-// block is (x0, y0): its index `at` in a coefficient plane (by rows of
-// bx*64), its index `pos` in the transform's dequant matrix, and its
-// storage row and block column (for the colour-correlation tile).
-struct SubPos {
-  size_t at;
-  int pos, row, col_block;
-};
-__device__ inline SubPos SubPosition(int k, int s, int ix, int iy, int x0,
-                                     int y0, size_t row_len) {
-  const int xx = s * (k & 7) + ix, yy = s * (k >> 3) + iy;
-  const int pos = yy * 8 * s + xx;
-  const int r = yy >> 3, col = pos - r * 64 * s;
-  SubPos p;
-  p.pos = pos;
-  p.row = y0 + r;
-  p.col_block = x0 + (col >> 6);
-  p.at = size_t(y0 + r) * row_len + size_t(x0) * 64 + col;
-  return p;
+// The dither chain of one sub-block and channel on eight lanes, lane r8 on
+// row r8: `val` points at the row's first scaled value in LDS (step j at
+// val[j * s]), which its quantized value replaces. Row r8 takes step j one
+// time step after row r8 - 1 took it, so the error handed down moves from
+// lane to lane by a DPP shift and the 64 dependent steps become 15. Every
+// lane of the wave calls.
+__device__ inline void DitherChain(float* val, int s, int r8, bool active,
+                                   float thres) {
+  double err = 0, below = 0;
+#pragma unroll 1
+  for (int t = 0; t < 15; ++t) {
+    // the lane of the row above (row_shr:1; lanes 0 and 8 of a DPP row
+    // start a sub-block)
+    const uint64_t bits = __builtin_bit_cast(uint64_t, below);
+    const uint32_t lo = uint32_t(__builtin_amdgcn_update_dpp(
+        0, int(uint32_t(bits)), 0x111, 0xF, 0xF, true));
+    const uint32_t hi = uint32_t(__builtin_amdgcn_update_dpp(
+        0, int(uint32_t(bits >> 32)), 0x111, 0xF, 0xF, true));
+    const double above =
+        r8 == 0 ? 0.0
+                : __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
+    const int j = t - r8;
+    if (active && j >= 0 && j < 8) {
+      float* p = val + j * s;
+      *p = float(DitherStep(j, *p, thres, r8 == 0 && j == 0, err, above,
+                            below));
+    }
+  }
 }
 
-// Y's 64 positions of the sub-block, then X and B with Y's dequantised
-// values' colour correlation removed (pik/compressed_image.cc:396-453).
-// `coef` holds the transforms' coefficients; the LLF position (k = 0 of
-// every sub-block: F[iy][ix]) comes from the group's LLF cache (CopyLlf,
-// pik/ac_predictions.cc:581-607). Y's dequantised values wait in LDS, one
-// column per thread.
-__global__ void __launch_bounds__(kEncQuantThreads)
+// Quantization of one 32x32 tile (pik/compressed_image.cc:396-453). Every
+// storage block (at most 16) is one 8x8 dither sub-block (ix, iy) of its
+// transform, with position k = 8 r8 + j at F[s r8 + iy][s j + ix]. `coef`
+// holds the transforms' coefficients; the LLF positions (k = 0 of every
+// sub-block) come from the group's LLF cache (CopyLlf,
+// pik/ac_predictions.cc:581-607).
+//
+// What bounds it is the chain of 64 dependent double-precision steps per
+// sub-block and channel. One thread per sub-block ran them one after the
+// other for Y, X and B (192 steps of strided reads: 82 us for 16384 blocks,
+// 112 us for 49152). Here the values are scaled in storage order with wide
+// loads, eight lanes walk a sub-block's rows as a wavefront (DitherChain, 15
+// steps), and X and B run at the same time on the two halves of the
+// workgroup once Y's dequantised values are out: 30 steps in all
+// (20 us and 43 us).
+__global__ void __launch_bounds__(256)
     KEncQuant(FrameParams P, FrameBuffers B, const float* coef,
               const float* itable, float gsf, int16_t* ac) {
-  __shared__ float s_ydec[64][kEncQuantThreads];
-  const int t = threadIdx.x;
-  const int i = blockIdx.x * kEncQuantThreads + t;
-  if (i >= P.bx * P.by) return;
-  const int y = i / P.bx, x = i - y * P.bx;
-  const uint8_t a = B.acs[i];
-  const int raw = a >> 4, idx = a & 15, s = AcsCovered(raw);
-  const int iy = idx / s, ix = idx - iy * s;
-  const int x0 = x - ix, y0 = y - iy;
-  const int quant = B.qf[size_t(y0) * P.bx + x0];
-  const int cf = B.dcf[(y0 >> 3) * P.tx + (x0 >> 3)];
-  const int table = B.dqmap[cf * 256 + quant];
-  const int kind = AcsQuantKind(raw);
-  const float qac = gsf * quant;
-  const float inv_qac = P.inv_global_scale / quant;
-  const size_t nb = size_t(P.bx) * P.by, row_len = size_t(P.bx) * 64;
-  const int g = (y0 / kGroupDimBlocks) * P.gx + x0 / kGroupDimBlocks;
-  const int lx = x0 % kGroupDimBlocks + 1 + ix,
-            ly = y0 % kGroupDimBlocks + 1 + iy;
+  __shared__ float s_val[2][kCoefPlane];
+  __shared__ uint32_t s_off[3][16];
+  __shared__ float s_qac[16], s_inv[16];
+  __shared__ uint8_t s_acs[16];
   constexpr float kZeroBias[3] = {0.65f, 0.6f, 0.7f};
-
-  // channel order Y, X, B: X and B need Y's dequantised values
-#pragma unroll 1
-  for (int ci = 0; ci < 3; ++ci) {
-    const int c = ci == 0 ? 1 : (ci == 1 ? 0 : 2);
-    const uint32_t off = B.offsets[(table * kNumQuantKinds + kind) * 3 + c];
-    const float* dm = B.table + off;
-    const float* qm = itable + off;
-    const int32_t* cmap = c == 0 ? B.ytox : B.ytob;
-    const int cmap_off = c == 0 ? 128 : 0;
-    const float cmap_scale = c == 0 ? 1.0f / 256 : 1.0f / 128;
-    const float llf =
-        B.llf[(size_t(g) * 3 + c) * kLlfPlane + ly * kLlfPitch + lx];
-    const float thres = kZeroBias[c];
-    const float* src = coef + c * nb * 64;
-    int16_t* dst = ac + c * nb * 64;
-    double err = 0, prev[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll 1
-    for (int r8 = 0; r8 < 8; ++r8) {
-#define PIKGPU_ENC_STEP(j)                                                   \
-  {                                                                          \
-    const int k = r8 * 8 + (j);                                              \
-    const SubPos p = SubPosition(k, s, ix, iy, x0, y0, row_len);             \
-    float v = k == 0 ? llf : src[p.at];                                      \
-    if (c != 1) {                                                            \
-      const float fac =                                                      \
-          1.0f * float(cmap[(p.row >> 3) * P.tx + (p.col_block >> 3)] -      \
-                       cmap_off) * cmap_scale;                               \
-      v = v - fac * s_ydec[k][t];                                            \
-    }                                                                        \
-    const float val = v * (qm[p.pos] * qac);                                 \
-    const int16_t q = DitherStep<j>(val, thres, k == 0, err, prev);          \
-    dst[p.at] = q;                                                           \
-    if (c == 1) s_ydec[k][t] = AdjustQuantBiasInt(1, q) * dm[p.pos] * inv_qac; \
+  const int tid = threadIdx.x;
+  const int tiles_x = (P.bx + 3) / 4;
+  const int tile = XcdTile(blockIdx.x, tiles_x * ((P.by + 3) / 4));
+  if (tile < 0) return;
+  const int tbx = (tile % tiles_x) * 4, tby = (tile / tiles_x) * 4;
+  // a 32x32 tile lies in one colour tile
+  const int ctile = (tby >> 3) * P.tx + (tbx >> 3);
+  if (tid < 16) {
+    const int x = tbx + (tid & 3), y = tby + (tid >> 2);
+    uint8_t a = 0xFF;
+    if (x < P.bx && y < P.by) {
+      a = B.acs[size_t(y) * P.bx + x];
+      const int raw = a >> 4, idx = a & 15, s = AcsCovered(raw);
+      const int x0 = x - idx % s, y0 = y - idx / s;
+      const int quant = B.qf[size_t(y0) * P.bx + x0];
+      const int table = B.dqmap[B.dcf[ctile] * 256 + quant];
+      for (int c = 0; c < 3; ++c) {
+        s_off[c][tid] =
+            B.offsets[(table * kNumQuantKinds + AcsQuantKind(raw)) * 3 + c];
+      }
+      s_qac[tid] = gsf * quant;
+      s_inv[tid] = P.inv_global_scale / quant;
+    }
+    s_acs[tid] = a;
   }
-      PIKGPU_ENC_STEP(0) PIKGPU_ENC_STEP(1) PIKGPU_ENC_STEP(2)
-      PIKGPU_ENC_STEP(3) PIKGPU_ENC_STEP(4) PIKGPU_ENC_STEP(5)
-      PIKGPU_ENC_STEP(6) PIKGPU_ENC_STEP(7)
-#undef PIKGPU_ENC_STEP
+  __syncthreads();
+  // four consecutive coefficients of one storage block per thread
+  const int gxi = tbx / kGroupDimBlocks, gyi = tby / kGroupDimBlocks;
+  const int g = gyi * P.gx + gxi;
+  const CoefSlot S = MakeSlot(P, s_acs, tbx, tby, gxi * kGroupDimBlocks,
+                              gyi * kGroupDimBlocks);
+  const int e = CoefAt(S.crow, S.ccol);
+  const size_t plane = size_t(P.by) * P.bx * 64;
+  const size_t at =
+      size_t(S.cby) * P.bx * 64 + size_t(S.cbx) * 64 + (S.ccol & 63);
+  float v[3][4], qm[3][4], dm[4];
+  float inv_qac = 0.0f;
+  if (S.valid) {
+    const int own = S.crow * 4 + (S.ccol >> 6);
+    const float qac = s_qac[own];
+    inv_qac = s_inv[own];
+    for (int c = 0; c < 3; ++c) {
+      const float4 q = *reinterpret_cast<const float4*>(coef + c * plane + at);
+      v[c][0] = q.x;
+      v[c][1] = q.y;
+      v[c][2] = q.z;
+      v[c][3] = q.w;
+      const float* m = itable + s_off[c][own] + S.cflat0;
+      const float* llf = B.llf + (size_t(g) * 3 + c) * kLlfPlane;
+      for (int j = 0; j < 4; ++j) {
+        qm[c][j] = m[j] * qac;
+        const int fi = (S.cflat0 + j) >> S.lgn, fj = (S.cflat0 + j) & (S.cN - 1);
+        if (fi < S.cs && fj < S.cs) {
+          v[c][j] = llf[(S.obyg + 1 + fi) * kLlfPitch + S.obxg + 1 + fj];
+        }
+      }
+    }
+    for (int j = 0; j < 4; ++j) {
+      dm[j] = B.table[s_off[1][own] + S.cflat0 + j];
+      s_val[0][e + j] = v[1][j] * qm[1][j];
+    }
+  }
+  __syncthreads();
+  // the chains: lanes 8 sub .. 8 sub + 7 of a half of the workgroup
+  const int sub = (tid >> 3) & 15, r8 = tid & 7, half = tid >> 7;
+  const uint8_t a = s_acs[sub];
+  int s = 1, row0 = 0;
+  if (a != 0xFF) {
+    s = AcsCovered(a >> 4);
+    const int iy = (a & 15) / s, ix = (a & 15) % s;
+    const int oby = (sub >> 2) - iy, obx = (sub & 3) - ix;
+    const int yy = s * r8 + iy;
+    row0 = CoefAt(oby + (yy >> 3), obx * 64 + (yy & 7) * 8 * s) + ix;
+  }
+  DitherChain(s_val[0] + row0, s, r8, a != 0xFF && half == 0, kZeroBias[1]);
+  __syncthreads();
+  if (S.valid) {
+    const float fac[3] = {
+        1.0f * float(B.ytox[ctile] - 128) * (1.0f / 256), 0.0f,
+        1.0f * float(B.ytob[ctile] - 0) * (1.0f / 128)};
+    short4 q;
+    float yd[4];
+    int16_t* qp = reinterpret_cast<int16_t*>(&q);
+    for (int j = 0; j < 4; ++j) {
+      qp[j] = int16_t(s_val[0][e + j]);
+      yd[j] = AdjustQuantBiasInt(1, qp[j]) * dm[j] * inv_qac;
+    }
+    *reinterpret_cast<short4*>(ac + plane + at) = q;
+    for (int j = 0; j < 4; ++j) {
+      s_val[0][e + j] = (v[0][j] - fac[0] * yd[j]) * qm[0][j];
+      s_val[1][e + j] = (v[2][j] - fac[2] * yd[j]) * qm[2][j];
+    }
+  }
+  __syncthreads();
+  DitherChain(s_val[half] + row0, s, r8, a != 0xFF,
+              half == 0 ? kZeroBias[0] : kZeroBias[2]);
+  __syncthreads();
+  if (S.valid) {
+    for (int h = 0; h < 2; ++h) {
+      short4 q;
+      int16_t* qp = reinterpret_cast<int16_t*>(&q);
+      for (int j = 0; j < 4; ++j) qp[j] = int16_t(s_val[h][e + j]);
+      *reinterpret_cast<short4*>(ac + 2 * h * plane + at) = q;
     }
   }
 }
@@ -325,7 +389,8 @@ __global__ void __launch_bounds__(256)
         B.llf[(size_t(g) * 3 + c) * kLlfPlane + (ly0 + iy) * kLlfPitch + lx0 + ix];
     float* cp = coef + c * nb * 64 + base;
     float dec[4];
-    double err = 0, prev[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    // errors along the row and left for the row below by steps 0 and 1
+    double err = 0, prev[2] = {0, 0};
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
       const int pos = fi[m] * 8 * s + fj[m];
@@ -338,16 +403,8 @@ __global__ void __launch_bounds__(256)
       const float val = v * (qm[pos] * qac);
       // k = 0, 1 are steps 0 and 1 of the first row, k = 8, 9 those of the
       // second (the steps between leave err and prev[0..1] as found)
-      int16_t q;
-      if (m == 0) {
-        q = DitherStep<0>(val, kZeroBias[c], true, err, prev);
-      } else if (m == 1) {
-        q = DitherStep<1>(val, kZeroBias[c], false, err, prev);
-      } else if (m == 2) {
-        q = DitherStep<0>(val, kZeroBias[c], false, err, prev);
-      } else {
-        q = DitherStep<1>(val, kZeroBias[c], false, err, prev);
-      }
+      const int16_t q = DitherStep(m & 1, val, kZeroBias[c], m == 0, err,
+                                   prev[m & 1], prev[m & 1]);
       if (m == 0) {
         // the LLF position keeps its value (through the colour correlation
         // taken out and put back for X and B)

@@ -524,6 +524,39 @@ __device__ inline void TileForward3(const TileTasks& T, const float* pix,
   TileForward3<kAdjoint, kAddHF, kSubHF>(AssignTasks(T), pix, coef, tmp);
 }
 
+// Coefficient ownership of a 256-thread tile pass, as in KBlocks: storage
+// row crow of the tile, columns ccol..ccol+3; 16 consecutive lanes own one
+// 8x8 storage block.
+struct CoefSlot {
+  int crow, ccol, cbx, cby;
+  bool valid;
+  int raw, cs, cN, lgn, cflat0, obxg, obyg;
+  uint8_t acs;
+};
+
+__device__ inline CoefSlot MakeSlot(const FrameParams& P, const uint8_t* s_acs,
+                                    int tbx, int tby, int gbx0, int gby0) {
+  CoefSlot s;
+  const int tid = threadIdx.x;
+  s.crow = tid >> 6;
+  s.ccol = (tid & 63) << 2;
+  s.cbx = tbx + (s.ccol >> 6);
+  s.cby = tby + s.crow;
+  s.valid = s.cbx < P.bx && s.cby < P.by;
+  s.acs = s_acs[s.crow * 4 + (s.ccol >> 6)];
+  s.raw = s.acs >> 4;
+  const int cidx = s.acs & 15;
+  s.cs = s.acs == 0xFF ? 1 : AcsCovered(s.raw);
+  const int lgs = s.cs >> 1;  // log2(cs): cs is 1, 2 or 4
+  s.lgn = 3 + lgs;
+  const int coby = s.crow - (cidx >> lgs), cobx = (s.ccol >> 6) - (cidx & (s.cs - 1));
+  s.cflat0 = (s.crow - coby) * 64 * s.cs + (s.ccol - cobx * 64);
+  s.cN = 8 * s.cs;
+  s.obxg = tbx + cobx - gbx0;
+  s.obyg = tby + coby - gby0;
+  return s;
+}
+
 // ---------------------------------------------------------------------------
 // Workgroup-to-tile order for the eight XCDs of an MI355X. Consecutive
 // workgroup ids are dealt round-robin to the XCDs, each with its own L2, so
@@ -711,9 +744,6 @@ __device__ inline void ReinterpIdct(const DeviceConsts* K, const float* in,
 struct EncDcScale {
   float scale[3];
 };
-// KEncQuant's workgroup size (its LDS holds 64 floats per thread).
-constexpr int kEncQuantThreads = 128;
-
 // ---------------------------------------------------------------------------
 // Kernels.
 __global__ void KDcDequant(FrameParams P, FrameBuffers B);
