@@ -1644,6 +1644,10 @@ int pikgpu_fwd_adj(pikgpu_ctx* ctx, const pikgpu_adj_io* io) {
     A.dqf = io->dl_dqf;
     A.dqf_pitch = int(io->dqf_stride);
     A.dc_pitch = io->dcoeffs_stride;
+    A.dcoef_vec = ndc && io->dcoeffs_stride % 4 == 0;
+    for (int c = 0; c < 3; ++c) {
+      if (reinterpret_cast<uintptr_t>(A.dcoef[c]) % 16 != 0) A.dcoef_vec = 0;
+    }
   } else {
     if ((rc = Grow(ctx, &ctx->adj_qf, bx * by * 4)) ||
         (rc = Grow(ctx, &ctx->adj_in, 3 * plane_in * 4)) ||
@@ -1677,6 +1681,7 @@ int pikgpu_fwd_adj(pikgpu_ctx* ctx, const pikgpu_adj_io* io) {
     A.dqf = static_cast<float*>(ctx->adj_dqf.p);
     A.dqf_pitch = int(bx);
     A.dc_pitch = bx * 64;
+    A.dcoef_vec = 1;
   }
   float* loss_part = static_cast<float*>(ctx->adj_loss.p);
   double* loss_dev = reinterpret_cast<double*>(
@@ -1879,6 +1884,7 @@ int pikgpu_search_quant_field(pikgpu_ctx* ctx,
   A.dqf = static_cast<float*>(ctx->adj_dqf.p);
   A.dqf_pitch = int(bx);
   A.dc_pitch = bx * 64;
+  A.dcoef_vec = 1;
   A.loss_part = static_cast<float*>(ctx->adj_loss.p);
   SearchArgs S;
   S.weight = io->weight ? st_w : nullptr;

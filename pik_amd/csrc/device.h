@@ -100,6 +100,7 @@ struct AdjArgs {
   int dqf_pitch;
   float* dcoef[3];           // optional dL/dd (before CfL)
   size_t dc_pitch;
+  int dcoef_vec;             // dcoef rows 16-byte aligned
   float* loss_part;          // per-tile sums of squared error, or null
 };
 

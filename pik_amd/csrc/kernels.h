@@ -31,6 +31,21 @@ __device__ inline float Symmetric3(const float* in, int pitch, int W, int H,
   return x2 * w2 + mul1;
 }
 
+// The same at p of an array whose neighbours all lie inside it.
+__device__ inline float Conv3(const float* p, int pitch, const float (&w)[3]) {
+  const float* t = p - pitch;
+  const float* b = p + pitch;
+  const float sum_tb = t[0] + b[0];
+  const float mul0 = p[0] * w[0];
+  const float sum_lr = p[-1] + p[1];
+  const float x1 = sum_tb + sum_lr;
+  const float mul1 = x1 * w[1] + mul0;
+  const float sum_t2 = t[-1] + t[1];
+  const float sum_b2 = b[-1] + b[1];
+  const float x2 = sum_t2 + sum_b2;
+  return x2 * w[2] + mul1;
+}
+
 // AdjustQuantBias, vector form (pik/quantizer.h:61-88).
 __device__ inline float AdjustQuantBias(int c, float q) {
   const float one_bias = c == 0 ? 0.05465007330715401f
@@ -68,6 +83,33 @@ __device__ inline BlockDq MakeBlockDq(const FrameParams& P,
   d.cc = c == 0 ? float(B.ytox[tile] - 128) * 0.00390625f
                 : (c == 2 ? float(B.ytob[tile]) * 0.0078125f : 0.0f);
   return d;
+}
+
+// Writes block i's two dequantisation descriptors (FrameBuffers::desc), so
+// the block kernels reach the dequant matrices with one dependent load
+// instead of the chain strategy -> quant field -> control field -> table
+// index -> table offset. qf, qfo: the quant values of the block and of its
+// transform's first block.
+__device__ inline void WriteBlockDesc(const FrameParams& P,
+                                      const FrameBuffers& B, int i, int qf,
+                                      int qfo) {
+  const int bxa = i % P.bx, bya = i / P.bx;
+  const uint8_t a = B.acs[i];
+  const int raw = a >> 4, idx = a & 15;
+  const int s = AcsCovered(raw);
+  const int kind = AcsQuantKind(raw);
+  const int obxa = bxa - (idx & (s - 1)), obya = bya - (idx >> (s >> 1));
+  const int qt = B.dqmap[B.dcf[(bya >> 3) * P.tx + (bxa >> 3)] * 256 + qf - 1];
+  const int qto =
+      B.dqmap[B.dcf[(obya >> 3) * P.tx + (obxa >> 3)] * 256 + qfo - 1];
+  const uint32_t* off = B.offsets + (qt * kNumQuantKinds + kind) * 3;
+  const uint32_t* offo = B.offsets + (qto * kNumQuantKinds + kind) * 3;
+  B.desc[2 * i] = make_uint4(
+      off[0] + idx * 64, off[1] + idx * 64, off[2] + idx * 64,
+      __float_as_uint(qf == 0 ? 1E10f : P.inv_global_scale / float(qf)));
+  B.desc[2 * i + 1] = make_uint4(
+      offo[0] + idx * 64, offo[1] + idx * 64, offo[2] + idx * 64,
+      __float_as_uint(P.inv_global_scale / float(qfo)));
 }
 
 // MakeBlockDq's values from the block's descriptor (KDcDequant).

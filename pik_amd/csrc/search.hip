@@ -26,8 +26,9 @@ namespace pikgpu {
 
 // Integer field from the log field: each block takes its transform's value
 // (stored at the transform's first block), rounded and clamped to
-// [1, qmax]; `qfr` receives it as float for the adjoint. Per workgroup the
-// sum of log(qf) (the rate proxy) goes to `part`.
+// [1, qmax]; `qfr` receives it as float for the adjoint, and the block's
+// dequantisation descriptors follow it. Per workgroup the sum of log(qf)
+// (the rate proxy) goes to `part`.
 __global__ void __launch_bounds__(256)
     KSearchRound(FrameParams P, FrameBuffers B, const float* u, int qmax,
                  int32_t* qf, float* qfr, float* part) {
@@ -43,6 +44,8 @@ __global__ void __launch_bounds__(256)
     const int q = int(fminf(fmaxf(v, 1.0f), float(qmax)));
     qf[i] = q;
     qfr[i] = float(q);
+    // every block of a transform has the same value
+    WriteBlockDesc(P, B, i, q, q);
     lq = __logf(float(q));
   }
   for (int m = 32; m >= 1; m >>= 1) lq += __shfl_xor(lq, m, 64);
