@@ -85,11 +85,10 @@ __device__ inline int16_t CoefQ(const uint2& q, int j) {
 }
 __device__ inline void LoadMatrix(const FrameBuffers& B, const CoefIn& in,
                                   float (&m)[3][4]) {
+  if (!in.valid) return;
   const uint32_t slot[3] = {in.desc.x, in.desc.y, in.desc.z};
   for (int c = 0; c < 3; ++c) {
-    for (int j = 0; j < 4; ++j) {
-      m[c][j] = in.valid ? B.table[slot[c] + (in.at & 63) + j] : 0.0f;
-    }
+    LoadFour(B.table + slot[c] + (in.at & 63), m[c]);
   }
 }
 __device__ inline uint8_t TileAcs(const FrameParams& P, const FrameBuffers& B,
@@ -127,7 +126,7 @@ __global__ void __launch_bounds__(256, 4)
                               gyi * kGroupDimBlocks);
   // the matrix entries and the LLF / LF values load while one wave builds
   // the task table
-  float mv[3][4], fixv[3][4];
+  float mv[3][4] = {}, fixv[3][4];
   int fix[4];
   LoadMatrix(B, in, mv);
   for (int j = 0; j < 4; ++j) {
@@ -387,7 +386,7 @@ __global__ void __launch_bounds__(256, 4)
       }
     }
   }
-  float mv[3][4];
+  float mv[3][4] = {};
   LoadMatrix(B, in, mv);
   __syncthreads();
 

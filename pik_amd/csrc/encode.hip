@@ -130,7 +130,7 @@ __device__ inline float AdjustQuantBiasInt(int c, int q) {
   if (q == 0) return 0.f;
   if (q == 1) return 1 - kOneBias[c];
   if (q == -1) return kOneBias[c] - 1;
-  return q - 0.145f / q;
+  return q - BiasOver(float(q));
 }
 
 // Step j of a row of QuantizeBlockAC's sub-block loop (pik/quantizer.h:

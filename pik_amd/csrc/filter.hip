@@ -967,7 +967,7 @@ __device__ __forceinline__ void KEpfBody(
   if (ar_valid) {
     const uint32_t slot[3] = {ar_desc.x, ar_desc.y, ar_desc.z};
     for (int c = 0; c < 3; ++c) {
-      for (int j = 0; j < 4; ++j) ar_m[c][j] = B.table[slot[c] + (ccol & 63) + j];
+      LoadFour(B.table + slot[c] + (ccol & 63), ar_m[c]);
     }
   }
   float orig[3][4];
@@ -1036,14 +1036,15 @@ __device__ __forceinline__ void KEpfBody(
   }
   __syncthreads();
   TileInverse3(my_tasks, &s_coef[0][0], &s_out[0][0], &s_tmp[0][0]);
-  const int y = y0 + r;
-  if (y < in.H) {
+  // (the width is a multiple of 8, the output rows are 128-byte aligned)
+  const int y = y0 + r, x = x0 + c0;
+  if (y < in.H && x < in.W) {
     for (int c = 0; c < 3; ++c) {
-      float* dst = out + c * out_plane + size_t(y) * out_pitch;
-      for (int j = 0; j < 4; ++j) {
-        const int x = x0 + c0 + j;
-        if (x < in.W) dst[x] = s_out[c][PixAt(r, c0 + j)] + orig[c][j];
-      }
+      const float* d = s_out[c] + PixAt(r, c0);
+      *reinterpret_cast<float4*>(out + c * out_plane + size_t(y) * out_pitch +
+                                 x) =
+          make_float4(d[0] + orig[c][0], d[1] + orig[c][1], d[2] + orig[c][2],
+                      d[3] + orig[c][3]);
     }
   }
 }

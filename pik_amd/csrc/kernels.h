@@ -46,15 +46,36 @@ __device__ inline float Conv3(const float* p, int pitch, const float (&w)[3]) {
   return x2 * w[2] + mul1;
 }
 
-// AdjustQuantBias, vector form (pik/quantizer.h:61-88).
+// 0.145f / q for an integer q != 0 with |q| <= 32768, correctly rounded: the
+// hardware's reciprocal (1 ulp), one residual step in fused arithmetic. The
+// generic division takes about 11 instructions to cover every exponent; for
+// these 65536 quotients this gives the same bits
+// (tests/test_gpu_dequant_values.py decodes every one of them). With the
+// division KBlocks spent a sixth of its VALU instructions here.
+__device__ inline float BiasOver(float q) {
+  const float r = __builtin_amdgcn_rcpf(q);
+  const float y = 0.145f * r;
+  return fmaf(fmaf(-q, y, 0.145f), r, y);
+}
+
+// AdjustQuantBias, vector form (pik/quantizer.h:61-88), of an integer q.
 __device__ inline float AdjustQuantBias(int c, float q) {
   const float one_bias = c == 0 ? 0.05465007330715401f
                                 : (c == 1 ? 0.07005449891748593f
                                           : 0.049935103337343655f);
   const float aq = fabsf(q);
-  if (aq >= 1.5f) return q - 0.145f / q;
-  if (aq >= 0.5f) return copysignf(1 - one_bias, q);
-  return q;
+  const float big = q - BiasOver(q);
+  const float one = copysignf(1 - one_bias, q);
+  return aq >= 1.5f ? big : (aq >= 0.5f ? one : q);
+}
+
+// Four consecutive floats at any 4-byte aligned address, in one load.
+struct __attribute__((packed, aligned(4))) Float4U {
+  float v[4];
+};
+__device__ inline void LoadFour(const float* p, float (&v)[4]) {
+  const Float4U q = *reinterpret_cast<const Float4U*>(p);
+  for (int j = 0; j < 4; ++j) v[j] = q.v[j];
 }
 
 // Per-storage-block dequantisation parameters of plane c: the dequant
@@ -197,22 +218,20 @@ __host__ __device__ inline int CoefAt(int row, int col) {
 
 // The tile's transforms in task order: grouped by kind (DCT8, DCT16,
 // DCT32, DCT4X4, direct), so that the lanes of a wave mostly run the same
-// line code. Position p holds the transform starting at tile block blk[p].
+// line code. A kind's transforms all have the same number of tasks, so task
+// t's transform follows from its kind's first task and a shift.
+constexpr int kTaskKinds = 5;
+// log2 of the tasks of one transform, kind k in bits 4k .. 4k + 3: 8, 16,
+// 32, 16 and 1
+constexpr uint32_t kTaskLog2 = 0x04543;
 struct TileTasks {
-  int off[17];      // first task of each position; off[16] = tasks per
-                    // channel (positions past the last transform: off = total)
-  uint8_t raw[16];  // strategy at each position (0xFF past the last)
-  uint8_t blk[16];  // tile block (by * 4 + bx) at each position
-  int has_dct4;     // a DCT4X4 transform is among them
+  int seg[kTaskKinds + 1];   // first task of each kind; the last entry: tasks
+                             // per channel
+  uint32_t kind[kTaskKinds]; // seg | first position << 16 | log2 tasks << 24
+  uint16_t at[16];           // raw | tile block (by * 4 + bx) << 4 of each
+                             // position
+  int has_dct4;              // a DCT4X4 transform is among them
 };
-
-__device__ inline int TaskCount(int raw) {
-  if (raw == kDCT || raw == kDCTNoHF) return 8;
-  if (raw == kDCT16) return 16;
-  if (raw == kDCT32) return 32;
-  if (AcsIsDCT4(raw)) return 16;
-  return 1;
-}
 
 __device__ inline int TaskKind(int raw) {
   if (raw == kDCT || raw == kDCTNoHF) return 0;
@@ -222,65 +241,46 @@ __device__ inline int TaskKind(int raw) {
   return 4;
 }
 
-// All threads call; `acs_t` holds the tile's 16 strategy bytes (0xFF
-// outside the image). hf_only keeps only strategies with HF prediction.
-// Lanes 0..15 of the first wave each place one block: its position is the
-// number of transforms of earlier kinds plus those of its kind at earlier
-// blocks (ballots), its first task the task count of the positions before
-// it (shuffles).
+// Wave `wave` of the workgroup fills T; `acs_t` holds the tile's 16 strategy
+// bytes (0xFF outside the image). hf_only keeps only strategies with HF
+// prediction. Lanes 0..15 each place one block: its position is the number
+// of transforms of earlier kinds plus those of its kind at earlier blocks
+// (ballots). The caller's next barrier publishes T.
+__device__ inline void BuildTasksWave(const uint8_t* acs_t, bool hf_only,
+                                      TileTasks* T, int wave) {
+  if (int(threadIdx.x >> 6) != wave) return;
+  const int b = threadIdx.x & 63;
+  int raw = 0, kind = kTaskKinds;
+  if (b < 16) {
+    const uint8_t a = acs_t[b];
+    if (a != 0xFF && (a & 15) == 0 && (!hf_only || AcsPredictHF(a >> 4))) {
+      raw = a >> 4;
+      kind = TaskKind(raw);
+    }
+  }
+  int seg = 0, first = 0;  // the running kind's first task and position
+#pragma unroll
+  for (int k = 0; k < kTaskKinds; ++k) {
+    const uint32_t m = uint32_t(__ballot(kind == k));
+    const uint32_t lg = (kTaskLog2 >> (4 * k)) & 15;
+    if (kind == k) {
+      T->at[first + __popc(m & ((1u << b) - 1))] = uint16_t(raw | (b << 4));
+    }
+    if (b == 0) {
+      T->seg[k] = seg;
+      T->kind[k] = uint32_t(seg) | (uint32_t(first) << 16) | (lg << 24);
+      if (k == 3) T->has_dct4 = m != 0;
+    }
+    seg += __popc(m) << lg;
+    first += __popc(m);
+  }
+  if (b == 0) T->seg[kTaskKinds] = seg;
+}
+// All threads call.
 __device__ inline void BuildTasks(const uint8_t* acs_t, bool hf_only,
                                   TileTasks* T) {
-  if (threadIdx.x < 64) {
-    const int b = threadIdx.x;
-    int raw = -1, kind = 5, cnt = 0;
-    if (b < 16) {
-      const uint8_t a = acs_t[b];
-      if (a != 0xFF && (a & 15) == 0 && (!hf_only || AcsPredictHF(a >> 4))) {
-        raw = a >> 4;
-        kind = TaskKind(raw);
-        cnt = TaskCount(raw);
-      }
-    }
-    int pos = 0, n = 0;
-    for (int k = 0; k < 5; ++k) {
-      const unsigned long long m = __ballot(kind == k);
-      n += __popcll(m);
-      if (k < kind) pos += __popcll(m);
-      if (k == kind) pos += __popcll(m & ((1ull << b) - 1));
-    }
-    int first = 0, total = 0;
-    for (int q = 0; q < 16; ++q) {
-      const int qc = __shfl(cnt, q, 64), qp = __shfl(pos, q, 64);
-      const int qk = __shfl(kind, q, 64);
-      total += qc;
-      if (qk < 5 && qp < pos) first += qc;
-    }
-    if (b < 16 && raw >= 0) {
-      T->off[pos] = first;
-      T->raw[pos] = uint8_t(raw);
-      T->blk[pos] = uint8_t(b);
-    }
-    if (b < 16 && b >= n) {  // positions past the last transform
-      T->off[b] = total;
-      T->raw[b] = 0xFF;
-      T->blk[b] = 0;
-    }
-    const unsigned long long m4 = __ballot(kind == 3);
-    if (b == 0) {
-      T->off[16] = total;
-      T->has_dct4 = m4 != 0;
-    }
-  }
+  BuildTasksWave(acs_t, hf_only, T, 0);
   __syncthreads();
-}
-
-// Position of task t (binary search over the offsets).
-__device__ inline int TaskBlock(const TileTasks& T, int t) {
-  int lo = 0;
-  for (int step = 8; step > 0; step >>= 1) {
-    if (T.off[lo + step] <= t) lo += step;
-  }
-  return lo;
 }
 
 // Column k of an N x N transform's F matrix (row-major, flat i * N + k)
@@ -496,7 +496,7 @@ struct ThreadTasks {
 };
 
 __device__ inline ThreadTasks AssignTasks(const TileTasks& T) {
-  const int total = T.off[16];
+  const int total = T.seg[kTaskKinds];
   ThreadTasks m;
   m.has_dct4 = T.has_dct4 != 0;
 #pragma unroll
@@ -505,10 +505,15 @@ __device__ inline ThreadTasks AssignTasks(const TileTasks& T) {
     m.t[i] = kNoTask;
     if (k < 3 * total) {
       const int c = (k >= total) + (k >= 2 * total), t = k - c * total;
-      const int p = TaskBlock(T, t), b = T.blk[p];
-      m.t[i] = uint32_t(c) | (uint32_t(T.raw[p]) << 2) |
-               (uint32_t(t - T.off[p]) << 6) | (uint32_t(b >> 2) << 11) |
-               (uint32_t(b & 3) << 13);
+      const int kd = (t >= T.seg[1]) + (t >= T.seg[2]) + (t >= T.seg[3]) +
+                     (t >= T.seg[4]);
+      const uint32_t w = T.kind[kd];
+      const uint32_t r = uint32_t(t) - (w & 0xFFFF), lg = w >> 24;
+      const uint32_t at = T.at[((w >> 16) & 0xFF) + (r >> lg)];
+      const uint32_t b = at >> 4;
+      m.t[i] = uint32_t(c) | ((at & 15) << 2) |
+               ((r & ((1u << lg) - 1)) << 6) | ((b >> 2) << 11) |
+               ((b & 3) << 13);
     }
   }
   return m;

@@ -117,7 +117,7 @@ __device__ __forceinline__ void KBlocksBody(
   if (cvalid) {
     const uint32_t slot[3] = {dsc.x, dsc.y, dsc.z};
     for (int c = 0; c < 3; ++c) {
-      for (int j = 0; j < 4; ++j) mv[c][j] = B.table[slot[c] + (ccol & 63) + j];
+      LoadFour(B.table + slot[c] + (ccol & 63), mv[c]);
     }
     for (int c = 0; c < 3; ++c) {
       const float* llf = B.llf + (size_t(g) * 3 + c) * kLlfPlane;
@@ -134,9 +134,12 @@ __device__ __forceinline__ void KBlocksBody(
       }
     }
   }
-  BuildTasks(s_acs, false, &s_inv);
-  if (P.predict_hf) BuildTasks(s_acs, true, &s_fwd);
+  BuildTasksWave(s_acs, false, &s_inv, 0);
+  if (P.predict_hf) BuildTasksWave(s_acs, true, &s_fwd, 1);
+  __syncthreads();
 
+  // Pixel quad of this thread: row pr, columns pc0..pc0+3.
+  const int pr = tid >> 3, pc0 = (tid & 7) << 2;
   // 1. dequantise Y, then X and B with their colour correlation
   //    (Dequant::DoAC, pik/compressed_image.cc:586-693), and 2. the LLF and
   //    LF predictions (UpdateLfForDecoder, pik/ac_predictions.cc:560-620).
@@ -187,36 +190,42 @@ __device__ __forceinline__ void KBlocksBody(
       }
     }
   }
-  // Pixel quad of this thread: row pr, columns pc0..pc0+3.
-  const int pr = tid >> 3, pc0 = (tid & 7) << 2;
   // 3. HF prediction (AddPredictions / UpSample4x4BlurDCT<true>,
   //    pik/ac_predictions.cc:263-374): 4x nearest-neighbour upsampling of
   //    pred2x2 with the separable 3-tap blur, forward transform, added to
-  //    all but the 2s x 2s low-frequency corner.
+  //    all but the 2s x 2s low-frequency corner. The horizontal taps run
+  //    once per window row (10 of them) and pixel column, not once per
+  //    pixel: a fifth of the instructions of three rows' taps in every
+  //    thread. Pixels of strategies without HF prediction get values no
+  //    transform reads.
   if (P.predict_hf) {
-    const uint8_t pa = s_acs[(pr >> 3) * 4 + (pc0 >> 3)];
-    if (pa != 0xFF && AcsPredictHF(pa >> 4)) {
-      // Pixel row pr of the tile reads pred2x2 rows rbase + 1 .. + 3 and
-      // its four columns (one upsampled pred2x2 column, q = j) columns
-      // xq + 1 .. + 3, where rbase = 2 * block row + (pr & 7 >= 4) and
-      // xq = pc0 / 4, both tile-local; in window coordinates that is rows
-      // rbase - 1 + 1 + t and columns xq + t.
+    float (*s_h)[10][32] = reinterpret_cast<float (*)[10][32]>(&s_tmp[0][0] + 320);
+    for (int k = tid; k < 3 * 10 * 8; k += 256) {
+      // window row t of channel c, the four pixel columns of one upsampled
+      // pred2x2 column xq: window columns xq .. xq + 2
+      const int c = k / 80, t = (k / 8) % 10, xq = k & 7;
+      const float* rw = s_p2[c] + t * 10 + xq;
+      const float r0 = rw[0], r1 = rw[1], r2 = rw[2];
+      for (int j = 0; j < 4; ++j) {
+        s_h[c][t][4 * xq + j] =
+            r0 * P.ub4[0][j] + r1 * P.ub4[1][j] + r2 * P.ub4[2][j];
+      }
+    }
+    __syncthreads();
+    {
+      // pixel row pr reads window rows wr .. wr + 2
       const int py = pr & 7, iy = py & 3;
-      const int wr = 2 * (pr >> 3) + (py < 4 ? 0 : 1);  // window row of t = 0
-      const int wc = pc0 >> 2;                         // window column
+      const int wr = 2 * (pr >> 3) + (py < 4 ? 0 : 1);
+      float w[3];
+      for (int t = 0; t < 3; ++t) {
+        w[t] = iy < 2 ? (iy == 0 ? P.ub4[t][0] : P.ub4[t][1])
+                      : (iy == 2 ? P.ub4[t][2] : P.ub4[t][3]);
+      }
       for (int c = 0; c < 3; ++c) {
-        float rw[3][3];
-        for (int t = 0; t < 3; ++t) {
-          for (int u = 0; u < 3; ++u) rw[t][u] = s_p2[c][(wr + t) * 10 + wc + u];
-        }
         for (int j = 0; j < 4; ++j) {
-          float v[3];
-          for (int t = 0; t < 3; ++t) {
-            v[t] = rw[t][0] * P.ub4[0][j] + rw[t][1] * P.ub4[1][j] +
-                   rw[t][2] * P.ub4[2][j];
-          }
-          s_pred[c][PixAt(pr, pc0 + j)] =
-              v[0] * P.ub4[0][iy] + v[1] * P.ub4[1][iy] + v[2] * P.ub4[2][iy];
+          s_pred[c][PixAt(pr, pc0 + j)] = s_h[c][wr][pc0 + j] * w[0] +
+                                          s_h[c][wr + 1][pc0 + j] * w[1] +
+                                          s_h[c][wr + 2][pc0 + j] * w[2];
         }
       }
     }
@@ -236,15 +245,13 @@ __device__ __forceinline__ void KBlocksBody(
   // 4. IDCT (InverseIntegralTransform, pik/compressed_image.cc:869-895)
   TileInverse3(s_inv, &s_coef[0][0], s_pix, &s_tmp[0][0]);
   if (P.downsample == 1) {
-    const int py = tby * 8 + pr;
-    if (py < P.py) {
+    // (the padded width is a multiple of 8, the rows are 128-byte aligned)
+    const int py = tby * 8 + pr, px = tbx * 8 + pc0;
+    if (py < P.py && px < P.px) {
       for (int c = 0; c < 3; ++c) {
-        float* dst = B.idct + (size_t(c) * P.py + py) * B.ipitch + tbx * 8 + pc0;
-        for (int j = 0; j < 4; ++j) {
-          if (tbx * 8 + pc0 + j < P.px) {
-            dst[j] = s_pix[c * kTilePlane + PixAt(pr, pc0 + j)];
-          }
-        }
+        const float* s = s_pix + c * kTilePlane + PixAt(pr, pc0);
+        *reinterpret_cast<float4*>(B.idct + (size_t(c) * P.py + py) * B.ipitch +
+                                   px) = make_float4(s[0], s[1], s[2], s[3]);
       }
     }
     return;
