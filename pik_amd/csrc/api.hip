@@ -702,8 +702,8 @@ int pikgpu_frame_upload(pikgpu_ctx* ctx, const pikgpu_frame* f) {
   const size_t gpitch = DivCeil(bx * 8, 32) * 32 + 64;
   GROW(gimg, 3 * grows * gpitch);
   GROW(out, 3 * opitch * f->ysize * 4);
-  GROW(mm_partial, kMinMaxMaxGroups * 6 * 4);
-  GROW(mm, 8 * 4);
+  GROW(mm_partial, kMinMaxMaxGroups * 2 * 4);
+  GROW(mm, 2 * 4);
 #undef GROW
 
   // --- copies ---
@@ -862,14 +862,9 @@ int pikgpu_frame_upload(pikgpu_ctx* ctx, const pikgpu_frame* f) {
 
 }  // extern "C"
 
-// Grid of KMinMaxPartial: 256-column strips, row ranges of >= 8 rows, at most
-// kMinMaxMaxGroups workgroups (the size of the partials buffer): 16 rows per
-// thread at 4096 x 4096, two waves of workgroups on 256 CUs.
-static dim3 MinMaxGrid(int w, int h) {
-  const int nx = int(DivCeil(w, 256));
-  const int ny =
-      std::max(1, std::min(int(DivCeil(h, 8)), kMinMaxMaxGroups / nx));
-  return dim3(nx, ny);
+// Workgroups of KDcDequant.
+static int DcGroups(int nblk) {
+  return std::min(kDcGroups, int(DivCeil(nblk, 256)));
 }
 // Grid of KMinMaxPartial4: 1024-column strips (four columns per thread),
 // row ranges of >= 8 rows.
@@ -898,25 +893,15 @@ static int EnsureStageBuffers(pikgpu_ctx* ctx) {
   return PIKGPU_OK;
 }
 
-// DC: dequant, min/max of the 8-padded DC image, EPF + clamp
+// DC: dequant with the DC image's range, EPF + clamp
 // (DequantDC + AdaptiveDCReconstruction).
 static void EnqueueDc(const FrameParams& P, const FrameBuffers& B,
                       const DeviceConsts* K, hipStream_t st) {
-  const int nblk = P.bx * P.by;
-  KDcDequant<<<DivCeil(nblk, 256), 256, 0, st>>>(P, B);
-  Img dci;
-  dci.p = B.dcq;
-  dci.plane = size_t(nblk);
-  dci.pitch = P.bx;
-  dci.W = int(DivCeil(P.bx, 8) * 8);
-  dci.H = int(DivCeil(P.by, 8) * 8);
-  dci.vw = P.bx;
-  dci.vh = P.by;
-  const dim3 mmg = MinMaxGrid(dci.W, dci.H);
-  KMinMaxPartial<<<mmg, 256, 0, st>>>(dci, 0, P, B.mm_partial);
-  KMinMaxFinal<<<1, 256, 0, st>>>(B.mm_partial, int(mmg.x * mmg.y), B.mm);
+  const int nblk = P.bx * P.by, groups = DcGroups(nblk);
+  KDcDequant<<<groups, 256, 0, st>>>(P, B);
+  const Img dci = DcImage(P, B);
   const int grid = XcdGrid(int(DivCeil(dci.W, 32) * DivCeil(dci.H, 32)));
-  KEpf<true><<<grid, 256, 0, st>>>(dci, P, B, K, B.mm, B.dc, P.bx,
+  KEpf<true><<<grid, 256, 0, st>>>(dci, P, B, K, groups, B.dc, P.bx,
                                    size_t(nblk));
 }
 
@@ -996,26 +981,19 @@ hipError_t pikgpu::EnqueueFullSize(const FrameParams& P,
   if ((e = (expr)) != hipSuccess) return e
   const size_t iplane = size_t(B.ipitch) * P.py;
   if (P.ar) {
-    Img ii;
-    ii.p = B.idct;
-    ii.plane = iplane;
-    ii.pitch = B.ipitch;
-    ii.W = P.px;
-    ii.H = P.py;
-    ii.vw = P.px;
-    ii.vh = P.py;
+    const Img ii = IdctImage(P, B);
     const int gab = P.gaborish && !P.use_sharpened;
     // the IDCT image: width a multiple of 8, rows 32-float aligned
     const dim3 mmg = MinMaxGrid4(ii.W, ii.H);
+    const int partials = int(mmg.x * mmg.y);
     KMinMaxPartial4<<<mmg, 256, 0, st>>>(ii, gab, P, B.mm_partial);
-    KMinMaxFinal<<<1, 256, 0, st>>>(B.mm_partial, int(mmg.x * mmg.y), B.mm);
+    if (MinMaxInline(partials) == 0) {
+      KMinMaxFinal<<<1, 256, 0, st>>>(B.mm_partial, partials, B.mm);
+    }
     const int grid = XcdGrid(int(DivCeil(P.px, 32) * DivCeil(P.py, 32)));
-    KGuide<<<grid, 256, 0, st>>>(ii, gab, P, B, B.mm);
-    const int ring = 3 * (2 * 6 * (P.px + 12) + 2 * 6 * P.py);
-    KGuideRing<<<DivCeil(ring, 256), 256, 0, st>>>(P, B);
+    KGuide<<<grid, 256, 0, st>>>(ii, gab, P, B, MinMaxInline(partials));
     REC(4);
-    KEpf<false><<<grid, 256, 0, st>>>(ii, P, B, K, B.mm, B.ar, B.ipitch,
-                                      iplane);
+    KEpf<false><<<grid, 256, 0, st>>>(ii, P, B, K, 0, B.ar, B.ipitch, iplane);
   } else {
     REC(4);
     KCopyPlanes<<<DivCeil(3 * iplane, 256), 256, 0, st>>>(B.idct, B.ar,
@@ -1969,8 +1947,9 @@ constexpr int kBranches = 32;
 typedef void (*BatchKernel)(const BatchFrame*, const BatchSpan*,
                             const uint32_t*, uint32_t, const DeviceConsts*);
 
-// The phases in launch order: name, kernel, whether it can loop
-// (persistent), and its minimum workgroups per CU for the loop's grid.
+// The phases in launch order: name, kernel (null: a phase whose work is part
+// of another one's kernel, kept for the schedules that name it) and whether
+// it can loop (persistent).
 struct BatchPhaseDef {
   const char* name;
   BatchKernel kernel;
@@ -1978,8 +1957,8 @@ struct BatchPhaseDef {
 };
 const BatchPhaseDef kBatchPhases[PIKGPU_BATCH_PHASES] = {
     {"dc_dequant", KDcDequantBatch, true},
-    {"dc_minmax", KMinMaxPartialDcBatch, true},
-    {"dc_minmax_final", KMinMaxFinalBatch, true},
+    {"dc_minmax", nullptr, true},        // in dc_dequant
+    {"dc_minmax_final", nullptr, true},  // in dc_epf
     {"dc_epf", KEpfDcBatch, false},
     {"llf", KComputeLlfBatch, true},
     {"lf_blur", KLfBlurBatch, true},
@@ -1991,7 +1970,7 @@ const BatchPhaseDef kBatchPhases[PIKGPU_BATCH_PHASES] = {
     {"minmax", KMinMaxPartial4Batch, true},
     {"minmax_final", KMinMaxFinalBatch, true},
     {"guide", KGuideBatch, false},
-    {"guide_ring", KGuideRingBatch, true},
+    {"guide_ring", nullptr, true},       // in guide
     {"epf", KEpfBatch, false},
     {"copy_planes", KCopyPlanesBatch, true},
     {"dots", KDotsBatch, true},
@@ -2069,21 +2048,11 @@ bool PhaseGrid(int p, const FrameParams& P, const FrameBuffers& B, int* nx,
   const bool hf = P.predict_hf != 0;
   switch (p) {
     case 0:  // dc_dequant
-      *nx = int(DivCeil(nblk, 256));
+      *nx = DcGroups(nblk);
       return true;
-    case 1: {  // dc_minmax
-      const dim3 g = MinMaxGrid(dci.W, dci.H);
-      *nx = int(g.x);
-      *ny = int(g.y);
-      return true;
-    }
-    case 2: {  // dc_minmax_final
-      const dim3 g = MinMaxGrid(dci.W, dci.H);
-      arg[0] = int(g.x * g.y);
-      return true;
-    }
     case 3:  // dc_epf
       *nx = XcdGrid(int(DivCeil(dci.W, 32) * DivCeil(dci.H, 32)));
+      arg[0] = DcGroups(nblk);
       return true;
     case 4:  // llf
       *nx = wg4 + wg2 + gcx * int(ngroups) * 3;
@@ -2131,15 +2100,15 @@ bool PhaseGrid(int p, const FrameParams& P, const FrameBuffers& B, int* nx,
     case 12: {  // minmax_final
       const dim3 g = MinMaxGrid4(ii.W, ii.H);
       arg[0] = int(g.x * g.y);
-      return P.ar != 0;
+      return P.ar != 0 && MinMaxInline(arg[0]) == 0;
     }
-    case 13:  // guide
+    case 13: {  // guide
+      const dim3 g = MinMaxGrid4(ii.W, ii.H);
       *nx = XcdGrid(int(DivCeil(P.px, 32) * DivCeil(P.py, 32)));
       arg[0] = P.gaborish && !P.use_sharpened;
+      arg[1] = MinMaxInline(int(g.x * g.y));
       return P.ar != 0;
-    case 14:  // guide_ring
-      *nx = int(DivCeil(3 * (2 * 6 * (P.px + 12) + 2 * 6 * P.py), 256));
-      return P.ar != 0;
+    }
     case 15:  // epf
       *nx = XcdGrid(int(DivCeil(P.px, 32) * DivCeil(P.py, 32)));
       return P.ar != 0;

@@ -69,15 +69,15 @@ struct FrameBuffers {
   float* epf;             // stage dump only
   float* ar;              // 3 planes py x ipitch
   // u8 EPF guide, 3 planes of grows rows x gpitch bytes; pixel (x, y) at
-  // (x + 6, y + 6), the 6-pixel border mirrored (KGuide, KGuideRing)
+  // (x + 6, y + 6), the 6-pixel border mirrored (KGuide)
   uint8_t* gimg;
   int gpitch, grows;
   float* dots_img;        // stage dump only
   float* gab;             // stage dump only
   float* out;             // 3 planes ysize x opitch
   uint8_t* srgb8;         // ysize rows of spitch bytes, interleaved RGB
-  float* mm_partial;      // [num_wg][6]
-  float* mm;              // [8]: min[3], max[3], stretch/mul, all_min
+  float* mm_partial;      // [num_wg][2]: min, max
+  float* mm;              // minimum over channels, guide multiplier
   int ipitch;             // floats per row of idct/ar
   int opitch;             // floats per row of out (dense: its width)
   int spitch;             // bytes per row of srgb8 (dense: 3 x its width)

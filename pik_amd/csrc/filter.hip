@@ -20,12 +20,6 @@ namespace pikgpu {
 
 namespace {
 
-__device__ inline float ImgAt(const Img& in, int c, int x, int y) {
-  const int mx = min(Mirror(x, in.W), in.vw - 1);
-  const int my = min(Mirror(y, in.H), in.vh - 1);
-  return in.p[c * in.plane + size_t(my) * in.pitch + mx];
-}
-
 // LUTs of SigmaFromQuant (pik/epf_target.cc:1161-1196).
 __constant__ float kSigmaLut[32] = {
     1.9815775622811198f, 1.9715084740908622f, 1.6819963065873933f,
@@ -141,128 +135,16 @@ __device__ inline uint32_t LdsDword(const uint8_t* p) {
 }  // namespace
 
 // ---------------------------------------------------------------------------
-// Partial per-channel min/max of the guide over a W x H image (MinMax,
-// pik/epf_target.cc:975-1004); one entry of 6 floats per workgroup. Thread
-// x walks column x of its row range with the 3x3 window of the Gaborish in
-// registers (Symmetric3's operation order, pik/convolve.h:605-621).
-__device__ __forceinline__ void KMinMaxPartialBody(
-    Img in, int gaborish, FrameParams P, float* partial, const VBlock& vb) {
-  __shared__ float s_mm[6][256];
-  const int tid = threadIdx.x;
-  const int x = vb.x * 256 + tid;
-  const int rows = (in.H + vb.ny - 1) / vb.ny;
-  const int ya = vb.y * rows, yb = min(in.H, ya + rows);
-  float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX};
-  float mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-  if (x < in.W) {
-    // Source columns and rows: mirrored at W x H, then replicated beyond
-    // the valid region (ImgAt). The three channels advance together so
-    // each row step issues nine independent loads.
-    const int xc = min(x, in.vw - 1);
-    const int xm = min(Mirror(x - 1, in.W), in.vw - 1);
-    const int xp = min(Mirror(x + 1, in.W), in.vw - 1);
-    if (!gaborish) {
-      for (int y = ya; y < yb; ++y) {
-        const size_t r = size_t(min(y, in.vh - 1)) * in.pitch;
-        for (int c = 0; c < 3; ++c) {
-          const float v = in.p[c * in.plane + r + xc];
-          mn[c] = fminf(mn[c], v);
-          mx[c] = fmaxf(mx[c], v);
-        }
-      }
-    } else {
-      float t[3][3], m[3][3];  // [channel][left, centre, right]
-      const size_t r0 = size_t(min(Mirror(ya - 1, in.H), in.vh - 1)) * in.pitch;
-      const size_t r1 = size_t(min(ya, in.vh - 1)) * in.pitch;
-      for (int c = 0; c < 3; ++c) {
-        const float* pc = in.p + c * in.plane;
-        t[c][0] = pc[r0 + xm];
-        t[c][1] = pc[r0 + xc];
-        t[c][2] = pc[r0 + xp];
-        m[c][0] = pc[r1 + xm];
-        m[c][1] = pc[r1 + xc];
-        m[c][2] = pc[r1 + xp];
-      }
-      // the row below, loaded one iteration ahead
-      float nb[3][3];
-      {
-        const int yn = ya + 1 < in.H ? ya + 1 : in.H - 1;
-        const size_t rb = size_t(min(yn, in.vh - 1)) * in.pitch;
-        for (int c = 0; c < 3; ++c) {
-          const float* pc = in.p + c * in.plane;
-          nb[c][0] = pc[rb + xm];
-          nb[c][1] = pc[rb + xc];
-          nb[c][2] = pc[rb + xp];
-        }
-      }
-      for (int y = ya; y < yb; ++y) {
-        float b[3][3];
-        for (int c = 0; c < 3; ++c) {
-          for (int i = 0; i < 3; ++i) b[c][i] = nb[c][i];
-        }
-        if (y + 1 < yb) {
-          const int yn = y + 2 < in.H ? y + 2 : in.H - 1;
-          const size_t rb = size_t(min(yn, in.vh - 1)) * in.pitch;
-          for (int c = 0; c < 3; ++c) {
-            const float* pc = in.p + c * in.plane;
-            nb[c][0] = pc[rb + xm];
-            nb[c][1] = pc[rb + xc];
-            nb[c][2] = pc[rb + xp];
-          }
-        }
-        for (int c = 0; c < 3; ++c) {
-          const float bl = b[c][0], bc = b[c][1], br = b[c][2];
-          const float sum_tb = t[c][1] + bc;
-          const float mul0 = m[c][1] * P.gab_w[0];
-          const float sum_lr = m[c][0] + m[c][2];
-          const float x1 = sum_tb + sum_lr;
-          const float mul1 = x1 * P.gab_w[1] + mul0;
-          const float sum_t2 = t[c][0] + t[c][2];
-          const float sum_b2 = bl + br;
-          const float x2 = sum_t2 + sum_b2;
-          const float v = x2 * P.gab_w[2] + mul1;
-          mn[c] = fminf(mn[c], v);
-          mx[c] = fmaxf(mx[c], v);
-          t[c][0] = m[c][0];
-          t[c][1] = m[c][1];
-          t[c][2] = m[c][2];
-          m[c][0] = bl;
-          m[c][1] = bc;
-          m[c][2] = br;
-        }
-      }
-    }
-  }
-  for (int c = 0; c < 3; ++c) {
-    s_mm[c][tid] = mn[c];
-    s_mm[3 + c][tid] = mx[c];
-  }
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (tid < s) {
-      for (int c = 0; c < 3; ++c) {
-        s_mm[c][tid] = fminf(s_mm[c][tid], s_mm[c][tid + s]);
-        s_mm[3 + c][tid] = fmaxf(s_mm[3 + c][tid], s_mm[3 + c][tid + s]);
-      }
-    }
-    __syncthreads();
-  }
-  if (tid < 6) {
-    partial[(vb.y * vb.nx + vb.x) * 6 + tid] = s_mm[tid][0];
-  }
-}
-__global__ void __launch_bounds__(256)
-    KMinMaxPartial(Img in, int gaborish, FrameParams P, float* partial) {
-  KMinMaxPartialBody(in, gaborish, P, partial, PlainBlock());
-}
-
-// KMinMaxPartial for an image whose rows are float4-aligned and whose width
-// is a multiple of 4 with no replicated margin (vw == W, vh == H): thread t
-// walks columns 4t .. 4t + 3 with one float4 and the two mirrored edge
-// columns per row and channel, the next row loaded one iteration ahead.
+// Partial minimum and maximum over the channels of the guide (MinMax,
+// pik/epf_target.cc:975-1004) of an image whose rows are float4-aligned and
+// whose width is a multiple of 4; two floats per workgroup. Thread t walks
+// columns 4t .. 4t + 3 with one float4 and the two mirrored edge columns per
+// row and channel, the 3x3 window of the Gaborish in registers (Symmetric3's
+// operation order, pik/convolve.h:605-621), the next row loaded one
+// iteration ahead.
 __device__ __forceinline__ void KMinMaxPartial4Body(
     Img in, int gaborish, FrameParams P, float* partial, const VBlock& vb) {
-  __shared__ float s_mm[6][256];
+  __shared__ float s_mm[8];
   const int tid = threadIdx.x;
   const int x = (vb.x * 256 + tid) * 4;
   const int rows = (in.H + vb.ny - 1) / vb.ny;
@@ -332,22 +214,12 @@ __device__ __forceinline__ void KMinMaxPartial4Body(
       }
     }
   }
-  for (int c = 0; c < 3; ++c) {
-    s_mm[c][tid] = mn[c];
-    s_mm[3 + c][tid] = mx[c];
-  }
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (tid < s) {
-      for (int c = 0; c < 3; ++c) {
-        s_mm[c][tid] = fminf(s_mm[c][tid], s_mm[c][tid + s]);
-        s_mm[3 + c][tid] = fmaxf(s_mm[3 + c][tid], s_mm[3 + c][tid + s]);
-      }
-    }
-    __syncthreads();
-  }
-  if (tid < 6) {
-    partial[(vb.y * vb.nx + vb.x) * 6 + tid] = s_mm[tid][0];
+  float lo = fminf(fminf(mn[0], mn[1]), mn[2]);
+  float hi = fmaxf(fmaxf(mx[0], mx[1]), mx[2]);
+  GroupMinMax(&lo, &hi, s_mm);
+  if (tid == 0) {
+    partial[2 * (vb.y * vb.nx + vb.x)] = lo;
+    partial[2 * (vb.y * vb.nx + vb.x) + 1] = hi;
   }
 }
 __global__ void __launch_bounds__(256)
@@ -355,42 +227,34 @@ __global__ void __launch_bounds__(256)
   KMinMaxPartial4Body(in, gaborish, P, partial, PlainBlock());
 }
 
-// Reduces the partials to mm[0..5] = min[3], max[3]; mm[6] = 255 / range
-// (the guide multiplier and the sigma stretch, both 1 for a flat image),
-// mm[7] = the minimum over channels.
+// The guide's scaling from n partials: the minimum over channels and 255 /
+// range (the guide multiplier and the sigma stretch, both 1 for a flat
+// image). All 256 threads call.
+struct GuideScale {
+  float all_min, gmul;
+};
+__device__ inline GuideScale ReducePartials(const float* partial, int n,
+                                            float* s_mm) {
+  float lo = FLT_MAX, hi = -FLT_MAX;
+  for (int i = threadIdx.x; i < n; i += 256) {
+    lo = fminf(lo, partial[2 * i]);
+    hi = fmaxf(hi, partial[2 * i + 1]);
+  }
+  GroupMinMax(&lo, &hi, s_mm);
+  const float range = hi - lo;
+  GuideScale g;
+  g.all_min = lo;
+  g.gmul = range == 0.0f ? 1.0f : 255.0f / range;
+  return g;
+}
+
 __device__ __forceinline__ void KMinMaxFinalBody(
     const float* partial, int n, float* mm, const VBlock& vb) {
-  __shared__ float s_mm[6][256];
-  const int tid = threadIdx.x;
-  float v[6] = {FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
-  for (int i = tid; i < n; i += 256) {
-    for (int c = 0; c < 3; ++c) {
-      v[c] = fminf(v[c], partial[i * 6 + c]);
-      v[3 + c] = fmaxf(v[3 + c], partial[i * 6 + 3 + c]);
-    }
-  }
-  for (int k = 0; k < 6; ++k) s_mm[k][tid] = v[k];
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (tid < s) {
-      for (int c = 0; c < 3; ++c) {
-        s_mm[c][tid] = fminf(s_mm[c][tid], s_mm[c][tid + s]);
-        s_mm[3 + c][tid] = fmaxf(s_mm[3 + c][tid], s_mm[3 + c][tid + s]);
-      }
-    }
-    __syncthreads();
-  }
-  if (tid == 0) {
-    float all_min = s_mm[0][0], all_max = s_mm[3][0];
-    for (int c = 0; c < 3; ++c) {
-      mm[c] = s_mm[c][0];
-      mm[3 + c] = s_mm[3 + c][0];
-      all_min = fminf(all_min, s_mm[c][0]);
-      all_max = fmaxf(all_max, s_mm[3 + c][0]);
-    }
-    const float range = all_max - all_min;
-    mm[6] = range == 0.0f ? 1.0f : 255.0f / range;
-    mm[7] = all_min;
+  __shared__ float s_mm[8];
+  const GuideScale g = ReducePartials(partial, n, s_mm);
+  if (threadIdx.x == 0) {
+    mm[0] = g.all_min;
+    mm[1] = g.gmul;
   }
 }
 __global__ void __launch_bounds__(256)
@@ -403,13 +267,21 @@ __global__ void __launch_bounds__(256)
 // pik/epf_target.cc:1129-1148): the Gaborish-smoothed image (the image
 // itself for the sharpened guide), minus the minimum over channels, times
 // the guide stretch, truncated to bytes. One 32x32 tile per workgroup,
-// written at (x + 6, y + 6) of the guide image; KGuideRing fills its
-// 6-pixel border.
+// written at (x + 6, y + 6) of the guide image. Tiles at the image's edge
+// also write the 6-pixel mirrored border (a kernel of its own took 4 to 5
+// us): each position takes the byte of the pixel it mirrors, which is its
+// own bit for bit (the 3x3 sums of the mirrored window only exchange the
+// operands of commutative additions).
+//
+// n_partial > 0: every workgroup reduces the n_partial min/max partials
+// itself, and the first one leaves the result in B.mm for KEpf; else
+// KMinMaxFinal did (MinMaxInline in host_api.h draws the line).
 __device__ __forceinline__ void KGuideBody(
-    Img in, int gaborish, FrameParams P, FrameBuffers B, const float* mm,
+    Img in, int gaborish, FrameParams P, FrameBuffers B, int n_partial,
     const VBlock& vb) {
   constexpr int kWP = 35;  // pitch of the 34 x 34 window rows
   __shared__ float s_w[3][34 * kWP];
+  __shared__ float s_mm[8];
   const int tid = threadIdx.x;
   const int tiles_x = (in.W + 31) / 32;
   const int tile = XcdTile(vb.x, tiles_x * ((in.H + 31) / 32));
@@ -489,10 +361,23 @@ __device__ __forceinline__ void KGuideBody(
       }
     }
   }
+  GuideScale gs;
+  if (n_partial > 0) {
+    gs = ReducePartials(B.mm_partial, n_partial, s_mm);
+    if (vb.x == 0 && tid == 0) {
+      B.mm[0] = gs.all_min;
+      B.mm[1] = gs.gmul;
+    }
+  } else {
+    gs.all_min = B.mm[0];
+    gs.gmul = B.mm[1];
+  }
   __syncthreads();
   // Each thread: pixels j0 .. j0 + 3 of tile row i, all three channels.
-  const float all_min = mm[7];
-  const float gmul = mm[6];
+  const float all_min = gs.all_min;
+  const float gmul = gs.gmul;
+  const bool edge = x0 < kEpfBorder || y0 < kEpfBorder ||
+                    x0 + 32 > in.W - kEpfBorder || y0 + 32 > in.H - kEpfBorder;
   const size_t gplane = size_t(B.grows) * B.gpitch;
   const int i = tid >> 3, j0 = (tid & 7) << 2;
   const int y = y0 + i, x = x0 + j0;
@@ -535,50 +420,33 @@ __device__ __forceinline__ void KGuideBody(
     } else {
       for (int k = 0; k < n; ++k) g8[k] = q[k];
     }
+    if (edge) {
+      // the border positions that mirror these pixels (images are at least
+      // 8 wide and high: one reflection, at most two per direction)
+      for (int k = 0; k < n; ++k) {
+        const int xm[3] = {x + k, x + k < kEpfBorder ? -1 - (x + k) : x + k,
+                           x + k >= in.W - kEpfBorder ? 2 * in.W - 1 - (x + k)
+                                                      : x + k};
+        const int ym[3] = {y, y < kEpfBorder ? -1 - y : y,
+                           y >= in.H - kEpfBorder ? 2 * in.H - 1 - y : y};
+        for (int my = 0; my < 3; ++my) {
+          for (int mx = 0; mx < 3; ++mx) {
+            if ((my > 0 && ym[my] == y) || (mx > 0 && xm[mx] == x + k) ||
+                (my == 0 && mx == 0)) {
+              continue;
+            }
+            B.gimg[c * gplane + size_t(ym[my] + kEpfBorder) * B.gpitch +
+                   xm[mx] + kEpfBorder] = q[k];
+          }
+        }
+      }
+    }
   }
 }
 __global__ void __launch_bounds__(256)
     KGuide(Img in, int gaborish, FrameParams P, FrameBuffers B,
-           const float* mm) {
-  KGuideBody(in, gaborish, P, B, mm, PlainBlock());
-}
-
-// The 6-pixel border of the guide image: each position takes the byte of
-// the pixel it mirrors. (The guide of a mirrored position equals its
-// source pixel's bit for bit: the 3x3 sums of the mirrored window only
-// exchange the operands of commutative additions.)
-__device__ __forceinline__ void KGuideRingBody(
-    FrameParams P, FrameBuffers B, const VBlock& vb) {
-  const int W = P.px, H = P.py;
-  const int pw = W + 12;
-  const int n_tb = 6 * pw, n_lr = 6 * H;
-  const int per_c = 2 * n_tb + 2 * n_lr;
-  const int k = vb.x * 256 + threadIdx.x;
-  if (k >= 3 * per_c) return;
-  const int c = k / per_c;
-  int r = k - c * per_c;
-  int X, Y;
-  if (r < n_tb) {
-    Y = r / pw;
-    X = r - Y * pw;
-  } else if ((r -= n_tb) < n_tb) {
-    Y = H + 6 + r / pw;
-    X = r - (r / pw) * pw;
-  } else if ((r -= n_tb) < n_lr) {
-    Y = 6 + r / 6;
-    X = r - (r / 6) * 6;
-  } else {
-    r -= n_lr;
-    Y = 6 + r / 6;
-    X = W + 6 + (r - (r / 6) * 6);
-  }
-  const int sx = Mirror(X - 6, W), sy = Mirror(Y - 6, H);
-  uint8_t* g = B.gimg + size_t(c) * B.grows * B.gpitch;
-  g[size_t(Y) * B.gpitch + X] = g[size_t(sy + 6) * B.gpitch + sx + 6];
-}
-__global__ void __launch_bounds__(256)
-    KGuideRing(FrameParams P, FrameBuffers B) {
-  KGuideRingBody(P, B, PlainBlock());
+           int n_partial) {
+  KGuideBody(in, gaborish, P, B, n_partial, PlainBlock());
 }
 
 // ---------------------------------------------------------------------------
@@ -596,7 +464,7 @@ __global__ void __launch_bounds__(256)
 template <bool kDc>
 __device__ __forceinline__ void KEpfBody(
     Img in, FrameParams P, FrameBuffers B, const DeviceConsts* K,
-    const float* mm, float* out, int out_pitch, size_t out_plane,
+    int n_partial, float* out, int out_pitch, size_t out_plane,
     const VBlock& vb) {
   constexpr int dc_mode = kDc;
   // Input window: the DC mode keeps the tile with a 7-pixel border (its
@@ -629,8 +497,19 @@ __device__ __forceinline__ void KEpfBody(
   const int tile = XcdTile(vb.x, tiles_x * ((in.H + 31) / 32));
   if (tile < 0) return;
   const int x0 = (tile % tiles_x) * 32, y0 = (tile / tiles_x) * 32;
-  const float all_min = mm[7];
-  const float gmul = mm[6];
+  // the DC mode reduces KDcDequant's min/max partials itself (at most
+  // kDcGroups of them), the image mode reads what KGuide's input was
+  // scaled by
+  GuideScale gs;
+  if (kDc) {
+    __shared__ float s_mm[8];
+    gs = ReducePartials(B.mm_partial, n_partial, s_mm);
+  } else {
+    gs.all_min = B.mm[0];
+    gs.gmul = B.mm[1];
+  }
+  const float all_min = gs.all_min;
+  const float gmul = gs.gmul;
 
   // AR (step 5) needs the descriptor of the storage block whose
   // coefficients this thread owns (the matrix slots and 1 / qf of the
@@ -1051,8 +930,8 @@ __device__ __forceinline__ void KEpfBody(
 template <bool kDc>
 __global__ void __launch_bounds__(256, kDc ? 3 : 4)
     KEpf(Img in, FrameParams P, FrameBuffers B, const DeviceConsts* K,
-         const float* mm, float* out, int out_pitch, size_t out_plane) {
-  KEpfBody<kDc>(in, P, B, K, mm, out, out_pitch, out_plane, PlainBlock());
+         int n_partial, float* out, int out_pitch, size_t out_plane) {
+  KEpfBody<kDc>(in, P, B, K, n_partial, out, out_pitch, out_plane, PlainBlock());
 }
 
 // ---------------------------------------------------------------------------
@@ -1350,19 +1229,15 @@ __global__ void __launch_bounds__(256)
 }
 
 template __global__ void KEpf<true>(Img, FrameParams, FrameBuffers,
-                                    const DeviceConsts*, const float*, float*,
-                                    int, size_t);
+                                    const DeviceConsts*, int, float*, int,
+                                    size_t);
 template __global__ void KEpf<false>(Img, FrameParams, FrameBuffers,
-                                     const DeviceConsts*, const float*, float*,
-                                     int, size_t);
+                                     const DeviceConsts*, int, float*, int,
+                                     size_t);
 
 // ---------------------------------------------------------------------------
 // Batched forms: one launch over every frame of a batch (BatchSpan), each
 // frame's images and buffers as the plain launches of pikgpu_run take them.
-__global__ void __launch_bounds__(256)
-    KMinMaxPartialDcBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_LOOP(KMinMaxPartialBody(DcImage(P, B), 0, P, B.mm_partial, vb));
-}
 __global__ void __launch_bounds__(256)
     KMinMaxPartial4Batch(PIKGPU_BATCH_PARAMS) {
   PIKGPU_BATCH_LOOP(KMinMaxPartial4Body(IdctImage(P, B), s.arg[0], P,
@@ -1372,17 +1247,14 @@ __global__ void __launch_bounds__(256) KMinMaxFinalBatch(PIKGPU_BATCH_PARAMS) {
   PIKGPU_BATCH_LOOP(KMinMaxFinalBody(B.mm_partial, s.arg[0], B.mm, vb));
 }
 __global__ void __launch_bounds__(256, 3) KEpfDcBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_ONE(KEpfBody<true>(DcImage(P, B), P, B, K, B.mm, B.dc, P.bx,
+  PIKGPU_BATCH_ONE(KEpfBody<true>(DcImage(P, B), P, B, K, s.arg[0], B.dc, P.bx,
                                    size_t(P.bx) * P.by, vb));
 }
 __global__ void __launch_bounds__(256) KGuideBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_ONE(KGuideBody(IdctImage(P, B), s.arg[0], P, B, B.mm, vb));
-}
-__global__ void __launch_bounds__(256) KGuideRingBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_LOOP(KGuideRingBody(P, B, vb));
+  PIKGPU_BATCH_ONE(KGuideBody(IdctImage(P, B), s.arg[0], P, B, s.arg[1], vb));
 }
 __global__ void __launch_bounds__(256, 4) KEpfBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_ONE(KEpfBody<false>(IdctImage(P, B), P, B, K, B.mm, B.ar,
+  PIKGPU_BATCH_ONE(KEpfBody<false>(IdctImage(P, B), P, B, K, 0, B.ar,
                                     B.ipitch, size_t(B.ipitch) * P.py, vb));
 }
 __global__ void __launch_bounds__(256) KCopyPlanesBatch(PIKGPU_BATCH_PARAMS) {

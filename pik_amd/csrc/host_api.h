@@ -12,8 +12,18 @@
 
 namespace pikgpu {
 
-// Most workgroups of a KMinMaxPartial launch (6 floats of partials each).
+// Most workgroups of a KMinMaxPartial4 launch (2 floats of partials each).
 constexpr int kMinMaxMaxGroups = 4096;
+// Most workgroups of KDcDequant, each of which leaves a partial of the DC
+// image's range: one per CU.
+constexpr int kDcGroups = 256;
+// Up to this many min/max partials every workgroup of KGuide reduces them
+// itself; beyond, KMinMaxFinal does it once. With 512 partials the 2048
+// workgroups of a 2-megapixel frame read 8 MB of L2 more, about 1 us, and
+// save a launch of 4 to 5 us; at 2048 partials (16 megapixels, 16384
+// workgroups) they would read 270 MB.
+constexpr int kMinMaxInline = 512;
+inline int MinMaxInline(int n) { return n <= kMinMaxInline ? n : 0; }
 
 // Checks that a frame is complete and self-consistent (what the reference
 // rejects as a decoding error); host-only. PIKGPU_OK or the error code,

@@ -182,6 +182,23 @@ __device__ inline float DequantPasses(const FrameParams& P,
   return acc;
 }
 
+// Minimum and maximum over the workgroup's 256 threads, in every thread; s
+// holds 8 floats of LDS that nothing else uses meanwhile. All threads call.
+__device__ inline void GroupMinMax(float* lo, float* hi, float* s) {
+  for (int m = 32; m >= 1; m >>= 1) {
+    *lo = fminf(*lo, __shfl_xor(*lo, m, 64));
+    *hi = fmaxf(*hi, __shfl_xor(*hi, m, 64));
+  }
+  const int wave = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    s[wave] = *lo;
+    s[4 + wave] = *hi;
+  }
+  __syncthreads();
+  *lo = fminf(fminf(s[0], s[1]), fminf(s[2], s[3]));
+  *hi = fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7]));
+}
+
 // ---------------------------------------------------------------------------
 // Cooperative transforms of the three channels of a 32x32 tile (256
 // threads). The 2-D transforms are the reference's two column passes with a
@@ -880,18 +897,15 @@ __host__ __device__ inline Img DcImage(const FrameParams& P,
   return dci;
 }
 
-__global__ void KMinMaxPartial(Img in, int gaborish, FrameParams P,
-                               float* partial);
 __global__ void KMinMaxPartial4(Img in, int gaborish, FrameParams P,
                                float* partial);
 __global__ void KMinMaxFinal(const float* partial, int n, float* mm);
 template <bool kDc>
 __global__ void KEpf(Img in, FrameParams P, FrameBuffers B,
-                     const DeviceConsts* K, const float* mm, float* out,
+                     const DeviceConsts* K, int n_partial, float* out,
                      int out_pitch, size_t out_plane);
 __global__ void KGuide(Img in, int gaborish, FrameParams P, FrameBuffers B,
-                       const float* mm);
-__global__ void KGuideRing(FrameParams P, FrameBuffers B);
+                       int n_partial);
 __global__ void KDots(FrameParams P, FrameBuffers B);
 // KFinal: rows per workgroup of its 256-column strips.
 constexpr int kFinalRows = 16;
@@ -901,7 +915,6 @@ __global__ void KCopyPlanes(const float* src, float* dst, size_t n);
 // Batched forms of the reconstruction's kernels (pikgpu_batch): one launch
 // per phase over every frame of a batch; see BatchSpan.
 __global__ void KDcDequantBatch(PIKGPU_BATCH_PARAMS);
-__global__ void KMinMaxPartialDcBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KMinMaxFinalBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KEpfDcBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KComputeLlfBatch(PIKGPU_BATCH_PARAMS);
@@ -913,7 +926,6 @@ __global__ void KPred2x2InteriorBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KBlocksBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KMinMaxPartial4Batch(PIKGPU_BATCH_PARAMS);
 __global__ void KGuideBatch(PIKGPU_BATCH_PARAMS);
-__global__ void KGuideRingBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KEpfBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KCopyPlanesBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KDotsBatch(PIKGPU_BATCH_PARAMS);

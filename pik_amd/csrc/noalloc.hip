@@ -105,8 +105,8 @@ size_t NoAllocLayout(const pikgpu_frame* f, const FrameParams& P,
   B->idct = c.Take<float>(3 * ipitch * P.py);
   B->ar = c.Take<float>(3 * ipitch * P.py);
   B->gimg = c.Take<uint8_t>(3 * grows * gpitch);
-  B->mm_partial = c.Take<float>(size_t(kMinMaxMaxGroups) * 6);
-  B->mm = c.Take<float>(8);
+  B->mm_partial = c.Take<float>(size_t(kMinMaxMaxGroups) * 2);
+  B->mm = c.Take<float>(2);
   // KFinal reads `ar` only, so the linear output reuses the IDCT image
   // (3 planes of ysize x opitch <= 3 planes of py x ipitch)
   B->out = B->idct;

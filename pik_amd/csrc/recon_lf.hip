@@ -11,33 +11,49 @@
 //   UpdateLfForDecoder (pred2x2)      pik/ac_predictions.cc:560-635
 // Every kernel is a flat grid over (group, plane, cache position); the group
 // caches have fixed pitches (device.h).
+#include <float.h>
+
 #include "device.h"
 #include "kernels.h"
 
 namespace pikgpu {
 
-// DequantDC; also writes each block's dequantisation descriptors.
+// DequantDC; also writes each block's dequantisation descriptors and, per
+// workgroup, the minimum and maximum of the DC image over the channels (the
+// DC EPF's guide has no Gaborish and its padding repeats pixels of the
+// image, so its range is the image's). At most kDcGroups workgroups, each
+// walking the blocks with a stride, so that every workgroup of the DC EPF
+// can reduce the partials itself: as two kernels of their own the min/max
+// and its reduction took 7 + 4 us of a 4096x4096 frame and 4 + 3 us and two
+// launches of any small one.
 __device__ __forceinline__ void KDcDequantBody(
-    FrameParams P, FrameBuffers B, const VBlock& vb) {
-  const int i = vb.x * blockDim.x + threadIdx.x;
+    const FrameParams& P, const FrameBuffers& B, const VBlock& vb) {
+  __shared__ float s_mm[8];
   const int n = P.bx * P.by;
-  if (i >= n) return;
-  {
+  float lo = FLT_MAX, hi = -FLT_MAX;
+  for (int i = vb.x * 256 + int(threadIdx.x); i < n; i += vb.nx * 256) {
     const uint8_t a = B.acs[i];
     const int s = AcsCovered(a >> 4), idx = a & 15;
     const int first = i - (idx >> (s >> 1)) * P.bx - (idx & (s - 1));
     WriteBlockDesc(P, B, i, B.qf[i], B.qf[first]);
+    // Y first, then X/B = ytox|ytob * Y + q * mul (the portable target's
+    // mul_add is a separate multiply and add).
+    const float y = float(B.dc16[n + i]) * P.mul_dc[1];
+    const float dqx = float(B.dc16[i]) * P.mul_dc[0];
+    const float dqb = float(B.dc16[2 * n + i]) * P.mul_dc[2];
+    const float x = P.ytox_dc * y + dqx;
+    const float b = P.ytob_dc * y + dqb;
+    B.dcq[i] = x;
+    B.dcq[n + i] = y;
+    B.dcq[2 * n + i] = b;
+    lo = fminf(lo, fminf(fminf(x, y), b));
+    hi = fmaxf(hi, fmaxf(fmaxf(x, y), b));
   }
-  // Y first, then X/B = ytox|ytob * Y + q * mul (the portable target's
-  // mul_add is a separate multiply and add).
-  const float y = float(B.dc16[n + i]) * P.mul_dc[1];
-  const float dqx = float(B.dc16[i]) * P.mul_dc[0];
-  const float dqb = float(B.dc16[2 * n + i]) * P.mul_dc[2];
-  const float x = P.ytox_dc * y + dqx;
-  const float b = P.ytob_dc * y + dqb;
-  B.dcq[i] = x;
-  B.dcq[n + i] = y;
-  B.dcq[2 * n + i] = b;
+  GroupMinMax(&lo, &hi, s_mm);
+  if (threadIdx.x == 0) {
+    B.mm_partial[2 * vb.x] = lo;
+    B.mm_partial[2 * vb.x + 1] = hi;
+  }
 }
 __global__ void __launch_bounds__(256)
     KDcDequant(FrameParams P, FrameBuffers B) {
