@@ -55,7 +55,7 @@ struct pikgpu_ctx {
   // device buffers (grown on demand)
   DevBuf ac, dc16, qf, acs, lut, dcf, ytox, ytob, dqmap, table, offsets, dots,
       dotbins, ac_extra;
-  DevBuf desc, dcq, dcv, llf, tmp2x2, lf2x2, pred2x2, coeffs, idct, guide, epf, ar,
+  DevBuf desc, dcq, dcv, llf, lf2x2, pred2x2, coeffs, idct, guide, epf, ar,
       dots_img, gab, out, mm_partial, mm, ar_keep, srgb8, gimg, predlist;
   // pikgpu_fwd_adj staging (host-pointer calls) and loss partials
   DevBuf adj_qf, adj_in, adj_lin, adj_dqf, adj_dc, adj_loss;
@@ -133,7 +133,7 @@ void FreeAll(pikgpu_ctx* ctx) {
                    &ctx->lut,     &ctx->dcf,    &ctx->ytox,    &ctx->ytob,
                    &ctx->dqmap,   &ctx->table,  &ctx->offsets, &ctx->dots,
                    &ctx->dotbins, &ctx->srgb8,
-                   &ctx->desc,    &ctx->dcq,     &ctx->dcv,    &ctx->llf,     &ctx->tmp2x2,
+                   &ctx->desc,    &ctx->dcq,     &ctx->dcv,    &ctx->llf,    
                    &ctx->lf2x2,   &ctx->pred2x2, &ctx->coeffs, &ctx->idct,
                    &ctx->guide,   &ctx->epf,    &ctx->ar,      &ctx->dots_img,
                    &ctx->gab,     &ctx->out,    &ctx->mm_partial, &ctx->mm,
@@ -691,7 +691,6 @@ int pikgpu_frame_upload(pikgpu_ctx* ctx, const pikgpu_frame* f) {
   GROW(dcq, 3 * nblk * 4);
   GROW(dcv, 3 * nblk * 4);
   GROW(llf, ngroups * 3 * kLlfPlane * 4);
-  GROW(tmp2x2, ngroups * 3 * kG2Plane * 4);
   GROW(lf2x2, ngroups * 3 * kG2Plane * 4);
   GROW(pred2x2, ngroups * 3 * kG2Plane * 4);
   GROW(idct, 3 * ipitch * by * 8 * 4);
@@ -842,7 +841,6 @@ int pikgpu_frame_upload(pikgpu_ctx* ctx, const pikgpu_frame* f) {
   B.dcq = static_cast<float*>(ctx->dcq.p);
   B.dc = static_cast<float*>(ctx->dcv.p);
   B.llf = static_cast<float*>(ctx->llf.p);
-  B.tmp2x2 = static_cast<float*>(ctx->tmp2x2.p);
   B.lf2x2 = static_cast<float*>(ctx->lf2x2.p);
   B.pred2x2 = static_cast<float*>(ctx->pred2x2.p);
   B.idct = static_cast<float*>(ctx->idct.p);
@@ -906,38 +904,21 @@ static void EnqueueDc(const FrameParams& P, const FrameBuffers& B,
 }
 
 // LF-domain predictions per group: LLF, LF predictions (predict_lf) and,
-// with `hf`, the pred2x2 image of the HF prediction.
+// with `hf`, the pred2x2 image of the HF prediction (`border`: only its
+// border, for the encoder, which forms the interior itself).
 static void EnqueueLf(const FrameParams& P, const FrameBuffers& B,
-                      const DeviceConsts* K, hipStream_t st, bool hf) {
-  const size_t ngroups = size_t(P.gx) * P.gy;
-  const int cache_pos = (kGroupDimBlocks + 2) * (kGroupDimBlocks + 2);
-  const int g2_pos = 4 * cache_pos;
-  dim3 gc(DivCeil(cache_pos, 256), ngroups, 3);
-  dim3 g2(DivCeil(g2_pos, 256), ngroups, 3);
-  // DCT32 / DCT16 first blocks on 8 / 4 lanes (32 / 64 units of block x
-  // plane per workgroup), then the cache positions
-  const int wg4 = int(DivCeil(3 * (P.pred_end[3] - P.pred_end[2]), 32));
-  const int wg2 = int(DivCeil(3 * (P.pred_end[2] - P.pred_end[1]), 64));
-  KComputeLlf<<<wg4 + wg2 + gc.x * gc.y * gc.z, 256, 0, st>>>(
-      P, B, K, P.predict_lf, wg4, wg2, int(gc.x), int(ngroups));
-  if (P.predict_lf) {
-    KLfBlur<<<g2, 256, 0, st>>>(P, B);
-    KLfFromDc2x2<<<wg4 + wg2 + gc.x * gc.y * gc.z, 256, 0, st>>>(
-        P, B, K, wg4, wg2, int(gc.x), int(ngroups));
-  }
-  if (hf) {
-    // (positions of pred2x2 no block writes were zeroed at upload)
-    if (P.predict_lf) {
-      KPred2x2Border<true><<<gc, 256, 0, st>>>(P, B, K);
-    } else {
-      KDc2x2Border<<<gc, 256, 0, st>>>(P, B, K);
-    }
-    if (P.pred_end[3] > 0) {
-      // segments as above, then one lane per unit
-      const int wg1 = int(DivCeil(3 * P.pred_end[1], 256));
-      KPred2x2Interior<false><<<wg4 + wg2 + wg1, 256, 0, st>>>(P, B, K, wg4,
-                                                               wg2, nullptr);
-    }
+                      const DeviceConsts* K, hipStream_t st, bool hf,
+                      bool border = false) {
+  // (positions of pred2x2 no block writes were zeroed at upload)
+  KLf<<<dim3(P.gx * P.gy * kLfStrips, 3), kLfThreads, 0, st>>>(P, B, K, hf || border);
+  if (hf && P.pred_end[3] > 0) {
+    // DCT32 / DCT16 first blocks on 8 / 4 lanes (32 / 64 units of block x
+    // plane per workgroup), then one lane per unit
+    const int wg4 = int(DivCeil(3 * (P.pred_end[3] - P.pred_end[2]), 32));
+    const int wg2 = int(DivCeil(3 * (P.pred_end[2] - P.pred_end[1]), 64));
+    const int wg1 = int(DivCeil(3 * P.pred_end[1], 256));
+    KPred2x2Interior<false><<<wg4 + wg2 + wg1, 256, 0, st>>>(P, B, K, wg4,
+                                                             wg2, nullptr);
   }
 }
 
@@ -1349,23 +1330,20 @@ int pikgpu_quantize(pikgpu_ctx* ctx, const float* const opsin[3],
   // dc_dec, the LLF and the LF prediction exactly as the decoder computes
   // them (the encoder calls the same ComputeLlf and PredictLf)
   EnqueueDc(P, B, K, st);
-  EnqueueLf(P, B, K, st, false);
+  EnqueueLf(P, B, K, st, false, P.predict_lf && P.predict_hf);
   const float* itable = static_cast<const float*>(ctx->itable.p);
   if (predict) {
     float* corner = static_cast<float*>(ctx->ecorner.p);
     KEncLf<<<DivCeil(nb, 256), 256, 0, st>>>(P, B, coef, itable, gsf,
                                              corner);
     if (P.predict_hf) {
-      // the encoder's pred2x2: the ring as the decoder forms it, the
-      // transforms from KEncLf's corners (positions no block writes were
-      // zeroed at upload)
-      const size_t ngroups = size_t(P.gx) * P.gy;
-      const int cache_pos = (kGroupDimBlocks + 2) * (kGroupDimBlocks + 2);
-      dim3 gc(DivCeil(cache_pos, 256), ngroups, 3);
-      if (P.predict_lf) {
-        KPred2x2Border<true><<<gc, 256, 0, st>>>(P, B, K);
-      } else {
-        KPred2x2Border<false><<<gc, 256, 0, st>>>(P, B, K);
+      // the encoder's pred2x2: the ring as the decoder forms it (KLf), or
+      // without LF prediction its own; the transforms from KEncLf's corners
+      // (positions no block writes were zeroed at upload)
+      if (!P.predict_lf) {
+        const int cache_pos = (kGroupDimBlocks + 2) * (kGroupDimBlocks + 2);
+        KEncPred2x2Border<<<dim3(DivCeil(cache_pos, 256), P.gx * P.gy, 3), 256,
+                            0, st>>>(P, B, K);
       }
       if (P.pred_end[3] > 0) {
         const int wg4 = int(DivCeil(3 * (P.pred_end[3] - P.pred_end[2]), 32));
@@ -1954,17 +1932,18 @@ struct BatchPhaseDef {
   const char* name;
   BatchKernel kernel;
   bool loop;
+  int threads = 256;
 };
 const BatchPhaseDef kBatchPhases[PIKGPU_BATCH_PHASES] = {
     {"dc_dequant", KDcDequantBatch, true},
     {"dc_minmax", nullptr, true},        // in dc_dequant
     {"dc_minmax_final", nullptr, true},  // in dc_epf
     {"dc_epf", KEpfDcBatch, false},
-    {"llf", KComputeLlfBatch, true},
-    {"lf_blur", KLfBlurBatch, true},
-    {"lf_from_dc2x2", KLfFromDc2x2Batch, true},
-    {"pred2x2_border", KPred2x2BorderBatch, true},
-    {"dc2x2_border", KDc2x2BorderBatch, true},
+    {"llf", KLfBatch, true, kLfThreads},
+    {"lf_blur", nullptr, true},          // in llf
+    {"lf_from_dc2x2", nullptr, true},    // in llf
+    {"pred2x2_border", nullptr, true},   // in llf
+    {"dc2x2_border", nullptr, true},     // in llf
     {"pred2x2_interior", KPred2x2InteriorBatch, false},
     {"blocks", KBlocksBatch, false},
     {"minmax", KMinMaxPartial4Batch, true},
@@ -2037,10 +2016,6 @@ bool PhaseGrid(int p, const FrameParams& P, const FrameBuffers& B, int* nx,
                int* ny, int* nz, int* arg) {
   *nx = *ny = *nz = 1;
   const int nblk = P.bx * P.by;
-  const size_t ngroups = size_t(P.gx) * P.gy;
-  const int cache_pos = (kGroupDimBlocks + 2) * (kGroupDimBlocks + 2);
-  const int gcx = int(DivCeil(cache_pos, 256));
-  const int g2x = int(DivCeil(4 * cache_pos, 256));
   const int wg4 = int(DivCeil(3 * (P.pred_end[3] - P.pred_end[2]), 32));
   const int wg2 = int(DivCeil(3 * (P.pred_end[2] - P.pred_end[1]), 64));
   const Img dci = DcImage(P, B);
@@ -2055,31 +2030,10 @@ bool PhaseGrid(int p, const FrameParams& P, const FrameBuffers& B, int* nx,
       arg[0] = DcGroups(nblk);
       return true;
     case 4:  // llf
-      *nx = wg4 + wg2 + gcx * int(ngroups) * 3;
-      arg[0] = P.predict_lf;
-      arg[1] = wg4;
-      arg[2] = wg2;
-      arg[3] = gcx;
-      arg[4] = int(ngroups);
+      *nx = P.gx * P.gy * kLfStrips;
+      *ny = 3;
+      arg[0] = hf;
       return true;
-    case 5:  // lf_blur
-      *nx = g2x;
-      *ny = int(ngroups);
-      *nz = 3;
-      return P.predict_lf != 0;
-    case 6:  // lf_from_dc2x2
-      *nx = wg4 + wg2 + gcx * int(ngroups) * 3;
-      arg[0] = wg4;
-      arg[1] = wg2;
-      arg[2] = gcx;
-      arg[3] = int(ngroups);
-      return P.predict_lf != 0;
-    case 7:  // pred2x2_border
-    case 8:  // dc2x2_border
-      *nx = gcx;
-      *ny = int(ngroups);
-      *nz = 3;
-      return hf && (P.predict_lf != 0) == (p == 7);
     case 9: {  // pred2x2_interior
       const int wg1 = int(DivCeil(3 * P.pred_end[1], 256));
       *nx = wg4 + wg2 + wg1;
@@ -2223,7 +2177,7 @@ int BuildQueueGraph(pikgpu_batch* b) {
     uint32_t total = L.total;
     void* args[] = {&F, &S, &M, &total, &K};
     e = hipLaunchKernel(reinterpret_cast<const void*>(d.kernel), dim3(grid),
-                        dim3(256), args, 0, b->main);
+                        dim3(d.threads), args, 0, b->main);
   }
   hipGraph_t g = nullptr;
   const hipError_t e_end = hipStreamEndCapture(b->main, &g);

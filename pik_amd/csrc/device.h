@@ -60,7 +60,6 @@ struct FrameBuffers {
   float* dcq;             // 3 planes by x bx (DequantDC)
   float* dc;              // 3 planes by x bx (after DC AR)
   float* llf;             // [group][3][kLlfPlane]
-  float* tmp2x2;          // [group][3][kG2Plane]
   float* lf2x2;           // [group][3][kG2Plane]
   float* pred2x2;         // [group][3][kG2Plane]
   float* coeffs;          // 3 planes by x (bx*64) (stage dump only)

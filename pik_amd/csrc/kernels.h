@@ -820,16 +820,15 @@ __global__ void KEncQuant(FrameParams P, FrameBuffers B, const float* coef,
 __global__ void KEncLf(FrameParams P, FrameBuffers B, float* coef,
                        const float* itable, float gsf, float* corner);
 __global__ void KEncHfResidual(FrameParams P, FrameBuffers B, float* coef);
-__global__ void KComputeLlf(FrameParams P, FrameBuffers B, const DeviceConsts* K,
-                            int dc2x2, int wg4, int wg2, int pos_blocks,
-                            int ngroups);
-__global__ void KDc2x2Border(FrameParams P, FrameBuffers B,
-                             const DeviceConsts* K);
-__global__ void KLfBlur(FrameParams P, FrameBuffers B);
-__global__ void KLfFromDc2x2(FrameParams P, FrameBuffers B, const DeviceConsts* K,
-                             int wg4, int wg2, int pos_blocks, int ngroups);
-template <bool kUseLf>
-__global__ void KPred2x2Border(FrameParams P, FrameBuffers B, const DeviceConsts* K);
+// KLf: workgroup size; strips of 16 block rows per group, each a workgroup
+// per plane (grid: groups x strips, planes).
+constexpr int kLfThreads = 1024;
+constexpr int kLfStrip = 16;
+constexpr int kLfStrips = kGroupDimBlocks / kLfStrip;
+__global__ void KLf(FrameParams P, FrameBuffers B, const DeviceConsts* K,
+                    int border);
+__global__ void KEncPred2x2Border(FrameParams P, FrameBuffers B,
+                                  const DeviceConsts* K);
 template <bool kEnc>
 __global__ void KPred2x2Interior(FrameParams P, FrameBuffers B, const DeviceConsts* K,
                                  int wg4, int wg2, const float* corner);
@@ -917,11 +916,7 @@ __global__ void KCopyPlanes(const float* src, float* dst, size_t n);
 __global__ void KDcDequantBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KMinMaxFinalBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KEpfDcBatch(PIKGPU_BATCH_PARAMS);
-__global__ void KComputeLlfBatch(PIKGPU_BATCH_PARAMS);
-__global__ void KLfBlurBatch(PIKGPU_BATCH_PARAMS);
-__global__ void KLfFromDc2x2Batch(PIKGPU_BATCH_PARAMS);
-__global__ void KPred2x2BorderBatch(PIKGPU_BATCH_PARAMS);
-__global__ void KDc2x2BorderBatch(PIKGPU_BATCH_PARAMS);
+__global__ void KLfBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KPred2x2InteriorBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KBlocksBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KMinMaxPartial4Batch(PIKGPU_BATCH_PARAMS);

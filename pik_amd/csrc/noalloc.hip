@@ -99,7 +99,6 @@ size_t NoAllocLayout(const pikgpu_frame* f, const FrameParams& P,
   B->dcq = c.Take<float>(3 * nblk);
   B->dc = c.Take<float>(3 * nblk);
   B->llf = c.Take<float>(ngroups * 3 * kLlfPlane);
-  B->tmp2x2 = c.Take<float>(ngroups * 3 * kG2Plane);
   B->lf2x2 = c.Take<float>(ngroups * 3 * kG2Plane);
   B->pred2x2 = c.Take<float>(ngroups * 3 * kG2Plane);
   B->idct = c.Take<float>(3 * ipitch * P.py);

@@ -9,9 +9,9 @@
 //   PredictLf                         pik/ac_predictions.cc:410-470
 //   border of pred2x2                 pik/compressed_image.cc:980-1039
 //   UpdateLfForDecoder (pred2x2)      pik/ac_predictions.cc:560-635
-// Every kernel is a flat grid over (group, plane, cache position); the group
-// caches have fixed pitches (device.h).
+// The group caches have fixed pitches (device.h).
 #include <float.h>
+#include <stddef.h>
 
 #include "device.h"
 #include "kernels.h"
@@ -103,391 +103,12 @@ __device__ inline uint8_t CacheAcs(const FrameParams& P, const FrameBuffers& B,
   return B.acs[(G.gby0 + y - 1) * P.bx + G.gbx0 + x - 1];
 }
 
-// ---------------------------------------------------------------------------
-// ComputeLlf: DC -> lowest-frequency coefficients of the first block at
-// cache position (x, y) (LowestFrequenciesFromDC, pik/ac_strategy.cc:
-// 850-887).
-__device__ inline void LlfAt(const FrameParams& P, const FrameBuffers& B,
-                             const DeviceConsts* K, const GroupGeom& G, int g,
-                             int c, int x, int y, int raw) {
-  float* llf = B.llf + (size_t(g) * 3 + c) * kLlfPlane + y * kLlfPitch + x;
-  if (raw == kDCT16 || raw == kDCT32) {
-    // ReinterpretingDCT<8s, s, s> of the s x s DC values.
-    float dc[16];
-    const int s = raw == kDCT16 ? 2 : 4;
-    for (int iy = 0; iy < 4; ++iy) {
-      for (int ix = 0; ix < 4; ++ix) {
-        dc[iy * 4 + ix] =
-            (iy < s && ix < s) ? GroupDc(P, K, B.dc, c, G, x + ix, y + iy) : 0.0f;
-      }
-    }
-    if (raw == kDCT16) {
-      const float a00 = dc[0], a01 = dc[1], a10 = dc[4], a11 = dc[5];
-      const float d[4] = {(a00 + a01 + a10 + a11) * 0.25f,
-                          (a00 + a01 - a10 - a11) * 0.25f,
-                          (a00 - a01 + a10 - a11) * 0.25f,
-                          (a00 - a01 - a10 + a11) * 0.25f};
-      for (int iy = 0; iy < 2; ++iy) {
-        for (int ix = 0; ix < 2; ++ix) {
-          const float v = d[iy * 2 + ix] * K->tscale[0][iy][ix];
-          llf[iy * kLlfPitch + ix] = v * K->ascale[3][iy][ix];
-        }
-      }
-    } else {
-      ReinterpDct<32, 4>(K, dc, 4, llf, kLlfPitch);
-    }
-    return;
-  }
-  llf[0] = GroupDc(P, K, B.dc, c, G, x, y);
-}
-
-// DC2x2FromLowestFrequencies of the first block at cache position (x, y)
-// into tmp2x2 or pred2x2 (pik/ac_strategy.cc:928-969).
-__device__ inline void Dc2x2At(const FrameParams& P, const FrameBuffers& B,
-                               const DeviceConsts* K, int g, int c, int x,
-                               int y, int raw, bool to_pred2x2) {
-  const float* llf = B.llf + (size_t(g) * 3 + c) * kLlfPlane + y * kLlfPitch + x;
-  float* o = (to_pred2x2 ? B.pred2x2 : B.tmp2x2) + (size_t(g) * 3 + c) * kG2Plane +
-             2 * y * kG2Pitch + 2 * x;
-  if (raw == kDCT16) {
-    ReinterpIdct<16, 2, 4>(K, llf, kLlfPitch, o, kG2Pitch);
-  } else if (raw == kDCT32) {
-    ReinterpIdct<32, 4, 8>(K, llf, kLlfPitch, o, kG2Pitch);
-  } else {
-    float v;
-    if (raw == kDCT || raw == kDCTNoHF || raw == kLines) {
-      // ReinterpretingIDCT<8, 1, 2>: one coefficient, 2-point IDCT of it.
-      v = (llf[0] * K->ascale[0][0][0]) * K->tscale[2][0][0];
-    } else {
-      v = llf[0];
-    }
-    o[0] = v;
-    o[1] = v;
-    o[kG2Pitch] = v;
-    o[kG2Pitch + 1] = v;
-  }
-}
-
-// LlfAt and, with dc2x2, Dc2x2At of a DCT16 (S = 2) or DCT32 (S = 4) first
-// block on N = 2S lanes, each element with the one-lane form's operations
-// in the same order. LLF: for S = 4 the 4x4 ReinterpretingDCT runs its
-// column pass on lanes 0..3 into the unit's LDS matrix t, then its row pass
-// there, lane l ending with LLF column l; for S = 2 every lane recomputes
-// the 2x2 Hadamard and keeps its column. The 2x image: the column pass of
-// Idct2D<N> over the zero-padded LLF, lane l on column l, into t, then the
-// row pass on column l of t. All threads of the workgroup call (barriers);
-// `active` is false past the last unit.
-template <int S>
-__device__ inline void LlfDc2x2Lanes(const FrameParams& P,
-                                     const FrameBuffers& B,
-                                     const DeviceConsts* K, bool active, int c,
-                                     int blk, int l, bool dc2x2, float* t) {
-  constexpr int N = 2 * S;
-  int g = 0, x = 0, y = 0;
-  GroupGeom G = {0, 0, 0, 0};
-  if (active) {
-    const int bxa = blk % P.bx, bya = blk / P.bx;
-    const int gxi = bxa / kGroupDimBlocks, gyi = bya / kGroupDimBlocks;
-    g = gyi * P.gx + gxi;
-    x = bxa - gxi * kGroupDimBlocks + 1;
-    y = bya - gyi * kGroupDimBlocks + 1;
-    G = Geom(P, g);
-  }
-  float* llf = B.llf + (size_t(g) * 3 + c) * kLlfPlane + y * kLlfPitch + x;
-  float col[S];  // LLF column l (lanes l < S)
-  if (S == 4) {
-    // ReinterpretingDCT<32, 4, 4> of the 4 x 4 DC values
-    float v[4], w[4];
-    if (active && l < 4) {
-#pragma unroll
-      for (int iy = 0; iy < 4; ++iy) v[iy] = GroupDc(P, K, B.dc, c, G, x + l, y + iy);
-      dct1d::Dct<4>(v, w);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) t[l * 5 + k] = w[k];
-    }
-    __syncthreads();
-    if (active && l < 4) {
-#pragma unroll
-      for (int xx = 0; xx < 4; ++xx) v[xx] = t[xx * 5 + l];
-      dct1d::Dct<4>(v, w);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float cf = w[j] * (1.0f / 16);
-        const float u = cf * K->tscale[1][j][l];
-        col[j] = u * K->ascale[4][j][l];
-        llf[j * kLlfPitch + l] = col[j];
-      }
-    }
-    __syncthreads();  // t is reused below
-  } else {
-    if (active) {
-      const float a00 = GroupDc(P, K, B.dc, c, G, x, y);
-      const float a01 = GroupDc(P, K, B.dc, c, G, x + 1, y);
-      const float a10 = GroupDc(P, K, B.dc, c, G, x, y + 1);
-      const float a11 = GroupDc(P, K, B.dc, c, G, x + 1, y + 1);
-      const float d[4] = {(a00 + a01 + a10 + a11) * 0.25f,
-                          (a00 + a01 - a10 - a11) * 0.25f,
-                          (a00 - a01 + a10 - a11) * 0.25f,
-                          (a00 - a01 - a10 + a11) * 0.25f};
-      if (l < 2) {
-#pragma unroll
-        for (int iy = 0; iy < 2; ++iy) {
-          const float v = d[iy * 2 + l] * K->tscale[0][iy][l];
-          col[iy] = v * K->ascale[3][iy][l];
-          llf[iy * kLlfPitch + l] = col[iy];
-        }
-      }
-    }
-  }
-  if (!dc2x2) return;  // the same for the whole launch
-  // ReinterpretingIDCT<8S, S, 2S>
-  constexpr int ai = ScaleIdx<N>(), ti = ScaleIdx<8 * S>();
-  float v[N], w[N];
-  if (active) {
-#pragma unroll
-    for (int r = 0; r < N; ++r) {
-      v[r] = (r < S && l < S) ? (col[r < S ? r : 0] * K->ascale[ai][r][l]) *
-                                    K->tscale[ti][r][l]
-                              : 0.0f;
-    }
-    dct1d::Idct<N>(v, w);
-#pragma unroll
-    for (int k = 0; k < N; ++k) t[l * (N + 1) + k] = w[k];
-  }
-  __syncthreads();
-  if (!active) return;
-#pragma unroll
-  for (int cc = 0; cc < N; ++cc) v[cc] = t[cc * (N + 1) + l];
-  dct1d::Idct<N>(v, w);
-  float* o = B.tmp2x2 + (size_t(g) * 3 + c) * kG2Plane + 2 * y * kG2Pitch + 2 * x;
-#pragma unroll
-  for (int yy = 0; yy < N; ++yy) o[yy * kG2Pitch + l] = w[yy];
-}
-
-// ComputeLlf (and with dc2x2 the LLF's 2x image in tmp2x2, the first step
-// of PredictLf). One launch: workgroups [0, wg4) take the DCT32 first
-// blocks of pred_list (32 units of block x plane on 8 lanes), [wg4, wg4 +
-// wg2) the DCT16 ones (64 units of 4 lanes), the rest one lane per cache
-// position of (position block, group, plane); there the thread turns its
-// block's LLF values into the 2x image reading back what it wrote.
-__device__ __forceinline__ void KComputeLlfBody(
-    FrameParams P, FrameBuffers B, const DeviceConsts* K, int dc2x2, int wg4,
-    int wg2, int pos_blocks, int ngroups, const VBlock& vb) {
-  __shared__ float s_t[32 * 8 * 9];
-  const int tid = threadIdx.x;
-  const int wg = vb.x;
-  if (wg < wg4 + wg2) {
-    const bool big = wg < wg4;
-    const int unit = big ? wg * 32 + (tid >> 3) : (wg - wg4) * 64 + (tid >> 2);
-    const int kb = unit / 3, c = unit - 3 * kb;
-    const int first = big ? P.pred_end[2] : P.pred_end[1];
-    const int n = big ? P.pred_end[3] - P.pred_end[2]
-                      : P.pred_end[2] - P.pred_end[1];
-    const bool active = kb < n;
-    const int blk = active ? int(B.pred_list[first + kb]) : 0;
-    if (big) {
-      LlfDc2x2Lanes<4>(P, B, K, active, c, blk, tid & 7, dc2x2 != 0,
-                       s_t + (tid >> 3) * 8 * 9);
-    } else {
-      LlfDc2x2Lanes<2>(P, B, K, active, c, blk, tid & 3, dc2x2 != 0,
-                       s_t + (tid >> 2) * 4 * 5);
-    }
-    return;
-  }
-  const int r = wg - wg4 - wg2;
-  const int pb = r % pos_blocks, g = (r / pos_blocks) % ngroups;
-  const int c = r / (pos_blocks * ngroups);
-  const int pos = pb * 256 + tid;
-  const GroupGeom G = Geom(P, g);
-  const int W = G.gw + 2, H = G.gh + 2;
-  if (pos >= W * H) return;
-  const int x = pos % W, y = pos / W;
-  const uint8_t a = CacheAcs(P, B, G, x, y);
-  if ((a & 15) != 0) return;  // written by the first block
-  const int raw = a >> 4;
-  if (raw == kDCT16 || raw == kDCT32) return;  // the lane segments
-  LlfAt(P, B, K, G, g, c, x, y, raw);
-  if (dc2x2) Dc2x2At(P, B, K, g, c, x, y, raw, false);
-}
-__global__ void __launch_bounds__(256)
-    KComputeLlf(FrameParams P, FrameBuffers B, const DeviceConsts* K,
-                int dc2x2, int wg4, int wg2, int pos_blocks, int ngroups) {
-  KComputeLlfBody(P, B, K, dc2x2, wg4, wg2, pos_blocks, ngroups, PlainBlock());
-}
-
-// The border of pred2x2 from the LLF cache without LF prediction
-// (pik/compressed_image.cc:980-1039; the interior is KPred2x2Interior's).
-__device__ __forceinline__ void KDc2x2BorderBody(
-    FrameParams P, FrameBuffers B, const DeviceConsts* K, const VBlock& vb) {
-  const int pos = vb.x * blockDim.x + threadIdx.x;
-  const int g = vb.y, c = vb.z;
-  const GroupGeom G = Geom(P, g);
-  const int W = G.gw + 2, H = G.gh + 2;
-  if (pos >= W * H) return;
-  const int x = pos % W, y = pos / W;
-  if (!(x == 0 || y == 0 || x == W - 1 || y == H - 1)) return;
-  const uint8_t a = CacheAcs(P, B, G, x, y);
-  if ((a & 15) != 0) return;
-  Dc2x2At(P, B, K, g, c, x, y, a >> 4, true);
-}
-__global__ void __launch_bounds__(256)
-    KDc2x2Border(FrameParams P, FrameBuffers B, const DeviceConsts* K) {
-  KDc2x2BorderBody(P, B, K, PlainBlock());
-}
-
-// 3x3 LF prediction blur with mirrored borders (Symmetric3,
-// pik/convolve.h:502-640).
-__device__ __forceinline__ void KLfBlurBody(
-    FrameParams P, FrameBuffers B, const VBlock& vb) {
-  const int pos = vb.x * blockDim.x + threadIdx.x;
-  const int g = vb.y, c = vb.z;
-  const GroupGeom G = Geom(P, g);
-  const int W = 2 * (G.gw + 2), H = 2 * (G.gh + 2);
-  if (pos >= W * H) return;
-  const int x = pos % W, y = pos / W;
-  const float* in = B.tmp2x2 + (size_t(g) * 3 + c) * kG2Plane;
-  float* out = B.lf2x2 + (size_t(g) * 3 + c) * kG2Plane;
-  out[y * kG2Pitch + x] =
-      Symmetric3(in, kG2Pitch, W, H, x, y, P.lfblur_w[0], P.lfblur_w[1],
-                 P.lfblur_w[2]);
-}
-__global__ void __launch_bounds__(256)
-    KLfBlur(FrameParams P, FrameBuffers B) {
-  KLfBlurBody(P, B, PlainBlock());
-}
-
-// ReinterpDct<8S, 2S> in place on the 2S x 2S block at p (pitch kG2Pitch)
-// on N = 2S lanes: lane l runs the first pass of Dct2D over column l into
-// row l of the unit's LDS matrix t (pitch N + 1), then, after the barrier,
-// the second pass over column l of t, scaling and writing column l. Every
-// element sees the one-lane form's operations in the same order. All
-// threads of the workgroup call; `active` is false past the last unit.
-template <int S>
-__device__ inline void ReinterpDctLanes(const DeviceConsts* K, bool active,
-                                        float* p, int l, float* t) {
-  constexpr int N = 2 * S;
-  constexpr int ti = ScaleIdx<N>(), ai = ScaleIdx<8 * S>();
-  float v[N], w[N];
-  if (active) {
-#pragma unroll
-    for (int y = 0; y < N; ++y) v[y] = p[y * kG2Pitch + l];
-    dct1d::Dct<N>(v, w);
-#pragma unroll
-    for (int k = 0; k < N; ++k) t[l * (N + 1) + k] = w[k];
-  }
-  __syncthreads();
-  if (!active) return;
-#pragma unroll
-  for (int x = 0; x < N; ++x) v[x] = t[x * (N + 1) + l];
-  dct1d::Dct<N>(v, w);
-  const float scale = 1.0f / (N * N);
-#pragma unroll
-  for (int j = 0; j < N; ++j) {
-    const float cf = w[j] * scale;
-    const float u = cf * K->tscale[ti][j][l];
-    p[j * kG2Pitch + l] = u * K->ascale[ai][j][l];
-  }
-}
-
-// LowFrequenciesFromDC2x2, in place on lf2x2 (pik/ac_strategy.cc:1019-1064).
-// One launch: workgroups [0, wg4) take the DCT32 first blocks of pred_list
-// (32 units of block x plane on 8 lanes each), [wg4, wg4 + wg2) the DCT16
-// ones (64 units of 4 lanes), the rest one lane per cache position of
-// (position block, group, plane) for the other strategies.
-__device__ __forceinline__ void KLfFromDc2x2Body(
-    FrameParams P, FrameBuffers B, const DeviceConsts* K, int wg4, int wg2,
-    int pos_blocks, int ngroups, const VBlock& vb) {
-  __shared__ float s_t[32 * 8 * 9];
-  const int tid = threadIdx.x;
-  const int wg = vb.x;
-  if (wg < wg4 + wg2) {
-    const bool big = wg < wg4;
-    const int lanes = big ? 8 : 4;
-    const int unit = big ? wg * 32 + (tid >> 3) : (wg - wg4) * 64 + (tid >> 2);
-    const int kb = unit / 3, c = unit - 3 * kb;
-    const int first = big ? P.pred_end[2] : P.pred_end[1];
-    const int n = big ? P.pred_end[3] - P.pred_end[2]
-                      : P.pred_end[2] - P.pred_end[1];
-    const bool active = kb < n;
-    float* p = nullptr;
-    if (active) {
-      const int blk = int(B.pred_list[first + kb]);
-      const int bxa = blk % P.bx, bya = blk / P.bx;
-      const int gxi = bxa / kGroupDimBlocks, gyi = bya / kGroupDimBlocks;
-      const int g = gyi * P.gx + gxi;
-      const int x = bxa - gxi * kGroupDimBlocks + 1;
-      const int y = bya - gyi * kGroupDimBlocks + 1;
-      p = B.lf2x2 + (size_t(g) * 3 + c) * kG2Plane + 2 * y * kG2Pitch + 2 * x;
-    }
-    if (big) {
-      ReinterpDctLanes<4>(K, active, p, tid & 7, s_t + (tid >> 3) * 8 * 9);
-    } else {
-      ReinterpDctLanes<2>(K, active, p, tid & 3, s_t + (tid >> 2) * 4 * 5);
-    }
-    (void)lanes;
-    return;
-  }
-  const int r = wg - wg4 - wg2;
-  const int pb = r % pos_blocks, g = (r / pos_blocks) % ngroups;
-  const int c = r / (pos_blocks * ngroups);
-  const int pos = pb * 256 + tid;
-  const GroupGeom G = Geom(P, g);
-  const int W = G.gw + 2, H = G.gh + 2;
-  if (pos >= W * H) return;
-  const int x = pos % W, y = pos / W;
-  const uint8_t a = CacheAcs(P, B, G, x, y);
-  if ((a & 15) != 0) return;
-  const int raw = a >> 4;
-  if (raw == kDCT16 || raw == kDCT32) return;  // the lane segments
-  float* p = B.lf2x2 + (size_t(g) * 3 + c) * kG2Plane + 2 * y * kG2Pitch + 2 * x;
-  const float b00 = p[0], b01 = p[1], b10 = p[kG2Pitch], b11 = p[kG2Pitch + 1];
-  const float d[4] = {(b00 + b01 + b10 + b11) * 0.25f,
-                      (b00 + b01 - b10 - b11) * 0.25f,
-                      (b00 - b01 + b10 - b11) * 0.25f,
-                      (b00 - b01 - b10 + b11) * 0.25f};
-  if (raw == kDCT || raw == kDCTNoHF || raw == kLines) {
-    // ReinterpretingDCT<8, 2, 2>
-    for (int iy = 0; iy < 2; ++iy) {
-      for (int ix = 0; ix < 2; ++ix) {
-        const float v = d[iy * 2 + ix] * K->tscale[0][iy][ix];
-        p[iy * kG2Pitch + ix] = v * K->ascale[2][iy][ix];
-      }
-    }
-  } else {
-    p[0] = d[0];
-    p[1] = d[1];
-    p[kG2Pitch] = d[2];
-    p[kG2Pitch + 1] = d[3];
-  }
-}
-__global__ void __launch_bounds__(256)
-    KLfFromDc2x2(FrameParams P, FrameBuffers B, const DeviceConsts* K,
-                 int wg4, int wg2, int pos_blocks, int ngroups) {
-  KLfFromDc2x2Body(P, B, K, wg4, wg2, pos_blocks, ngroups, PlainBlock());
-}
-
-// Border of pred2x2 from llf and lf2x2 as DCT8 blocks
-// (pik/compressed_image.cc:980-1039).
-template <bool kUseLf>
-__device__ __forceinline__ void KPred2x2BorderBody(
-    FrameParams P, FrameBuffers B, const DeviceConsts* K, const VBlock& vb) {
-  const int pos = vb.x * blockDim.x + threadIdx.x;
-  const int g = vb.y, c = vb.z;
-  const GroupGeom G = Geom(P, g);
-  const int W = G.gw + 2, H = G.gh + 2;
-  if (pos >= W * H) return;
-  const int x = pos % W, y = pos / W;
-  if (!(x == 0 || y == 0 || x == W - 1 || y == H - 1)) return;
-  const float* llf = B.llf + (size_t(g) * 3 + c) * kLlfPlane;
-  const float* lf = B.lf2x2 + (size_t(g) * 3 + c) * kG2Plane;
-  float* o = B.pred2x2 + (size_t(g) * 3 + c) * kG2Plane + 2 * y * kG2Pitch + 2 * x;
-  // ReinterpretingIDCT<8, 2, 2> of {llf, lf(0,1), lf(1,0), lf(1,1)}; the
-  // encoder without LF prediction forms the same with zeros in place of
-  // the LF values (pik/ac_predictions.cc:187-198).
-  const float l01 = kUseLf ? lf[2 * y * kG2Pitch + 2 * x + 1] : 0.0f;
-  const float l10 = kUseLf ? lf[(2 * y + 1) * kG2Pitch + 2 * x] : 0.0f;
-  const float l11 = kUseLf ? lf[(2 * y + 1) * kG2Pitch + 2 * x + 1] : 0.0f;
-  const float a00 = (llf[y * kLlfPitch + x] * K->ascale[0][0][0]) * K->tscale[2][0][0];
+// A border position of pred2x2 as a DCT8 block: ReinterpretingIDCT<8, 2, 2>
+// of {llf, lf(0,1), lf(1,0), lf(1,1)} (pik/compressed_image.cc:980-1039).
+__device__ inline void Pred2x2BorderAt(const DeviceConsts* K, float llf,
+                                       float l01, float l10, float l11,
+                                       float* o) {
+  const float a00 = (llf * K->ascale[0][0][0]) * K->tscale[2][0][0];
   const float a01 = (l01 * K->ascale[0][0][1]) * K->tscale[2][0][1];
   const float a10 = (l10 * K->ascale[0][1][0]) * K->tscale[2][1][0];
   const float a11 = (l11 * K->ascale[0][1][1]) * K->tscale[2][1][1];
@@ -496,10 +117,442 @@ __device__ __forceinline__ void KPred2x2BorderBody(
   o[kG2Pitch] = a00 - a01 + a10 - a11;
   o[kG2Pitch + 1] = a00 - a01 - a10 + a11;
 }
-template <bool kUseLf>
+
+// ---------------------------------------------------------------------------
+// The LF domain of one group and plane: ComputeLlf (LowestFrequenciesFromDC,
+// pik/ac_strategy.cc:850-887), then with predict_lf the steps of PredictLf
+// (pik/ac_predictions.cc:410-470) -- the LLF's 2x image
+// (DC2x2FromLowestFrequencies, pik/ac_strategy.cc:928-969), its 3x3 blur with
+// mirrored borders (Symmetric3, pik/convolve.h:502-640), the LF coefficients
+// (LowFrequenciesFromDC2x2, pik/ac_strategy.cc:1019-1064) -- and with
+// `border` the border of pred2x2 (pik/compressed_image.cc:980-1039).
+//
+// Every step reads its neighbours' results of the one before; a strip of 16
+// block rows keeps them all in LDS, with the four rows above and below
+// recomputed (the blur needs the 2x row next to the strip, which may belong
+// to a 32x32 transform; strips are aligned to those). The DC and the
+// strategies come in once, LLF and LF go out once. As four kernels over the
+// group caches in memory it took 54 us of a 4096x4096 frame and four launches
+// of 3 to 5 us of a small one; one workgroup for a whole group and plane (91
+// KB) 28 us and, for want of workgroups, 24 us of an 803x533 frame; strips
+// 23 us and 10 us.
+constexpr int kLfRows = kLfStrip + 8;  // block rows of a strip in LDS
+
+struct LfShared {
+  float g2[2 * kLfRows * kG2Pitch];  // the 2x image, then the LF coefficients
+  float dc[kLfRows * kLlfPitch];     // the cache's DC, then the LLF
+  float tscale[5][8][8], ascale[5][8][8];  // DeviceConsts'
+  uint8_t acs[kLfRows * kLlfPitch];
+};
+
+// The strip's rows of the group cache: [lo, hi) are in LDS, [first, last)
+// are its own (the group's border rows 0 and gh + 1 belong to the first and
+// the last strip).
+struct LfStrip {
+  int lo, hi, first, last;
+};
+
+// Orders the LDS accesses of a wave's lanes around it (they run in lockstep
+// and LDS accesses of a wave are in order; this keeps the compiler from
+// moving them).
+__device__ inline void WaveSync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// One DCT16 (S = 2) or DCT32 (S = 4) transform on N = 2S lanes of a wave.
+struct LfUnit {
+  bool active;
+  int x, y, l;  // cache column and LDS row of the first block, lane
+};
+// Slots of the S-aligned first-block positions of kLfRows block rows.
+template <int S>
+constexpr int LfSlots() {
+  return kLfRows / S * (kGroupDimBlocks / S) * 2 * S;
+}
+// Unit `slot / N` of those in cache rows [from, to) of the strip; the first
+// position at or after its first row is S-aligned.
+template <int S>
+__device__ inline LfUnit LfUnitAt(const LfShared& s, const GroupGeom& G,
+                                  const LfStrip& R, int from, int to,
+                                  int slot) {
+  constexpr int N = 2 * S, kPer = kGroupDimBlocks / S;
+  const int u = slot / N;
+  const int x = 1 + S * (u % kPer), y = max(R.lo, 1) + S * (u / kPer);
+  LfUnit f;
+  f.l = slot % N;
+  f.x = x;
+  f.y = y - R.lo;
+  f.active = x <= G.gw && y >= from && y < to && y <= G.gh &&
+             s.acs[f.y * kLlfPitch + x] ==
+                 uint8_t((S == 4 ? kDCT32 : kDCT16) << 4);
+  return f;
+}
+
+// LLF of a unit in place of its DC and, with lf, its 2x image. Each element
+// sees the operations of LowestFrequenciesFromDC and
+// DC2x2FromLowestFrequencies in their order: for S = 4 the 4x4
+// ReinterpretingDCT as a column pass on lanes 0..3 and a row pass after the
+// transpose, for S = 2 the 2x2 Hadamard in every lane; then the column and
+// row passes of Idct2D<N> over the zero-padded LLF. The transposes go
+// through the unit's own region of the 2x image. Every lane of the wave
+// calls.
+template <int S>
+__device__ inline void LlfUnit(const LfUnit& f, bool lf, LfShared* s) {
+  constexpr int N = 2 * S;
+  constexpr int ai = ScaleIdx<N>(), ti = ScaleIdx<8 * S>();
+  const int l = f.l;
+  float* t = s->g2 + 2 * f.y * kG2Pitch + 2 * f.x;  // rows of kG2Pitch
+  float* dc = s->dc + f.y * kLlfPitch + f.x;
+  float col[S];  // LLF column l (lanes l < S)
+  if (S == 4) {
+    float v[4], w[4];
+    if (f.active && l < 4) {
+#pragma unroll
+      for (int iy = 0; iy < 4; ++iy) v[iy] = dc[iy * kLlfPitch + l];
+      dct1d::Dct<4>(v, w);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) t[l * kG2Pitch + k] = w[k];
+    }
+    WaveSync();
+    if (f.active && l < 4) {
+#pragma unroll
+      for (int xx = 0; xx < 4; ++xx) v[xx] = t[xx * kG2Pitch + l];
+      dct1d::Dct<4>(v, w);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float cf = w[j] * (1.0f / 16);
+        const float u = cf * s->tscale[1][j][l];
+        col[j] = u * s->ascale[4][j][l];
+        dc[j * kLlfPitch + l] = col[j];
+      }
+    }
+  } else {
+    float d[4];
+    if (f.active) {
+      const float a00 = dc[0], a01 = dc[1];
+      const float a10 = dc[kLlfPitch], a11 = dc[kLlfPitch + 1];
+      d[0] = (a00 + a01 + a10 + a11) * 0.25f;
+      d[1] = (a00 + a01 - a10 - a11) * 0.25f;
+      d[2] = (a00 - a01 + a10 - a11) * 0.25f;
+      d[3] = (a00 - a01 - a10 + a11) * 0.25f;
+    }
+    WaveSync();
+    if (f.active && l < 2) {
+#pragma unroll
+      for (int iy = 0; iy < 2; ++iy) {
+        const float v = (l == 0 ? d[iy * 2] : d[iy * 2 + 1]) *
+                        s->tscale[0][iy][l];
+        col[iy] = v * s->ascale[3][iy][l];
+        dc[iy * kLlfPitch + l] = col[iy];
+      }
+    }
+  }
+  if (!lf) return;
+  WaveSync();
+  float v[N], w[N];
+  if (f.active) {
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+      v[r] = (r < S && l < S) ? (col[r < S ? r : 0] * s->ascale[ai][r][l]) *
+                                    s->tscale[ti][r][l]
+                              : 0.0f;
+    }
+    dct1d::Idct<N>(v, w);
+#pragma unroll
+    for (int k = 0; k < N; ++k) t[l * kG2Pitch + k] = w[k];
+  }
+  WaveSync();
+  if (f.active) {
+#pragma unroll
+    for (int cc = 0; cc < N; ++cc) v[cc] = t[cc * kG2Pitch + l];
+    dct1d::Idct<N>(v, w);
+  }
+  WaveSync();
+  if (f.active) {
+#pragma unroll
+    for (int yy = 0; yy < N; ++yy) t[yy * kG2Pitch + l] = w[yy];
+  }
+}
+
+// LowFrequenciesFromDC2x2 of a unit, in place: ReinterpDct<8S, 2S> as a
+// column pass, the transpose and a row pass.
+template <int S>
+__device__ inline void LfCoefUnit(const LfUnit& f, LfShared* s) {
+  constexpr int N = 2 * S;
+  constexpr int ti = ScaleIdx<N>(), ai = ScaleIdx<8 * S>();
+  const int l = f.l;
+  float* t = s->g2 + 2 * f.y * kG2Pitch + 2 * f.x;
+  float v[N], w[N];
+  if (f.active) {
+#pragma unroll
+    for (int y = 0; y < N; ++y) v[y] = t[y * kG2Pitch + l];
+    dct1d::Dct<N>(v, w);
+  }
+  WaveSync();
+  if (f.active) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) t[l * kG2Pitch + k] = w[k];
+  }
+  WaveSync();
+  if (f.active) {
+#pragma unroll
+    for (int x = 0; x < N; ++x) v[x] = t[x * kG2Pitch + l];
+    dct1d::Dct<N>(v, w);
+  }
+  WaveSync();
+  if (f.active) {
+    const float scale = 1.0f / (N * N);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const float cf = w[j] * scale;
+      const float u = cf * s->tscale[ti][j][l];
+      t[j * kG2Pitch + l] = u * s->ascale[ai][j][l];
+    }
+  }
+}
+
+// Copies `floats` (a multiple of 4) from LDS to memory, both 16-byte aligned.
+__device__ inline void StoreRows(const float* from, float* to, int floats) {
+  for (int i = threadIdx.x; 4 * i < floats; i += kLfThreads) {
+    reinterpret_cast<float4*>(to)[i] =
+        reinterpret_cast<const float4*>(from)[i];
+  }
+}
+
+__device__ __forceinline__ void KLfBody(const FrameParams& P,
+                                        const FrameBuffers& B,
+                                        const DeviceConsts* K, int border,
+                                        const VBlock& vb) {
+  __shared__ __attribute__((aligned(16))) LfShared s;
+  const int tid = threadIdx.x;
+  const int g = vb.x / kLfStrips, k = vb.x % kLfStrips, c = vb.y;
+  const GroupGeom G = Geom(P, g);
+  if (k * kLfStrip >= G.gh) return;
+  const int W = G.gw + 2, H = G.gh + 2;
+  const bool lf = P.predict_lf != 0;
+  LfStrip R;
+  R.first = k == 0 ? 0 : 1 + k * kLfStrip;
+  R.last = (k + 1) * kLfStrip >= G.gh ? H : 1 + (k + 1) * kLfStrip;
+  R.lo = max(R.first - 4, 0);
+  R.hi = min(R.last + 4, H);
+  // Positions of the strip's rows, kLfThreads apart: the quotient and
+  // remainder of the step are the same for all.
+  const int y0 = tid / W, x0 = tid - y0 * W;
+  const int dy = kLfThreads / W, dx = kLfThreads - dy * W;
+  auto next = [&](int* x, int* y) {
+    *x += dx;
+    *y += dy;
+    if (*x >= W) {
+      *x -= W;
+      *y += 1;
+    }
+  };
+  // the DC, the strategies and the scale tables, every load issued before
+  // the first store
+  {
+    constexpr int kPos =
+        (kLfRows * kLlfPitch + kLfThreads - 1) / kLfThreads;
+    float v[kPos];
+    uint8_t a[kPos];
+    int at[kPos];
+    float sc = 0.0f;
+    constexpr int kScales = 2 * 5 * 8 * 8;
+    static_assert(kScales <= kLfThreads && offsetof(DeviceConsts, ascale) ==
+                                               5 * 8 * 8 * sizeof(float) &&
+                      offsetof(LfShared, ascale) - offsetof(LfShared, tscale) ==
+                          5 * 8 * 8 * sizeof(float),
+                  "one scale per thread");
+    if (tid < kScales) sc = (&K->tscale[0][0][0])[tid];
+    int x = x0, y = R.lo + y0;
+#pragma unroll
+    for (int u = 0; u < kPos; ++u) {
+      at[u] = -1;
+      v[u] = 0.0f;
+      a[u] = 0;
+      if (y < R.hi) {
+        at[u] = (y - R.lo) * kLlfPitch + x;
+        v[u] = GroupDc(P, K, B.dc, c, G, x, y);
+        a[u] = CacheAcs(P, B, G, x, y);
+      }
+      next(&x, &y);
+    }
+    if (tid < kScales) (&s.tscale[0][0][0])[tid] = sc;
+#pragma unroll
+    for (int u = 0; u < kPos; ++u) {
+      if (at[u] >= 0) {
+        s.dc[at[u]] = v[u];
+        s.acs[at[u]] = a[u];
+      }
+    }
+  }
+  __syncthreads();
+  const size_t gc = size_t(g) * 3 + c;
+  float* pred = B.pred2x2 + gc * kG2Plane;
+  // LLF and the 2x image: the strategies of one DC value (whose LLF is that
+  // value), then the lane units
+  {
+    int x = x0, y = R.lo + y0;
+#pragma unroll 1
+    for (; y < R.hi; next(&x, &y)) {
+      const int yl = y - R.lo;
+      const uint8_t a = s.acs[yl * kLlfPitch + x];
+      const int raw = a >> 4;
+      if ((a & 15) != 0 || raw == kDCT16 || raw == kDCT32) continue;
+      float v = s.dc[yl * kLlfPitch + x];
+      if (raw == kDCT || raw == kDCTNoHF || raw == kLines) {
+        // ReinterpretingIDCT<8, 1, 2>: one coefficient, 2-point IDCT of it.
+        v = (v * s.ascale[0][0][0]) * s.tscale[2][0][0];
+      }
+      if (lf) {
+        float* o = s.g2 + 2 * yl * kG2Pitch + 2 * x;
+        o[0] = v;
+        o[1] = v;
+        o[kG2Pitch] = v;
+        o[kG2Pitch + 1] = v;
+      } else if (border && y >= R.first && y < R.last &&
+                 (x == 0 || y == 0 || x == W - 1 || y == H - 1)) {
+        float* o = pred + 2 * y * kG2Pitch + 2 * x;
+        o[0] = v;
+        o[1] = v;
+        o[kG2Pitch] = v;
+        o[kG2Pitch + 1] = v;
+      }
+    }
+  }
+#pragma unroll 1
+  for (int slot = tid; slot - tid < LfSlots<4>(); slot += kLfThreads) {
+    const LfUnit f = LfUnitAt<4>(s, G, R, R.lo, R.hi, slot);
+    if (__ballot(f.active)) LlfUnit<4>(f, lf, &s);
+  }
+#pragma unroll 1
+  for (int slot = tid; slot - tid < LfSlots<2>(); slot += kLfThreads) {
+    const LfUnit f = LfUnitAt<2>(s, G, R, R.lo, R.hi, slot);
+    if (__ballot(f.active)) LlfUnit<2>(f, lf, &s);
+  }
+  __syncthreads();
+  {
+    float* llf = B.llf + gc * kLlfPlane;
+    for (int i = R.first * kLlfPitch + tid; i < R.last * kLlfPitch;
+         i += kLfThreads) {
+      llf[i] = s.dc[i - R.lo * kLlfPitch];
+    }
+  }
+  if (!lf) return;
+  // the blur of the strip's own rows, whose results wait in registers until
+  // every window is read
+  {
+    const int W2 = 2 * W, H2 = 2 * H;
+    const int per = kLfThreads / W2;  // rows per pass
+    constexpr int kOwn = 2 * (kLfStrip + 2);
+    constexpr int kPer = kLfThreads / kG2Pitch;
+    constexpr int kRows = (kOwn + kPer - 1) / kPer;
+    const int r0 = tid / W2, x = tid - r0 * W2;
+    const int xm = max(x - 1, 0), xp = min(x + 1, W2 - 1);
+    const float* g2 = s.g2 - 2 * R.lo * kG2Pitch;
+    float o[kRows];
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+      const int y = 2 * R.first + r0 + u * per;
+      o[u] = 0.0f;
+      if (r0 < per && y < 2 * R.last) {
+        // Symmetric3's operation order; one mirrored step past an edge is
+        // the edge itself
+        const float* rt = g2 + max(y - 1, 0) * kG2Pitch;
+        const float* rm = g2 + y * kG2Pitch;
+        const float* rb = g2 + min(y + 1, H2 - 1) * kG2Pitch;
+        const float sum_tb = rt[x] + rb[x];
+        const float mul0 = rm[x] * P.lfblur_w[0];
+        const float sum_lr = rm[xm] + rm[xp];
+        const float x1 = sum_tb + sum_lr;
+        const float mul1 = x1 * P.lfblur_w[1] + mul0;
+        const float sum_t2 = rt[xm] + rt[xp];
+        const float sum_b2 = rb[xm] + rb[xp];
+        const float x2 = sum_t2 + sum_b2;
+        o[u] = x2 * P.lfblur_w[2] + mul1;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+      const int y = 2 * R.first + r0 + u * per;
+      if (r0 < per && y < 2 * R.last) {
+        s.g2[(y - 2 * R.lo) * kG2Pitch + x] = o[u];
+      }
+    }
+  }
+  __syncthreads();
+  // LF coefficients of the own rows in place, and the border of pred2x2
+  {
+    int x = x0, y = R.first + y0;
+#pragma unroll 1
+    for (; y < R.last; next(&x, &y)) {
+      const int yl = y - R.lo;
+      const uint8_t a = s.acs[yl * kLlfPitch + x];
+      const int raw = a >> 4;
+      if ((a & 15) != 0 || raw == kDCT16 || raw == kDCT32) continue;
+      float* p = s.g2 + 2 * yl * kG2Pitch + 2 * x;
+      const float b00 = p[0], b01 = p[1];
+      const float b10 = p[kG2Pitch], b11 = p[kG2Pitch + 1];
+      float d[4] = {(b00 + b01 + b10 + b11) * 0.25f,
+                    (b00 + b01 - b10 - b11) * 0.25f,
+                    (b00 - b01 + b10 - b11) * 0.25f,
+                    (b00 - b01 - b10 + b11) * 0.25f};
+      if (raw == kDCT || raw == kDCTNoHF || raw == kLines) {
+        // ReinterpretingDCT<8, 2, 2>
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float v = d[i] * s.tscale[0][i >> 1][i & 1];
+          d[i] = v * s.ascale[2][i >> 1][i & 1];
+        }
+      }
+      p[0] = d[0];
+      p[1] = d[1];
+      p[kG2Pitch] = d[2];
+      p[kG2Pitch + 1] = d[3];
+      if (border && (x == 0 || y == 0 || x == W - 1 || y == H - 1)) {
+        Pred2x2BorderAt(K, s.dc[yl * kLlfPitch + x], d[1], d[2], d[3],
+                        pred + 2 * y * kG2Pitch + 2 * x);
+      }
+    }
+  }
+#pragma unroll 1
+  for (int slot = tid; slot - tid < LfSlots<4>(); slot += kLfThreads) {
+    const LfUnit f = LfUnitAt<4>(s, G, R, R.first, R.last, slot);
+    if (__ballot(f.active)) LfCoefUnit<4>(f, &s);
+  }
+#pragma unroll 1
+  for (int slot = tid; slot - tid < LfSlots<2>(); slot += kLfThreads) {
+    const LfUnit f = LfUnitAt<2>(s, G, R, R.first, R.last, slot);
+    if (__ballot(f.active)) LfCoefUnit<2>(f, &s);
+  }
+  __syncthreads();
+  static_assert(kG2Plane % 4 == 0 && 2 * kG2Pitch % 4 == 0, "float4 rows");
+  StoreRows(s.g2 + 2 * (R.first - R.lo) * kG2Pitch,
+            B.lf2x2 + gc * kG2Plane + 2 * R.first * kG2Pitch,
+            2 * (R.last - R.first) * kG2Pitch);
+}
+__global__ void __launch_bounds__(kLfThreads)
+    KLf(FrameParams P, FrameBuffers B, const DeviceConsts* K, int border) {
+  KLfBody(P, B, K, border, PlainBlock());
+}
+
+// The border of pred2x2 as the encoder without LF prediction forms it: zeros
+// in place of the LF values (pik/ac_predictions.cc:187-198; everyone else's
+// border is KLf's).
 __global__ void __launch_bounds__(256)
-    KPred2x2Border(FrameParams P, FrameBuffers B, const DeviceConsts* K) {
-  KPred2x2BorderBody<kUseLf>(P, B, K, PlainBlock());
+    KEncPred2x2Border(FrameParams P, FrameBuffers B, const DeviceConsts* K) {
+  const int pos = blockIdx.x * 256 + threadIdx.x;
+  const int g = blockIdx.y, c = blockIdx.z;
+  const GroupGeom G = Geom(P, g);
+  const int W = G.gw + 2, H = G.gh + 2;
+  if (pos >= W * H) return;
+  const int x = pos % W, y = pos / W;
+  if (!(x == 0 || y == 0 || x == W - 1 || y == H - 1)) return;
+  const size_t gc = size_t(g) * 3 + c;
+  Pred2x2BorderAt(K, B.llf[gc * kLlfPlane + y * kLlfPitch + x], 0.0f, 0.0f,
+                  0.0f, B.pred2x2 + gc * kG2Plane + 2 * y * kG2Pitch + 2 * x);
 }
 
 // Interior of pred2x2: per first block and plane, the decoder-side LF
@@ -720,10 +773,6 @@ __global__ void __launch_bounds__(256)
   KPred2x2InteriorBody<kEnc>(P, B, K, wg4, wg2, corner, PlainBlock());
 }
 
-template __global__ void KPred2x2Border<true>(FrameParams, FrameBuffers,
-                                              const DeviceConsts*);
-template __global__ void KPred2x2Border<false>(FrameParams, FrameBuffers,
-                                               const DeviceConsts*);
 template __global__ void KPred2x2Interior<false>(FrameParams, FrameBuffers,
                                                  const DeviceConsts*, int, int,
                                                  const float*);
@@ -738,23 +787,8 @@ template __global__ void KPred2x2Interior<true>(FrameParams, FrameBuffers,
 __global__ void __launch_bounds__(256) KDcDequantBatch(PIKGPU_BATCH_PARAMS) {
   PIKGPU_BATCH_LOOP(KDcDequantBody(P, B, vb));
 }
-__global__ void __launch_bounds__(256) KComputeLlfBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_LOOP(KComputeLlfBody(P, B, K, s.arg[0], s.arg[1], s.arg[2],
-                                    s.arg[3], s.arg[4], vb));
-}
-__global__ void __launch_bounds__(256) KDc2x2BorderBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_LOOP(KDc2x2BorderBody(P, B, K, vb));
-}
-__global__ void __launch_bounds__(256) KLfBlurBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_LOOP(KLfBlurBody(P, B, vb));
-}
-__global__ void __launch_bounds__(256) KLfFromDc2x2Batch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_LOOP(KLfFromDc2x2Body(P, B, K, s.arg[0], s.arg[1], s.arg[2],
-                                     s.arg[3], vb));
-}
-__global__ void __launch_bounds__(256)
-    KPred2x2BorderBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_LOOP(KPred2x2BorderBody<true>(P, B, K, vb));
+__global__ void __launch_bounds__(kLfThreads) KLfBatch(PIKGPU_BATCH_PARAMS) {
+  PIKGPU_BATCH_LOOP(KLfBody(P, B, K, s.arg[0], vb));
 }
 __global__ void __launch_bounds__(256)
     KPred2x2InteriorBatch(PIKGPU_BATCH_PARAMS) {
