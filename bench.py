@@ -12,7 +12,7 @@ timed steps run back to back on the library's stream, the host
 synchronised before the first and after the last.
 
 Prints one JSON line. `roofline` covers the dominant kernel, timed with the
-library's HIP events on the stream it launches on; `cpu_baseline` times the
+library's device-clock timings; `cpu_baseline` times the
 reference's own AVX2 build (oracle/_ref, the reference's ThreadPool) on the
 same frame on this host's cores.
 
@@ -30,7 +30,7 @@ Two further figures ride on the same line:
            image with the LF and HF prediction residuals (the reference
            encoder's default; a figure without them beside it): forward
            transforms, DC, residuals and dithered AC quantization; MP/s of
-           the kernels (HIP events), and the rate with the host-to-device
+           the kernels (device clock), and the rate with the host-to-device
            copy of the float image and the int16 downloads included.
   search   gradient quant-field search (pikgpu_search_quant_field) of 64
            1024x1024 images at Butteraugli distance 1.0, 20 Adam steps each
@@ -691,11 +691,11 @@ def main():
     R.sync()
     el = time.perf_counter() - t0
     ms_step = el * 1000.0 / a.steps
-    # the last timed run's kernel-family times (HIP events on the library's
+    # the last timed run's kernel-family times (device clock, on the library's
     # stream): the roofline's launch duration
     timed_ms = R.timings()
     # Per-family device times averaged: the same K runs again, each
-    # synchronised so that its HIP events can be read (not timed).
+    # synchronised so that its times can be read (not timed).
     fams = {}
     for _ in range(a.steps):
         R.run()
@@ -711,7 +711,7 @@ def main():
     # Dominant single-kernel family. `achieved` divides the path's
     # algorithmic bytes per pixel (int16 AC in, per-block side data, f32
     # linear out: PATH_BYTES_PER_PX) times the frame's pixels by that
-    # kernel's average HIP-event time; the kernel's own input / output
+    # kernel's average device time; the kernel's own input / output
     # bytes (BYTES_PER_PX) ride along as `kernel_bytes`. The kernel is
     # limited by VALU issue, not HBM: `valu` gives its issue rate from the
     # SQ counter record of the same workload (VALU instructions per wave x

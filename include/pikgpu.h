@@ -337,8 +337,10 @@ PIKGPU_API int pikgpu_stage_dump(pikgpu_ctx* ctx, int stage, float* planes[3],
                       size_t stride_bytes);
 
 /* Device-side timing of the last pikgpu_run (and, in the adj_* entries, of
- * the last pikgpu_fwd_adj), per kernel family, in milliseconds, measured
- * with HIP events on the context stream.
+ * the last pikgpu_fwd_adj, in enc_quantize of the last pikgpu_quantize), per
+ * kernel family, in milliseconds of the device clock: from the start of a
+ * family's first kernel to the start of the next family's (the last one's:
+ * to its end). Waits for the context stream.
  * names[i] points to static strings. Returns the number of entries written
  * (<= max_entries). */
 PIKGPU_API int pikgpu_last_timings(pikgpu_ctx* ctx, const char** names, float* ms,

@@ -115,6 +115,7 @@ __global__ void __launch_bounds__(256, 4)
   const int tile = XcdTile(blockIdx.x, tiles_x * ((P.by + 3) / 4));
   if (tile < 0) return;
   const int tbx = (tile % tiles_x) * 4, tby = (tile / tiles_x) * 4;
+  if (B.stamps) StampStart(&B.stamps->adj[0], blockIdx.x);
   const uint8_t a_own = TileAcs(P, B, tbx, tby);
   const CoefIn in = LoadCoefIn(P, B, A, tbx, tby);
   if (tid < 16) s_acs[tid] = a_own;
@@ -211,6 +212,7 @@ __global__ void __launch_bounds__(256, 4)
   if (tile < 0) return;
   const int tbx = (tile % tiles_x) * 4, tby = (tile / tiles_x) * 4;
   const int ox = tbx * 8, oy = tby * 8;
+  if (B.stamps) StampStart(&B.stamps->adj[1], blockIdx.x);
   const uint8_t a_own = TileAcs(P, B, tbx, tby);
 
   // 1. P ring (mirrored at the 8-padded image edge, as the Gaborish
@@ -452,6 +454,7 @@ __global__ void __launch_bounds__(256, 4)
       A.loss_part[tile] = (s_loss[0] + s_loss[1]) + (s_loss[2] + s_loss[3]);
     }
   }
+  if (B.stamps) StampEnd(B.stamps->end[1], blockIdx.x, gridDim.x);
 }
 
 // Sum of the per-tile loss partials in double (one workgroup).

@@ -24,8 +24,8 @@ using namespace pikgpu;
 
 namespace {
 
-// Kernel families timed by pikgpu_run (events ev[0..kNumRunTimers]), by
-// pikgpu_fwd_adj (adj_ev[0..2]) and by pikgpu_quantize (enc_ev[0..1]).
+// Kernel families timed by pikgpu_run, pikgpu_fwd_adj and pikgpu_quantize
+// (DeviceStamps).
 enum Timer {
   kTDc, kTLf, kTBlocks, kTMinMax, kTEpf, kTDots, kTFinal, kNumRunTimers,
   kTAdjForward = kNumRunTimers, kTAdjBackward, kTEncQuantize, kNumTimers
@@ -71,7 +71,6 @@ struct pikgpu_ctx {
   int global_scale = 0, quant_dc = 0;  // the uploaded frame's
   float dc_matrix0[3] = {0, 0, 0};     // DequantMatrix(0, DCT8, c)[0]
   bool adj_ready = false;  // LLF / LF caches hold the uploaded frame's
-  bool adj_timed = false;
   bool uploaded = false;
   bool ran = false;
   bool kept = false;
@@ -80,13 +79,15 @@ struct pikgpu_ctx {
   int ran_flags = 0;
   int out_xsize = 0, out_ysize = 0;  // output size of the last run
   bool ran_downsampled = false;
-  bool timed = false;   // the last run recorded timing events
   FrameParams P;
   FrameBuffers B;
   int num_tables = 0;
-  hipEvent_t ev[kNumRunTimers + 1] = {};
-  hipEvent_t adj_ev[3] = {};
-  hipEvent_t enc_ev[2] = {};
+  DeviceStamps* stamps = nullptr;  // behind consts, in its allocation
+  int clock_khz = 100000;  // of wall_clock64
+  // calls whose stamps pikgpu_last_timings has not read yet, and the families
+  // the last pikgpu_run had (others take no time)
+  bool run_due = false, adj_due = false, enc_due = false;
+  bool ran_guide = false, ran_epf = false, ran_dots = false;
   float timings[kNumTimers] = {};
   // Pinned host staging for strided host planes with short rows (packed
   // here, then one linear copy): [0, stage_used) may still be in flight
@@ -278,43 +279,41 @@ pikgpu_ctx* pikgpu_create(int device, const pikgpu_config* config) {
     delete ctx;
     return nullptr;
   }
-  for (int i = 0; i <= kNumRunTimers + 3; ++i) {
-    hipEvent_t* e = i <= kNumRunTimers ? &ctx->ev[i]
-                                       : &ctx->adj_ev[i - kNumRunTimers - 1];
-    if (hipEventCreate(e) != hipSuccess) {
-      delete ctx;
-      return nullptr;
-    }
-  }
-  for (hipEvent_t& e : ctx->enc_ev) {
-    if (hipEventCreate(&e) != hipSuccess) {
-      delete ctx;
-      return nullptr;
-    }
-  }
+  (void)hipDeviceGetAttribute(&ctx->clock_khz,
+                              hipDeviceAttributeWallClockRate, device);
   if (hipEventCreateWithFlags(&ctx->stage_ev, hipEventDisableTiming) !=
       hipSuccess) {
     delete ctx;
     return nullptr;
   }
-  // Constant tables.
-  DeviceConsts* h = new DeviceConsts;
-  memset(h, 0, sizeof(*h));
+  // Constant tables, and the timing stamps behind them (one allocation, one
+  // copy).
+  struct Tables {
+    DeviceConsts consts;
+    DeviceStamps stamps;
+  };
+  Tables* t = new Tables;
+  memset(t, 0, sizeof(*t));
+  DeviceConsts* h = &t->consts;
   FillScaleTables(&h->tscale[0][0][0], &h->ascale[0][0][0]);
   ComputeHostTables(&ctx->host);
   memcpy(h->mul_table, ctx->host.mul_table, sizeof(h->mul_table));
   OpsinInverse(h->opsin_inv);
   AdjointNorms(h->adj_norm);
   ComputeGrayXyb(&h->gray);
-  if (hipMalloc(&ctx->consts, sizeof(DeviceConsts)) != hipSuccess ||
-      hipMemcpy(ctx->consts, h, sizeof(DeviceConsts), hipMemcpyHostToDevice) !=
-          hipSuccess) {
-    delete h;
+  Tables* dev = nullptr;
+  const bool ok =
+      hipMalloc(&dev, sizeof(Tables)) == hipSuccess &&
+      hipMemcpy(dev, t, sizeof(Tables), hipMemcpyHostToDevice) == hipSuccess;
+  delete t;
+  if (!ok) {
+    if (dev) (void)hipFree(dev);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return nullptr;
   }
-  delete h;
+  ctx->consts = &dev->consts;
+  ctx->stamps = &dev->stamps;
   return ctx;
 }
 
@@ -325,15 +324,6 @@ void pikgpu_destroy(pikgpu_ctx* ctx) {
   FreeAll(ctx);
   pikgpu_parsed_free(ctx->parsed);
   if (ctx->consts) (void)hipFree(ctx->consts);
-  for (int i = 0; i <= kNumRunTimers; ++i) {
-    if (ctx->ev[i]) (void)hipEventDestroy(ctx->ev[i]);
-  }
-  for (hipEvent_t e : ctx->adj_ev) {
-    if (e) (void)hipEventDestroy(e);
-  }
-  for (hipEvent_t e : ctx->enc_ev) {
-    if (e) (void)hipEventDestroy(e);
-  }
   if (ctx->stage_ev) (void)hipEventDestroy(ctx->stage_ev);
   if (ctx->stage) (void)hipHostFree(ctx->stage);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -923,41 +913,25 @@ static void EnqueueLf(const FrameParams& P, const FrameBuffers& B,
 }
 
 // DC, LF predictions and the block kernel: everything before the pixel
-// filters (the same for full-size and downsampled runs). `ev` (may be
-// null) receives events 0..3 around the families.
+// filters (the same for full-size and downsampled runs).
 static hipError_t EnqueuePrefix(const FrameParams& P, const FrameBuffers& B,
-                                const DeviceConsts* K, hipStream_t st,
-                                const hipEvent_t* ev) {
-  hipError_t e = hipSuccess;
-#define REC(i) \
-  if (ev && (e = hipEventRecord(ev[i], st)) != hipSuccess) return e
-  REC(0);
+                                const DeviceConsts* K, hipStream_t st) {
   EnqueueDc(P, B, K, st);
-  REC(1);
   EnqueueLf(P, B, K, st, P.predict_hf != 0);
-  REC(2);
-  {
-    const int grid = XcdGrid(int(DivCeil(P.bx, 4) * DivCeil(P.by, 4)));
-    KBlocks<<<grid, 256, 0, st>>>(P, B, K);
-  }
-  REC(3);
-#undef REC
+  const int grid = XcdGrid(int(DivCeil(P.bx, 4) * DivCeil(P.by, 4)));
+  KBlocks<<<grid, 256, 0, st>>>(P, B, K);
   return hipGetLastError();
 }
 
 // The full-size reconstruction of a frame whose inputs are in device
 // memory (B): DC, predictions, IDCT, EPF + AR (or the plain copy without
 // AR), dots, Gaborish and OpsinToLinear into B.out; with B.keep the stage
-// copies for pikgpu_stage_dump. Allocates nothing. `ev` (may be null)
-// receives events 0..7 between the kernel families.
+// copies for pikgpu_stage_dump. Allocates nothing.
 hipError_t pikgpu::EnqueueFullSize(const FrameParams& P,
                                    const FrameBuffers& B,
-                                   const DeviceConsts* K, hipStream_t st,
-                                   const hipEvent_t* ev) {
-  hipError_t e = EnqueuePrefix(P, B, K, st, ev);
+                                   const DeviceConsts* K, hipStream_t st) {
+  hipError_t e = EnqueuePrefix(P, B, K, st);
   if (e != hipSuccess) return e;
-#define REC(i) \
-  if (ev && (e = hipEventRecord(ev[i], st)) != hipSuccess) return e
 #define TRY(expr) \
   if ((e = (expr)) != hipSuccess) return e
   const size_t iplane = size_t(B.ipitch) * P.py;
@@ -967,20 +941,16 @@ hipError_t pikgpu::EnqueueFullSize(const FrameParams& P,
     // the IDCT image: width a multiple of 8, rows 32-float aligned
     const dim3 mmg = MinMaxGrid4(ii.W, ii.H);
     const int partials = int(mmg.x * mmg.y);
-    KMinMaxPartial4<<<mmg, 256, 0, st>>>(ii, gab, P, B.mm_partial);
+    KMinMaxPartial4<<<mmg, 256, 0, st>>>(ii, gab, P, B);
     if (MinMaxInline(partials) == 0) {
       KMinMaxFinal<<<1, 256, 0, st>>>(B.mm_partial, partials, B.mm);
     }
     const int grid = XcdGrid(int(DivCeil(P.px, 32) * DivCeil(P.py, 32)));
     KGuide<<<grid, 256, 0, st>>>(ii, gab, P, B, MinMaxInline(partials));
-    REC(4);
     KEpf<false><<<grid, 256, 0, st>>>(ii, P, B, K, 0, B.ar, B.ipitch, iplane);
   } else {
-    REC(4);
-    KCopyPlanes<<<DivCeil(3 * iplane, 256), 256, 0, st>>>(B.idct, B.ar,
-                                                          3 * iplane);
+    KCopyPlanes<<<DivCeil(3 * iplane, 256), 256, 0, st>>>(B, 3 * iplane);
   }
-  REC(5);
   if (B.keep) {
     if (!P.ar) {
       TRY(hipMemcpyAsync(B.guide, B.idct, 3 * iplane * 4,
@@ -993,23 +963,20 @@ hipError_t pikgpu::EnqueueFullSize(const FrameParams& P,
                        hipMemcpyDeviceToDevice, st));
   }
   if (P.dot_tiles) KDots<<<P.dot_tiles, 256, 0, st>>>(P, B);
-  REC(6);
   {
     const int grid =
         XcdGrid(int(DivCeil(P.px, 256) * DivCeil(P.py, kFinalRows)));
     KFinal<<<grid, 256, 0, st>>>(P, B, K);
   }
-  REC(7);
-#undef REC
 #undef TRY
   return hipGetLastError();
 }
 
 // Enqueues the whole reconstruction of the uploaded frame on stream `st`.
-// With `timing`, HIP events between the kernel families record their
-// durations (pikgpu_last_timings). Allocates nothing unless stage dumps or
-// the 8-bit output need buffers that do not exist yet, so a batch can
-// capture it into a graph.
+// With `timing` the kernel families leave their start times
+// (pikgpu_last_timings). Allocates nothing unless stage dumps or the 8-bit
+// output need buffers that do not exist yet, so a batch can capture it into
+// a graph.
 static int Enqueue(pikgpu_ctx* ctx, hipStream_t st, bool keep_stages,
                    bool timing) {
   int rc;
@@ -1038,16 +1005,19 @@ static int Enqueue(pikgpu_ctx* ctx, hipStream_t st, bool keep_stages,
     B.srgb8 = static_cast<uint8_t*>(ctx->srgb8.p);
   }
   const DeviceConsts* K = ctx->consts;
-  const hipEvent_t* ev = timing ? ctx->ev : nullptr;
+  if (timing) {
+    B.stamps = ctx->stamps;
+    ctx->run_due = true;
+    ctx->ran_guide = ds == 1 && P.ar;
+    ctx->ran_epf = ds == 1;
+    ctx->ran_dots = ds == 1 && P.dot_tiles > 0;
+  }
 
   if (ds != 1) {
-    HIP_TRY(ctx, EnqueuePrefix(P, B, K, st, ev));
+    HIP_TRY(ctx, EnqueuePrefix(P, B, K, st));
     // The downsampled branch of FinalizeFrameDecoding: KBlocks wrote the
     // averaged image into B.idct (planes of (py / ds) x ipitch); no AR, no
     // Gaborish, no dots; ShrinkTo and OpsinToLinear in KFinal.
-    if (timing) {
-      for (int e = 4; e <= 6; ++e) HIP_TRY(ctx, hipEventRecord(ctx->ev[e], st));
-    }
     FrameParams Pd = P;
     Pd.px = P.px / ds;
     Pd.py = P.py / ds;
@@ -1059,10 +1029,9 @@ static int Enqueue(pikgpu_ctx* ctx, hipStream_t st, bool keep_stages,
     const int grid =
         XcdGrid(int(DivCeil(Pd.px, 256) * DivCeil(Pd.py, kFinalRows)));
     KFinal<<<grid, 256, 0, st>>>(Pd, Bd, K);
-    if (timing) HIP_TRY(ctx, hipEventRecord(ctx->ev[7], st));
     HIP_TRY(ctx, hipGetLastError());
   } else {
-    HIP_TRY(ctx, EnqueueFullSize(P, B, K, st, ev));
+    HIP_TRY(ctx, EnqueueFullSize(P, B, K, st));
   }
   ctx->ran = true;
   ctx->kept = B.keep;
@@ -1121,7 +1090,6 @@ int pikgpu_run(pikgpu_ctx* ctx, int keep_stages) {
   if (ctx == nullptr) return PIKGPU_EINVAL;
   if (!ctx->uploaded) return Fail(ctx, PIKGPU_ESTATE, "no frame uploaded");
   HIP_TRY(ctx, hipSetDevice(ctx->device));
-  ctx->timed = true;
   return Enqueue(ctx, ctx->stream, keep_stages != 0, true);
 }
 
@@ -1129,24 +1097,6 @@ int pikgpu_sync(pikgpu_ctx* ctx) {
   if (ctx == nullptr) return PIKGPU_EINVAL;
   HIP_TRY(ctx, hipSetDevice(ctx->device));
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-  if (ctx->adj_timed) {
-    for (int i = 0; i < 2; ++i) {
-      float ms = 0.0f;
-      if (hipEventElapsedTime(&ms, ctx->adj_ev[i], ctx->adj_ev[i + 1]) ==
-          hipSuccess) {
-        ctx->timings[kTAdjForward + i] = ms;
-      }
-    }
-    ctx->adj_timed = false;
-  }
-  if (ctx->ran && ctx->timed) {
-    for (int i = 0; i < kNumRunTimers; ++i) {
-      float ms = 0.0f;
-      if (hipEventElapsedTime(&ms, ctx->ev[i], ctx->ev[i + 1]) == hipSuccess) {
-        ctx->timings[i] = ms;
-      }
-    }
-  }
   return PIKGPU_OK;
 }
 
@@ -1316,8 +1266,10 @@ int pikgpu_quantize(pikgpu_ctx* ctx, const float* const opsin[3],
   int16_t* ac16 = static_cast<int16_t*>(ctx->ac.p);
   int16_t* dc16 = static_cast<int16_t*>(ctx->dc16.p);
   const int tiles = int(DivCeil(P.bx, 4) * DivCeil(P.by, 4));
-  HIP_TRY(ctx, hipEventRecord(ctx->enc_ev[0], st));
-  KEncForward<<<tiles, 256, 0, st>>>(P, B, K, dev_opsin, coef, dcf);
+  FrameBuffers Bt = B;  // with the timing stamps
+  Bt.stamps = ctx->stamps;
+  ctx->enc_due = true;
+  KEncForward<<<tiles, 256, 0, st>>>(P, Bt, K, dev_opsin, coef, dcf);
   // Quantizer::QuantizeDC's factors (float arithmetic as the reference's)
   const float gsf = static_cast<float>(ctx->global_scale * (1.0 / 65536));
   const float qdc = gsf * ctx->quant_dc;
@@ -1355,9 +1307,8 @@ int pikgpu_quantize(pikgpu_ctx* ctx, const float* const opsin[3],
       KEncHfResidual<<<XcdGrid(tiles), 256, 0, st>>>(P, B, coef);
     }
   }
-  KEncQuant<<<XcdGrid(tiles), 256, 0, st>>>(P, B, coef, itable, gsf, ac16);
+  KEncQuant<<<XcdGrid(tiles), 256, 0, st>>>(P, Bt, coef, itable, gsf, ac16);
   HIP_TRY(ctx, hipGetLastError());
-  HIP_TRY(ctx, hipEventRecord(ctx->enc_ev[1], st));
   for (int c = 0; c < 3; ++c) {
     if (ac_out) {
       HIP_TRY(ctx, Copy2D(ac_out[c], ac_stride * 2,
@@ -1371,10 +1322,6 @@ int pikgpu_quantize(pikgpu_ctx* ctx, const float* const opsin[3],
     }
   }
   HIP_TRY(ctx, hipStreamSynchronize(st));
-  float ms = 0.0f;
-  if (hipEventElapsedTime(&ms, ctx->enc_ev[0], ctx->enc_ev[1]) == hipSuccess) {
-    ctx->timings[kTEncQuantize] = ms;
-  }
   return PIKGPU_OK;
 }
 
@@ -1507,6 +1454,38 @@ int pikgpu_stage_dump(pikgpu_ctx* ctx, int stage, float* planes[3],
 int pikgpu_last_timings(pikgpu_ctx* ctx, const char** names, float* ms,
                         int max_entries) {
   if (ctx == nullptr) return PIKGPU_EINVAL;
+  if (ctx->run_due || ctx->adj_due || ctx->enc_due) {
+    // every clock value of the calls since the last look, once the stream
+    // has passed them
+    std::vector<DeviceStamps> h(1);
+    HIP_TRY(ctx, hipSetDevice(ctx->device));
+    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    HIP_TRY(ctx, hipMemcpy(h.data(), ctx->stamps, sizeof(DeviceStamps),
+                           hipMemcpyDeviceToHost));
+    DeviceStamps& S = h[0];
+    const auto ms_between = [&](unsigned long long a, unsigned long long b) {
+      return b > a ? float(double(b - a) / ctx->clock_khz) : 0.0f;
+    };
+    const auto end = [&](int k) {
+      return *std::max_element(S.end[k], S.end[k] + kEndStamps);
+    };
+    if (ctx->run_due) {
+      // a family that did not run ends where it starts
+      if (!ctx->ran_dots) S.run[kTDots] = S.run[kTFinal];
+      if (!ctx->ran_epf) S.run[kTEpf] = S.run[kTDots];
+      if (!ctx->ran_guide) S.run[kTMinMax] = S.run[kTEpf];
+      for (int i = 0; i < kNumRunTimers; ++i) {
+        ctx->timings[i] = ms_between(
+            S.run[i], i + 1 < kNumRunTimers ? S.run[i + 1] : end(0));
+      }
+    }
+    if (ctx->adj_due) {
+      ctx->timings[kTAdjForward] = ms_between(S.adj[0], S.adj[1]);
+      ctx->timings[kTAdjBackward] = ms_between(S.adj[1], end(1));
+    }
+    if (ctx->enc_due) ctx->timings[kTEncQuantize] = ms_between(S.enc, end(2));
+    ctx->run_due = ctx->adj_due = ctx->enc_due = false;
+  }
   int n = 0;
   for (int i = 0; i < kNumTimers && n < max_entries; ++i, ++n) {
     if (names) names[n] = kTimerNames[i];
@@ -1654,14 +1633,12 @@ int pikgpu_fwd_adj(pikgpu_ctx* ctx, const pikgpu_adj_io* io) {
     ctx->adj_ready = true;
   }
   const int grid = XcdGrid(tiles);
-  HIP_TRY(ctx, hipEventRecord(ctx->adj_ev[0], st));
+  B.stamps = ctx->stamps;
+  ctx->adj_due = true;
   KAdjForward<<<grid, 256, 0, st>>>(P, B, K, A);
-  HIP_TRY(ctx, hipEventRecord(ctx->adj_ev[1], st));
   KAdjBackward<<<grid, 256, 0, st>>>(P, B, K, A);
-  HIP_TRY(ctx, hipEventRecord(ctx->adj_ev[2], st));
   if (io->loss) KAdjLoss<<<1, 256, 0, st>>>(loss_part, tiles, loss_dev);
   HIP_TRY(ctx, hipGetLastError());
-  ctx->adj_timed = true;
   // pikgpu_run's output is not what the device buffers hold any more.
   ctx->ran = false;
   if (dev) {
@@ -2198,7 +2175,7 @@ int BuildQueueGraph(pikgpu_batch* b) {
     c->out_xsize = int(c->P.xsize);
     c->out_ysize = int(c->P.ysize);
     c->ran_downsampled = false;
-    c->timed = false;
+    c->run_due = false;
   }
   return PIKGPU_OK;
 }

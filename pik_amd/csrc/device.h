@@ -25,6 +25,8 @@ constexpr int kG2Pitch = 2 * (kGroupDimBlocks + 2);  // 132
 constexpr int kLlfPlane = kLlfPitch * kLlfPitch;
 constexpr int kG2Plane = kG2Pitch * kG2Pitch;
 
+struct DeviceStamps;
+
 // Device pointers and sizes of one frame.
 struct FrameBuffers {
   // inputs
@@ -81,6 +83,21 @@ struct FrameBuffers {
   int opitch;             // floats per row of out (dense: its width)
   int spitch;             // bytes per row of srgb8 (dense: 3 x its width)
   int keep;               // write stage dumps
+  DeviceStamps* stamps;  // device clock per kernel family, or null
+};
+
+// Device clock (wall_clock64) at the start of each kernel family and at the
+// end of the last workgroups of the last one: what pikgpu_last_timings
+// reports, without an event between two kernels (each took 5 to 10 us of the
+// stream, up to 40 us of a decode). Starts are written by a launch's first
+// workgroup; ends by its last kEndStamps ones, a slot each, of which the host
+// takes the latest.
+constexpr int kEndStamps = 512;
+struct DeviceStamps {
+  unsigned long long run[7];       // dc, lf, blocks, guide, epf, dots, final
+  unsigned long long adj[2];       // forward, backward
+  unsigned long long enc;          // quantize
+  unsigned long long end[3][kEndStamps];  // of run, adj, enc
 };
 
 // Inputs and outputs of one forward + adjoint evaluation (device memory).

@@ -39,6 +39,7 @@ __global__ void __launch_bounds__(256)
   __shared__ float s_coef[3][kCoefPlane];
   __shared__ uint8_t s_acs[16];
   __shared__ TileTasks s_tasks;
+  if (B.stamps) StampStart(&B.stamps->enc, blockIdx.x);
   const int tiles_x = (P.bx + 3) / 4;
   const int tx4 = blockIdx.x % tiles_x, ty4 = blockIdx.x / tiles_x;
   const size_t plane = size_t(P.px) * P.py;
@@ -327,6 +328,7 @@ __global__ void __launch_bounds__(256)
       *reinterpret_cast<short4*>(ac + 2 * h * plane + at) = q;
     }
   }
+  if (B.stamps) StampEnd(B.stamps->end[2], blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------

@@ -143,8 +143,11 @@ __device__ inline uint32_t LdsDword(const uint8_t* p) {
 // operation order, pik/convolve.h:605-621), the next row loaded one
 // iteration ahead.
 __device__ __forceinline__ void KMinMaxPartial4Body(
-    Img in, int gaborish, FrameParams P, float* partial, const VBlock& vb) {
+    Img in, int gaborish, const FrameParams& P, const FrameBuffers& B,
+    const VBlock& vb) {
   __shared__ float s_mm[8];
+  float* partial = B.mm_partial;
+  if (B.stamps) StampStart(&B.stamps->run[3], vb.x + vb.y);
   const int tid = threadIdx.x;
   const int x = (vb.x * 256 + tid) * 4;
   const int rows = (in.H + vb.ny - 1) / vb.ny;
@@ -223,8 +226,8 @@ __device__ __forceinline__ void KMinMaxPartial4Body(
   }
 }
 __global__ void __launch_bounds__(256)
-    KMinMaxPartial4(Img in, int gaborish, FrameParams P, float* partial) {
-  KMinMaxPartial4Body(in, gaborish, P, partial, PlainBlock());
+    KMinMaxPartial4(Img in, int gaborish, FrameParams P, FrameBuffers B) {
+  KMinMaxPartial4Body(in, gaborish, P, B, PlainBlock());
 }
 
 // The guide's scaling from n partials: the minimum over channels and 255 /
@@ -497,6 +500,7 @@ __device__ __forceinline__ void KEpfBody(
   const int tile = XcdTile(vb.x, tiles_x * ((in.H + 31) / 32));
   if (tile < 0) return;
   const int x0 = (tile % tiles_x) * 32, y0 = (tile / tiles_x) * 32;
+  if (!kDc && B.stamps) StampStart(&B.stamps->run[4], vb.x);
   // the DC mode reduces KDcDequant's min/max partials itself (at most
   // kDcGroups of them), the image mode reads what KGuide's input was
   // scaled by
@@ -943,6 +947,7 @@ __global__ void __launch_bounds__(256, kDc ? 3 : 4)
 __device__ __forceinline__ void KDotsBody(
     FrameParams P, FrameBuffers B, const VBlock& vb) {
   __shared__ float s_blk[3][21 * 21];
+  if (B.stamps) StampStart(&B.stamps->run[5], vb.x);
   const int tid = threadIdx.x;
   const int tile = B.dot_tile_ids[vb.x];
   const int tx0 = (tile % P.dot_tiles_x) * 32, ty0 = (tile / P.dot_tiles_x) * 32;
@@ -1079,6 +1084,7 @@ __device__ __forceinline__ void KFinalBody(
   const int tile =
       XcdTile(vb.x, strips * ((P.py + kFinalRows - 1) / kFinalRows));
   if (tile < 0) return;
+  if (B.stamps) StampStart(&B.stamps->run[6], vb.x);
   const int x = (tile % strips) * 256 + threadIdx.x;
   const int ya = (tile / strips) * kFinalRows;
   const int yb = min(P.py, ya + kFinalRows);
@@ -1212,20 +1218,23 @@ __device__ __forceinline__ void KFinalBody(
       }
     }
   }
+  if (B.stamps) StampEnd(B.stamps->end[0], vb.x, vb.nx);
 }
 __global__ void __launch_bounds__(256)
     KFinal(FrameParams P, FrameBuffers B, const DeviceConsts* K) {
   KFinalBody(P, B, K, PlainBlock());
 }
 
-__device__ __forceinline__ void KCopyPlanesBody(
-    const float* src, float* dst, size_t n, const VBlock& vb) {
+// The IDCT image as the AR output (frames without adaptive
+// reconstruction).
+__device__ __forceinline__ void KCopyPlanesBody(const FrameBuffers& B,
+                                                size_t n, const VBlock& vb) {
+  if (B.stamps) StampStart(&B.stamps->run[4], vb.x);
   const size_t i = size_t(vb.x) * 256 + threadIdx.x;
-  if (i < n) dst[i] = src[i];
+  if (i < n) B.ar[i] = B.idct[i];
 }
-__global__ void __launch_bounds__(256)
-    KCopyPlanes(const float* src, float* dst, size_t n) {
-  KCopyPlanesBody(src, dst, n, PlainBlock());
+__global__ void __launch_bounds__(256) KCopyPlanes(FrameBuffers B, size_t n) {
+  KCopyPlanesBody(B, n, PlainBlock());
 }
 
 template __global__ void KEpf<true>(Img, FrameParams, FrameBuffers,
@@ -1240,8 +1249,7 @@ template __global__ void KEpf<false>(Img, FrameParams, FrameBuffers,
 // frame's images and buffers as the plain launches of pikgpu_run take them.
 __global__ void __launch_bounds__(256)
     KMinMaxPartial4Batch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_LOOP(KMinMaxPartial4Body(IdctImage(P, B), s.arg[0], P,
-                                        B.mm_partial, vb));
+  PIKGPU_BATCH_LOOP(KMinMaxPartial4Body(IdctImage(P, B), s.arg[0], P, B, vb));
 }
 __global__ void __launch_bounds__(256) KMinMaxFinalBatch(PIKGPU_BATCH_PARAMS) {
   PIKGPU_BATCH_LOOP(KMinMaxFinalBody(B.mm_partial, s.arg[0], B.mm, vb));
@@ -1258,8 +1266,7 @@ __global__ void __launch_bounds__(256, 4) KEpfBatch(PIKGPU_BATCH_PARAMS) {
                                     B.ipitch, size_t(B.ipitch) * P.py, vb));
 }
 __global__ void __launch_bounds__(256) KCopyPlanesBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_LOOP(KCopyPlanesBody(B.idct, B.ar, 3 * size_t(B.ipitch) * P.py,
-                                    vb));
+  PIKGPU_BATCH_LOOP(KCopyPlanesBody(B, 3 * size_t(B.ipitch) * P.py, vb));
 }
 __global__ void __launch_bounds__(256) KDotsBatch(PIKGPU_BATCH_PARAMS) {
   PIKGPU_BATCH_LOOP(KDotsBody(P, B, vb));

@@ -56,10 +56,8 @@ hipError_t Copy2D(void* dst, size_t dpitch, const void* src, size_t spitch,
                   hipStream_t stream);
 
 // The full-size reconstruction of a frame whose inputs are in device memory
-// (B), asynchronous on `st`; allocates nothing. `ev` (may be null) receives
-// events 0..7 between the kernel families.
+// (B), asynchronous on `st`; allocates nothing.
 hipError_t EnqueueFullSize(const FrameParams& P, const FrameBuffers& B,
-                           const DeviceConsts* K, hipStream_t st,
-                           const hipEvent_t* ev);
+                           const DeviceConsts* K, hipStream_t st);
 
 }  // namespace pikgpu

@@ -182,6 +182,16 @@ __device__ inline float DequantPasses(const FrameParams& P,
   return acc;
 }
 
+// Thread 0 of workgroup wg of n: the launch's start, its end.
+__device__ inline void StampStart(unsigned long long* at, int wg) {
+  if (wg == 0 && threadIdx.x == 0) *at = wall_clock64();
+}
+__device__ inline void StampEnd(unsigned long long* at, int wg, int n) {
+  if (wg >= n - kEndStamps && threadIdx.x == 0) {
+    at[wg % kEndStamps] = wall_clock64();
+  }
+}
+
 // Minimum and maximum over the workgroup's 256 threads, in every thread; s
 // holds 8 floats of LDS that nothing else uses meanwhile. All threads call.
 __device__ inline void GroupMinMax(float* lo, float* hi, float* s) {
@@ -897,7 +907,7 @@ __host__ __device__ inline Img DcImage(const FrameParams& P,
 }
 
 __global__ void KMinMaxPartial4(Img in, int gaborish, FrameParams P,
-                               float* partial);
+                                FrameBuffers B);
 __global__ void KMinMaxFinal(const float* partial, int n, float* mm);
 template <bool kDc>
 __global__ void KEpf(Img in, FrameParams P, FrameBuffers B,
@@ -909,7 +919,7 @@ __global__ void KDots(FrameParams P, FrameBuffers B);
 // KFinal: rows per workgroup of its 256-column strips.
 constexpr int kFinalRows = 16;
 __global__ void KFinal(FrameParams P, FrameBuffers B, const DeviceConsts* K);
-__global__ void KCopyPlanes(const float* src, float* dst, size_t n);
+__global__ void KCopyPlanes(FrameBuffers B, size_t n);
 
 // Batched forms of the reconstruction's kernels (pikgpu_batch): one launch
 // per phase over every frame of a batch; see BatchSpan.

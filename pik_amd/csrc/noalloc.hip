@@ -249,7 +249,7 @@ int NoAllocRun(const pikgpu_frame* f, float* const out_planes[3],
     const size_t n = size_t(P.gx) * P.gy * 3 * kG2Plane;
     KFillZero<<<DivCeil(n, 256), 256, 0, st>>>(B.pred2x2, n);
   }
-  TRY(EnqueueFullSize(P, B, K, st, nullptr));
+  TRY(EnqueueFullSize(P, B, K, st));
   const size_t oplane = size_t(B.opitch) * P.ysize;
   for (int c = 0; c < 3; ++c) {
     TRY(Copy2D(out_planes[c], out_stride_bytes, B.out + c * oplane,

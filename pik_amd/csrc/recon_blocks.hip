@@ -30,6 +30,7 @@ __device__ __forceinline__ void KBlocksBody(
   const int tiles_x = (P.bx + 3) / 4;
   const int tile = XcdTile(vb.x, tiles_x * ((P.by + 3) / 4));
   if (tile < 0) return;
+  if (B.stamps) StampStart(&B.stamps->run[2], vb.x);
   const int tbx = (tile % tiles_x) * 4, tby = (tile / tiles_x) * 4;  // blocks
   // pred2x2 window of the tile's HF prediction, 10 x 10 values per channel
   // (the tile's 8 x 8 plus the blur's one-value ring). It lives in the

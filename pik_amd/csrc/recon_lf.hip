@@ -29,6 +29,7 @@ namespace pikgpu {
 __device__ __forceinline__ void KDcDequantBody(
     const FrameParams& P, const FrameBuffers& B, const VBlock& vb) {
   __shared__ float s_mm[8];
+  if (B.stamps) StampStart(&B.stamps->run[0], vb.x);
   const int n = P.bx * P.by;
   float lo = FLT_MAX, hi = -FLT_MAX;
   for (int i = vb.x * 256 + int(threadIdx.x); i < n; i += vb.nx * 256) {
@@ -329,6 +330,7 @@ __device__ __forceinline__ void KLfBody(const FrameParams& P,
   const int tid = threadIdx.x;
   const int g = vb.x / kLfStrips, k = vb.x % kLfStrips, c = vb.y;
   const GroupGeom G = Geom(P, g);
+  if (B.stamps) StampStart(&B.stamps->run[1], vb.x + c);
   if (k * kLfStrip >= G.gh) return;
   const int W = G.gw + 2, H = G.gh + 2;
   const bool lf = P.predict_lf != 0;
