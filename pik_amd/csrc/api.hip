@@ -56,7 +56,7 @@ struct pikgpu_ctx {
   DevBuf ac, dc16, qf, acs, lut, dcf, ytox, ytob, dqmap, table, offsets, dots,
       dotbins, ac_extra;
   DevBuf desc, dcq, dcv, llf, lf2x2, pred2x2, coeffs, idct, guide, epf, ar,
-      dots_img, gab, out, mm_partial, mm, ar_keep, srgb8, gimg, predlist;
+      dots_img, gab, out, mm_partial, mm, ar_keep, srgb8, gimg;
   // pikgpu_fwd_adj staging (host-pointer calls) and loss partials
   DevBuf adj_qf, adj_in, adj_lin, adj_dqf, adj_dc, adj_loss;
   // pikgpu_quantize: XYB input, coefficients, DC, the inverse dequant table
@@ -138,7 +138,7 @@ void FreeAll(pikgpu_ctx* ctx) {
                    &ctx->lf2x2,   &ctx->pred2x2, &ctx->coeffs, &ctx->idct,
                    &ctx->guide,   &ctx->epf,    &ctx->ar,      &ctx->dots_img,
                    &ctx->gab,     &ctx->out,    &ctx->mm_partial, &ctx->mm,
-                   &ctx->ar_keep, &ctx->gimg,   &ctx->predlist, &ctx->adj_qf, &ctx->adj_in, &ctx->adj_lin,
+                   &ctx->ar_keep, &ctx->gimg, &ctx->adj_qf, &ctx->adj_in, &ctx->adj_lin,
                    &ctx->adj_dqf, &ctx->adj_dc, &ctx->adj_loss,
                    &ctx->eopsin, &ctx->ecoef, &ctx->edcf, &ctx->itable,
                    &ctx->ecorner,
@@ -522,32 +522,6 @@ void FillParams(const pikgpu_frame* f, FrameParams* Pp) {
   P.neg_bias[2] = -ToF(0.14255999980363571 / kScale);
 }
 
-// First blocks grouped by the class of their pred2x2 computation
-// (KPred2x2Interior): DCT8-like, 2x2 Hadamard, DCT16, DCT32; `end` receives
-// the end of each class in `list`.
-void PredClasses(const pikgpu_frame* f, std::vector<uint32_t>* list,
-                 int end[4]) {
-  const size_t bx = DivCeil(f->xsize, 8), by = DivCeil(f->ysize, 8);
-  std::vector<uint32_t> plist[4];
-  for (size_t y = 0; y < by; ++y) {
-    const uint8_t* row = f->ac_strategy + y * f->ac_strategy_stride;
-    for (size_t x = 0; x < bx; ++x) {
-      if ((row[x] & 15) != 0) continue;
-      const int raw = row[x] >> 4;
-      const int cls = raw == kDCT16 ? 2
-                      : raw == kDCT32 ? 3
-                      : (raw == kDCT || raw == kDCTNoHF || raw == kLines) ? 0
-                                                                           : 1;
-      plist[cls].push_back(uint32_t(y * bx + x));
-    }
-  }
-  list->clear();
-  for (int k = 0; k < 4; ++k) {
-    list->insert(list->end(), plist[k].begin(), plist[k].end());
-    end[k] = int(list->size());
-  }
-}
-
 // Bins the dots into 32x32 tiles of the padded image. Every dot goes to
 // each tile its footprint may touch (transformed dots: the bounding box of
 // the splat's four corners, widened by two pixels), and each tile's list
@@ -778,9 +752,6 @@ int pikgpu_frame_upload(pikgpu_ctx* ctx, const pikgpu_frame* f) {
                                 dot_list.data(), dot_list.size() * 4,
                                 hipMemcpyHostToDevice, ctx->stream));
   }
-  std::vector<uint32_t> pred_list;
-  int pred_end[4];
-  PredClasses(f, &pred_list, pred_end);
   ctx->has_lines = false;
   for (size_t y = 0; y < by && !ctx->has_lines; ++y) {
     for (size_t x = 0; x < bx; ++x) {
@@ -790,10 +761,6 @@ int pikgpu_frame_upload(pikgpu_ctx* ctx, const pikgpu_frame* f) {
       }
     }
   }
-  if ((rc = Grow(ctx, &ctx->predlist, pred_list.size() * 4))) return rc;
-  HIP_TRY(ctx, hipMemcpyAsync(ctx->predlist.p, pred_list.data(),
-                              pred_list.size() * 4, hipMemcpyHostToDevice,
-                              ctx->stream));
   // pred2x2 positions that no block writes (ZeroFillImage,
   // pik/compressed_image.cc:976): the same ones on every run of this frame,
   // so once here rather than per run
@@ -817,8 +784,6 @@ int pikgpu_frame_upload(pikgpu_ctx* ctx, const pikgpu_frame* f) {
   B.offsets = static_cast<const uint32_t*>(ctx->offsets.p);
   B.num_tables = num_tables;
   B.dots = static_cast<const pikgpu_dot*>(ctx->dots.p);
-  B.pred_list = static_cast<const uint32_t*>(ctx->predlist.p);
-  for (int k = 0; k < 4; ++k) P.pred_end[k] = pred_end[k];
   P.dot_tiles = int(dot_ids.size());
   P.dot_tiles_x = int(DivCeil(bx * 8, 32));
   if (P.dot_tiles) {
@@ -893,23 +858,12 @@ static void EnqueueDc(const FrameParams& P, const FrameBuffers& B,
                                    size_t(nblk));
 }
 
-// LF-domain predictions per group: LLF, LF predictions (predict_lf) and,
-// with `hf`, the pred2x2 image of the HF prediction (`border`: only its
-// border, for the encoder, which forms the interior itself).
+// LF-domain predictions per group: LLF, LF predictions (predict_lf) and with
+// `border` the border of the HF prediction's pred2x2 image.
 static void EnqueueLf(const FrameParams& P, const FrameBuffers& B,
-                      const DeviceConsts* K, hipStream_t st, bool hf,
-                      bool border = false) {
-  // (positions of pred2x2 no block writes were zeroed at upload)
-  KLf<<<dim3(P.gx * P.gy * kLfStrips, 3), kLfThreads, 0, st>>>(P, B, K, hf || border);
-  if (hf && P.pred_end[3] > 0) {
-    // DCT32 / DCT16 first blocks on 8 / 4 lanes (32 / 64 units of block x
-    // plane per workgroup), then one lane per unit
-    const int wg4 = int(DivCeil(3 * (P.pred_end[3] - P.pred_end[2]), 32));
-    const int wg2 = int(DivCeil(3 * (P.pred_end[2] - P.pred_end[1]), 64));
-    const int wg1 = int(DivCeil(3 * P.pred_end[1], 256));
-    KPred2x2Interior<false><<<wg4 + wg2 + wg1, 256, 0, st>>>(P, B, K, wg4,
-                                                             wg2, nullptr);
-  }
+                      const DeviceConsts* K, hipStream_t st, bool border) {
+  KLf<<<dim3(P.gx * P.gy * kLfStrips, 3), kLfThreads, 0, st>>>(P, B, K,
+                                                               border);
 }
 
 // DC, LF predictions and the block kernel: everything before the pixel
@@ -918,6 +872,9 @@ static hipError_t EnqueuePrefix(const FrameParams& P, const FrameBuffers& B,
                                 const DeviceConsts* K, hipStream_t st) {
   EnqueueDc(P, B, K, st);
   EnqueueLf(P, B, K, st, P.predict_hf != 0);
+  if (P.predict_hf) {
+    KPred2x2<false><<<PredGrid(P.gx * P.gy), 256, 0, st>>>(P, B, K, nullptr);
+  }
   const int grid = XcdGrid(int(DivCeil(P.bx, 4) * DivCeil(P.by, 4)));
   KBlocks<<<grid, 256, 0, st>>>(P, B, K);
   return hipGetLastError();
@@ -1282,7 +1239,7 @@ int pikgpu_quantize(pikgpu_ctx* ctx, const float* const opsin[3],
   // dc_dec, the LLF and the LF prediction exactly as the decoder computes
   // them (the encoder calls the same ComputeLlf and PredictLf)
   EnqueueDc(P, B, K, st);
-  EnqueueLf(P, B, K, st, false, P.predict_lf && P.predict_hf);
+  EnqueueLf(P, B, K, st, P.predict_lf && P.predict_hf);
   const float* itable = static_cast<const float*>(ctx->itable.p);
   if (predict) {
     float* corner = static_cast<float*>(ctx->ecorner.p);
@@ -1297,13 +1254,7 @@ int pikgpu_quantize(pikgpu_ctx* ctx, const float* const opsin[3],
         KEncPred2x2Border<<<dim3(DivCeil(cache_pos, 256), P.gx * P.gy, 3), 256,
                             0, st>>>(P, B, K);
       }
-      if (P.pred_end[3] > 0) {
-        const int wg4 = int(DivCeil(3 * (P.pred_end[3] - P.pred_end[2]), 32));
-        const int wg2 = int(DivCeil(3 * (P.pred_end[2] - P.pred_end[1]), 64));
-        const int wg1 = int(DivCeil(3 * P.pred_end[1], 256));
-        KPred2x2Interior<true><<<wg4 + wg2 + wg1, 256, 0, st>>>(
-            P, B, K, wg4, wg2, corner);
-      }
+      KPred2x2<true><<<PredGrid(P.gx * P.gy), 256, 0, st>>>(P, B, K, corner);
       KEncHfResidual<<<XcdGrid(tiles), 256, 0, st>>>(P, B, coef);
     }
   }
@@ -1913,20 +1864,20 @@ struct BatchPhaseDef {
 };
 const BatchPhaseDef kBatchPhases[PIKGPU_BATCH_PHASES] = {
     {"dc_dequant", KDcDequantBatch, true},
-    {"dc_minmax", nullptr, true},        // in dc_dequant
-    {"dc_minmax_final", nullptr, true},  // in dc_epf
+    {"dc_minmax", nullptr, false},        // in dc_dequant
+    {"dc_minmax_final", nullptr, false},  // in dc_epf
     {"dc_epf", KEpfDcBatch, false},
-    {"llf", KLfBatch, true, kLfThreads},
-    {"lf_blur", nullptr, true},          // in llf
-    {"lf_from_dc2x2", nullptr, true},    // in llf
-    {"pred2x2_border", nullptr, true},   // in llf
-    {"dc2x2_border", nullptr, true},     // in llf
-    {"pred2x2_interior", KPred2x2InteriorBatch, false},
+    {"llf", KLfBatch, false, kLfThreads},
+    {"lf_blur", nullptr, false},          // in llf
+    {"lf_from_dc2x2", nullptr, false},    // in llf
+    {"pred2x2_border", nullptr, false},   // in llf
+    {"dc2x2_border", nullptr, false},     // in llf
+    {"pred2x2_interior", KPred2x2Batch, false},
     {"blocks", KBlocksBatch, false},
     {"minmax", KMinMaxPartial4Batch, true},
     {"minmax_final", KMinMaxFinalBatch, true},
     {"guide", KGuideBatch, false},
-    {"guide_ring", nullptr, true},       // in guide
+    {"guide_ring", nullptr, false},       // in guide
     {"epf", KEpfBatch, false},
     {"copy_planes", KCopyPlanesBatch, true},
     {"dots", KDotsBatch, true},
@@ -1993,11 +1944,8 @@ bool PhaseGrid(int p, const FrameParams& P, const FrameBuffers& B, int* nx,
                int* ny, int* nz, int* arg) {
   *nx = *ny = *nz = 1;
   const int nblk = P.bx * P.by;
-  const int wg4 = int(DivCeil(3 * (P.pred_end[3] - P.pred_end[2]), 32));
-  const int wg2 = int(DivCeil(3 * (P.pred_end[2] - P.pred_end[1]), 64));
   const Img dci = DcImage(P, B);
   const Img ii = IdctImage(P, B);
-  const bool hf = P.predict_hf != 0;
   switch (p) {
     case 0:  // dc_dequant
       *nx = DcGroups(nblk);
@@ -2009,15 +1957,11 @@ bool PhaseGrid(int p, const FrameParams& P, const FrameBuffers& B, int* nx,
     case 4:  // llf
       *nx = P.gx * P.gy * kLfStrips;
       *ny = 3;
-      arg[0] = hf;
+      arg[0] = P.predict_hf;
       return true;
-    case 9: {  // pred2x2_interior
-      const int wg1 = int(DivCeil(3 * P.pred_end[1], 256));
-      *nx = wg4 + wg2 + wg1;
-      arg[0] = wg4;
-      arg[1] = wg2;
-      return hf && P.pred_end[3] > 0;
-    }
+    case 9:  // pred2x2_interior
+      *nx = PredGrid(P.gx * P.gy);
+      return P.predict_hf != 0;
     case 10:  // blocks
       *nx = XcdGrid(int(DivCeil(P.bx, 4) * DivCeil(P.by, 4)));
       return true;

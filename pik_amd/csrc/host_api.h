@@ -33,11 +33,6 @@ int ValidateFrame(const pikgpu_frame* f, std::string* err);
 // Geometry and derived scalars of a validated frame.
 void FillParams(const pikgpu_frame* f, FrameParams* P);
 
-// First blocks grouped by the class of their pred2x2 computation; end[k]
-// is the end of class k in `list`.
-void PredClasses(const pikgpu_frame* f, std::vector<uint32_t>* list,
-                 int end[4]);
-
 // Dots binned into 32x32 tiles of the padded image (px x py): tile ids, CSR
 // starts and dot indices in application order.
 void BinDots(const pikgpu_frame* f, int px, int py, std::vector<int32_t>* ids,

@@ -839,9 +839,15 @@ __global__ void KLf(FrameParams P, FrameBuffers B, const DeviceConsts* K,
                     int border);
 __global__ void KEncPred2x2Border(FrameParams P, FrameBuffers B,
                                   const DeviceConsts* K);
+// KPred2x2: block rows per strip, workgroups per strip; the grid of a frame's
+// groups.
+constexpr int kPredRows = 4;
+constexpr int kPredStrips = kGroupDimBlocks / kPredRows;
+constexpr int kPredRoles = 3;
+inline int PredGrid(int groups) { return groups * kPredStrips * kPredRoles; }
 template <bool kEnc>
-__global__ void KPred2x2Interior(FrameParams P, FrameBuffers B, const DeviceConsts* K,
-                                 int wg4, int wg2, const float* corner);
+__global__ void KPred2x2(FrameParams P, FrameBuffers B, const DeviceConsts* K,
+                         const float* corner);
 __global__ void KBlocks(FrameParams P, FrameBuffers B, const DeviceConsts* K);
 __global__ void KAdjForward(FrameParams P, FrameBuffers B,
                             const DeviceConsts* K, AdjArgs A);
@@ -927,7 +933,7 @@ __global__ void KDcDequantBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KMinMaxFinalBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KEpfDcBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KLfBatch(PIKGPU_BATCH_PARAMS);
-__global__ void KPred2x2InteriorBatch(PIKGPU_BATCH_PARAMS);
+__global__ void KPred2x2Batch(PIKGPU_BATCH_PARAMS);
 __global__ void KBlocksBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KMinMaxPartial4Batch(PIKGPU_BATCH_PARAMS);
 __global__ void KGuideBatch(PIKGPU_BATCH_PARAMS);

@@ -67,10 +67,9 @@ struct Carve {
 };
 
 // Lays the frame's buffers out from `base` (the constants first) and
-// returns the bytes they span. Host-side lists: the pred2x2 classes and the
-// dot bins.
+// returns the bytes they span; `bins` entries of host-side dot bins.
 size_t NoAllocLayout(const pikgpu_frame* f, const FrameParams& P,
-                     size_t pred_count, size_t bins, uintptr_t base,
+                     size_t bins, uintptr_t base,
                      FrameBuffers* B, DeviceConsts** K) {
   const size_t nblk = size_t(P.bx) * P.by;
   const size_t ngroups = size_t(P.gx) * P.gy;
@@ -94,7 +93,6 @@ size_t NoAllocLayout(const pikgpu_frame* f, const FrameParams& P,
   B->offsets = c.Take<uint32_t>(f->num_dequant_offsets);
   B->dots = c.Take<pikgpu_dot>(f->num_dots);
   B->dot_tile_ids = c.Take<int32_t>(bins);
-  B->pred_list = c.Take<uint32_t>(pred_count);
   B->desc = c.Take<uint4>(2 * nblk);
   B->dcq = c.Take<float>(3 * nblk);
   B->dc = c.Take<float>(3 * nblk);
@@ -165,8 +163,6 @@ int NoAllocRun(const pikgpu_frame* f, float* const out_planes[3],
   }
   FrameParams P;
   FillParams(f, &P);
-  std::vector<uint32_t> pred_list;
-  PredClasses(f, &pred_list, P.pred_end);
   std::vector<int32_t> dot_ids, dot_starts, dot_list;
   if (f->num_dots) {
     BinDots(f, P.px, P.py, &dot_ids, &dot_starts, &dot_list);
@@ -175,7 +171,7 @@ int NoAllocRun(const pikgpu_frame* f, float* const out_planes[3],
   FrameBuffers B;
   DeviceConsts* K = nullptr;
   const size_t need =
-      NoAllocLayout(f, P, pred_list.size(), bins, 0, &B, &K);
+      NoAllocLayout(f, P, bins, 0, &B, &K);
   if (need > kNoAllocBytes) {
     *err = "frame needs " + std::to_string(need) +
            " bytes of device scratch; the no-allocation entry point has " +
@@ -190,8 +186,7 @@ int NoAllocRun(const pikgpu_frame* f, float* const out_planes[3],
   }
   unsigned char* base = nullptr;
   if ((rc = NoAllocDeviceInit(dev, &base, err)) != PIKGPU_OK) return rc;
-  NoAllocLayout(f, P, pred_list.size(), bins, reinterpret_cast<uintptr_t>(base),
-                &B, &K);
+  NoAllocLayout(f, P, bins, reinterpret_cast<uintptr_t>(base), &B, &K);
   B.num_tables = int(f->num_dequant_offsets / (kNumQuantKinds * 3));
   P.dot_tiles = int(dot_ids.size());
   P.dot_tiles_x = int(DivCeil(size_t(P.px), 32));
@@ -229,7 +224,6 @@ int NoAllocRun(const pikgpu_frame* f, float* const out_planes[3],
   TRY(up(B.dqmap, f->dequant_map, 16 * 256));
   TRY(up(B.table, f->dequant_table, f->dequant_table_size * 4));
   TRY(up(B.offsets, f->dequant_offsets, f->num_dequant_offsets * 4));
-  TRY(up(B.pred_list, pred_list.data(), pred_list.size() * 4));
   if (f->num_dots) {
     int32_t* bin = const_cast<int32_t*>(B.dot_tile_ids);
     TRY(up(B.dots, f->dots, f->num_dots * sizeof(pikgpu_dot)));

@@ -322,6 +322,18 @@ __device__ inline void StoreRows(const float* from, float* to, int floats) {
   }
 }
 
+// The strip of workgroup (group, strip); false when the group has no such
+// strip.
+__device__ inline bool LfStripAt(const GroupGeom& G, int k, LfStrip* R) {
+  if (k * kLfStrip >= G.gh) return false;
+  const int H = G.gh + 2;
+  R->first = k == 0 ? 0 : 1 + k * kLfStrip;
+  R->last = (k + 1) * kLfStrip >= G.gh ? H : 1 + (k + 1) * kLfStrip;
+  R->lo = max(R->first - 4, 0);
+  R->hi = min(R->last + 4, H);
+  return true;
+}
+
 __device__ __forceinline__ void KLfBody(const FrameParams& P,
                                         const FrameBuffers& B,
                                         const DeviceConsts* K, int border,
@@ -331,14 +343,10 @@ __device__ __forceinline__ void KLfBody(const FrameParams& P,
   const int g = vb.x / kLfStrips, k = vb.x % kLfStrips, c = vb.y;
   const GroupGeom G = Geom(P, g);
   if (B.stamps) StampStart(&B.stamps->run[1], vb.x + c);
-  if (k * kLfStrip >= G.gh) return;
+  LfStrip R;
+  if (!LfStripAt(G, k, &R)) return;
   const int W = G.gw + 2, H = G.gh + 2;
   const bool lf = P.predict_lf != 0;
-  LfStrip R;
-  R.first = k == 0 ? 0 : 1 + k * kLfStrip;
-  R.last = (k + 1) * kLfStrip >= G.gh ? H : 1 + (k + 1) * kLfStrip;
-  R.lo = max(R.first - 4, 0);
-  R.hi = min(R.last + 4, H);
   // Positions of the strip's rows, kLfThreads apart: the quotient and
   // remainder of the step are the same for all.
   const int y0 = tid / W, x0 = tid - y0 * W;
@@ -540,6 +548,198 @@ __global__ void __launch_bounds__(kLfThreads)
   KLfBody(P, B, K, border, PlainBlock());
 }
 
+// The interior of pred2x2: per first block, the decoder-side LF coefficients
+// (dequantised + LLF + LF prediction) reinterpreted as a 2x upsampled DC
+// block (DC2x2FromLowFrequencies, pik/ac_strategy.cc:971-1017, as called by
+// UpdateLfForDecoder, pik/ac_predictions.cc:621-633).
+//
+// kEnc: the encoder's side (ComputeDecoderBlockAnd2x2DC, pik/ac_predictions.
+// cc:136-199): the corner's values were formed by KEncLf and wait in
+// `corner` (coefficient layout).
+//
+// Three workgroups per four block rows of a group -- the 8x8 strategies, the
+// DCT32 and the DCT16 transforms, which wait for their loads at the same time
+// instead of one after the other -- each for all three planes: X and B take
+// the dequantised Y of their colour correlation from the same thread.
+// Bound by the scattered corners' memory sectors (97 MB of a 4096x4096
+// frame). One thread per block and plane, from a list of the blocks by class
+// that the host built at every upload (0.4 ms at that size), took 40 us;
+// inside KLf, whose large workgroups wait for these loads together, 70 us;
+// PRED_US us so.
+// The three planes' corner value of F-matrix row i, column j of the transform
+// of S x S blocks at frame block (bxa, bya), group block (bxg, byg).
+template <int S, bool kEnc>
+__device__ inline void Corner3(const FrameParams& P, const FrameBuffers& B,
+                               int g, int bxa, int bya, int bxg, int byg,
+                               int i, int j, float ccx, float ccb,
+                               const float* corner, float (&v)[3]) {
+  const int flat = i * 8 * S + j, sb = flat >> 6, k = flat & 63;
+  const size_t at = size_t(bya) * P.bx * 64 + size_t(bxa) * 64 + flat;
+  if (kEnc) {
+    for (int c = 0; c < 3; ++c) {
+      v[c] = corner[size_t(c) * P.by * P.bx * 64 + at];
+    }
+    return;
+  }
+  if (i < S && j < S) {
+    for (int c = 0; c < 3; ++c) {
+      v[c] = B.llf[(size_t(g) * 3 + c) * kLlfPlane +
+                   (byg + 1 + i) * kLlfPitch + bxg + 1 + j];
+    }
+    return;
+  }
+  const uint4 d = B.desc[2 * (bya * P.bx + bxa + sb)];
+  const float scaled = __uint_as_float(d.w);
+  const BlockDq dq[3] = {{B.table + d.x, scaled, ccx},
+                         {B.table + d.y, scaled, 0.0f},
+                         {B.table + d.z, scaled, ccb}};
+  for (int p = 0; p < P.num_passes; ++p) {
+    // each later pass adds its own value, with its own colour correlation
+    // (Dequant<false>::DoAC, pik/compressed_image.cc:695-703)
+    const float y = DequantWith(dq[1], 1, AcPlane(P, B, p, 1)[at], k, 0.0f);
+    const float x = DequantWith(dq[0], 0, AcPlane(P, B, p, 0)[at], k, y);
+    const float b = DequantWith(dq[2], 2, AcPlane(P, B, p, 2)[at], k, y);
+    v[0] = p == 0 ? x : x + v[0];
+    v[1] = p == 0 ? y : y + v[1];
+    v[2] = p == 0 ? b : b + v[2];
+  }
+  if (P.predict_lf) {
+    for (int c = 0; c < 3; ++c) {
+      v[c] += B.lf2x2[(size_t(g) * 3 + c) * kG2Plane +
+                      (2 * (byg + 1) + i) * kG2Pitch + 2 * (bxg + 1) + j];
+    }
+  }
+}
+
+// The DCT16 (S = 2) and DCT32 (S = 4) transforms of the workgroup's rows on
+// N = 2S lanes each: lane l builds column l of the corner and runs the column
+// pass of Idct2D, then the row pass after the transpose through the unit's
+// N x N floats at t. Every thread calls.
+template <int S, bool kEnc>
+__device__ inline void PredUnits(const FrameParams& P, const FrameBuffers& B,
+                                 const DeviceConsts* K, const GroupGeom& G,
+                                 int g, int byg0, float ccx, float ccb,
+                                 const float* corner, float* s_t) {
+  constexpr int N = 2 * S, kPer = kGroupDimBlocks / S;
+  constexpr int ai = ScaleIdx<N>(), ti = ScaleIdx<8 * S>();
+  const int unit = int(threadIdx.x) / N, l = int(threadIdx.x) % N;
+  const int bxg = S * (unit % kPer), byg = byg0 + S * (unit / kPer);
+  const bool inside =
+      byg < byg0 + kPredRows && bxg < G.gw && byg < G.gh;
+  const int bxa = G.gbx0 + bxg, bya = G.gby0 + byg;
+  const bool active =
+      inside && B.acs[bya * P.bx + bxa] ==
+                    uint8_t((S == 4 ? kDCT32 : kDCT16) << 4);
+  if (__ballot(active) == 0) return;  // the same for the wave
+  float* t = s_t + unit * N * (N + 1);
+  float v[3][N], w[N];
+  if (active) {
+#pragma unroll
+    for (int y = 0; y < N; ++y) {
+      float q[3];
+      Corner3<S, kEnc>(P, B, g, bxa, bya, bxg, byg, y, l, ccx, ccb, corner, q);
+      // ReinterpretingIDCT<8S, 2S, 2S>'s scaling
+      for (int c = 0; c < 3; ++c) {
+        v[c][y] = (q[c] * K->ascale[ai][y][l]) * K->tscale[ti][y][l];
+      }
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    if (active) {
+      dct1d::Idct<N>(v[c], w);
+#pragma unroll
+      for (int x = 0; x < N; ++x) t[l * (N + 1) + x] = w[x];
+    }
+    WaveSync();
+    if (active) {
+#pragma unroll
+      for (int cc = 0; cc < N; ++cc) v[c][cc] = t[cc * (N + 1) + l];
+      dct1d::Idct<N>(v[c], w);
+      float* o = B.pred2x2 + (size_t(g) * 3 + c) * kG2Plane +
+                 2 * (byg + 1) * kG2Pitch + 2 * (bxg + 1);
+#pragma unroll
+      for (int y = 0; y < N; ++y) o[y * kG2Pitch + l] = w[y];
+    }
+    WaveSync();
+  }
+}
+
+template <bool kEnc>
+__device__ __forceinline__ void KPred2x2Body(const FrameParams& P,
+                                             const FrameBuffers& B,
+                                             const DeviceConsts* K,
+                                             const float* corner,
+                                             const VBlock& vb) {
+  // the transposes: 16 DCT32 units of 8 x 9 or 64 DCT16 units of 4 x 5
+  __shared__ float s_t[64 * 4 * 5];
+  const int role = vb.x % kPredRoles, strip = vb.x / kPredRoles;
+  const int g = strip / kPredStrips, byg0 = strip % kPredStrips * kPredRows;
+  const GroupGeom G = Geom(P, g);
+  if (byg0 >= G.gh) return;
+  const auto cfl = [&](int bxg, float* ccx, float* ccb) {
+    const int tile = ((G.gby0 + byg0) >> 3) * P.tx + ((G.gbx0 + bxg) >> 3);
+    *ccx = float(B.ytox[tile] - 128) * 0.00390625f;
+    *ccb = float(B.ytob[tile]) * 0.0078125f;
+  };
+  float ccx = 0.0f, ccb = 0.0f;
+  if (role == 1) {
+    const int bxg = int(threadIdx.x) / 8 % 16 * 4;
+    if (!kEnc && bxg < G.gw) cfl(bxg, &ccx, &ccb);
+    PredUnits<4, kEnc>(P, B, K, G, g, byg0, ccx, ccb, corner, s_t);
+    return;
+  }
+  if (role == 2) {
+    const int bxg = int(threadIdx.x) / 4 % 32 * 2;
+    if (!kEnc && bxg < G.gw) cfl(bxg, &ccx, &ccb);
+    PredUnits<2, kEnc>(P, B, K, G, g, byg0, ccx, ccb, corner, s_t);
+    return;
+  }
+  // one block of the rows per thread
+  const int bxg = threadIdx.x & 63, byg = byg0 + int(threadIdx.x >> 6);
+  if (bxg < G.gw && byg < G.gh) {
+    const int bxa = G.gbx0 + bxg, bya = G.gby0 + byg;
+    const uint8_t a = B.acs[bya * P.bx + bxa];
+    const int raw = a >> 4;
+    if ((a & 15) == 0 && raw != kDCT16 && raw != kDCT32) {
+      if (!kEnc) cfl(bxg, &ccx, &ccb);
+      float F[4][3];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        Corner3<1, kEnc>(P, B, g, bxa, bya, bxg, byg, i >> 1, i & 1, ccx, ccb,
+                         corner, F[i]);
+      }
+      const bool dct = raw == kDCT || raw == kDCTNoHF || raw == kLines;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        float f[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          // ReinterpretingIDCT<8, 2, 2>'s scaling; the others (DCT2X2,
+          // DCT4X4(_NOHF), IDENTITY) take the 2x2 Hadamard as it is
+          f[i] = dct ? (F[i][c] * K->ascale[0][i >> 1][i & 1]) *
+                           K->tscale[2][i >> 1][i & 1]
+                     : F[i][c];
+        }
+        Idct2x2(f[0], f[1], f[2], f[3],
+                B.pred2x2 + (size_t(g) * 3 + c) * kG2Plane +
+                    2 * (byg + 1) * kG2Pitch + 2 * (bxg + 1),
+                kG2Pitch);
+      }
+    }
+  }
+}
+template <bool kEnc>
+__global__ void __launch_bounds__(256)
+    KPred2x2(FrameParams P, FrameBuffers B, const DeviceConsts* K,
+             const float* corner) {
+  KPred2x2Body<kEnc>(P, B, K, corner, PlainBlock());
+}
+template __global__ void KPred2x2<false>(FrameParams, FrameBuffers,
+                                         const DeviceConsts*, const float*);
+template __global__ void KPred2x2<true>(FrameParams, FrameBuffers,
+                                        const DeviceConsts*, const float*);
+
 // The border of pred2x2 as the encoder without LF prediction forms it: zeros
 // in place of the LF values (pik/ac_predictions.cc:187-198; everyone else's
 // border is KLf's).
@@ -557,231 +757,6 @@ __global__ void __launch_bounds__(256)
                   0.0f, B.pred2x2 + gc * kG2Plane + 2 * y * kG2Pitch + 2 * x);
 }
 
-// Interior of pred2x2: per first block and plane, the decoder-side LF
-// coefficients (dequantised + LLF + LF prediction) reinterpreted as a 2x
-// upsampled DC block (DC2x2FromLowFrequencies, pik/ac_strategy.cc:971-1017,
-// as called by UpdateLfForDecoder, pik/ac_predictions.cc:621-633). X and B
-// recompute the dequantised Y values their colour correlation needs.
-//
-// kEnc: the encoder's side (ComputeDecoderBlockAnd2x2DC, pik/ac_predictions.
-// cc:136-199): the corner's values were formed by KEncLf and wait in
-// `corner` (coefficient layout).
-template <int S, bool kEnc = false>
-__device__ inline void Pred2x2Block(const FrameParams& P, const FrameBuffers& B,
-                                    const DeviceConsts* K, int c, int bxa,
-                                    int bya, int bxg, int byg, int g,
-                                    const float* corner) {
-  constexpr int N = 2 * S;  // LF corner size
-  const float* llf = B.llf + (size_t(g) * 3 + c) * kLlfPlane;
-  const float* lf = B.lf2x2 + (size_t(g) * 3 + c) * kG2Plane;
-  // Dequantisation parameters of the storage blocks the corner touches:
-  // coefficient F[i][j] (flat i*8S + j) lies in storage block
-  // (bxa + flat / 64, bya) for these sizes.
-  constexpr int kStore = S == 4 ? 4 : 1;
-  BlockDq dq[kStore], dqy[kStore];
-#pragma unroll
-  for (int k = 0; k < kStore; ++k) {
-    dq[k] = DescBlockDq(P, B, c, bya, bxa + k);
-    if (c != 1) dqy[k] = DescBlockDq(P, B, 1, bya, bxa + k);
-  }
-  const size_t row0 = size_t(bya) * P.bx * 64 + size_t(bxa) * 64;
-  const size_t cplane = size_t(c) * P.by * P.bx * 64;
-  float F[N * N];
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-      float v;
-      if (kEnc) {
-        v = corner[cplane + row0 + i * 8 * S + j];
-      } else if (i < S && j < S) {
-        v = llf[(byg + 1 + i) * kLlfPitch + bxg + 1 + j];
-      } else {
-        const int flat = i * 8 * S + j;
-        const int sb = S == 4 ? flat >> 6 : 0, k = flat & 63;
-        v = DequantPasses(P, B, dq[sb], dqy[sb], c, row0 + flat, k);
-        if (P.predict_lf) {
-          v += lf[(2 * (byg + 1) + i) * kG2Pitch + 2 * (bxg + 1) + j];
-        }
-      }
-      F[i * N + j] = v;
-    }
-  }
-  float* o = B.pred2x2 + (size_t(g) * 3 + c) * kG2Plane +
-             2 * (byg + 1) * kG2Pitch + 2 * (bxg + 1);
-  // ReinterpretingIDCT<8S, 2S, 2S>
-  if (S == 1) {
-    const float a00 = (F[0] * K->ascale[0][0][0]) * K->tscale[2][0][0];
-    const float a01 = (F[1] * K->ascale[0][0][1]) * K->tscale[2][0][1];
-    const float a10 = (F[2] * K->ascale[0][1][0]) * K->tscale[2][1][0];
-    const float a11 = (F[3] * K->ascale[0][1][1]) * K->tscale[2][1][1];
-    Idct2x2(a00, a01, a10, a11, o, kG2Pitch);
-  } else {
-    ReinterpIdct<8 * S, N, N>(K, F, N, o, kG2Pitch);
-  }
-}
-
-// Location of a first block in its group.
-struct FirstBlock {
-  int bxa, bya, bxg, byg, g;
-};
-__device__ inline FirstBlock LocateBlock(const FrameParams& P, int blk) {
-  FirstBlock f;
-  f.bxa = blk % P.bx;
-  f.bya = blk / P.bx;
-  const int gxi = f.bxa / kGroupDimBlocks, gyi = f.bya / kGroupDimBlocks;
-  f.g = gyi * P.gx + gxi;
-  f.bxg = f.bxa - gxi * kGroupDimBlocks;
-  f.byg = f.bya - gyi * kGroupDimBlocks;
-  return f;
-}
-
-// Pred2x2Block<S> for S = 2, 4 on N = 2S lanes of a workgroup: lane l
-// builds column l of the corner F, scales it and runs the column pass of
-// Idct2D into row l of the unit's LDS matrix t (pitch N + 1); after the
-// barrier lane l runs the row pass over column l of t and writes column l
-// of the output. Each element sees the operations of the one-lane form in
-// the same order. Every thread of the workgroup calls (the barrier);
-// `active` is false for lanes past the last unit.
-template <int S, bool kEnc = false>
-__device__ inline void Pred2x2Lanes(const FrameParams& P, const FrameBuffers& B,
-                                    const DeviceConsts* K, bool active, int c,
-                                    int blk, int l, float* t,
-                                    const float* corner) {
-  constexpr int N = 2 * S;
-  constexpr int ai = ScaleIdx<N>(), ti = ScaleIdx<8 * S>();
-  FirstBlock f = {0, 0, 0, 0, 0};
-  float v[N], w[N];
-  if (active) {
-    f = LocateBlock(P, blk);
-    const float* llf = B.llf + (size_t(f.g) * 3 + c) * kLlfPlane;
-    const float* lf = B.lf2x2 + (size_t(f.g) * 3 + c) * kG2Plane;
-    const size_t row0 = size_t(f.bya) * P.bx * 64 + size_t(f.bxa) * 64;
-    const size_t cplane = size_t(c) * P.by * P.bx * 64;
-#pragma unroll
-    for (int y = 0; y < N; ++y) {
-      float x;
-      if (kEnc) {
-        x = corner[cplane + row0 + y * 8 * S + l];
-      } else if (y < S && l < S) {
-        x = llf[(f.byg + 1 + y) * kLlfPitch + f.bxg + 1 + l];
-      } else {
-        // F[y][l] is flat y * 8S + l, in storage block bxa + flat / 64
-        const int flat = y * 8 * S + l;
-        const int sb = flat >> 6, k = flat & 63;
-        const BlockDq d = DescBlockDq(P, B, c, f.bya, f.bxa + sb);
-        BlockDq dy = d;
-        if (c != 1) dy = DescBlockDq(P, B, 1, f.bya, f.bxa + sb);
-        x = DequantPasses(P, B, d, dy, c, row0 + flat, k);
-        if (P.predict_lf) {
-          x += lf[(2 * (f.byg + 1) + y) * kG2Pitch + 2 * (f.bxg + 1) + l];
-        }
-      }
-      // ReinterpretingIDCT<8S, 2S, 2S>'s scaling
-      v[y] = (x * K->ascale[ai][y][l]) * K->tscale[ti][y][l];
-    }
-    dct1d::Idct<N>(v, w);
-#pragma unroll
-    for (int x = 0; x < N; ++x) t[l * (N + 1) + x] = w[x];
-  }
-  __syncthreads();
-  if (!active) return;
-#pragma unroll
-  for (int cc = 0; cc < N; ++cc) v[cc] = t[cc * (N + 1) + l];
-  dct1d::Idct<N>(v, w);
-  float* o = B.pred2x2 + (size_t(f.g) * 3 + c) * kG2Plane +
-             2 * (f.byg + 1) * kG2Pitch + 2 * (f.bxg + 1);
-#pragma unroll
-  for (int y = 0; y < N; ++y) o[y * kG2Pitch + l] = w[y];
-}
-
-// Interior of pred2x2 over the first blocks of pred_list, binned on the
-// host by class (DCT8-like, 2x2 Hadamard, DCT16, DCT32; P.pred_end holds
-// the class ends). One launch in three segments, the longest work first:
-// workgroups [0, wg4) take the DCT32 blocks, 32 units (block x plane) of 8
-// lanes; [wg4, wg4 + wg2) the DCT16 blocks, 64 units of 4 lanes; the rest
-// one lane per unit for the DCT8-like and Hadamard classes. The three
-// planes of a block are adjacent units (X and B read the block's Y
-// coefficients and descriptors with the Y unit).
-template <bool kEnc>
-__device__ __forceinline__ void KPred2x2InteriorBody(
-    FrameParams P, FrameBuffers B, const DeviceConsts* K, int wg4, int wg2,
-    const float* corner, const VBlock& vb) {
-  __shared__ float s_t[32 * 8 * 9];
-  const int tid = threadIdx.x;
-  const int wg = vb.x;
-  if (wg < wg4) {
-    const int unit = wg * 32 + (tid >> 3);
-    const int kb = unit / 3, c = unit - 3 * kb;
-    const bool active = kb < P.pred_end[3] - P.pred_end[2];
-    const int blk = active ? int(B.pred_list[P.pred_end[2] + kb]) : 0;
-    Pred2x2Lanes<4, kEnc>(P, B, K, active, c, blk, tid & 7,
-                          s_t + (tid >> 3) * 8 * 9, corner);
-    return;
-  }
-  if (wg < wg4 + wg2) {
-    const int unit = (wg - wg4) * 64 + (tid >> 2);
-    const int kb = unit / 3, c = unit - 3 * kb;
-    const bool active = kb < P.pred_end[2] - P.pred_end[1];
-    const int blk = active ? int(B.pred_list[P.pred_end[1] + kb]) : 0;
-    Pred2x2Lanes<2, kEnc>(P, B, K, active, c, blk, tid & 3,
-                          s_t + (tid >> 2) * 4 * 5, corner);
-    return;
-  }
-  const int lane = (wg - wg4 - wg2) * 256 + tid;
-  const int k = lane / 3, c = lane - 3 * k;
-  if (k >= P.pred_end[1]) return;
-  const FirstBlock f = LocateBlock(P, int(B.pred_list[k]));
-  if (k < P.pred_end[0]) {
-    Pred2x2Block<1, kEnc>(P, B, K, c, f.bxa, f.bya, f.bxg, f.byg, f.g,
-                          corner);
-    return;
-  }
-  // DCT2X2, DCT4X4(_NOHF), IDENTITY: 2x2 Hadamard of the LF corner.
-  const int bxa = f.bxa, bya = f.bya, bxg = f.bxg, byg = f.byg, g = f.g;
-  const BlockDq dq = DescBlockDq(P, B, c, bya, bxa);
-  BlockDq dqy;
-  if (c != 1) dqy = DescBlockDq(P, B, 1, bya, bxa);
-  const size_t row0 = size_t(bya) * P.bx * 64 + size_t(bxa) * 64;
-  const float* llf = B.llf + (size_t(g) * 3 + c) * kLlfPlane;
-  const float* lf = B.lf2x2 + (size_t(g) * 3 + c) * kG2Plane;
-  float F[4];
-  const size_t cplane = size_t(c) * P.by * P.bx * 64;
-  for (int i = 0; i < 2; ++i) {
-    for (int j = 0; j < 2; ++j) {
-      float v;
-      if (kEnc) {
-        v = corner[cplane + row0 + i * 8 + j];
-      } else if (i == 0 && j == 0) {
-        v = llf[(byg + 1) * kLlfPitch + bxg + 1];
-      } else {
-        const int flat = i * 8 + j;
-        v = DequantPasses(P, B, dq, dqy, c, row0 + flat, flat);
-        if (P.predict_lf) {
-          v += lf[(2 * (byg + 1) + i) * kG2Pitch + 2 * (bxg + 1) + j];
-        }
-      }
-      F[i * 2 + j] = v;
-    }
-  }
-  float* o = B.pred2x2 + (size_t(g) * 3 + c) * kG2Plane +
-             2 * (byg + 1) * kG2Pitch + 2 * (bxg + 1);
-  Idct2x2(F[0], F[1], F[2], F[3], o, kG2Pitch);
-}
-template <bool kEnc>
-__global__ void __launch_bounds__(256)
-    KPred2x2Interior(FrameParams P, FrameBuffers B, const DeviceConsts* K,
-                     int wg4, int wg2, const float* corner) {
-  KPred2x2InteriorBody<kEnc>(P, B, K, wg4, wg2, corner, PlainBlock());
-}
-
-template __global__ void KPred2x2Interior<false>(FrameParams, FrameBuffers,
-                                                 const DeviceConsts*, int, int,
-                                                 const float*);
-template __global__ void KPred2x2Interior<true>(FrameParams, FrameBuffers,
-                                                const DeviceConsts*, int, int,
-                                                const float*);
-
 // ---------------------------------------------------------------------------
 // Batched forms: one launch over every frame of a batch, each frame's part
 // of the launch running the plain kernel's grid (BatchSpan, with the
@@ -789,13 +764,11 @@ template __global__ void KPred2x2Interior<true>(FrameParams, FrameBuffers,
 __global__ void __launch_bounds__(256) KDcDequantBatch(PIKGPU_BATCH_PARAMS) {
   PIKGPU_BATCH_LOOP(KDcDequantBody(P, B, vb));
 }
-__global__ void __launch_bounds__(kLfThreads) KLfBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_LOOP(KLfBody(P, B, K, s.arg[0], vb));
+__global__ void __launch_bounds__(256) KPred2x2Batch(PIKGPU_BATCH_PARAMS) {
+  PIKGPU_BATCH_ONE(KPred2x2Body<false>(P, B, K, nullptr, vb));
 }
-__global__ void __launch_bounds__(256)
-    KPred2x2InteriorBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_ONE(KPred2x2InteriorBody<false>(P, B, K, s.arg[0], s.arg[1],
-                                                nullptr, vb));
+__global__ void __launch_bounds__(kLfThreads) KLfBatch(PIKGPU_BATCH_PARAMS) {
+  PIKGPU_BATCH_ONE(KLfBody(P, B, K, s.arg[0], vb));
 }
 
 }  // namespace pikgpu
