@@ -41,6 +41,15 @@ struct DevBuf {
 };
 
 
+// What the walk over the blocks finds besides errors.
+struct BlockScan {
+  bool lines = false;       // a LINES block (no adjoint: fwd_adj, search)
+  bool enc_map_ok = true;   // the encoder's dequant-map lookups, which index
+                            // the map by the quant value itself
+                            // (pik/compressed_image.cc:417, 445), stay
+                            // inside it
+};
+
 // Most AC passes of a frame (pikgpu_frame_add_pass).
 constexpr int kMaxPasses = 16;
 
@@ -53,8 +62,8 @@ struct pikgpu_ctx {
   DeviceConsts* consts = nullptr;
   HostTables host;
   // device buffers (grown on demand)
-  DevBuf ac, dc16, qf, acs, lut, dcf, ytox, ytob, dqmap, table, offsets, dots,
-      dotbins, ac_extra;
+  DevBuf ac, ac_extra;
+  DevBuf side;  // every other input of the frame (SidePack)
   DevBuf desc, dcq, dcv, llf, lf2x2, pred2x2, coeffs, idct, guide, epf, ar,
       dots_img, gab, out, mm_partial, mm, ar_keep, srgb8, gimg;
   // pikgpu_fwd_adj staging (host-pointer calls) and loss partials
@@ -66,8 +75,9 @@ struct pikgpu_ctx {
   // pikgpu_search_quant_field: log field, Adam moments, weights, per-block
   // distortion, rate partials, the rate weight, loss / rate histories
   DevBuf srch;
-  bool enc_map_ok = false;  // every quant_table index of the frame in range
-  bool has_lines = false;   // a LINES block (no adjoint: fwd_adj, search)
+  BlockScan scan;               // of the uploaded frame
+  bool itable_ready = false;    // itable holds the uploaded frame's
+  size_t table_size = 0;        // floats of its dequant table
   int global_scale = 0, quant_dc = 0;  // the uploaded frame's
   float dc_matrix0[3] = {0, 0, 0};     // DequantMatrix(0, DCT8, c)[0]
   bool adj_ready = false;  // LLF / LF caches hold the uploaded frame's
@@ -129,11 +139,7 @@ int Grow(pikgpu_ctx* ctx, DevBuf* b, size_t bytes) {
 }
 
 void FreeAll(pikgpu_ctx* ctx) {
-  DevBuf* all[] = {&ctx->ac,      &ctx->ac_extra, &ctx->dc16, &ctx->qf,
-                   &ctx->acs,
-                   &ctx->lut,     &ctx->dcf,    &ctx->ytox,    &ctx->ytob,
-                   &ctx->dqmap,   &ctx->table,  &ctx->offsets, &ctx->dots,
-                   &ctx->dotbins, &ctx->srgb8,
+  DevBuf* all[] = {&ctx->ac,      &ctx->ac_extra, &ctx->side,   &ctx->srgb8,
                    &ctx->desc,    &ctx->dcq,     &ctx->dcv,    &ctx->llf,    
                    &ctx->lf2x2,   &ctx->pred2x2, &ctx->coeffs, &ctx->idct,
                    &ctx->guide,   &ctx->epf,    &ctx->ar,      &ctx->dots_img,
@@ -154,6 +160,10 @@ void FreeAll(pikgpu_ctx* ctx) {
 // the host plane is strided; longer ones go row by row (per-row copy cost
 // is then small against the row's own transfer).
 constexpr size_t kStageRowMax = 32 << 10;
+// AC planes of at most this many bytes together are uploaded with the other
+// inputs, in one copy: a host memcpy of 256 KB takes about 25 us, three
+// copies of their own 35 to 50.
+constexpr size_t kStageAc = 256 << 10;
 // Dense planes of at most this many bytes together are downloaded as one
 // staged copy instead of one copy each.
 constexpr size_t kStageSmall = 128 << 10;
@@ -352,10 +362,9 @@ int VFail(std::string* err, int code, const char* msg) {
 
 namespace pikgpu {
 
-// Checks that a frame is complete and self-consistent (what the reference's
-// decoder establishes while reading the bitstream; a violation there is a
-// decoding error). Host-only; touches no device.
-int ValidateFrame(const pikgpu_frame* f, std::string* err) {
+// The checks that read only the frame's scalars and pointers (enough to size
+// buffers and to read the planes).
+static int ValidateHeader(const pikgpu_frame* f, std::string* err) {
   if (f == nullptr) return VFail(err, PIKGPU_EINVAL, "null frame");
   if (f->xsize == 0 || f->ysize == 0 || f->xsize > (1u << 16) ||
       f->ysize > (1u << 16)) {
@@ -384,8 +393,7 @@ int ValidateFrame(const pikgpu_frame* f, std::string* err) {
     return VFail(err, PIKGPU_EUNSUPPORTED,
                 "fixed-sigma EPF (enable_adaptive = false) is not supported");
   }
-  const size_t bx = DivCeil(f->xsize, 8), by = DivCeil(f->ysize, 8);
-  const size_t tx = DivCeil(f->xsize, 64), ty = DivCeil(f->ysize, 64);
+  const size_t bx = DivCeil(f->xsize, 8), tx = DivCeil(f->xsize, 64);
   if (!f->ac[0] || !f->ac[1] || !f->ac[2] || !f->dc[0] || !f->dc[1] ||
       !f->dc[2] || !f->quant_field || !f->ac_strategy || !f->sigma_lut_ids ||
       !f->dequant_cf || !f->ytox_map || !f->ytob_map || !f->dequant_map ||
@@ -402,6 +410,14 @@ int ValidateFrame(const pikgpu_frame* f, std::string* err) {
       f->num_dequant_offsets % (kNumQuantKinds * 3) != 0) {
     return VFail(err, PIKGPU_EINVAL, "dequant offsets not a multiple of 21");
   }
+  return PIKGPU_OK;
+}
+
+// The checks of the arrays' contents, after ValidateHeader.
+static int ValidateArrays(const pikgpu_frame* f, std::string* err,
+                          BlockScan* scan) {
+  const size_t bx = DivCeil(f->xsize, 8), by = DivCeil(f->ysize, 8);
+  const size_t tx = DivCeil(f->xsize, 64), ty = DivCeil(f->ysize, 64);
   const int num_tables = int(f->num_dequant_offsets / (kNumQuantKinds * 3));
   // Every table entry a kind can address must lie in the table.
   const int kind_size[kNumQuantKinds] = {64, 64, 64, 64, 256, 1024, 64};
@@ -429,33 +445,45 @@ int ValidateFrame(const pikgpu_frame* f, std::string* err) {
   }
   // AC strategy: valid raw types, multi-block transforms complete, aligned
   // and inside the image (as AcStrategyImage::SetFromRaw establishes).
+  // Covered sizes are powers of two: shifts and masks, no divisions.
   for (size_t y = 0; y < by; ++y) {
+    const uint8_t* acs = f->ac_strategy + y * f->ac_strategy_stride;
+    const int32_t* qf = f->quant_field + y * f->quant_field_stride;
+    const uint8_t* lut = f->sigma_lut_ids + y * f->sigma_lut_stride;
+    const uint8_t* cf = f->dequant_cf + (y / 8) * f->dequant_cf_stride;
     for (size_t x = 0; x < bx; ++x) {
-      const uint8_t a = f->ac_strategy[y * f->ac_strategy_stride + x];
+      const uint8_t a = acs[x];
       const int raw = a >> 4, idx = a & 15;
-      const int qfv = f->quant_field[y * f->quant_field_stride + x];
-      if (qfv < 1 || qfv > 256) {
+      if (qf[x] < 1 || qf[x] > 256) {
         return VFail(err, PIKGPU_EINVAL, "quant field outside [1, 256]");
       }
-      if (f->sigma_lut_ids[y * f->sigma_lut_stride + x] > 1) {
-        return VFail(err, PIKGPU_EINVAL, "sigma lut id > 1");
-      }
+      if (qf[x] == 256 && cf[x / 8] == 15) scan->enc_map_ok = false;
+      if (lut[x] > 1) return VFail(err, PIKGPU_EINVAL, "sigma lut id > 1");
       if (raw > 8) return VFail(err, PIKGPU_EINVAL, "invalid AC strategy");
-      const int s = AcsCovered(raw);
-      if (idx >= s * s) return VFail(err, PIKGPU_EINVAL, "invalid block index");
-      const size_t ox = x - idx % s, oy = y - idx / s;
-      if (idx % s > int(x) || idx / s > int(y) || ox % s || oy % s ||
+      if (raw == kLines) scan->lines = true;
+      const unsigned s = AcsCovered(raw), lg = s >> 1;
+      if (s == 1) {
+        if (idx != 0) return VFail(err, PIKGPU_EINVAL, "invalid block index");
+        continue;
+      }
+      if (unsigned(idx) >= s * s) {
+        return VFail(err, PIKGPU_EINVAL, "invalid block index");
+      }
+      const size_t ix = idx & (s - 1), iy = size_t(idx) >> lg;
+      const size_t ox = x - ix, oy = y - iy;
+      if (ix > x || iy > y || (ox & (s - 1)) || (oy & (s - 1)) ||
           ox + s > bx || oy + s > by) {
         return VFail(err, PIKGPU_EINVAL, "misaligned multi-block transform");
       }
       // A transform's first block checks the whole transform; every other
       // block only that its first block is one of the same kind, whose own
       // check then covers it.
-      const int kmax = idx == 0 ? s * s : 1;
-      for (int k = 0; k < kmax; ++k) {
-        const uint8_t e =
-            f->ac_strategy[(oy + k / s) * f->ac_strategy_stride + ox + k % s];
-        if (e != ((raw << 4) | k)) {
+      const unsigned kmax = idx == 0 ? s * s : 1;
+      for (unsigned k = 0; k < kmax; ++k) {
+        const uint8_t e = f->ac_strategy[(oy + (k >> lg)) *
+                                             f->ac_strategy_stride +
+                                         ox + (k & (s - 1))];
+        if (e != ((unsigned(raw) << 4) | k)) {
           return VFail(err, PIKGPU_EINVAL, "inconsistent multi-block transform");
         }
       }
@@ -475,6 +503,15 @@ int ValidateFrame(const pikgpu_frame* f, std::string* err) {
   }
 
   return PIKGPU_OK;
+}
+
+// Checks that a frame is complete and self-consistent (what the reference's
+// decoder establishes while reading the bitstream; a violation there is a
+// decoding error). Host-only; touches no device.
+int ValidateFrame(const pikgpu_frame* f, std::string* err) {
+  BlockScan scan;
+  const int rc = ValidateHeader(f, err);
+  return rc != PIKGPU_OK ? rc : ValidateArrays(f, err, &scan);
 }
 
 // Geometry and derived scalars of a validated frame.
@@ -613,44 +650,85 @@ int pikgpu_validate_frame(const pikgpu_frame* frame, char* msg,
   return rc;
 }
 
-int pikgpu_frame_upload(pikgpu_ctx* ctx, const pikgpu_frame* f) {
-  if (ctx == nullptr) return PIKGPU_EINVAL;
-  HIP_TRY(ctx, hipSetDevice(ctx->device));
-  ctx->uploaded = false;
-  ctx->ran = false;
-  ctx->adj_ready = false;
-  {
-    std::string err;
-    const int rc = ValidateFrame(f, &err);
-    if (rc != PIKGPU_OK) return Fail(ctx, rc, err);
+}  // extern "C"
+
+namespace {
+
+// The frame's inputs other than large AC planes, packed one after the other
+// (256-byte aligned) into pinned staging and copied to the device as one
+// piece: each copy of its own costs 10 to 20 us whatever its size, and there
+// are sixteen (a frame of one block, upload to download: 255 us with them,
+// 156 us with one; 1024x683: 725 and 488 us).
+class SidePack {
+ public:
+  struct Plane {
+    const void* src;
+    size_t stride_b, row_b, rows, at;
+  };
+  // Rows of row_b bytes, stride_b apart; `follow`: right behind the one
+  // before (the planes of one image). Returns the place on the device.
+  size_t Add(const void* src, size_t stride_b, size_t row_b, size_t rows,
+             bool follow = false) {
+    const size_t at = follow ? bytes_ : (bytes_ + 255) & ~size_t(255);
+    planes_.push_back(Plane{src, stride_b, row_b, rows, at});
+    bytes_ = at + row_b * rows;
+    return at;
   }
-  const size_t bx = DivCeil(f->xsize, 8), by = DivCeil(f->ysize, 8);
-  const size_t tx = DivCeil(f->xsize, 64), ty = DivCeil(f->ysize, 64);
-  const int num_tables = int(f->num_dequant_offsets / (kNumQuantKinds * 3));
+  size_t bytes() const { return bytes_; }
+  // To `base`: staged when it fits a chunk, else plane by plane.
+  int Upload(pikgpu_ctx* ctx, uint8_t* base) {
+    int rc;
+    if (bytes_ > kStageChunk) {
+      for (const Plane& p : planes_) {
+        if (p.row_b * p.rows == 0) continue;
+        if ((rc = Upload2D(ctx, base + p.at, p.src, p.stride_b, p.row_b,
+                           p.rows))) {
+          return rc;
+        }
+      }
+      return PIKGPU_OK;
+    }
+    if ((rc = StageReserve(ctx, bytes_)) != PIKGPU_OK) return rc;
+    uint8_t* stage = static_cast<uint8_t*>(ctx->stage);
+    for (const Plane& p : planes_) {
+      uint8_t* to = stage + p.at;
+      const uint8_t* from = static_cast<const uint8_t*>(p.src);
+      if (p.rows <= 1 || p.stride_b == p.row_b) {
+        if (p.row_b * p.rows) memcpy(to, from, p.row_b * p.rows);
+        continue;
+      }
+      for (size_t y = 0; y < p.rows; ++y) {
+        memcpy(to + y * p.row_b, from + y * p.stride_b, p.row_b);
+      }
+    }
+    HIP_TRY(ctx, hipMemcpyAsync(base, stage, bytes_, hipMemcpyHostToDevice,
+                                ctx->stream));
+    return PIKGPU_OK;
+  }
+
+ private:
+  std::vector<Plane> planes_;
+  size_t bytes_ = 0;
+};
+
+// Everything of an upload after the AC planes: parameters, buffers, the other
+// inputs, the frame's buffer table. The copies may still be in flight.
+int UploadRest(pikgpu_ctx* ctx, const pikgpu_frame* f, bool ac_packed,
+               int num_tables, size_t bx, size_t by, size_t tx, size_t ty,
+               size_t ngroups) {
   FrameParams& P = ctx->P;
   FillParams(f, &P);
-
-  // --- buffers ---
   const size_t nblk = bx * by;
-  const size_t ngroups = size_t(P.gx) * P.gy;
   const size_t ipitch = DivCeil(bx * 8, 32) * 32;
   // dense output rows: a download is one linear copy per plane
   const size_t opitch = f->xsize;
+  // guide image: 6-pixel border, rows and pitch cover the 44-row, 44-byte
+  // windows of every (possibly partial) 32x32 tile
+  const size_t grows = DivCeil(by * 8, 32) * 32 + 16;
+  const size_t gpitch = DivCeil(bx * 8, 32) * 32 + 64;
   int rc;
 #define GROW(buf, bytes) \
   if ((rc = Grow(ctx, &ctx->buf, (bytes))) != PIKGPU_OK) return rc
-  GROW(ac, 3 * nblk * 64 * sizeof(int16_t));
-  GROW(dc16, 3 * nblk * sizeof(int16_t));
-  GROW(qf, nblk * 4);
-  GROW(acs, nblk);
-  GROW(lut, nblk);
-  GROW(dcf, tx * ty);
-  GROW(ytox, tx * ty * 4);
-  GROW(ytob, tx * ty * 4);
-  GROW(dqmap, 16 * 256);
-  GROW(table, f->dequant_table_size * 4);
-  GROW(offsets, f->num_dequant_offsets * 4);
-  GROW(dots, f->num_dots * sizeof(pikgpu_dot));
   GROW(desc, 2 * nblk * 16);
   GROW(dcq, 3 * nblk * 4);
   GROW(dcv, 3 * nblk * 4);
@@ -659,138 +737,78 @@ int pikgpu_frame_upload(pikgpu_ctx* ctx, const pikgpu_frame* f) {
   GROW(pred2x2, ngroups * 3 * kG2Plane * 4);
   GROW(idct, 3 * ipitch * by * 8 * 4);
   GROW(ar, 3 * ipitch * by * 8 * 4);
-  // guide image: 6-pixel border, rows and pitch cover the 44-row, 44-byte
-  // windows of every (possibly partial) 32x32 tile
-  const size_t grows = DivCeil(by * 8, 32) * 32 + 16;
-  const size_t gpitch = DivCeil(bx * 8, 32) * 32 + 64;
   GROW(gimg, 3 * grows * gpitch);
   GROW(out, 3 * opitch * f->ysize * 4);
   GROW(mm_partial, kMinMaxMaxGroups * 2 * 4);
   GROW(mm, 2 * 4);
-#undef GROW
 
-  // --- copies ---
-  const size_t nb = nblk;
-  for (int c = 0; c < 3; ++c) {
-    if ((rc = Upload2D(ctx, static_cast<int16_t*>(ctx->ac.p) + c * nb * 64,
-                       f->ac[c], f->ac_stride * 2, bx * 64 * 2, by)))
-      return rc;
-    if ((rc = Upload2D(ctx, static_cast<int16_t*>(ctx->dc16.p) + c * nb,
-                       f->dc[c], f->dc_stride * 2, bx * 2, by)))
-      return rc;
-  }
-  if ((rc = Upload2D(ctx, ctx->qf.p, f->quant_field, f->quant_field_stride * 4,
-                     bx * 4, by)))
-    return rc;
-  if ((rc = Upload2D(ctx, ctx->acs.p, f->ac_strategy, f->ac_strategy_stride,
-                     bx, by)))
-    return rc;
-  if ((rc = Upload2D(ctx, ctx->lut.p, f->sigma_lut_ids, f->sigma_lut_stride,
-                     bx, by)))
-    return rc;
-  if ((rc = Upload2D(ctx, ctx->dcf.p, f->dequant_cf, f->dequant_cf_stride, tx,
-                     ty)))
-    return rc;
-  if ((rc = Upload2D(ctx, ctx->ytox.p, f->ytox_map, f->ytox_stride * 4, tx * 4,
-                     ty)))
-    return rc;
-  if ((rc = Upload2D(ctx, ctx->ytob.p, f->ytob_map, f->ytob_stride * 4, tx * 4,
-                     ty)))
-    return rc;
-  HIP_TRY(ctx, hipMemcpyAsync(ctx->dqmap.p, f->dequant_map, 16 * 256,
-                              hipMemcpyHostToDevice, ctx->stream));
-  HIP_TRY(ctx, hipMemcpyAsync(ctx->table.p, f->dequant_table,
-                              f->dequant_table_size * 4, hipMemcpyHostToDevice,
-                              ctx->stream));
-  HIP_TRY(ctx, hipMemcpyAsync(ctx->offsets.p, f->dequant_offsets,
-                              f->num_dequant_offsets * 4,
-                              hipMemcpyHostToDevice, ctx->stream));
-  // The encoder's inverse table (DequantMatrices, pik/quant_weights.cc:
-  // 918-923) and whether its quant_table lookups, which index the map by
-  // the quant value itself (pik/compressed_image.cc:417, 445), stay inside
-  // the 16 x 256 map.
-  {
-    std::vector<float> inv(f->dequant_table_size);
-    for (size_t i = 0; i < inv.size(); ++i) inv[i] = 1.0f / f->dequant_table[i];
-    if ((rc = Grow(ctx, &ctx->itable, inv.size() * 4))) return rc;
-    HIP_TRY(ctx, hipMemcpyAsync(ctx->itable.p, inv.data(), inv.size() * 4,
-                                hipMemcpyHostToDevice, ctx->stream));
-    HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
-    bool ok = true;
-    for (size_t y = 0; y < by && ok; ++y) {
-      for (size_t x = 0; x < bx; ++x) {
-        const int q = f->quant_field[y * f->quant_field_stride + x];
-        const int cf = f->dequant_cf[(y / 8) * f->dequant_cf_stride + x / 8];
-        if (cf * 256 + q >= 16 * 256) {
-          ok = false;
-          break;
-        }
-      }
-    }
-    ctx->enc_map_ok = ok;
-    ctx->global_scale = int(f->global_scale);
-    ctx->quant_dc = int(f->quant_dc);
-    for (int c = 0; c < 3; ++c) {
-      ctx->dc_matrix0[c] = f->dequant_table[f->dequant_offsets[c]];
-    }
-  }
   std::vector<int32_t> dot_ids, dot_starts, dot_list;
   if (f->num_dots) {
-    HIP_TRY(ctx, hipMemcpyAsync(ctx->dots.p, f->dots,
-                                f->num_dots * sizeof(pikgpu_dot),
-                                hipMemcpyHostToDevice, ctx->stream));
     BinDots(f, int(bx * 8), int(by * 8), &dot_ids, &dot_starts, &dot_list);
-    const size_t nbin = dot_ids.size() + dot_starts.size() + dot_list.size();
-    if ((rc = Grow(ctx, &ctx->dotbins, nbin * 4))) return rc;
-    int32_t* dst = static_cast<int32_t*>(ctx->dotbins.p);
-    HIP_TRY(ctx, hipMemcpyAsync(dst, dot_ids.data(), dot_ids.size() * 4,
-                                hipMemcpyHostToDevice, ctx->stream));
-    HIP_TRY(ctx, hipMemcpyAsync(dst + dot_ids.size(), dot_starts.data(),
-                                dot_starts.size() * 4, hipMemcpyHostToDevice,
-                                ctx->stream));
-    HIP_TRY(ctx, hipMemcpyAsync(dst + dot_ids.size() + dot_starts.size(),
-                                dot_list.data(), dot_list.size() * 4,
-                                hipMemcpyHostToDevice, ctx->stream));
   }
-  ctx->has_lines = false;
-  for (size_t y = 0; y < by && !ctx->has_lines; ++y) {
-    for (size_t x = 0; x < bx; ++x) {
-      if ((f->ac_strategy[y * f->ac_strategy_stride + x] >> 4) == kLines) {
-        ctx->has_lines = true;
-        break;
-      }
+  SidePack pack;
+  const auto planes = [&](const int16_t* const src[3], size_t stride,
+                          size_t row) {
+    size_t at = 0;
+    for (int c = 0; c < 3; ++c) {
+      const size_t a = pack.Add(src[c], stride * 2, row * 2, by, c > 0);
+      if (c == 0) at = a;
     }
-  }
-  // pred2x2 positions that no block writes (ZeroFillImage,
-  // pik/compressed_image.cc:976): the same ones on every run of this frame,
-  // so once here rather than per run
-  HIP_TRY(ctx, hipMemsetAsync(ctx->pred2x2.p, 0, ngroups * 3 * kG2Plane * 4,
-                              ctx->stream));
-  HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    return at;
+  };
+  const size_t at_ac = ac_packed ? planes(f->ac, f->ac_stride, bx * 64) : 0;
+  const size_t at_dc = planes(f->dc, f->dc_stride, bx);
+  const size_t at_qf = pack.Add(f->quant_field, f->quant_field_stride * 4,
+                                bx * 4, by);
+  const size_t at_acs = pack.Add(f->ac_strategy, f->ac_strategy_stride, bx, by);
+  const size_t at_lut = pack.Add(f->sigma_lut_ids, f->sigma_lut_stride, bx, by);
+  const size_t at_dcf = pack.Add(f->dequant_cf, f->dequant_cf_stride, tx, ty);
+  const size_t at_ytox = pack.Add(f->ytox_map, f->ytox_stride * 4, tx * 4, ty);
+  const size_t at_ytob = pack.Add(f->ytob_map, f->ytob_stride * 4, tx * 4, ty);
+  const size_t at_map = pack.Add(f->dequant_map, 0, 16 * 256, 1);
+  const size_t at_table = pack.Add(f->dequant_table, 0,
+                                   f->dequant_table_size * 4, 1);
+  const size_t at_off = pack.Add(f->dequant_offsets, 0,
+                                 f->num_dequant_offsets * 4, 1);
+  const size_t at_dots = pack.Add(f->dots, 0,
+                                  f->num_dots * sizeof(pikgpu_dot), 1);
+  const size_t at_ids = pack.Add(dot_ids.data(), 0, dot_ids.size() * 4, 1);
+  const size_t at_starts = pack.Add(dot_starts.data(), 0,
+                                    dot_starts.size() * 4, 1);
+  const size_t at_list = pack.Add(dot_list.data(), 0, dot_list.size() * 4, 1);
+  GROW(side, pack.bytes());
+#undef GROW
+  uint8_t* base = static_cast<uint8_t*>(ctx->side.p);
+  if ((rc = pack.Upload(ctx, base)) != PIKGPU_OK) return rc;
 
+  ctx->table_size = f->dequant_table_size;
+  ctx->global_scale = int(f->global_scale);
+  ctx->quant_dc = int(f->quant_dc);
+  for (int c = 0; c < 3; ++c) {
+    ctx->dc_matrix0[c] = f->dequant_table[f->dequant_offsets[c]];
+  }
   FrameBuffers& B = ctx->B;
   memset(&B, 0, sizeof(B));
-  B.ac = static_cast<const int16_t*>(ctx->ac.p);
-  B.ac_extra = nullptr;
-  B.dc16 = static_cast<const int16_t*>(ctx->dc16.p);
-  B.qf = static_cast<const int32_t*>(ctx->qf.p);
-  B.acs = static_cast<const uint8_t*>(ctx->acs.p);
-  B.lut = static_cast<const uint8_t*>(ctx->lut.p);
-  B.dcf = static_cast<const uint8_t*>(ctx->dcf.p);
-  B.ytox = static_cast<const int32_t*>(ctx->ytox.p);
-  B.ytob = static_cast<const int32_t*>(ctx->ytob.p);
-  B.dqmap = static_cast<const uint8_t*>(ctx->dqmap.p);
-  B.table = static_cast<const float*>(ctx->table.p);
-  B.offsets = static_cast<const uint32_t*>(ctx->offsets.p);
+  B.ac = reinterpret_cast<const int16_t*>(
+      ac_packed ? base + at_ac : static_cast<uint8_t*>(ctx->ac.p));
+  B.dc16 = reinterpret_cast<const int16_t*>(base + at_dc);
+  B.qf = reinterpret_cast<const int32_t*>(base + at_qf);
+  B.acs = base + at_acs;
+  B.lut = base + at_lut;
+  B.dcf = base + at_dcf;
+  B.ytox = reinterpret_cast<const int32_t*>(base + at_ytox);
+  B.ytob = reinterpret_cast<const int32_t*>(base + at_ytob);
+  B.dqmap = base + at_map;
+  B.table = reinterpret_cast<const float*>(base + at_table);
+  B.offsets = reinterpret_cast<const uint32_t*>(base + at_off);
   B.num_tables = num_tables;
-  B.dots = static_cast<const pikgpu_dot*>(ctx->dots.p);
+  B.dots = reinterpret_cast<const pikgpu_dot*>(base + at_dots);
   P.dot_tiles = int(dot_ids.size());
   P.dot_tiles_x = int(DivCeil(bx * 8, 32));
   if (P.dot_tiles) {
-    const int32_t* bins = static_cast<const int32_t*>(ctx->dotbins.p);
-    B.dot_tile_ids = bins;
-    B.dot_tile_start = bins + dot_ids.size();
-    B.dot_list = bins + dot_ids.size() + dot_starts.size();
+    B.dot_tile_ids = reinterpret_cast<const int32_t*>(base + at_ids);
+    B.dot_tile_start = reinterpret_cast<const int32_t*>(base + at_starts);
+    B.dot_list = reinterpret_cast<const int32_t*>(base + at_list);
   }
   B.desc = static_cast<uint4*>(ctx->desc.p);
   B.dcq = static_cast<float*>(ctx->dcq.p);
@@ -809,6 +827,57 @@ int pikgpu_frame_upload(pikgpu_ctx* ctx, const pikgpu_frame* f) {
   B.ipitch = int(ipitch);
   B.opitch = int(opitch);
   ctx->num_tables = num_tables;
+  return PIKGPU_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int pikgpu_frame_upload(pikgpu_ctx* ctx, const pikgpu_frame* f) {
+  if (ctx == nullptr) return PIKGPU_EINVAL;
+  HIP_TRY(ctx, hipSetDevice(ctx->device));
+  ctx->uploaded = false;
+  ctx->ran = false;
+  ctx->adj_ready = false;
+  ctx->itable_ready = false;
+  ctx->scan = BlockScan();
+  std::string err;
+  int rc = ValidateHeader(f, &err);
+  if (rc != PIKGPU_OK) return Fail(ctx, rc, err);
+  const size_t bx = DivCeil(f->xsize, 8), by = DivCeil(f->ysize, 8);
+  const size_t tx = DivCeil(f->xsize, 64), ty = DivCeil(f->ysize, 64);
+  const int num_tables = int(f->num_dequant_offsets / (kNumQuantKinds * 3));
+  const size_t nblk = bx * by;
+  const size_t ngroups =
+      DivCeil(bx, kGroupDimBlocks) * DivCeil(by, kGroupDimBlocks);
+  const size_t ac_b = nblk * 64 * sizeof(int16_t);  // of a plane
+
+  // The AC planes first: from pinned memory they copy while the host checks
+  // the frame's arrays and packs the other inputs (a 4096x4096 frame's 1.8
+  // ms of copies against 0.6 ms of host work). Tiny ones go with the rest.
+  const bool ac_packed = 3 * ac_b <= kStageAc;
+  rc = ac_packed ? PIKGPU_OK : Grow(ctx, &ctx->ac, 3 * ac_b);
+  bool in_flight = false;
+  if (rc == PIKGPU_OK && !ac_packed) {
+    for (int c = 0; c < 3 && rc == PIKGPU_OK; ++c) {
+      in_flight = true;
+      rc = Upload2D(ctx, static_cast<uint8_t*>(ctx->ac.p) + c * ac_b, f->ac[c],
+                    f->ac_stride * 2, bx * 128, by);
+    }
+  }
+  // (a refused frame: nothing may still read the caller's planes)
+  const int valid = ValidateArrays(f, &err, &ctx->scan);
+  if (valid != PIKGPU_OK || rc != PIKGPU_OK) {
+    if (in_flight) (void)hipStreamSynchronize(ctx->stream);
+    return valid != PIKGPU_OK ? Fail(ctx, valid, err) : rc;
+  }
+  rc = UploadRest(ctx, f, ac_packed, num_tables, bx, by, tx, ty, ngroups);
+  // The caller's arrays are free once the copies are done.
+  const hipError_t e = hipStreamSynchronize(ctx->stream);
+  ctx->stage_used = 0;
+  if (rc != PIKGPU_OK) return rc;
+  HIP_TRY(ctx, e);
   ctx->uploaded = true;
   return PIKGPU_OK;
 }
@@ -1168,6 +1237,20 @@ int pikgpu_decode_frame(pikgpu_ctx* ctx, const uint8_t* data, size_t size,
   return rc;
 }
 
+// The encoder's inverse table (DequantMatrices, pik/quant_weights.cc:
+// 918-923) of the uploaded frame, formed on the device by the first call that
+// quantizes with it.
+static int EnsureInverseTable(pikgpu_ctx* ctx) {
+  if (ctx->itable_ready) return PIKGPU_OK;
+  const int rc = Grow(ctx, &ctx->itable, ctx->table_size * 4);
+  if (rc != PIKGPU_OK) return rc;
+  KEncInverseTable<<<DivCeil(ctx->table_size, 256), 256, 0, ctx->stream>>>(
+      ctx->B.table, int(ctx->table_size), static_cast<float*>(ctx->itable.p));
+  HIP_TRY(ctx, hipGetLastError());
+  ctx->itable_ready = true;
+  return PIKGPU_OK;
+}
+
 // Encoder-side quantization of an XYB image under the uploaded frame's side
 // information (see pikgpu.h). The quantized AC and DC replace the frame's,
 // so pikgpu_run then decodes the round trip.
@@ -1187,7 +1270,7 @@ int pikgpu_quantize(pikgpu_ctx* ctx, const float* const opsin[3],
     return Fail(ctx, PIKGPU_EUNSUPPORTED,
                 "quantization of frames with dots or grayscale");
   }
-  if (!ctx->enc_map_ok) {
+  if (!ctx->scan.enc_map_ok) {
     return Fail(ctx, PIKGPU_EUNSUPPORTED, "quant value past the dequant map");
   }
   const size_t nb = size_t(P.bx) * P.by, row = size_t(P.bx) * 64;
@@ -1202,6 +1285,7 @@ int pikgpu_quantize(pikgpu_ctx* ctx, const float* const opsin[3],
   if ((rc = Grow(ctx, &ctx->eopsin, 3 * plane * 4))) return rc;
   if ((rc = Grow(ctx, &ctx->ecoef, 3 * nb * 64 * 4))) return rc;
   if ((rc = Grow(ctx, &ctx->edcf, 3 * nb * 4))) return rc;
+  if ((rc = EnsureInverseTable(ctx))) return rc;
   const bool predict = P.predict_lf || P.predict_hf;
   if (predict && (rc = Grow(ctx, &ctx->ecorner, 3 * nb * 64 * 4))) return rc;
   float* dev_opsin = static_cast<float*>(ctx->eopsin.p);
@@ -1220,8 +1304,8 @@ int pikgpu_quantize(pikgpu_ctx* ctx, const float* const opsin[3],
   hipStream_t st = ctx->stream;
   float* coef = static_cast<float*>(ctx->ecoef.p);
   float* dcf = static_cast<float*>(ctx->edcf.p);
-  int16_t* ac16 = static_cast<int16_t*>(ctx->ac.p);
-  int16_t* dc16 = static_cast<int16_t*>(ctx->dc16.p);
+  int16_t* ac16 = const_cast<int16_t*>(ctx->B.ac);
+  int16_t* dc16 = const_cast<int16_t*>(ctx->B.dc16);
   const int tiles = int(DivCeil(P.bx, 4) * DivCeil(P.by, 4));
   FrameBuffers Bt = B;  // with the timing stamps
   Bt.stamps = ctx->stamps;
@@ -1457,7 +1541,7 @@ int pikgpu_fwd_adj(pikgpu_ctx* ctx, const pikgpu_adj_io* io) {
     return Fail(ctx, PIKGPU_EUNSUPPORTED,
                 "the forward model takes single-pass colour frames");
   }
-  if (ctx->has_lines) {
+  if (ctx->scan.lines) {
     return Fail(ctx, PIKGPU_EUNSUPPORTED,
                 "the forward model has no adjoint of the LINES transform");
   }
@@ -1637,7 +1721,7 @@ int pikgpu_search_quant_field(pikgpu_ctx* ctx,
     return Fail(ctx, PIKGPU_EUNSUPPORTED,
                 "search of frames with predictions, dots or grayscale");
   }
-  if (ctx->has_lines) {
+  if (ctx->scan.lines) {
     return Fail(ctx, PIKGPU_EUNSUPPORTED,
                 "the search has no adjoint of the LINES transform");
   }
@@ -1693,6 +1777,7 @@ int pikgpu_search_quant_field(pikgpu_ctx* ctx,
   if ((rc = Grow(ctx, &ctx->eopsin, 3 * plane * 4)) ||
       (rc = Grow(ctx, &ctx->ecoef, 3 * nb * 64 * 4)) ||
       (rc = Grow(ctx, &ctx->edcf, 3 * nb * 4)) ||
+      (rc = EnsureInverseTable(ctx)) ||
       (rc = Grow(ctx, &ctx->adj_qf, nb * 4)) ||
       (rc = Grow(ctx, &ctx->adj_in, 3 * tplane * 4)) ||
       (rc = Grow(ctx, &ctx->adj_dqf, nb * 4)) ||
@@ -1736,9 +1821,9 @@ int pikgpu_search_quant_field(pikgpu_ctx* ctx,
   const DeviceConsts* K = ctx->consts;
   float* coef = static_cast<float*>(ctx->ecoef.p);
   float* dcf = static_cast<float*>(ctx->edcf.p);
-  int16_t* ac16 = static_cast<int16_t*>(ctx->ac.p);
-  int16_t* dc16 = static_cast<int16_t*>(ctx->dc16.p);
-  int32_t* qf = static_cast<int32_t*>(ctx->qf.p);
+  int16_t* ac16 = const_cast<int16_t*>(ctx->B.ac);
+  int16_t* dc16 = const_cast<int16_t*>(ctx->B.dc16);
+  int32_t* qf = const_cast<int32_t*>(ctx->B.qf);
   float* qfr = static_cast<float*>(ctx->adj_qf.p);
   float* grad = static_cast<float*>(ctx->adj_dc.p);
   // forward transforms and the DC: independent of the AC field

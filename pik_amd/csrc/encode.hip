@@ -124,6 +124,13 @@ __global__ void __launch_bounds__(256)
   dc16[2 * nb + i] = int16_t(int(roundf(bv * S.scale[2])));
 }
 
+// Reciprocals of the dequant table's n entries.
+__global__ void __launch_bounds__(256)
+    KEncInverseTable(const float* table, int n, float* out) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) out[i] = 1.0f / table[i];
+}
+
 // AdjustQuantBiasVar (pik/quantizer.h:66-74) of an integer.
 __device__ inline float AdjustQuantBiasInt(int c, int q) {
   constexpr float kOneBias[3] = {0.05465007330715401f, 0.07005449891748593f,

@@ -823,6 +823,7 @@ struct EncDcScale {
 __global__ void KDcDequant(FrameParams P, FrameBuffers B);
 __global__ void KEncForward(FrameParams P, FrameBuffers B, const DeviceConsts* K,
                             const float* opsin, float* coef, float* dcf);
+__global__ void KEncInverseTable(const float* table, int n, float* out);
 __global__ void KEncDc(FrameParams P, const float* dcf, EncDcScale S,
                        int16_t* dc16);
 __global__ void KEncQuant(FrameParams P, FrameBuffers B, const float* coef,

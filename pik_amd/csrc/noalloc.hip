@@ -28,12 +28,6 @@ namespace {
 
 size_t DivCeil(size_t a, size_t b) { return (a + b - 1) / b; }
 
-// Zero fill of n floats.
-__global__ void __launch_bounds__(256) KFillZero(float* p, size_t n) {
-  const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
-  if (i < n) p[i] = 0.0f;
-}
-
 constexpr size_t kNoAllocBytes = size_t(PIKGPU_NOALLOC_SCRATCH_BYTES);
 constexpr size_t kNoAllocAlign = 256;
 constexpr int kNoAllocMaxDevices = 64;
@@ -235,13 +229,6 @@ int NoAllocRun(const pikgpu_frame* f, float* const out_planes[3],
     B.dot_list = bin + dot_ids.size() + dot_starts.size();
   } else {
     B.dot_tile_ids = nullptr;
-  }
-  // the pred2x2 positions no block writes must read zero (ZeroFillImage,
-  // pik/compressed_image.cc:976); the array keeps the last call's
-  // contents, so they are cleared on every call, by a kernel
-  {
-    const size_t n = size_t(P.gx) * P.gy * 3 * kG2Plane;
-    KFillZero<<<DivCeil(n, 256), 256, 0, st>>>(B.pred2x2, n);
   }
   TRY(EnqueueFullSize(P, B, K, st));
   const size_t oplane = size_t(B.opitch) * P.ysize;

@@ -564,8 +564,9 @@ __global__ void __launch_bounds__(kLfThreads)
 // Bound by the scattered corners' memory sectors (97 MB of a 4096x4096
 // frame). One thread per block and plane, from a list of the blocks by class
 // that the host built at every upload (0.4 ms at that size), took 40 us;
-// inside KLf, whose large workgroups wait for these loads together, 70 us;
-// PRED_US us so.
+// inside KLf, whose large workgroups wait for these loads together, 70 us; in
+// one workgroup for the three kinds of a strip 40 us;
+// 37 us so.
 // The three planes' corner value of F-matrix row i, column j of the transform
 // of S x S blocks at frame block (bxa, bya), group block (bxg, byg).
 template <int S, bool kEnc>
