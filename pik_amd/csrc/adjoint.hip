@@ -188,9 +188,10 @@ constexpr int kPW = 36;
 constexpr int kGW = 34;
 constexpr int kGPer = (kGW * kGW + 255) / 256;  // dG positions per thread
 
+template <bool kSearch>
 __global__ void __launch_bounds__(256, 4)
     KAdjBackward(FrameParams P, FrameBuffers B, const DeviceConsts* K,
-                 AdjArgs A) {
+                 AdjArgs A, SearchDist D) {
   // One LDS array for the buffers of all phases, 39 KB, so that four
   // workgroups share a CU (three with a buffer each): P's ring from 0,
   // dG's ring from kDg; then dP from 0 over the dead P, the transform's
@@ -388,8 +389,13 @@ __global__ void __launch_bounds__(256, 4)
       }
     }
   }
-  float mv[3][4] = {};
+  float mv[3][4] = {}, x[3][4];
   LoadMatrix(B, in, mv);
+  if (kSearch && in.valid) {
+    for (int c = 0; c < 3; ++c) {
+      LoadFour(D.coef + c * size_t(P.by) * P.bx * 64 + in.at, x[c]);
+    }
+  }
   __syncthreads();
 
   // 5. Transform transposes: forward transform, then the per-coefficient
@@ -402,6 +408,7 @@ __global__ void __launch_bounds__(256, 4)
   const CoefSlot S = MakeSlot(P, s_acs, tbx, tby, gxi * kGroupDimBlocks,
                               gyi * kGroupDimBlocks);
   float part = 0.0f;
+  float dist[4] = {};
   if (in.valid) {
     const float scaled = P.inv_global_scale / in.qf;
     float out[3][4];
@@ -421,12 +428,22 @@ __global__ void __launch_bounds__(256, 4)
       const float vx = DequantPlain(mv[0][j], scaled, 0, CoefQ(in.q4[0], j));
       const float vy = DequantPlain(mv[1][j], scaled, 1, CoefQ(in.q4[1], j));
       const float vb = DequantPlain(mv[2][j], scaled, 2, CoefQ(in.q4[2], j));
-      part += gx * vx + gyt * vy + gb * vb;
-      out[0][j] = gx;
-      out[1][j] = gyt;
-      out[2][j] = gb;
+      if (!kSearch) {
+        part += gx * vx + gyt * vy + gb * vb;
+        out[0][j] = gx;
+        out[1][j] = gyt;
+        out[2][j] = gb;
+        continue;
+      }
+      // the search's distortion (search.hip): gradient times quantization
+      // error in the total (after colour correlation) coefficient domain,
+      // where Y's gradient is its pre-correlation one minus the factors
+      // times X's and B's
+      dist[j] = gx * (in.cfx * vy + vx - x[0][j]) +
+                (gyt - in.cfx * gx - in.cfb * gb) * (vy - x[1][j]) +
+                gb * (in.cfb * vy + vb - x[2][j]);
     }
-    if (A.dcoef[0]) {
+    if (!kSearch && A.dcoef[0]) {
       for (int c = 0; c < 3; ++c) {
         float* dst = A.dcoef[c] + size_t(S.cby) * A.dc_pitch +
                      size_t(S.cbx) * 64 + (S.ccol & 63);
@@ -439,10 +456,20 @@ __global__ void __launch_bounds__(256, 4)
       }
     }
   }
-  // Sum over the 16 lanes of the block (all lanes take part).
-  for (int m = 8; m >= 1; m >>= 1) part += __shfl_xor(part, m, 64);
-  if (in.valid && (tid & 15) == 0) {
-    A.dqf[size_t(S.cby) * A.dqf_pitch + S.cbx] = -part / in.qf;
+  if (kSearch) {
+    // the block's 64 slots, pairwise over slot distances 32, 16, .. 1 (slot
+    // k = 4 lane + j)
+    for (int m = 8; m >= 1; m >>= 1) {
+      for (int j = 0; j < 4; ++j) dist[j] += __shfl_xor(dist[j], m, 64);
+    }
+    const float d = (dist[0] + dist[2]) + (dist[1] + dist[3]);
+    if (in.valid && (tid & 15) == 0) D.dist[S.cby * P.bx + S.cbx] = 0.5f * d;
+  } else {
+    // Sum over the 16 lanes of the block (all lanes take part).
+    for (int m = 8; m >= 1; m >>= 1) part += __shfl_xor(part, m, 64);
+    if (in.valid && (tid & 15) == 0) {
+      A.dqf[size_t(S.cby) * A.dqf_pitch + S.cbx] = -part / in.qf;
+    }
   }
 
   // 7. Tile loss partial.
@@ -456,20 +483,14 @@ __global__ void __launch_bounds__(256, 4)
   }
   if (B.stamps) StampEnd(B.stamps->end[1], blockIdx.x, gridDim.x);
 }
+template __global__ void KAdjBackward<false>(FrameParams, FrameBuffers,
+                                             const DeviceConsts*, AdjArgs, SearchDist);
+template __global__ void KAdjBackward<true>(FrameParams, FrameBuffers,
+                                            const DeviceConsts*, AdjArgs, SearchDist);
 
-// Sum of the per-tile loss partials in double (one workgroup).
 __global__ void __launch_bounds__(256)
     KAdjLoss(const float* part, int n, double* out) {
-  __shared__ double s[256];
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) acc += double(part[i]);
-  s[threadIdx.x] = acc;
-  __syncthreads();
-  for (int w = 128; w >= 1; w >>= 1) {
-    if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *out = s[0];
+  SumPartials(part, n, out);
 }
 
 }  // namespace pikgpu

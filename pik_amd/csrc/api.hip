@@ -1671,7 +1671,7 @@ int pikgpu_fwd_adj(pikgpu_ctx* ctx, const pikgpu_adj_io* io) {
   B.stamps = ctx->stamps;
   ctx->adj_due = true;
   KAdjForward<<<grid, 256, 0, st>>>(P, B, K, A);
-  KAdjBackward<<<grid, 256, 0, st>>>(P, B, K, A);
+  KAdjBackward<false><<<grid, 256, 0, st>>>(P, B, K, A, SearchDist());
   if (io->loss) KAdjLoss<<<1, 256, 0, st>>>(loss_part, tiles, loss_dev);
   HIP_TRY(ctx, hipGetLastError());
   // pikgpu_run's output is not what the device buffers hold any more.
@@ -1706,8 +1706,8 @@ int pikgpu_fwd_adj(pikgpu_ctx* ctx, const pikgpu_adj_io* io) {
 
 
 // Gradient quant-field search (see pikgpu.h): device-resident loop of
-// quantization (KEncQuant), forward + adjoint (KAdjForward / KAdjBackward),
-// distortion attribution (KSearchDist) and Adam (KSearchUpdate).
+// quantization and forward model (KSearchForward), adjoint with the
+// distortion's attribution (KAdjBackward) and Adam (KSearchStep).
 int pikgpu_search_quant_field(pikgpu_ctx* ctx,
                               const pikgpu_search_params* prm,
                               const pikgpu_search_io* io) {
@@ -1770,9 +1770,11 @@ int pikgpu_search_quant_field(pikgpu_ctx* ctx,
   const int steps = prm->steps;
   const int round_groups = int(DivCeil(nb, 256));
   const int tiles = int(DivCeil(bx, 4) * DivCeil(by, 4));
-  // search state: u, m, v, weight, dist, u0 (nb floats each), lambda, rate
-  // partials (round_groups floats), loss / rate histories (steps + 1 doubles)
-  const size_t hist_off = DivCeil((6 * nb + 1 + size_t(round_groups)) * 4, 8) * 8;
+  // search state: two copies of u, m, v, then weight, dist, u0 (nb floats
+  // each), lambda, two sets of rate partials (round_groups floats), loss /
+  // rate histories (steps + 1 doubles)
+  const size_t hist_off =
+      DivCeil((9 * nb + 1 + 2 * size_t(round_groups)) * 4, 8) * 8;
   int rc;
   if ((rc = Grow(ctx, &ctx->eopsin, 3 * plane * 4)) ||
       (rc = Grow(ctx, &ctx->ecoef, 3 * nb * 64 * 4)) ||
@@ -1780,8 +1782,6 @@ int pikgpu_search_quant_field(pikgpu_ctx* ctx,
       (rc = EnsureInverseTable(ctx)) ||
       (rc = Grow(ctx, &ctx->adj_qf, nb * 4)) ||
       (rc = Grow(ctx, &ctx->adj_in, 3 * tplane * 4)) ||
-      (rc = Grow(ctx, &ctx->adj_dqf, nb * 4)) ||
-      (rc = Grow(ctx, &ctx->adj_dc, 3 * nb * 64 * 4)) ||
       (rc = Grow(ctx, &ctx->adj_loss, size_t(tiles) * 4 + 16)) ||
       (rc = Grow(ctx, &ctx->srch, hist_off + 2 * size_t(steps + 1) * 8))) {
     return rc;
@@ -1796,14 +1796,23 @@ int pikgpu_search_quant_field(pikgpu_ctx* ctx,
       return rc;
     }
   }
-  float* st_u = static_cast<float*>(ctx->srch.p);
-  float* st_m = st_u + nb;
-  float* st_v = st_m + nb;
-  float* st_w = st_v + nb;
-  float* st_d = st_w + nb;
-  float* st_u0 = st_d + nb;
-  float* st_lam = st_u0 + nb;
-  float* st_rate = st_lam + 1;
+  float* at = static_cast<float*>(ctx->srch.p);
+  const auto take = [&](size_t n) {
+    float* p = at;
+    at += n;
+    return p;
+  };
+  SearchState state[2];
+  for (SearchState& q : state) {
+    q.u = take(nb);
+    q.m = take(nb);
+    q.v = take(nb);
+  }
+  float* st_w = take(nb);
+  float* st_d = take(nb);
+  float* st_u0 = take(nb);
+  float* st_lam = take(1);
+  float* const st_rate[2] = {take(round_groups), take(round_groups)};
   double* h_loss = reinterpret_cast<double*>(
       static_cast<char*>(ctx->srch.p) + hist_off);
   double* h_rate = h_loss + (steps + 1);
@@ -1825,7 +1834,6 @@ int pikgpu_search_quant_field(pikgpu_ctx* ctx,
   int16_t* dc16 = const_cast<int16_t*>(ctx->B.dc16);
   int32_t* qf = const_cast<int32_t*>(ctx->B.qf);
   float* qfr = static_cast<float*>(ctx->adj_qf.p);
-  float* grad = static_cast<float*>(ctx->adj_dc.p);
   // forward transforms and the DC: independent of the AC field
   KEncForward<<<tiles, 256, 0, st>>>(P, B, K, dev_opsin, coef, dcf);
   const float gsf = static_cast<float>(ctx->global_scale * (1.0 / 65536));
@@ -1838,8 +1846,8 @@ int pikgpu_search_quant_field(pikgpu_ctx* ctx,
   EnqueueDc(P, B, K, st);
   EnqueueLf(P, B, K, st, false);  // the LLF (CopyLlf) and the LF caches
   ctx->adj_ready = true;
-  KSearchInit<<<DivCeil(nb, 256), 256, 0, st>>>(P, B, st_u0, st_u, st_m,
-                                                  st_v);
+  KSearchInit<<<DivCeil(nb, 256), 256, 0, st>>>(P, B, st_u0, state[0].u,
+                                                state[0].m, state[0].v);
 
   AdjArgs A;
   memset(&A, 0, sizeof(A));
@@ -1847,14 +1855,10 @@ int pikgpu_search_quant_field(pikgpu_ctx* ctx,
   A.qf_pitch = int(bx);
   for (int c = 0; c < 3; ++c) {
     A.target[c] = target + c * tplane;
-    A.dcoef[c] = grad + c * nb * 64;
   }
   A.in_pitch = int(xs);
-  A.dqf = static_cast<float*>(ctx->adj_dqf.p);
-  A.dqf_pitch = int(bx);
-  A.dc_pitch = bx * 64;
-  A.dcoef_vec = 1;
   A.loss_part = static_cast<float*>(ctx->adj_loss.p);
+  const SearchDist D = {st_d, coef};
   SearchArgs S;
   S.weight = io->weight ? st_w : nullptr;
   S.lambda = st_lam;
@@ -1868,23 +1872,28 @@ int pikgpu_search_quant_field(pikgpu_ctx* ctx,
   S.dhi = std::log(prm->trust_high);
   const float* itable = static_cast<const float*>(ctx->itable.p);
   const int grid = XcdGrid(tiles);
+  KSearchRound<<<round_groups, 256, 0, st>>>(P, B, state[0].u, qmax, qf, qfr,
+                                             st_rate[0]);
   for (int t = 0; t <= steps; ++t) {
-    KSearchRound<<<round_groups, 256, 0, st>>>(P, B, st_u, qmax, qf, qfr,
-                                               st_rate);
-    KAdjLoss<<<1, 256, 0, st>>>(st_rate, round_groups, h_rate + t);
-    KEncQuant<<<grid, 256, 0, st>>>(P, B, coef, itable, gsf, ac16);
-    KAdjForward<<<grid, 256, 0, st>>>(P, B, K, A);
-    KAdjBackward<<<grid, 256, 0, st>>>(P, B, K, A);
-    KAdjLoss<<<1, 256, 0, st>>>(A.loss_part, tiles, h_loss + t);
-    if (t == steps) break;
-    KSearchDist<<<DivCeil(nb, 4), 256, 0, st>>>(P, B, coef, grad, st_d);
+    const SearchState &now = state[t & 1], &then = state[1 - (t & 1)];
+    float *rate = st_rate[t & 1], *next_rate = st_rate[1 - (t & 1)];
+    KSearchForward<<<grid, 256, 0, st>>>(P, B, coef, itable, gsf, ac16);
+    KAdjBackward<true><<<grid, 256, 0, st>>>(P, B, K, A, D);
+    if (t == steps) {
+      KAdjLoss<<<1, 256, 0, st>>>(A.loss_part, tiles, h_loss + t);
+      KAdjLoss<<<1, 256, 0, st>>>(rate, round_groups, h_rate + t);
+      break;
+    }
     if (t == 0) {
       KSearchLambda<<<1, 256, 0, st>>>(
           st_d, S.weight, int(nb), prm->lambda,
           prm->lambda < 0.0f ? -prm->lambda : 1.0f, st_lam);
     }
-    KSearchUpdate<<<DivCeil(nb, 256), 256, 0, st>>>(P, B, S, t + 1, st_d,
-                                                    st_u0, st_u, st_m, st_v);
+    const SearchSums sums = {A.loss_part, rate,       tiles, round_groups,
+                             h_loss + t,  h_rate + t};
+    KSearchStep<<<round_groups + 2, 256, 0, st>>>(P, B, S, t + 1, st_d, st_u0,
+                                                  now, then, qmax, qf, qfr,
+                                                  next_rate, sums);
   }
   HIP_TRY(ctx, hipGetLastError());
   // outputs

@@ -222,19 +222,21 @@ __device__ inline void DitherChain(float* val, int s, int r8, bool active,
 // steps), and X and B run at the same time on the two halves of the
 // workgroup once Y's dequantised values are out: 30 steps in all
 // (20 us and 43 us).
-__global__ void __launch_bounds__(256)
-    KEncQuant(FrameParams P, FrameBuffers B, const float* coef,
-              const float* itable, float gsf, int16_t* ac) {
-  __shared__ float s_val[2][kCoefPlane];
-  __shared__ uint32_t s_off[3][16];
-  __shared__ float s_qac[16], s_inv[16];
-  __shared__ uint8_t s_acs[16];
+//
+// Block (tbx, tby) is the tile's first; s_val holds two coefficient planes.
+// The thread's four quantized values of each channel (of slot S) are left in
+// q. All 256 threads call.
+struct EncShared {
+  uint32_t off[3][16];
+  float qac[16], inv[16];
+  uint8_t acs[16];
+};
+__device__ inline CoefSlot QuantizeTile(
+    const FrameParams& P, const FrameBuffers& B, const float* coef,
+    const float* itable, float gsf, int16_t* ac, int tbx, int tby,
+    float (*s_val)[kCoefPlane], EncShared* sh, int16_t (&q)[3][4]) {
   constexpr float kZeroBias[3] = {0.65f, 0.6f, 0.7f};
   const int tid = threadIdx.x;
-  const int tiles_x = (P.bx + 3) / 4;
-  const int tile = XcdTile(blockIdx.x, tiles_x * ((P.by + 3) / 4));
-  if (tile < 0) return;
-  const int tbx = (tile % tiles_x) * 4, tby = (tile / tiles_x) * 4;
   // a 32x32 tile lies in one colour tile
   const int ctile = (tby >> 3) * P.tx + (tbx >> 3);
   if (tid < 16) {
@@ -247,19 +249,19 @@ __global__ void __launch_bounds__(256)
       const int quant = B.qf[size_t(y0) * P.bx + x0];
       const int table = B.dqmap[B.dcf[ctile] * 256 + quant];
       for (int c = 0; c < 3; ++c) {
-        s_off[c][tid] =
+        sh->off[c][tid] =
             B.offsets[(table * kNumQuantKinds + AcsQuantKind(raw)) * 3 + c];
       }
-      s_qac[tid] = gsf * quant;
-      s_inv[tid] = P.inv_global_scale / quant;
+      sh->qac[tid] = gsf * quant;
+      sh->inv[tid] = P.inv_global_scale / quant;
     }
-    s_acs[tid] = a;
+    sh->acs[tid] = a;
   }
   __syncthreads();
   // four consecutive coefficients of one storage block per thread
   const int gxi = tbx / kGroupDimBlocks, gyi = tby / kGroupDimBlocks;
   const int g = gyi * P.gx + gxi;
-  const CoefSlot S = MakeSlot(P, s_acs, tbx, tby, gxi * kGroupDimBlocks,
+  const CoefSlot S = MakeSlot(P, sh->acs, tbx, tby, gxi * kGroupDimBlocks,
                               gyi * kGroupDimBlocks);
   const int e = CoefAt(S.crow, S.ccol);
   const size_t plane = size_t(P.by) * P.bx * 64;
@@ -269,15 +271,15 @@ __global__ void __launch_bounds__(256)
   float inv_qac = 0.0f;
   if (S.valid) {
     const int own = S.crow * 4 + (S.ccol >> 6);
-    const float qac = s_qac[own];
-    inv_qac = s_inv[own];
+    const float qac = sh->qac[own];
+    inv_qac = sh->inv[own];
     for (int c = 0; c < 3; ++c) {
       const float4 q = *reinterpret_cast<const float4*>(coef + c * plane + at);
       v[c][0] = q.x;
       v[c][1] = q.y;
       v[c][2] = q.z;
       v[c][3] = q.w;
-      const float* m = itable + s_off[c][own] + S.cflat0;
+      const float* m = itable + sh->off[c][own] + S.cflat0;
       const float* llf = B.llf + (size_t(g) * 3 + c) * kLlfPlane;
       for (int j = 0; j < 4; ++j) {
         qm[c][j] = m[j] * qac;
@@ -288,14 +290,14 @@ __global__ void __launch_bounds__(256)
       }
     }
     for (int j = 0; j < 4; ++j) {
-      dm[j] = B.table[s_off[1][own] + S.cflat0 + j];
+      dm[j] = B.table[sh->off[1][own] + S.cflat0 + j];
       s_val[0][e + j] = v[1][j] * qm[1][j];
     }
   }
   __syncthreads();
   // the chains: lanes 8 sub .. 8 sub + 7 of a half of the workgroup
   const int sub = (tid >> 3) & 15, r8 = tid & 7, half = tid >> 7;
-  const uint8_t a = s_acs[sub];
+  const uint8_t a = sh->acs[sub];
   int s = 1, row0 = 0;
   if (a != 0xFF) {
     s = AcsCovered(a >> 4);
@@ -310,14 +312,13 @@ __global__ void __launch_bounds__(256)
     const float fac[3] = {
         1.0f * float(B.ytox[ctile] - 128) * (1.0f / 256), 0.0f,
         1.0f * float(B.ytob[ctile] - 0) * (1.0f / 128)};
-    short4 q;
     float yd[4];
-    int16_t* qp = reinterpret_cast<int16_t*>(&q);
     for (int j = 0; j < 4; ++j) {
-      qp[j] = int16_t(s_val[0][e + j]);
-      yd[j] = AdjustQuantBiasInt(1, qp[j]) * dm[j] * inv_qac;
+      q[1][j] = int16_t(s_val[0][e + j]);
+      yd[j] = AdjustQuantBiasInt(1, q[1][j]) * dm[j] * inv_qac;
     }
-    *reinterpret_cast<short4*>(ac + plane + at) = q;
+    *reinterpret_cast<short4*>(ac + plane + at) =
+        make_short4(q[1][0], q[1][1], q[1][2], q[1][3]);
     for (int j = 0; j < 4; ++j) {
       s_val[0][e + j] = (v[0][j] - fac[0] * yd[j]) * qm[0][j];
       s_val[1][e + j] = (v[2][j] - fac[2] * yd[j]) * qm[2][j];
@@ -329,13 +330,92 @@ __global__ void __launch_bounds__(256)
   __syncthreads();
   if (S.valid) {
     for (int h = 0; h < 2; ++h) {
-      short4 q;
-      int16_t* qp = reinterpret_cast<int16_t*>(&q);
-      for (int j = 0; j < 4; ++j) qp[j] = int16_t(s_val[h][e + j]);
-      *reinterpret_cast<short4*>(ac + 2 * h * plane + at) = q;
+      int16_t (&v)[4] = q[2 * h];
+      for (int j = 0; j < 4; ++j) v[j] = int16_t(s_val[h][e + j]);
+      *reinterpret_cast<short4*>(ac + 2 * h * plane + at) =
+          make_short4(v[0], v[1], v[2], v[3]);
     }
   }
+  return S;
+}
+
+__global__ void __launch_bounds__(256)
+    KEncQuant(FrameParams P, FrameBuffers B, const float* coef,
+              const float* itable, float gsf, int16_t* ac) {
+  __shared__ float s_val[2][kCoefPlane];
+  __shared__ EncShared sh;
+  const int tiles_x = (P.bx + 3) / 4;
+  const int tile = XcdTile(blockIdx.x, tiles_x * ((P.by + 3) / 4));
+  if (tile < 0) return;
+  int16_t q[3][4];
+  QuantizeTile(P, B, coef, itable, gsf, ac, (tile % tiles_x) * 4,
+               (tile / tiles_x) * 4, s_val, &sh, q);
   if (B.stamps) StampEnd(B.stamps->end[2], blockIdx.x, gridDim.x);
+}
+
+// A step's quantization and forward model in one (KEncQuant, KAdjForward
+// without predictions): the tile's quantized values go from registers through
+// the dequantisation of the decoder (the descriptors of the current field)
+// and the inverse transforms to the IDCT image. Bound by the dither
+// chains' latency (as KEncQuant); on a 1024x1024 image 33 us, 21 + 18 us as two
+// kernels with the values through memory.
+__global__ void __launch_bounds__(256, 4)
+    KSearchForward(FrameParams P, FrameBuffers B, const float* coef,
+                   const float* itable, float gsf, int16_t* ac) {
+  __shared__ float s_coef[3][kCoefPlane];
+  __shared__ float s_pix[3][kTilePlane];
+  __shared__ float s_tmp[3][kTilePlane];
+  __shared__ EncShared sh;
+  __shared__ TileTasks s_inv;
+  static_assert(2 * kCoefPlane <= 3 * kTilePlane, "s_val in s_tmp");
+  float (*s_val)[kCoefPlane] = reinterpret_cast<float (*)[kCoefPlane]>(&s_tmp[0][0]);
+  const int tid = threadIdx.x;
+  const int tiles_x = (P.bx + 3) / 4;
+  const int tile = XcdTile(blockIdx.x, tiles_x * ((P.by + 3) / 4));
+  if (tile < 0) return;
+  const int tbx = (tile % tiles_x) * 4, tby = (tile / tiles_x) * 4;
+  int16_t q[3][4];
+  const CoefSlot S = QuantizeTile(P, B, coef, itable, gsf, ac, tbx, tby, s_val,
+                                  &sh, q);
+  if (S.valid) {
+    const uint4 d = B.desc[2 * (S.cby * P.bx + S.cbx)];
+    const uint32_t slot[3] = {d.x, d.y, d.z};
+    const float scaled = __uint_as_float(d.w);
+    const int ctile = (tby >> 3) * P.tx + (tbx >> 3);
+    const float cc[3] = {float(B.ytox[ctile] - 128) * 0.00390625f, 0.0f,
+                         float(B.ytob[ctile]) * 0.0078125f};
+    const int g = (tby / kGroupDimBlocks) * P.gx + tbx / kGroupDimBlocks;
+    float yv[4];
+    for (int ci = 0; ci < 3; ++ci) {
+      const int c = ci == 0 ? 1 : (ci == 1 ? 0 : 2);
+      const float* llf = B.llf + (size_t(g) * 3 + c) * kLlfPlane;
+      float m[4];
+      LoadFour(B.table + slot[c] + (S.ccol & 63), m);
+      for (int j = 0; j < 4; ++j) {
+        // DequantWith's operation order
+        const float v0 = AdjustQuantBias(c, float(q[c][j])) * (m[j] * scaled);
+        float v = c == 1 ? v0 : cc[c] * yv[j] + v0;
+        if (c == 1) yv[j] = v;
+        const int flat = S.cflat0 + j;
+        const int fi = flat >> S.lgn, fj = flat & (S.cN - 1);
+        if (fi < S.cs && fj < S.cs) {
+          v = llf[(S.obyg + 1 + fi) * kLlfPitch + S.obxg + 1 + fj];
+        }
+        s_coef[c][CoefAt(S.crow, S.ccol + j)] = v;
+      }
+    }
+  }
+  BuildTasks(sh.acs, false, &s_inv);
+  TileInverse3(s_inv, &s_coef[0][0], &s_pix[0][0], &s_tmp[0][0]);
+  const int pr = tid >> 3, pc0 = (tid & 7) << 2;
+  const int py = tby * 8 + pr, px = tbx * 8 + pc0;
+  if (py < P.py && px < P.px) {
+    for (int c = 0; c < 3; ++c) {
+      const float* s = s_pix[c] + PixAt(pr, pc0);
+      *reinterpret_cast<float4*>(B.idct + (size_t(c) * P.py + py) * B.ipitch +
+                                 px) = make_float4(s[0], s[1], s[2], s[3]);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------

@@ -209,6 +209,20 @@ __device__ inline void GroupMinMax(float* lo, float* hi, float* s) {
   *hi = fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7]));
 }
 
+// Sum of n partials in double by one workgroup of 256 threads.
+__device__ inline void SumPartials(const float* part, int n, double* out) {
+  __shared__ double s[256];
+  double acc = 0.0;
+  for (int i = threadIdx.x; i < n; i += 256) acc += double(part[i]);
+  s[threadIdx.x] = acc;
+  __syncthreads();
+  for (int w = 128; w >= 1; w >>= 1) {
+    if (threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *out = s[0];
+}
+
 // ---------------------------------------------------------------------------
 // Cooperative transforms of the three channels of a 32x32 tile (256
 // threads). The 2-D transforms are the reference's two column passes with a
@@ -548,7 +562,7 @@ __device__ inline ThreadTasks AssignTasks(const TileTasks& T) {
 
 // coef (3 x kCoefPlane) -> pix (3 x kTilePlane), tmp 3 x kTilePlane. All
 // 256 threads must call.
-__device__ inline void TileInverse3(const ThreadTasks& m, const float* coef,
+__device__ __forceinline__ void TileInverse3(const ThreadTasks& m, const float* coef,
                                     float* pix, float* tmp) {
   for (int pass = 0; pass < 2; ++pass) {
 #pragma unroll 1
@@ -564,7 +578,7 @@ __device__ inline void TileInverse3(const ThreadTasks& m, const float* coef,
     __syncthreads();
   }
 }
-__device__ inline void TileInverse3(const TileTasks& T, const float* coef,
+__device__ __forceinline__ void TileInverse3(const TileTasks& T, const float* coef,
                                     float* pix, float* tmp) {
   TileInverse3(AssignTasks(T), coef, pix, tmp);
 }
@@ -573,7 +587,7 @@ __device__ inline void TileInverse3(const TileTasks& T, const float* coef,
 // (others keep their coefficient entries), tmp 3 x kTilePlane. All 256
 // threads must call.
 template <bool kAdjoint = false, bool kAddHF = false, bool kSubHF = false>
-__device__ inline void TileForward3(const ThreadTasks& m, const float* pix,
+__device__ __forceinline__ void TileForward3(const ThreadTasks& m, const float* pix,
                                     float* coef, float* tmp) {
   // pass 2 (the DCT4X4 DC Hadamard) only when the tile has a DCT4X4
   const int passes = kAddHF ? 2 : (m.has_dct4 ? 3 : 2);
@@ -593,7 +607,7 @@ __device__ inline void TileForward3(const ThreadTasks& m, const float* pix,
   }
 }
 template <bool kAdjoint = false, bool kAddHF = false, bool kSubHF = false>
-__device__ inline void TileForward3(const TileTasks& T, const float* pix,
+__device__ __forceinline__ void TileForward3(const TileTasks& T, const float* pix,
                                     float* coef, float* tmp) {
   TileForward3<kAdjoint, kAddHF, kSubHF>(AssignTasks(T), pix, coef, tmp);
 }
@@ -828,6 +842,9 @@ __global__ void KEncDc(FrameParams P, const float* dcf, EncDcScale S,
                        int16_t* dc16);
 __global__ void KEncQuant(FrameParams P, FrameBuffers B, const float* coef,
                           const float* itable, float gsf, int16_t* ac);
+__global__ void KSearchForward(FrameParams P, FrameBuffers B,
+                               const float* coef, const float* itable,
+                               float gsf, int16_t* ac);
 __global__ void KEncLf(FrameParams P, FrameBuffers B, float* coef,
                        const float* itable, float gsf, float* corner);
 __global__ void KEncHfResidual(FrameParams P, FrameBuffers B, float* coef);
@@ -852,8 +869,16 @@ __global__ void KPred2x2(FrameParams P, FrameBuffers B, const DeviceConsts* K,
 __global__ void KBlocks(FrameParams P, FrameBuffers B, const DeviceConsts* K);
 __global__ void KAdjForward(FrameParams P, FrameBuffers B,
                             const DeviceConsts* K, AdjArgs A);
+// <true>: the quant-field search's, which leaves each block's distortion (from
+// the unquantized coefficients, three planes in the AC layout) instead of the
+// gradients.
+struct SearchDist {
+  float* dist;
+  const float* coef;
+};
+template <bool kSearch>
 __global__ void KAdjBackward(FrameParams P, FrameBuffers B,
-                             const DeviceConsts* K, AdjArgs A);
+                             const DeviceConsts* K, AdjArgs A, SearchDist D);
 __global__ void KAdjLoss(const float* part, int n, double* out);
 
 // Parameters of one Adam step of the quant-field search (search.hip).
@@ -866,11 +891,22 @@ struct SearchArgs {
 };
 __global__ void KSearchRound(FrameParams P, FrameBuffers B, const float* u,
                              int qmax, int32_t* qf, float* qfr, float* part);
-__global__ void KSearchDist(FrameParams P, FrameBuffers B, const float* coef,
-                            const float* grad, float* dist);
-__global__ void KSearchUpdate(FrameParams P, FrameBuffers B, SearchArgs S,
-                              int t, const float* dist, const float* u0,
-                              float* u, float* m, float* v);
+// The search's state at each transform's first block: log field and Adam
+// moments. A step reads one copy and writes the other.
+struct SearchState {
+  float *u, *m, *v;
+};
+// The partials of the evaluation before a step, and where their sums go.
+struct SearchSums {
+  const float *loss_part, *rate_part;
+  int loss_n, rate_n;
+  double *loss, *rate;
+};
+__global__ void KSearchStep(FrameParams P, FrameBuffers B, SearchArgs S, int t,
+                            const float* dist, const float* u0,
+                            SearchState from, SearchState to, int qmax,
+                            int32_t* qf, float* qfr, float* rate_part,
+                            SearchSums sums);
 __global__ void KSearchInit(FrameParams P, FrameBuffers B, float* u0, float* u,
                             float* m, float* v);
 __global__ void KSearchLambda(const float* dist, const float* weight, int n,

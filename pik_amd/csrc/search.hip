@@ -1,7 +1,7 @@
 // Gradient quant-field search (pikgpu_search_quant_field): the kernels of
-// one Adam step on the log quant field, between the encoder's quantization
-// (KEncQuant) and the forward + adjoint of the decode (KAdjForward /
-// KAdjBackward).
+// one Adam step on the log quant field, beside the quantization with the
+// forward model (KSearchForward) and the adjoint (KAdjBackward, which also
+// attributes the distortion below).
 //
 // The reference searches the field by repeated round trips judged by
 // Butteraugli (FindBestQuantization, pik/adaptive_quantization.cc:677-853);
@@ -24,98 +24,111 @@
 
 namespace pikgpu {
 
-// Integer field from the log field: each block takes its transform's value
-// (stored at the transform's first block), rounded and clamped to
-// [1, qmax]; `qfr` receives it as float for the adjoint, and the block's
-// dequantisation descriptors follow it. Per workgroup the sum of log(qf)
-// (the rate proxy) goes to `part`.
-__global__ void __launch_bounds__(256)
-    KSearchRound(FrameParams P, FrameBuffers B, const float* u, int qmax,
-                 int32_t* qf, float* qfr, float* part) {
+// Block i's integer field value from its transform's log field u, rounded and
+// clamped to [1, qmax]; `qfr` receives it as float for the adjoint, and the
+// block's dequantisation descriptors follow it. Returns its log (the rate
+// proxy).
+__device__ inline float RoundField(const FrameParams& P, const FrameBuffers& B,
+                                   int i, float u, int qmax, int32_t* qf,
+                                   float* qfr) {
+  const float v = rintf(__expf(u));
+  const int q = int(fminf(fmaxf(v, 1.0f), float(qmax)));
+  qf[i] = q;
+  qfr[i] = float(q);
+  // every block of a transform has the same value
+  WriteBlockDesc(P, B, i, q, q);
+  return __logf(float(q));
+}
+// The workgroup's sum of lq to part[wg].
+__device__ inline void RatePartial(float lq, int wg, float* part) {
   __shared__ float s[4];
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  float lq = 0.0f;
-  if (i < P.bx * P.by) {
-    const int y = i / P.bx, x = i - y * P.bx;
-    const uint8_t a = B.acs[i];
-    const int sc = AcsCovered(a >> 4), idx = a & 15;
-    const int fy = y - idx / sc, fx = x - idx % sc;
-    const float v = rintf(__expf(u[fy * P.bx + fx]));
-    const int q = int(fminf(fmaxf(v, 1.0f), float(qmax)));
-    qf[i] = q;
-    qfr[i] = float(q);
-    // every block of a transform has the same value
-    WriteBlockDesc(P, B, i, q, q);
-    lq = __logf(float(q));
-  }
   for (int m = 32; m >= 1; m >>= 1) lq += __shfl_xor(lq, m, 64);
   if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = lq;
   __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = (s[0] + s[1]) + (s[2] + s[3]);
+  if (threadIdx.x == 0) part[wg] = (s[0] + s[1]) + (s[2] + s[3]);
 }
 
-// Distortion attributed to each storage block (one wave per block, lane k
-// = coefficient slot k; `coef` and `grad` hold three planes in the AC
-// layout): D_b = 1/2 sum over k and the three channels of
-// g e, in the total (after colour correlation) coefficient domain. The
-// adjoint's gradients for X and B are already in that domain; Y's total
-// gradient is its pre-correlation one minus the correlation factors times
-// X's and B's. LLF slots have g = 0.
-__global__ void __launch_bounds__(256)
-    KSearchDist(FrameParams P, FrameBuffers B, const float* coef,
-                const float* grad, float* dist) {
-  const int b = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int k = threadIdx.x & 63;
-  if (b >= P.bx * P.by) return;
-  const int y = b / P.bx, x = b - y * P.bx;
-  const size_t plane = size_t(P.by) * P.bx * 64;
-  const size_t at = size_t(b) * 64 + k;
-  const BlockDq dx = MakeBlockDq(P, B, 0, y, x);
-  const BlockDq dy = MakeBlockDq(P, B, 1, y, x);
-  const BlockDq db = MakeBlockDq(P, B, 2, y, x);
-  const float vy = DequantWith(dy, 1, B.ac[plane + at], k, 0.0f);
-  const float vx = DequantWith(dx, 0, B.ac[at], k, vy);
-  const float vb = DequantWith(db, 2, B.ac[2 * plane + at], k, vy);
-  const float gx = grad[at], gyt = grad[plane + at], gb = grad[2 * plane + at];
-  const float gy = gyt - dx.cc * gx - db.cc * gb;
-  float d = gx * (vx - coef[at]) + gy * (vy - coef[plane + at]) +
-            gb * (vb - coef[2 * plane + at]);
-  for (int m = 32; m >= 1; m >>= 1) d += __shfl_xor(d, m, 64);
-  if (k == 0) dist[b] = 0.5f * d;
-}
-
-// One Adam step (step number t >= 1) on each transform's log field, at its
-// first block: gradient sum over the covered blocks of -2 w D + lambda;
-// u clamped to [ulo, uhi] and to the trust region [u0 + dlo, u0 + dhi]
-// around its initial value u0.
-__global__ void __launch_bounds__(256)
-    KSearchUpdate(FrameParams P, FrameBuffers B, SearchArgs S, int t,
-                  const float* dist, const float* u0, float* u, float* m,
-                  float* v) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= P.bx * P.by) return;
+// First block of block i's transform.
+struct FirstOf {
+  int x, y, size;  // first block, covered blocks per side
+};
+__device__ inline FirstOf FirstBlockOf(const FrameParams& P,
+                                       const FrameBuffers& B, int i) {
   const uint8_t a = B.acs[i];
-  if ((a & 15) != 0) return;
-  const int sc = AcsCovered(a >> 4);
-  const int y = i / P.bx, x = i - y * P.bx;
-  float g = 0.0f;
-  for (int iy = 0; iy < sc; ++iy) {
-    for (int ix = 0; ix < sc; ++ix) {
-      const int j = (y + iy) * P.bx + x + ix;
-      const float w = S.weight ? S.weight[j] : 1.0f;
-      g += *S.lambda - 2.0f * w * dist[j];
-    }
+  FirstOf f;
+  f.size = AcsCovered(a >> 4);
+  const int idx = a & 15, y = i / P.bx, x = i - y * P.bx;
+  f.y = y - idx / f.size;
+  f.x = x - idx % f.size;
+  return f;
+}
+
+// The integer field of the initial log field.
+__global__ void __launch_bounds__(256)
+    KSearchRound(FrameParams P, FrameBuffers B, const float* u, int qmax,
+                 int32_t* qf, float* qfr, float* part) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  float lq = 0.0f;
+  if (i < P.bx * P.by) {
+    const FirstOf f = FirstBlockOf(P, B, i);
+    lq = RoundField(P, B, i, u[f.y * P.bx + f.x], qmax, qf, qfr);
   }
-  const float mi = S.beta1 * m[i] + (1.0f - S.beta1) * g;
-  const float vi = S.beta2 * v[i] + (1.0f - S.beta2) * g * g;
-  m[i] = mi;
-  v[i] = vi;
-  const float mh = mi / (1.0f - powf(S.beta1, float(t)));
-  const float vh = vi / (1.0f - powf(S.beta2, float(t)));
-  const float ui = u[i] - S.lr * mh / (sqrtf(vh) + S.eps);
-  const float lo = fmaxf(S.ulo, u0[i] + S.dlo);
-  const float hi = fminf(S.uhi, u0[i] + S.dhi);
-  u[i] = fminf(fmaxf(ui, lo), hi);
+  RatePartial(lq, blockIdx.x, part);
+}
+
+// One Adam step (step number t >= 1) on each transform's log field and the
+// integer field of the result: gradient sum over the transform's blocks of
+// -2 w D + lambda; u clamped to [ulo, uhi] and to the trust region [u0 + dlo,
+// u0 + dhi] around its initial value u0. Every block of a transform computes
+// its step from the old state (at the first block), so that the rounding
+// needs no other block's result, and the first block keeps it; the last two
+// workgroups sum the partials of the evaluation before. An update, a
+// rounding and two sums of their own took 20 us in four launches, this 7 us
+// (1024x1024 image); a step with the distortion in KAdjBackward and the
+// forward model in KSearchForward 69 us instead of 98.
+__global__ void __launch_bounds__(256)
+    KSearchStep(FrameParams P, FrameBuffers B, SearchArgs S, int t,
+                const float* dist, const float* u0, SearchState from,
+                SearchState to, int qmax, int32_t* qf, float* qfr,
+                float* rate_part, SearchSums sums) {
+  const int groups = int(gridDim.x) - 2;
+  if (int(blockIdx.x) >= groups) {
+    if (int(blockIdx.x) == groups) {
+      SumPartials(sums.loss_part, sums.loss_n, sums.loss);
+    } else {
+      SumPartials(sums.rate_part, sums.rate_n, sums.rate);
+    }
+    return;
+  }
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  float lq = 0.0f;
+  if (i < P.bx * P.by) {
+    const FirstOf f = FirstBlockOf(P, B, i);
+    const int i0 = f.y * P.bx + f.x;
+    float g = 0.0f;
+    for (int iy = 0; iy < f.size; ++iy) {
+      for (int ix = 0; ix < f.size; ++ix) {
+        const int j = (f.y + iy) * P.bx + f.x + ix;
+        const float w = S.weight ? S.weight[j] : 1.0f;
+        g += *S.lambda - 2.0f * w * dist[j];
+      }
+    }
+    const float mi = S.beta1 * from.m[i0] + (1.0f - S.beta1) * g;
+    const float vi = S.beta2 * from.v[i0] + (1.0f - S.beta2) * g * g;
+    const float mh = mi / (1.0f - powf(S.beta1, float(t)));
+    const float vh = vi / (1.0f - powf(S.beta2, float(t)));
+    const float ui = from.u[i0] - S.lr * mh / (sqrtf(vh) + S.eps);
+    const float lo = fmaxf(S.ulo, u0[i0] + S.dlo);
+    const float hi = fminf(S.uhi, u0[i0] + S.dhi);
+    const float u = fminf(fmaxf(ui, lo), hi);
+    if (i == i0) {
+      to.m[i] = mi;
+      to.v[i] = vi;
+      to.u[i] = u;
+    }
+    lq = RoundField(P, B, i, u, qmax, qf, qfr);
+  }
+  RatePartial(lq, blockIdx.x, rate_part);
 }
 
 // The rate weight: `fixed` when positive, else kappa times the mean over
