@@ -915,6 +915,10 @@ static int EnsureStageBuffers(pikgpu_ctx* ctx) {
   return PIKGPU_OK;
 }
 
+static int DcEpfGrid(const Img& dci) {
+  return XcdGrid(int(DivCeil(dci.W, 32) * DivCeil(dci.H, kDcEpfRows)));
+}
+
 // DC: dequant with the DC image's range, EPF + clamp
 // (DequantDC + AdaptiveDCReconstruction).
 static void EnqueueDc(const FrameParams& P, const FrameBuffers& B,
@@ -922,9 +926,7 @@ static void EnqueueDc(const FrameParams& P, const FrameBuffers& B,
   const int nblk = P.bx * P.by, groups = DcGroups(nblk);
   KDcDequant<<<groups, 256, 0, st>>>(P, B);
   const Img dci = DcImage(P, B);
-  const int grid = XcdGrid(int(DivCeil(dci.W, 32) * DivCeil(dci.H, 32)));
-  KEpf<true><<<grid, 256, 0, st>>>(dci, P, B, K, groups, B.dc, P.bx,
-                                   size_t(nblk));
+  KDcEpf<<<DcEpfGrid(dci), 256, 0, st>>>(dci, P, B, K, groups);
 }
 
 // LF-domain predictions per group: LLF, LF predictions (predict_lf) and with
@@ -973,7 +975,7 @@ hipError_t pikgpu::EnqueueFullSize(const FrameParams& P,
     }
     const int grid = XcdGrid(int(DivCeil(P.px, 32) * DivCeil(P.py, 32)));
     KGuide<<<grid, 256, 0, st>>>(ii, gab, P, B, MinMaxInline(partials));
-    KEpf<false><<<grid, 256, 0, st>>>(ii, P, B, K, 0, B.ar, B.ipitch, iplane);
+    KEpf<<<grid, 256, 0, st>>>(ii, P, B, K);
   } else {
     KCopyPlanes<<<DivCeil(3 * iplane, 256), 256, 0, st>>>(B, 3 * iplane);
   }
@@ -1960,7 +1962,7 @@ const BatchPhaseDef kBatchPhases[PIKGPU_BATCH_PHASES] = {
     {"dc_dequant", KDcDequantBatch, true},
     {"dc_minmax", nullptr, false},        // in dc_dequant
     {"dc_minmax_final", nullptr, false},  // in dc_epf
-    {"dc_epf", KEpfDcBatch, false},
+    {"dc_epf", KDcEpfBatch, false},
     {"llf", KLfBatch, false, kLfThreads},
     {"lf_blur", nullptr, false},          // in llf
     {"lf_from_dc2x2", nullptr, false},    // in llf
@@ -2045,7 +2047,7 @@ bool PhaseGrid(int p, const FrameParams& P, const FrameBuffers& B, int* nx,
       *nx = DcGroups(nblk);
       return true;
     case 3:  // dc_epf
-      *nx = XcdGrid(int(DivCeil(dci.W, 32) * DivCeil(dci.H, 32)));
+      *nx = DcEpfGrid(dci);
       arg[0] = DcGroups(nblk);
       return true;
     case 4:  // llf

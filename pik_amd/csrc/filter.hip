@@ -453,39 +453,168 @@ __global__ void __launch_bounds__(256)
 }
 
 // ---------------------------------------------------------------------------
-// EPF (+ AR clamp) on one 32x32 tile. dc_mode: the image is the 8-padded DC
-// image (constant quant field QuantDC/2, lut 0, DCT8 everywhere), no AR, and
-// the result is clamped to +-half a DC step and written to B.dc.
+// EPF of the 8-padded DC image (constant quant field QuantDC/2, lut 0), the
+// result clamped to +-half a DC step, to B.dc. A workgroup filters 32 x 8
+// pixels, one per thread, and quantises its guide itself (no Gaborish on the
+// DC image) with the range of KDcDequant's min/max partials (at most kDcGroups
+// of them). Every decode waits for this kernel, and the DC image of all but
+// the largest frames leaves most of the chip idle: bound by latency, so the
+// tile is small and a thread's chain short. On tiles of 32 x 32 with four
+// pixels per thread (as KEpf) it took 20 us for frames up to 1024 x 1024 and
+// 22 us for 4096 x 4096, 11 and 20 us so.
+__device__ __forceinline__ void KDcEpfBody(
+    Img in, const FrameParams& P, const FrameBuffers& B,
+    const DeviceConsts* K, int n_partial, const VBlock& vb) {
+  // the pixels with a 7-pixel border; the guide with a 6-pixel one
+  constexpr int kRows = kDcEpfRows + 14, kCols = 46, kP = 48;
+  constexpr int kGRows = kDcEpfRows + 12;
+  __shared__ float s_in[3][kRows * kP];
+  __shared__ __attribute__((aligned(4))) uint8_t s_g[3][kGRows * kP];
+  __shared__ float s_mm[8];
+  const int tid = threadIdx.x;
+  const int tiles_x = (in.W + 31) / 32;
+  const int tile =
+      XcdTile(vb.x, tiles_x * ((in.H + kDcEpfRows - 1) / kDcEpfRows));
+  if (tile < 0) return;
+  const int x0 = (tile % tiles_x) * 32, y0 = (tile / tiles_x) * kDcEpfRows;
+  // One reflection gives the mirror for every position within 7 of the image
+  // (at least 8 wide and high); positions further out are only clamped into
+  // it, their values are never used.
+  constexpr int kWin = 3 * kRows * kCols, kPer = (kWin + 255) / 256;
+  float wv[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int i = tid + u * 256;
+    wv[u] = 0.0f;
+    if (i < kWin) {
+      const int row = i / kCols, lx = i - row * kCols;
+      const int c = row / kRows, ly = row - c * kRows;
+      int x = x0 - 7 + lx, y = y0 - 7 + ly;
+      x = x < 0 ? -x - 1 : (x >= in.W ? 2 * in.W - 1 - x : x);
+      y = y < 0 ? -y - 1 : (y >= in.H ? 2 * in.H - 1 - y : y);
+      x = min(max(x, 0), in.vw - 1);
+      y = min(max(y, 0), in.vh - 1);
+      wv[u] = in.p[c * in.plane + size_t(y) * in.pitch + x];
+    }
+  }
+  const GuideScale gs = ReducePartials(B.mm_partial, n_partial, s_mm);
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int i = tid + u * 256;
+    if (i < kWin) {
+      const int row = i / kCols, lx = i - row * kCols;
+      const int c = row / kRows, ly = row - c * kRows;
+      s_in[c][ly * kP + lx] = wv[u];
+      // MakeGuide
+      if (ly >= 1 && ly <= kGRows && lx >= 1 && lx <= 44) {
+        const float scaled = (wv[u] - gs.all_min) * gs.gmul;
+        s_g[c][(ly - 1) * kP + lx - 1] =
+            static_cast<uint8_t>(static_cast<int>(scaled));
+      }
+    }
+  }
+  __syncthreads();
+  const int r = tid >> 5, col = tid & 31;
+  const int x = x0 + col, y = y0 + r;
+  if (x >= P.bx || y >= P.by) return;  // the unpadded region
+  const int sigma =
+      SigmaFromQuant(float(P.dc_qf) * 1.0f * 0.039324273f, gs.gmul, 0);
+  float d[3];
+  const float* mid = &s_in[0][(r + 7) * kP + col + 7];
+  if (sigma < kMinSigma) {
+    for (int c = 0; c < 3; ++c) d[c] = mid[c * kRows * kP];
+  } else {
+    // KEpf's filter: the neighbours' SADs from quad-SADs of byte-shifted
+    // windows, maximum over the channels, weights, weighted mean
+    const int mul64 = (K->mul_table[sigma] * 64 << 8) >> 8;
+    const int wq = (col + 2) & ~3, ws = (col + 2) & 3;
+    const int rq = (col + 5) & ~3, rs = (col + 5) & 3;
+    uint32_t ref[3][3];
+    for (int c = 0; c < 3; ++c) {
+      for (int iy = 0; iy < 3; ++iy) {
+        const uint8_t* row = s_g[c] + (r + 5 + iy) * kP + rq;
+        ref[c][iy] = __builtin_amdgcn_alignbyte(LdsDword(row + 4),
+                                                LdsDword(row), rs);
+      }
+    }
+    float acc[3] = {0.0f, 0.0f, 0.0f}, sw = 0.0f;
+    for (int cy = -3; cy <= 3; ++cy) {
+      uint32_t msad[4];
+      for (int c = 0; c < 3; ++c) {
+        uint64_t sad[2] = {0, 0};
+        for (int iy = 0; iy < 3; ++iy) {
+          const uint8_t* row = s_g[c] + (r + 5 + cy + iy) * kP + wq;
+          const uint32_t q[4] = {LdsDword(row), LdsDword(row + 4),
+                                 LdsDword(row + 8), LdsDword(row + 12)};
+          uint32_t a[3];
+          for (int k = 0; k < 3; ++k) {
+            a[k] = __builtin_amdgcn_alignbyte(q[k + 1], q[k], ws);
+          }
+          for (int h = 0; h < 2; ++h) {
+            sad[h] = __builtin_amdgcn_qsad_pk_u16_u8(
+                uint64_t(a[h]) | (uint64_t(a[h + 1]) << 32), ref[c][iy],
+                sad[h]);
+          }
+        }
+        const uint32_t w4[4] = {uint32_t(sad[0]), uint32_t(sad[0] >> 32),
+                                uint32_t(sad[1]), uint32_t(sad[1] >> 32)};
+        for (int w = 0; w < 4; ++w) {
+          msad[w] = c == 0 ? w4[w] : PkMaxU16(msad[w], w4[w]);
+        }
+      }
+      for (int cx = -3; cx <= 4; ++cx) {
+        const uint32_t word = PkMinU16(msad[(cx + 3) >> 1], 0x01FB01FBu);
+        const uint32_t s16 = ((cx + 3) & 1) ? (word >> 16) : (word & 0xFFFFu);
+        float wt = WeightOfClamped(int(s16), mul64);
+        wt = wt >= 0.05f ? wt : 0.0f;
+        for (int c = 0; c < 3; ++c) {
+          acc[c] = acc[c] + mid[c * kRows * kP + cy * kP + cx] * wt;
+        }
+        sw = sw + wt;
+      }
+    }
+    for (int c = 0; c < 3; ++c) d[c] = acc[c] / sw;
+  }
+  // Clamp to +-half a quantization step around the dequantised DC
+  // (pik/adaptive_reconstruction.cc:320-331).
+  const size_t plane = size_t(P.bx) * P.by;
+  for (int c = 0; c < 3; ++c) {
+    const float dc = mid[c * kRows * kP];
+    const float hs = P.dc_half_step[c];
+    const float lo = dc - hs, hi = dc + hs;
+    const float mn = hi < d[c] ? hi : d[c];
+    B.dc[c * plane + size_t(y) * P.bx + x] = lo < mn ? mn : lo;
+  }
+}
+__global__ void __launch_bounds__(256)
+    KDcEpf(Img in, FrameParams P, FrameBuffers B, const DeviceConsts* K,
+           int n_partial) {
+  KDcEpfBody(in, P, B, K, n_partial, PlainBlock());
+}
+
+// ---------------------------------------------------------------------------
+// EPF + AR clamp on one 32x32 tile, with the u8 guide of the guide image
+// KGuide wrote; the result goes to B.ar.
 //
-// LDS: the input window (46 x 46 per channel) is dead once the filter has
-// run -- each thread keeps the 12 original values it needs for AR in
-// registers -- so AR's coefficients and transform scratch reuse it; with
-// ~45 KB per workgroup three workgroups share a CU.
-//
-// Image mode (!kDc) reads the u8 guide from the guide image KGuide wrote;
-// the DC mode quantises its input itself (no Gaborish on the DC image).
-template <bool kDc>
+// LDS: the input window is dead once the filter has run -- each thread keeps
+// the 12 original values it needs for AR in registers -- so AR's coefficients
+// and transform scratch reuse it.
 __device__ __forceinline__ void KEpfBody(
     Img in, FrameParams P, FrameBuffers B, const DeviceConsts* K,
-    int n_partial, float* out, int out_pitch, size_t out_plane,
     const VBlock& vb) {
-  constexpr int dc_mode = kDc;
-  // Input window: the DC mode keeps the tile with a 7-pixel border (its
-  // guide is computed from it); the image mode only the filter's window,
-  // pixels -3 .. +35 in x and -3 .. +34 in y. Window row / column 0 is
-  // pixel -kOrg of the tile.
-  constexpr int kOrg = kDc ? 7 : 3;
-  constexpr int kRows = kDc ? 46 : 38;
-  constexpr int kCols = kDc ? 46 : 39;
-  constexpr int kInP = kDc ? 48 : 40;  // pitch of s_in rows
+  // Input window: pixels -3 .. +35 of the tile in x and -3 .. +34 in y.
+  // Window row / column 0 is pixel -kOrg of the tile.
+  constexpr int kOrg = 3;
+  constexpr int kRows = 38;
+  constexpr int kCols = 39;
+  constexpr int kInP = 40;             // pitch of s_in rows
   constexpr int kGP = 48;              // pitch of s_g rows (44 used)
   constexpr int kInPlane = kRows * kInP;
   constexpr int kGuideFloats = 3 * 44 * kGP / 4;
   constexpr int kBig = 3 * kInPlane + kGuideFloats > 3 * (kCoefPlane + kTilePlane)
                            ? 3 * kInPlane + kGuideFloats
                            : 3 * (kCoefPlane + kTilePlane);
-  // s_in and s_g, then (AR) s_coef and s_tmp; ~39 KB in the image mode:
-  // four workgroups per CU.
+  // s_in and s_g, then (AR) s_coef and s_tmp; ~39 KB: four workgroups per CU.
   __shared__ __attribute__((aligned(16))) float s_big[kBig];
   __shared__ float s_out[3][kTilePlane];
   __shared__ uint8_t s_acs[16];
@@ -500,29 +629,18 @@ __device__ __forceinline__ void KEpfBody(
   const int tile = XcdTile(vb.x, tiles_x * ((in.H + 31) / 32));
   if (tile < 0) return;
   const int x0 = (tile % tiles_x) * 32, y0 = (tile / tiles_x) * 32;
-  if (!kDc && B.stamps) StampStart(&B.stamps->run[4], vb.x);
-  // the DC mode reduces KDcDequant's min/max partials itself (at most
-  // kDcGroups of them), the image mode reads what KGuide's input was
-  // scaled by
-  GuideScale gs;
-  if (kDc) {
-    __shared__ float s_mm[8];
-    gs = ReducePartials(B.mm_partial, n_partial, s_mm);
-  } else {
-    gs.all_min = B.mm[0];
-    gs.gmul = B.mm[1];
-  }
-  const float all_min = gs.all_min;
-  const float gmul = gs.gmul;
+  if (B.stamps) StampStart(&B.stamps->run[4], vb.x);
+  // the scale of KGuide's guide, for the blocks' sigmas
+  const float gmul = B.mm[1];
 
-  // AR (step 5) needs the descriptor of the storage block whose
+  // AR (step 4) needs the descriptor of the storage block whose
   // coefficients this thread owns (the matrix slots and 1 / qf of the
   // transform's first block); it loads with the input window.
   const int crow = tid >> 6, ccol = (tid & 63) << 2;
   const int ar_blk =
       (y0 / 8 + crow) * P.bx + x0 / 8 + (ccol >> 6);
   const bool ar_valid =
-      !dc_mode && x0 / 8 + (ccol >> 6) < P.bx && y0 / 8 + crow < P.by;
+      x0 / 8 + (ccol >> 6) < P.bx && y0 / 8 + crow < P.by;
   uint4 ar_desc = make_uint4(0, 0, 0, 0);
   if (ar_valid) ar_desc = B.desc[2 * ar_blk + 1];
   // inputs of the per-block sigma (step 2), loaded with the window
@@ -530,24 +648,21 @@ __device__ __forceinline__ void KEpfBody(
   int sg_qf = 0, sg_lut = 0;
   const bool sg_valid = tid < 16 && (x0 / 8 + (tid & 3)) * 8 < in.W &&
                         (y0 / 8 + (tid >> 2)) * 8 < in.H;
-  if (!kDc && sg_valid) {
+  if (sg_valid) {
     const int blk = (y0 / 8 + (tid >> 2)) * P.bx + x0 / 8 + (tid & 3);
     sg_acs = B.acs[blk];
     sg_qf = B.qf[blk];
     sg_lut = B.lut[blk];
   }
 
-  // 1. input tile with a 7-pixel mirrored border (the DC mode computes its
-  //    guide from it); the image mode only needs the filter's window,
-  //    pixels -3 .. +35 of the tile in x and -3 .. +34 in y. One reflection
-  //    gives the mirror for every position within 7 of the image (both
-  //    images are at least 8 wide and high); positions further out (a tile
-  //    wider than a small image reaches up to 38 past its origin) are only
-  //    clamped into the image, their values are never used. All loads are
-  //    issued before the LDS stores. Image-mode tiles whose window columns
-  //    all lie inside the image load aligned float4s (columns -4 .. +35,
-  //    the first one dropped) and mirror only the rows.
-  if (!kDc && x0 >= 4 && x0 + 36 <= in.W && in.vw == in.W) {
+  // 1. input window, mirrored. One reflection gives the mirror for every
+  //    position within 7 of the image (it is at least 8 wide and high);
+  //    positions further out (a tile wider than a small image reaches up to
+  //    38 past its origin) are only clamped into the image, their values are
+  //    never used. All loads are issued before the LDS stores. Tiles whose
+  //    window columns all lie inside the image load aligned float4s (columns
+  //    -4 .. +35, the first one dropped) and mirror only the rows.
+  if (x0 >= 4 && x0 + 36 <= in.W && in.vw == in.W) {
     constexpr int kVec = 3 * kRows * 10;  // float4s per tile
     constexpr int kPer = (kVec + 255) / 256;
     float4 wv[kPer];
@@ -608,7 +723,7 @@ __device__ __forceinline__ void KEpfBody(
       }
     }
   }
-  if (!kDc) {
+  {
     // the guide window: 44 rows of 11 aligned dwords per channel (the guide
     // image's 6-pixel border makes window column 0 the padded column x0)
     const size_t gplane = size_t(B.grows) * B.gpitch;
@@ -625,40 +740,18 @@ __device__ __forceinline__ void KEpfBody(
     int sigma = 0;
     uint8_t a = 0xFF;
     if (sg_valid) {
-      float ac_q, scale;
-      int lut_id;
-      if (dc_mode) {
-        ac_q = float(P.dc_qf);
-        scale = 1.0f;
-        lut_id = 0;
-        a = 0;
-      } else {
-        a = sg_acs;
-        ac_q = float(sg_qf);
-        scale = ARQuantScale(a >> 4);
-        lut_id = sg_lut;
-      }
+      a = sg_acs;
+      const float ac_q = float(sg_qf);
+      const float scale = ARQuantScale(a >> 4);
       const float quant = ac_q * scale * 0.039324273f;
-      sigma = SigmaFromQuant(quant, gmul, lut_id);
+      sigma = SigmaFromQuant(quant, gmul, sg_lut);
     }
     s_sigma[tid] = sigma;
     s_acs[tid] = a;
   }
   __syncthreads();
-  // 3. DC mode: u8 guide over the tile plus a 6-pixel border (MakeGuide,
-  //    no Gaborish on the DC image).
-  if (kDc) {
-    for (int i = tid; i < 3 * 44 * 44; i += 256) {
-      const int c = i / (44 * 44), rem = i % (44 * 44);
-      const int ly = rem / 44, lx = rem % 44;
-      const float g = s_in[c][(ly + 1) * kInP + (lx + 1)];
-      const float scaled = (g - all_min) * gmul;
-      s_g[c][ly * kGP + lx] = static_cast<uint8_t>(static_cast<int>(scaled));
-    }
-    __syncthreads();
-  }
 
-  // 4. EPF (AdaptiveFilter, pik/epf_target.cc:1113-1277): each thread
+  // 3. EPF (AdaptiveFilter, pik/epf_target.cc:1113-1277): each thread
   //    filters 4 horizontally adjacent pixels of one block row. For every
   //    neighbour row offset cy the SADs of the 3x4 patches against the 8
   //    neighbours cx = -3..4 come from two quad-SAD instructions per patch
@@ -810,25 +903,6 @@ __device__ __forceinline__ void KEpfBody(
   }
   __syncthreads();
 
-  if (dc_mode) {
-    // Clamp to +-half a quantization step around the dequantised DC
-    // (pik/adaptive_reconstruction.cc:320-331); only the unpadded region.
-    const int y = y0 + r;
-    for (int j = 0; j < 4; ++j) {
-      const int x = x0 + c0 + j;
-      if (x < P.bx && y < P.by) {
-        for (int c = 0; c < 3; ++c) {
-          const float dc = s_in[c][(r + kOrg) * kInP + c0 + kOrg + j];
-          const float hs = P.dc_half_step[c];
-          const float lo = dc - hs, hi = dc + hs;
-          const float d = s_out[c][PixAt(r, c0 + j)];
-          const float mn = hi < d ? hi : d;
-          out[c * out_plane + size_t(y) * out_pitch + x] = lo < mn ? mn : lo;
-        }
-      }
-    }
-    return;
-  }
   if (B.keep) {
     const int y = y0 + r;
     for (int j = 0; j < 4; ++j) {
@@ -842,7 +916,7 @@ __device__ __forceinline__ void KEpfBody(
     }
   }
 
-  // 5. AR: clamp the DCT of (filtered - original) to half the quantization
+  // 4. AR: clamp the DCT of (filtered - original) to half the quantization
   //    interval with one ratio per coefficient shared by X, Y, B. The
   //    matrix entries of this thread's coefficients load during the forward
   //    transform.
@@ -924,18 +998,15 @@ __device__ __forceinline__ void KEpfBody(
   if (y < in.H && x < in.W) {
     for (int c = 0; c < 3; ++c) {
       const float* d = s_out[c] + PixAt(r, c0);
-      *reinterpret_cast<float4*>(out + c * out_plane + size_t(y) * out_pitch +
-                                 x) =
+      *reinterpret_cast<float4*>(B.ar + (size_t(c) * P.py + y) * B.ipitch + x) =
           make_float4(d[0] + orig[c][0], d[1] + orig[c][1], d[2] + orig[c][2],
                       d[3] + orig[c][3]);
     }
   }
 }
-template <bool kDc>
-__global__ void __launch_bounds__(256, kDc ? 3 : 4)
-    KEpf(Img in, FrameParams P, FrameBuffers B, const DeviceConsts* K,
-         int n_partial, float* out, int out_pitch, size_t out_plane) {
-  KEpfBody<kDc>(in, P, B, K, n_partial, out, out_pitch, out_plane, PlainBlock());
+__global__ void __launch_bounds__(256, 4)
+    KEpf(Img in, FrameParams P, FrameBuffers B, const DeviceConsts* K) {
+  KEpfBody(in, P, B, K, PlainBlock());
 }
 
 // ---------------------------------------------------------------------------
@@ -1237,13 +1308,6 @@ __global__ void __launch_bounds__(256) KCopyPlanes(FrameBuffers B, size_t n) {
   KCopyPlanesBody(B, n, PlainBlock());
 }
 
-template __global__ void KEpf<true>(Img, FrameParams, FrameBuffers,
-                                    const DeviceConsts*, int, float*, int,
-                                    size_t);
-template __global__ void KEpf<false>(Img, FrameParams, FrameBuffers,
-                                     const DeviceConsts*, int, float*, int,
-                                     size_t);
-
 // ---------------------------------------------------------------------------
 // Batched forms: one launch over every frame of a batch (BatchSpan), each
 // frame's images and buffers as the plain launches of pikgpu_run take them.
@@ -1254,16 +1318,14 @@ __global__ void __launch_bounds__(256)
 __global__ void __launch_bounds__(256) KMinMaxFinalBatch(PIKGPU_BATCH_PARAMS) {
   PIKGPU_BATCH_LOOP(KMinMaxFinalBody(B.mm_partial, s.arg[0], B.mm, vb));
 }
-__global__ void __launch_bounds__(256, 3) KEpfDcBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_ONE(KEpfBody<true>(DcImage(P, B), P, B, K, s.arg[0], B.dc, P.bx,
-                                   size_t(P.bx) * P.by, vb));
+__global__ void __launch_bounds__(256) KDcEpfBatch(PIKGPU_BATCH_PARAMS) {
+  PIKGPU_BATCH_ONE(KDcEpfBody(DcImage(P, B), P, B, K, s.arg[0], vb));
 }
 __global__ void __launch_bounds__(256) KGuideBatch(PIKGPU_BATCH_PARAMS) {
   PIKGPU_BATCH_ONE(KGuideBody(IdctImage(P, B), s.arg[0], P, B, s.arg[1], vb));
 }
 __global__ void __launch_bounds__(256, 4) KEpfBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_ONE(KEpfBody<false>(IdctImage(P, B), P, B, K, 0, B.ar,
-                                    B.ipitch, size_t(B.ipitch) * P.py, vb));
+  PIKGPU_BATCH_ONE(KEpfBody(IdctImage(P, B), P, B, K, vb));
 }
 __global__ void __launch_bounds__(256) KCopyPlanesBatch(PIKGPU_BATCH_PARAMS) {
   PIKGPU_BATCH_LOOP(KCopyPlanesBody(B, 3 * size_t(B.ipitch) * P.py, vb));

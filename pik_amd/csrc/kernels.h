@@ -952,10 +952,12 @@ __host__ __device__ inline Img DcImage(const FrameParams& P,
 __global__ void KMinMaxPartial4(Img in, int gaborish, FrameParams P,
                                 FrameBuffers B);
 __global__ void KMinMaxFinal(const float* partial, int n, float* mm);
-template <bool kDc>
+// KDcEpf: rows per workgroup of 32 columns.
+constexpr int kDcEpfRows = 8;
+__global__ void KDcEpf(Img in, FrameParams P, FrameBuffers B,
+                       const DeviceConsts* K, int n_partial);
 __global__ void KEpf(Img in, FrameParams P, FrameBuffers B,
-                     const DeviceConsts* K, int n_partial, float* out,
-                     int out_pitch, size_t out_plane);
+                     const DeviceConsts* K);
 __global__ void KGuide(Img in, int gaborish, FrameParams P, FrameBuffers B,
                        int n_partial);
 __global__ void KDots(FrameParams P, FrameBuffers B);
@@ -968,7 +970,7 @@ __global__ void KCopyPlanes(FrameBuffers B, size_t n);
 // per phase over every frame of a batch; see BatchSpan.
 __global__ void KDcDequantBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KMinMaxFinalBatch(PIKGPU_BATCH_PARAMS);
-__global__ void KEpfDcBatch(PIKGPU_BATCH_PARAMS);
+__global__ void KDcEpfBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KLfBatch(PIKGPU_BATCH_PARAMS);
 __global__ void KPred2x2Batch(PIKGPU_BATCH_PARAMS);
 __global__ void KBlocksBatch(PIKGPU_BATCH_PARAMS);
