@@ -1146,19 +1146,20 @@ __global__ void __launch_bounds__(256)
 // ---------------------------------------------------------------------------
 // Final Gaborish (on the 8-padded image) and XYB -> linear RGB of the
 // xsize x ysize output (pik/compressed_image.cc:1164-1179). Thread x of a
-// workgroup walks kFinalRows rows of column x of its 256-column strip with
+// workgroup walks `rows` rows (FinalRows) of column x of its 256-column strip
+// with
 // the 3x3 window of each channel in registers, so every input value is
 // loaded three times (left, centre, right) instead of nine.
 __device__ __forceinline__ void KFinalBody(
-    FrameParams P, FrameBuffers B, const DeviceConsts* K, const VBlock& vb) {
+    FrameParams P, FrameBuffers B, const DeviceConsts* K, int rows,
+    const VBlock& vb) {
   const int strips = (P.px + 255) / 256;
-  const int tile =
-      XcdTile(vb.x, strips * ((P.py + kFinalRows - 1) / kFinalRows));
+  const int tile = XcdTile(vb.x, strips * ((P.py + rows - 1) / rows));
   if (tile < 0) return;
   if (B.stamps) StampStart(&B.stamps->run[6], vb.x);
   const int x = (tile % strips) * 256 + threadIdx.x;
-  const int ya = (tile / strips) * kFinalRows;
-  const int yb = min(P.py, ya + kFinalRows);
+  const int ya = (tile / strips) * rows;
+  const int yb = min(P.py, ya + rows);
   if (x >= P.px) return;
   const size_t plane = size_t(P.py) * B.ipitch;
   const int xm = Mirror(x - 1, P.px), xp = Mirror(x + 1, P.px);
@@ -1292,8 +1293,8 @@ __device__ __forceinline__ void KFinalBody(
   if (B.stamps) StampEnd(B.stamps->end[0], vb.x, vb.nx);
 }
 __global__ void __launch_bounds__(256)
-    KFinal(FrameParams P, FrameBuffers B, const DeviceConsts* K) {
-  KFinalBody(P, B, K, PlainBlock());
+    KFinal(FrameParams P, FrameBuffers B, const DeviceConsts* K, int rows) {
+  KFinalBody(P, B, K, rows, PlainBlock());
 }
 
 // The IDCT image as the AR output (frames without adaptive
@@ -1334,7 +1335,7 @@ __global__ void __launch_bounds__(256) KDotsBatch(PIKGPU_BATCH_PARAMS) {
   PIKGPU_BATCH_LOOP(KDotsBody(P, B, vb));
 }
 __global__ void __launch_bounds__(256) KFinalBatch(PIKGPU_BATCH_PARAMS) {
-  PIKGPU_BATCH_LOOP(KFinalBody(P, B, K, vb));
+  PIKGPU_BATCH_LOOP(KFinalBody(P, B, K, kFinalRows, vb));
 }
 
 }  // namespace pikgpu

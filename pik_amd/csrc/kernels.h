@@ -961,9 +961,20 @@ __global__ void KEpf(Img in, FrameParams P, FrameBuffers B,
 __global__ void KGuide(Img in, int gaborish, FrameParams P, FrameBuffers B,
                        int n_partial);
 __global__ void KDots(FrameParams P, FrameBuffers B);
-// KFinal: rows per workgroup of its 256-column strips.
+// KFinal: rows per workgroup of its 256-column strips. A thread walks them
+// one after the other, about 1 us each where the chip is not full, and reads
+// two more: kFinalRows where that leaves four workgroups per CU (and in a
+// batch, whose frames fill the chip together), else as many as do, at least 2
+// (803x533: 18 us with 16 rows, 8 us with 2; one tile: 9 and 4 us).
 constexpr int kFinalRows = 16;
-__global__ void KFinal(FrameParams P, FrameBuffers B, const DeviceConsts* K);
+inline int FinalRows(int px, int py) {
+  const int strips = (px + 255) / 256;
+  int rows = kFinalRows;
+  while (rows > 2 && strips * ((py + rows - 1) / rows) < 1024) rows /= 2;
+  return rows;
+}
+__global__ void KFinal(FrameParams P, FrameBuffers B, const DeviceConsts* K,
+                       int rows);
 __global__ void KCopyPlanes(FrameBuffers B, size_t n);
 
 // Batched forms of the reconstruction's kernels (pikgpu_batch): one launch
