@@ -655,6 +655,28 @@ __device__ __forceinline__ void KEpfBody(
     sg_lut = B.lut[blk];
   }
 
+  // The guide window: 44 rows of 11 aligned dwords per channel (the guide
+  // image's 6-pixel border makes window column 0 the padded column x0). Like
+  // the input window's, all its loads are issued before the first LDS store
+  // (one tile 35 us waiting for each of a thread's 6 in turn, 34 us so; 803x533
+  // 49.3 and 47.5 us).
+  constexpr int kGDwords = 3 * 44 * 11, kGPer = (kGDwords + 255) / 256;
+  uint32_t gv[kGPer];
+  {
+    const size_t gplane = size_t(B.grows) * B.gpitch;
+#pragma unroll
+    for (int u = 0; u < kGPer; ++u) {
+      const int k = tid + u * 256;
+      gv[u] = 0;
+      if (k < kGDwords) {
+        const int row = k / 11, d = k - row * 11;
+        const int c = row / 44, ly = row - c * 44;
+        gv[u] = *reinterpret_cast<const uint32_t*>(
+            B.gimg + c * gplane + size_t(y0 + ly) * B.gpitch + x0 + 4 * d);
+      }
+    }
+  }
+
   // 1. input window, mirrored. One reflection gives the mirror for every
   //    position within 7 of the image (it is at least 8 wide and high);
   //    positions further out (a tile wider than a small image reaches up to
@@ -723,16 +745,13 @@ __device__ __forceinline__ void KEpfBody(
       }
     }
   }
-  {
-    // the guide window: 44 rows of 11 aligned dwords per channel (the guide
-    // image's 6-pixel border makes window column 0 the padded column x0)
-    const size_t gplane = size_t(B.grows) * B.gpitch;
-    for (int k = tid; k < 3 * 44 * 11; k += 256) {
-      const int c = k / (44 * 11), rem = k - c * (44 * 11);
-      const int row = rem / 11, d = rem - row * 11;
-      const uint32_t v = *reinterpret_cast<const uint32_t*>(
-          B.gimg + c * gplane + size_t(y0 + row) * B.gpitch + x0 + 4 * d);
-      *reinterpret_cast<uint32_t*>(&s_g[c][row * kGP + 4 * d]) = v;
+#pragma unroll
+  for (int u = 0; u < kGPer; ++u) {
+    const int k = tid + u * 256;
+    if (k < kGDwords) {
+      const int row = k / 11, d = k - row * 11;
+      const int c = row / 44, ly = row - c * 44;
+      *reinterpret_cast<uint32_t*>(&s_g[c][ly * kGP + 4 * d]) = gv[u];
     }
   }
   // 2. per-block sigma and strategy
