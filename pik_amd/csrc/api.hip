@@ -243,6 +243,82 @@ hipError_t Copy2D(void* dst, size_t dpitch, const void* src, size_t spitch,
                           stream);
 }
 
+// Whether the n bytes at p are of one allocation, as far as the runtime knows
+// the memory (ordinary host memory it copies through buffers of its own).
+bool OneAllocation(const void* p, size_t n) {
+  const hipDeviceptr_t q = const_cast<void*>(p);
+  void* base = nullptr;
+  size_t size = 0;
+  if (hipPointerGetAttribute(&base, HIP_POINTER_ATTRIBUTE_RANGE_START_ADDR,
+                             q) != hipSuccess ||
+      hipPointerGetAttribute(&size, HIP_POINTER_ATTRIBUTE_RANGE_SIZE, q) !=
+          hipSuccess ||
+      base == nullptr) {
+    (void)hipGetLastError();
+    return true;
+  }
+  const uintptr_t a = reinterpret_cast<uintptr_t>(p);
+  const uintptr_t b = reinterpret_cast<uintptr_t>(base);
+  return a >= b && a + n <= b + size;
+}
+
+// Whether dense host planes lie one behind the other, as they do on the
+// device: they take one copy then, not one each with 10 to 20 us between
+// them. Allocations of their own that happen to touch don't (and were they
+// taken for one, the runtime would refuse the copy).
+template <typename T>
+bool OnePiece(T* const* p, int planes, size_t stride_b, size_t row_b,
+              size_t rows) {
+  if (planes < 2 || (rows > 1 && stride_b != row_b)) return false;
+  for (int c = 1; c < planes; ++c) {
+    if (reinterpret_cast<uintptr_t>(p[c]) !=
+        reinterpret_cast<uintptr_t>(p[0]) + c * row_b * rows) {
+      return false;
+    }
+  }
+  return OneAllocation(p[0], planes * row_b * rows);
+}
+
+// Upload2D of three planes into dense planes one behind the other.
+template <typename T>
+int UploadPlanes(pikgpu_ctx* ctx, void* dst, T* const* src,
+                 size_t src_stride_b, size_t row_b, size_t rows) {
+  if (OnePiece(src, 3, src_stride_b, row_b, rows)) {
+    if (hipMemcpyAsync(dst, src[0], 3 * row_b * rows, hipMemcpyHostToDevice,
+                       ctx->stream) == hipSuccess) {
+      return PIKGPU_OK;
+    }
+    (void)hipGetLastError();
+  }
+  int rc = PIKGPU_OK;
+  for (int c = 0; c < 3 && rc == PIKGPU_OK; ++c) {
+    rc = Upload2D(ctx, static_cast<uint8_t*>(dst) + c * row_b * rows, src[c],
+                  src_stride_b, row_b, rows);
+  }
+  return rc;
+}
+
+// Queues the copies of dense device planes one behind the other to host
+// planes.
+template <typename T>
+int DownloadPlanes(pikgpu_ctx* ctx, T* const* dst, int planes, size_t stride_b,
+                   const void* src, size_t row_b, size_t rows) {
+  if (OnePiece(dst, planes, stride_b, row_b, rows)) {
+    if (hipMemcpyAsync(dst[0], src, planes * row_b * rows,
+                       hipMemcpyDeviceToHost, ctx->stream) == hipSuccess) {
+      return PIKGPU_OK;
+    }
+    (void)hipGetLastError();
+  }
+  for (int c = 0; c < planes; ++c) {
+    HIP_TRY(ctx,
+            Copy2D(dst[c], stride_b,
+                   static_cast<const uint8_t*>(src) + c * row_b * rows, row_b,
+                   row_b, rows, hipMemcpyDeviceToHost, ctx->stream));
+  }
+  return PIKGPU_OK;
+}
+
 // Inverse of the opsin absorbance matrix as Inv3x3Matrix<float> computes it
 // (pik/linalg.h:153-170, pik/opsin_params.cc:13-26).
 void OpsinInverse(float out[9]) {
@@ -860,11 +936,8 @@ int pikgpu_frame_upload(pikgpu_ctx* ctx, const pikgpu_frame* f) {
   rc = ac_packed ? PIKGPU_OK : Grow(ctx, &ctx->ac, 3 * ac_b);
   bool in_flight = false;
   if (rc == PIKGPU_OK && !ac_packed) {
-    for (int c = 0; c < 3 && rc == PIKGPU_OK; ++c) {
-      in_flight = true;
-      rc = Upload2D(ctx, static_cast<uint8_t*>(ctx->ac.p) + c * ac_b, f->ac[c],
-                    f->ac_stride * 2, bx * 128, by);
-    }
+    in_flight = true;
+    rc = UploadPlanes(ctx, ctx->ac.p, f->ac, f->ac_stride * 2, bx * 128, by);
   }
   // (a refused frame: nothing may still read the caller's planes)
   const int valid = ValidateArrays(f, &err, &ctx->scan);
@@ -1119,11 +1192,8 @@ static int DownloadRows(pikgpu_ctx* ctx, uint8_t* const* dst, int planes,
     }
     return PIKGPU_OK;
   }
-  for (int c = 0; c < planes; ++c) {
-    HIP_TRY(ctx, Copy2D(dst[c], stride_b, from + c * plane_b, row_b, row_b,
-                        rows, hipMemcpyDeviceToHost, ctx->stream));
-  }
-  return pikgpu_sync(ctx);
+  const int rc = DownloadPlanes(ctx, dst, planes, stride_b, src, row_b, rows);
+  return rc != PIKGPU_OK ? rc : pikgpu_sync(ctx);
 }
 
 extern "C" {
@@ -1213,12 +1283,9 @@ int pikgpu_frame_add_pass(pikgpu_ctx* ctx, const int16_t* const ac[3],
   }
   int16_t* dst = static_cast<int16_t*>(ctx->ac_extra.p) + extra * 3 * row * P.by;
   int rc;
-  for (int c = 0; c < 3; ++c) {
-    if ((rc = Upload2D(ctx, dst + c * row * P.by, ac[c],
-                       ac_stride * sizeof(int16_t), row * sizeof(int16_t),
-                       P.by))) {
-      return rc;
-    }
+  if ((rc = UploadPlanes(ctx, dst, ac, ac_stride * sizeof(int16_t),
+                         row * sizeof(int16_t), P.by))) {
+    return rc;
   }
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
   P.num_passes += 1;
@@ -1305,10 +1372,9 @@ int pikgpu_quantize(pikgpu_ctx* ctx, const float* const opsin[3],
   const bool predict = P.predict_lf || P.predict_hf;
   if (predict && (rc = Grow(ctx, &ctx->ecorner, 3 * nb * 64 * 4))) return rc;
   float* dev_opsin = static_cast<float*>(ctx->eopsin.p);
-  for (int c = 0; c < 3; ++c) {
-    if ((rc = Upload2D(ctx, dev_opsin + c * plane, opsin[c], opsin_stride * 4,
-                       size_t(P.px) * 4, size_t(P.py))))
-      return rc;
+  if ((rc = UploadPlanes(ctx, dev_opsin, opsin, opsin_stride * 4,
+                         size_t(P.px) * 4, size_t(P.py)))) {
+    return rc;
   }
   // the quantized values replace the frame's own (and any later passes)
   P.num_passes = 1;
@@ -1360,17 +1426,13 @@ int pikgpu_quantize(pikgpu_ctx* ctx, const float* const opsin[3],
   }
   KEncQuant<<<XcdGrid(tiles), 256, 0, st>>>(P, Bt, coef, itable, gsf, ac16);
   HIP_TRY(ctx, hipGetLastError());
-  for (int c = 0; c < 3; ++c) {
-    if (ac_out) {
-      HIP_TRY(ctx, Copy2D(ac_out[c], ac_stride * 2,
-                                    ac16 + c * nb * 64, row * 2, row * 2,
-                                    size_t(P.by), hipMemcpyDeviceToHost, st));
-    }
-    if (dc_out) {
-      HIP_TRY(ctx, Copy2D(dc_out[c], dc_stride * 2, dc16 + c * nb,
-                                    size_t(P.bx) * 2, size_t(P.bx) * 2,
-                                    size_t(P.by), hipMemcpyDeviceToHost, st));
-    }
+  if (ac_out && (rc = DownloadPlanes(ctx, ac_out, 3, ac_stride * 2, ac16,
+                                     row * 2, size_t(P.by)))) {
+    return rc;
+  }
+  if (dc_out && (rc = DownloadPlanes(ctx, dc_out, 3, dc_stride * 2, dc16,
+                                     size_t(P.bx) * 2, size_t(P.by)))) {
+    return rc;
   }
   HIP_TRY(ctx, hipStreamSynchronize(st));
   return PIKGPU_OK;
@@ -1647,11 +1709,8 @@ int pikgpu_fwd_adj(pikgpu_ctx* ctx, const pikgpu_adj_io* io) {
     if ((rc = Upload2D(ctx, qf, io->qf, io->qf_stride * 4, bx * 4, by))) {
       return rc;
     }
-    for (int c = 0; c < 3; ++c) {
-      if ((rc = Upload2D(ctx, inb + c * plane_in, in[c], io->in_stride * 4,
-                         xs * 4, ys))) {
-        return rc;
-      }
+    if ((rc = UploadPlanes(ctx, inb, in, io->in_stride * 4, xs * 4, ys))) {
+      return rc;
     }
     A.qf = qf;
     A.qf_pitch = int(bx);
@@ -1707,17 +1766,14 @@ int pikgpu_fwd_adj(pikgpu_ctx* ctx, const pikgpu_adj_io* io) {
   }
   HIP_TRY(ctx, Copy2D(io->dl_dqf, io->dqf_stride * 4, A.dqf, bx * 4,
                                 bx * 4, by, hipMemcpyDeviceToHost, st));
-  for (int c = 0; c < 3; ++c) {
-    if (nlin) {
-      HIP_TRY(ctx, Copy2D(io->linear[c], io->linear_stride * 4,
-                                    A.linear[c], xs * 4, xs * 4, ys,
-                                    hipMemcpyDeviceToHost, st));
-    }
-    if (ndc) {
-      HIP_TRY(ctx, Copy2D(io->dl_dcoeffs[c], io->dcoeffs_stride * 4,
-                                    A.dcoef[c], bx * 64 * 4, bx * 64 * 4, by,
-                                    hipMemcpyDeviceToHost, st));
-    }
+  if (nlin && (rc = DownloadPlanes(ctx, io->linear, 3, io->linear_stride * 4,
+                                   A.linear[0], xs * 4, ys))) {
+    return rc;
+  }
+  if (ndc && (rc = DownloadPlanes(ctx, io->dl_dcoeffs, 3,
+                                  io->dcoeffs_stride * 4, A.dcoef[0],
+                                  bx * 64 * 4, by))) {
+    return rc;
   }
   if (io->loss) {
     HIP_TRY(ctx, hipMemcpyAsync(io->loss, loss_dev, 8, hipMemcpyDeviceToHost,
@@ -1810,13 +1866,11 @@ int pikgpu_search_quant_field(pikgpu_ctx* ctx,
   }
   float* dev_opsin = static_cast<float*>(ctx->eopsin.p);
   float* target = static_cast<float*>(ctx->adj_in.p);
-  for (int c = 0; c < 3; ++c) {
-    if ((rc = Upload2D(ctx, dev_opsin + c * plane, io->opsin[c],
-                       io->opsin_stride * 4, size_t(P.px) * 4, size_t(P.py))) ||
-        (rc = Upload2D(ctx, target + c * tplane, io->target[c],
-                       io->target_stride * 4, xs * 4, ys))) {
-      return rc;
-    }
+  if ((rc = UploadPlanes(ctx, dev_opsin, io->opsin, io->opsin_stride * 4,
+                         size_t(P.px) * 4, size_t(P.py))) ||
+      (rc = UploadPlanes(ctx, target, io->target, io->target_stride * 4,
+                         xs * 4, ys))) {
+    return rc;
   }
   float* at = static_cast<float*>(ctx->srch.p);
   const auto take = [&](size_t n) {
@@ -1924,17 +1978,13 @@ int pikgpu_search_quant_field(pikgpu_ctx* ctx,
                                   qf, bx * 4, bx * 4, by,
                                   hipMemcpyDeviceToHost, st));
   }
-  for (int c = 0; c < 3; ++c) {
-    if (nac) {
-      HIP_TRY(ctx, Copy2D(io->ac[c], io->ac_stride * 2,
-                                    ac16 + c * nb * 64, bx * 128, bx * 128, by,
-                                    hipMemcpyDeviceToHost, st));
-    }
-    if (ndc) {
-      HIP_TRY(ctx, Copy2D(io->dc[c], io->dc_stride * 2,
-                                    dc16 + c * nb, bx * 2, bx * 2, by,
-                                    hipMemcpyDeviceToHost, st));
-    }
+  if (nac && (rc = DownloadPlanes(ctx, io->ac, 3, io->ac_stride * 2, ac16,
+                                  bx * 128, by))) {
+    return rc;
+  }
+  if (ndc && (rc = DownloadPlanes(ctx, io->dc, 3, io->dc_stride * 2, dc16,
+                                  bx * 2, by))) {
+    return rc;
   }
   if (io->loss) {
     HIP_TRY(ctx, hipMemcpyAsync(io->loss, h_loss, size_t(steps + 1) * 8,

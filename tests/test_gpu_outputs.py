@@ -55,3 +55,22 @@ def test_linear_and_srgb8_downloads(rec, w, h):
         diff = np.abs(out.reshape(h, w, 3).astype(np.int32) - bytes_)
         assert diff.max() <= 1 and (diff != 0).mean() < 1e-3, pad
         assert np.all(base[..., 3 * w:] == 7)
+
+
+@pytest.mark.parametrize("w,h", [(105, 104), (203, 131), (203, 132)])
+def test_planes_one_by_one(rec, w, h):
+    """Dense host planes behind one another, apart, and in another order."""
+    frame = synth.make_frame(w, h, seed=w + h)
+    want, _, _ = checker_recon(frame, stages=False)
+    rec.upload(frame)
+    rec.run()
+    for order in ((0, 1, 2), (2, 1, 0), (0, 2, 4), (0, 1, 3)):
+        base = np.full((5, h, w), 7, np.float32)
+        planes = (abi.c_float_p * 3)(
+            *[base[i].ctypes.data_as(abi.c_float_p) for i in order])
+        rec._check(rec._lib.pikgpu_download(rec._ctx, planes, w * 4))
+        for c, i in enumerate(order):
+            assert np.array_equal(base[i].view(np.uint32),
+                                  want[c].view(np.uint32)), order
+        for i in set(range(5)) - set(order):
+            assert np.all(base[i] == 7), order
