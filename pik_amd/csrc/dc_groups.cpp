@@ -4,7 +4,7 @@
 // and the control fields -- AC strategy, quant field and AR sigma LUT ids
 // under one ANS state. This is DecodeDCGroups / DecodeDCGroup
 // (pik/compressed_dc.cc:276-345, 436-507) without DequantDC and the DC
-// smoothing, which run on the GPU (KDcDequant, KEpf<true>); the int16 DC
+// smoothing, which run on the GPU (KDcDequant, KDcEpf); the int16 DC
 // and the side information land in the frame-wide arrays pikgpu_frame
 // takes.
 #include <smmintrin.h>

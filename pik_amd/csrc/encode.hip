@@ -15,7 +15,7 @@
 //    PredictLf then give dc_dec, the LLF that CopyLlf puts into the
 //    coefficients and the LF prediction)
 //   KEncLf       per block: LF residuals and the decoder-side LF corner
-//                (PredictLfForEncoder), whose 2x DC image KPred2x2Interior
+//                (PredictLfForEncoder), whose 2x DC image KPred2x2
 //                forms; KEncHfResidual per tile: the HF residuals
 //                (ComputePredictionResiduals);
 //   KEncQuant    per 32x32 tile: Y quantized and dequantised
@@ -435,7 +435,7 @@ __global__ void __launch_bounds__(256, 4)
 // dequantised with Y's colour correlation; with the LF prediction added
 // back (and the LLF position restored) they are the decoder-side corner
 // values that DC2x2FromLowFrequencies reads. They go to `corner` (the
-// coefficient layout), for KPred2x2Interior<true>.
+// coefficient layout), for KPred2x2<true>.
 __global__ void __launch_bounds__(256)
     KEncLf(FrameParams P, FrameBuffers B, float* coef, const float* itable,
            float gsf, float* corner) {
