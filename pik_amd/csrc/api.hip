@@ -962,13 +962,16 @@ static int DcGroups(int nblk) {
   return std::min(kDcGroups, int(DivCeil(nblk, 256)));
 }
 // Grid of KMinMaxPartial4: 1024-column strips (four columns per thread), row
-// ranges of >= 8 rows, or of >= 2 while KGuide can still reduce the partials
-// itself: a thread's rows follow one another, which is all the time that the
-// kernel takes where the chip is not full (803x533: 9.4 us with 8 rows,
-// 5.8 us with 2).
-static dim3 MinMaxGrid4(int w, int h) {
+// ranges of >= 8 rows, or for a frame decoded alone of >= 2 while KGuide can
+// still reduce the partials itself: a thread's rows follow one another, which
+// is all the time that the kernel takes where the chip is not full (803x533:
+// 9.4 us with 8 rows, 5.8 us with 2). A batch's frames fill the chip together:
+// there the shorter ranges' halo rows and partials cost more (64 frames of 256
+// to 2048 pixels a side: 220 us with 8 rows, 254 us with 2).
+static dim3 MinMaxGrid4(int w, int h, bool alone) {
   const int nx = int(DivCeil(w, 1024));
-  const int fine = std::min(int(DivCeil(h, 2)), kMinMaxInline / nx);
+  const int fine =
+      alone ? std::min(int(DivCeil(h, 2)), kMinMaxInline / nx) : 1;
   const int ny = std::max(
       {1, fine, std::min(int(DivCeil(h, 8)), kMinMaxMaxGroups / nx)});
   return dim3(nx, ny);
@@ -1060,7 +1063,7 @@ hipError_t pikgpu::EnqueueFullSize(const FrameParams& P,
     const Img ii = IdctImage(P, B);
     const int gab = P.gaborish && !P.use_sharpened;
     // the IDCT image: width a multiple of 8, rows 32-float aligned
-    const dim3 mmg = MinMaxGrid4(ii.W, ii.H);
+    const dim3 mmg = MinMaxGrid4(ii.W, ii.H, true);
     const int partials = int(mmg.x * mmg.y);
     KMinMaxPartial4<<<mmg, 256, 0, st>>>(ii, gab, P, B);
     if (MinMaxInline(partials) == 0) {
@@ -2132,19 +2135,19 @@ bool PhaseGrid(int p, const FrameParams& P, const FrameBuffers& B, int* nx,
       *nx = XcdGrid(int(DivCeil(P.bx, 4) * DivCeil(P.by, 4)));
       return true;
     case 11: {  // minmax
-      const dim3 g = MinMaxGrid4(ii.W, ii.H);
+      const dim3 g = MinMaxGrid4(ii.W, ii.H, false);
       *nx = int(g.x);
       *ny = int(g.y);
       arg[0] = P.gaborish && !P.use_sharpened;
       return P.ar != 0;
     }
     case 12: {  // minmax_final
-      const dim3 g = MinMaxGrid4(ii.W, ii.H);
+      const dim3 g = MinMaxGrid4(ii.W, ii.H, false);
       arg[0] = int(g.x * g.y);
       return P.ar != 0 && MinMaxInline(arg[0]) == 0;
     }
     case 13: {  // guide
-      const dim3 g = MinMaxGrid4(ii.W, ii.H);
+      const dim3 g = MinMaxGrid4(ii.W, ii.H, false);
       *nx = XcdGrid(int(DivCeil(P.px, 32) * DivCeil(P.py, 32)));
       arg[0] = P.gaborish && !P.use_sharpened;
       arg[1] = MinMaxInline(int(g.x * g.y));
