@@ -751,7 +751,8 @@ class SidePack {
     return at;
   }
   size_t bytes() const { return bytes_; }
-  // To `base`: staged when it fits a chunk, else plane by plane.
+  // To `base`: staged when it fits a chunk, else plane by plane, each read in
+  // place until the stream is waited for: every `src` outlives that wait.
   int Upload(pikgpu_ctx* ctx, uint8_t* base) {
     int rc;
     if (bytes_ > kStageChunk) {
@@ -787,11 +788,18 @@ class SidePack {
   size_t bytes_ = 0;
 };
 
+// The frame's dots binned into tiles (BinDots).
+struct DotBins {
+  std::vector<int32_t> ids, starts, list;
+};
+
 // Everything of an upload after the AC planes: parameters, buffers, the other
-// inputs, the frame's buffer table. The copies may still be in flight.
+// inputs, the frame's buffer table. The copies may still be in flight, from
+// the frame's arrays and from `bins`, which receives the dots' tiles: both
+// outlive the caller's wait.
 int UploadRest(pikgpu_ctx* ctx, const pikgpu_frame* f, bool ac_packed,
                int num_tables, size_t bx, size_t by, size_t tx, size_t ty,
-               size_t ngroups) {
+               size_t ngroups, DotBins* bins) {
   FrameParams& P = ctx->P;
   FillParams(f, &P);
   const size_t nblk = bx * by;
@@ -818,9 +826,9 @@ int UploadRest(pikgpu_ctx* ctx, const pikgpu_frame* f, bool ac_packed,
   GROW(mm_partial, kMinMaxMaxGroups * 2 * 4);
   GROW(mm, 2 * 4);
 
-  std::vector<int32_t> dot_ids, dot_starts, dot_list;
   if (f->num_dots) {
-    BinDots(f, int(bx * 8), int(by * 8), &dot_ids, &dot_starts, &dot_list);
+    BinDots(f, int(bx * 8), int(by * 8), &bins->ids, &bins->starts,
+            &bins->list);
   }
   SidePack pack;
   const auto planes = [&](const int16_t* const src[3], size_t stride,
@@ -848,10 +856,11 @@ int UploadRest(pikgpu_ctx* ctx, const pikgpu_frame* f, bool ac_packed,
                                  f->num_dequant_offsets * 4, 1);
   const size_t at_dots = pack.Add(f->dots, 0,
                                   f->num_dots * sizeof(pikgpu_dot), 1);
-  const size_t at_ids = pack.Add(dot_ids.data(), 0, dot_ids.size() * 4, 1);
-  const size_t at_starts = pack.Add(dot_starts.data(), 0,
-                                    dot_starts.size() * 4, 1);
-  const size_t at_list = pack.Add(dot_list.data(), 0, dot_list.size() * 4, 1);
+  const size_t at_ids = pack.Add(bins->ids.data(), 0, bins->ids.size() * 4, 1);
+  const size_t at_starts = pack.Add(bins->starts.data(), 0,
+                                    bins->starts.size() * 4, 1);
+  const size_t at_list = pack.Add(bins->list.data(), 0, bins->list.size() * 4,
+                                  1);
   GROW(side, pack.bytes());
 #undef GROW
   uint8_t* base = static_cast<uint8_t*>(ctx->side.p);
@@ -879,7 +888,7 @@ int UploadRest(pikgpu_ctx* ctx, const pikgpu_frame* f, bool ac_packed,
   B.offsets = reinterpret_cast<const uint32_t*>(base + at_off);
   B.num_tables = num_tables;
   B.dots = reinterpret_cast<const pikgpu_dot*>(base + at_dots);
-  P.dot_tiles = int(dot_ids.size());
+  P.dot_tiles = int(bins->ids.size());
   P.dot_tiles_x = int(DivCeil(bx * 8, 32));
   if (P.dot_tiles) {
     B.dot_tile_ids = reinterpret_cast<const int32_t*>(base + at_ids);
@@ -945,8 +954,10 @@ int pikgpu_frame_upload(pikgpu_ctx* ctx, const pikgpu_frame* f) {
     if (in_flight) (void)hipStreamSynchronize(ctx->stream);
     return valid != PIKGPU_OK ? Fail(ctx, valid, err) : rc;
   }
-  rc = UploadRest(ctx, f, ac_packed, num_tables, bx, by, tx, ty, ngroups);
-  // The caller's arrays are free once the copies are done.
+  DotBins bins;
+  rc = UploadRest(ctx, f, ac_packed, num_tables, bx, by, tx, ty, ngroups,
+                  &bins);
+  // The caller's arrays, and the bins, are free once the copies are done.
   const hipError_t e = hipStreamSynchronize(ctx->stream);
   ctx->stage_used = 0;
   if (rc != PIKGPU_OK) return rc;

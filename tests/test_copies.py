@@ -1,0 +1,91 @@
+"""The library's host <-> device copies against a runtime that carries every
+one of them out as late as it may (tests/native/deferred_hip.cc, on the CPU):
+what a copy reads must stay as it was until the wait that covers it. Each test
+runs in a process of its own, with freed memory overwritten (MALLOC_PERTURB_)."""
+import ctypes
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SOURCE = os.path.join(ROOT, "tests", "native", "deferred_hip.cc")
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    so = str(tmp_path_factory.mktemp("hip") / "libdeferred_hip.so")
+    r = subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC",
+                        "-fvisibility=hidden", "-Wall", "-o", so, SOURCE],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return so
+
+
+def in_child(runtime, name, *args):
+    """Runs child_<name> of this file on the deferred runtime."""
+    r = subprocess.run(
+        [sys.executable, os.path.abspath(__file__), runtime, name] +
+        [str(a) for a in args], capture_output=True, text=True, timeout=300,
+        cwd=ROOT, env=dict(os.environ, MALLOC_PERTURB_="165"))
+    assert r.returncode == 0, r.stdout[-1000:] + r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("w,h,table_mb,dots,pad", [
+    (8, 8, 0, 0, 0), (72, 40, 0, 9, 0), (72, 40, 0, 9, 1),
+    (520, 264, 0, 40, 0), (520, 264, 0, 40, 3),
+    (72, 40, 17, 0, 0), (72, 40, 17, 9, 0), (520, 264, 17, 40, 3)])
+def test_sources_live_until_the_copies_are_done(runtime, w, h, table_mb, dots,
+                                                pad):
+    in_child(runtime, "upload", w, h, table_mb, dots, pad)
+
+
+# --- in the child -----------------------------------------------------------
+
+def large_table(fr, mb):
+    """The frame with `mb` MB of dequant table (the tail is never addressed)."""
+    import numpy as np
+    table = np.ones((mb << 20) // 4, np.float32)
+    table[:fr.dequant_table.size] = fr.dequant_table
+    fr.dequant_table = table
+
+
+def child_upload(hip, w, h, table_mb, dots, pad):
+    """Uploads, a refused one between: nothing waits after either, and no
+    source changed while it waited."""
+    import numpy as np
+    from pik_amd import synth
+    from pik_amd.runtime import PikGpuError, Reconstructor
+    fr = synth.make_frame(w, h, seed=w + h, num_dots=dots)
+    assert len(fr.dots) == dots
+    if table_mb:
+        large_table(fr, table_mb)
+    if pad:
+        for name in ("ac", "dc", "quant_field", "ac_strategy"):
+            a = getattr(fr, name)
+            wide = np.zeros(a.shape[:-1] + (a.shape[-1] + pad,), a.dtype)
+            wide[..., :a.shape[-1]] = a
+            setattr(fr, name, wide[..., :a.shape[-1]])
+    bad = fr.copy()
+    bad.quant_field = bad.quant_field.copy()
+    bad.quant_field[-1, -1] = 0
+    with Reconstructor(0) as rec:
+        for f, good in ((fr, True), (bad, False), (fr, True)):
+            if good:
+                rec.upload(f)
+            else:
+                with pytest.raises(PikGpuError):
+                    rec.upload(f)
+            assert hip.deferred_hip_waiting() == 0
+            assert hip.deferred_hip_changed() == 0
+    assert hip.deferred_hip_copies() > 0
+
+
+if __name__ == "__main__":
+    sys.path.insert(0, ROOT)
+    HIP = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+    globals()["child_" + sys.argv[2]](HIP, *(int(a) for a in sys.argv[3:]))

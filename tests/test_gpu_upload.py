@@ -49,6 +49,17 @@ def test_large_side_inputs():
         assert same(rec.reconstruct(fr), want)
 
 
+def test_large_side_inputs_with_dots():
+    """The dots' tile lists go from host memory of the library's own."""
+    fr = synth.make_frame(520, 264, seed=3, num_dots=40)
+    want, _, _ = checker_recon(fr, stages=False)
+    table = np.ones((17 << 20) // 4, np.float32)
+    table[:fr.dequant_table.size] = fr.dequant_table
+    fr.dequant_table = table
+    with Reconstructor(0) as rec:
+        assert same(rec.reconstruct(fr), want)
+
+
 def test_refused_frame_between_two():
     good = synth.make_frame(320, 200, seed=1)
     bad = synth.make_frame(320, 200, seed=2)
