@@ -27,6 +27,8 @@ HEADERS = ["common.h", "device.h", "kernels.h", "xform.h", "dct1d.h",
 HOST_OUT = os.path.join(HERE, "libpikgpu_host.so")
 HOST_SOURCES = ["host_check.cpp", "host_tables.cpp", "entropy.cpp",
                 "dc_groups.cpp"]
+CHECK_OUT = os.path.join(HERE, "libpikgpu_check.so")
+CHECK_SOURCES = ["device_check.hip"]
 
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
           "-fvisibility=hidden", "-Wall", "-Wno-unused-function",
@@ -46,8 +48,8 @@ def _run(cmd):
 
 def build(verbose=False):
     os.makedirs(BUILD, exist_ok=True)
-    objs = []
-    for src in SOURCES:
+    objs = {}
+    for src in SOURCES + CHECK_SOURCES:
         path = os.path.join(CSRC, src)
         obj = os.path.join(BUILD, src + ".o")
         cmd = [HIPCC] + COMMON
@@ -59,11 +61,15 @@ def build(verbose=False):
         if verbose:
             print(" ".join(cmd))
         _run(cmd)
-        objs.append(obj)
-    tmp = OUT + ".tmp"
-    _run([HIPCC, "-shared", "-fPIC", "--offload-arch=" + ARCH, "-o", tmp] +
-         objs + ["-Wl,--no-undefined", "-Wl,-soname,libpikgpu.so"])
-    os.replace(tmp, OUT)
+        objs[src] = obj
+    # The library, and the device functions that the GPU tests call by
+    # themselves.
+    for out, sources in ((OUT, SOURCES), (CHECK_OUT, CHECK_SOURCES)):
+        tmp = out + ".tmp"
+        _run([HIPCC, "-shared", "-fPIC", "--offload-arch=" + ARCH, "-o", tmp] +
+             [objs[s] for s in sources] +
+             ["-Wl,--no-undefined", "-Wl,-soname," + os.path.basename(out)])
+        os.replace(tmp, out)
     # Host build of the transforms and tables for the CPU test suite.
     tmp = HOST_OUT + ".tmp"
     _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off",

@@ -482,7 +482,7 @@ __global__ void __launch_bounds__(256, 4)
       A.loss_part[tile] = (s_loss[0] + s_loss[1]) + (s_loss[2] + s_loss[3]);
     }
   }
-  if (B.stamps) StampEnd(B.stamps->end[1], blockIdx.x, gridDim.x);
+  if (B.stamps) StampEnd(B.stamps->end[1], blockIdx.x);
 }
 template __global__ void KAdjBackward<false>(FrameParams, FrameBuffers,
                                              const DeviceConsts*, AdjArgs, SearchDist);

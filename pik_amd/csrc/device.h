@@ -84,11 +84,11 @@ struct FrameBuffers {
 };
 
 // Device clock (wall_clock64) at the start of each kernel family and at the
-// end of the last workgroups of the last one: what pikgpu_last_timings
-// reports, without an event between two kernels (each took 5 to 10 us of the
-// stream, up to 40 us of a decode). Starts are written by a launch's first
-// workgroup; ends by its last kEndStamps ones, a slot each, of which the host
-// takes the latest.
+// end of the last one: what pikgpu_last_timings reports, without an event
+// between two kernels (each took 5 to 10 us of the stream, up to 40 us of a
+// decode). Starts are written by a launch's first workgroup; for the end
+// every wave raises one of kEndStamps slots, of which the host takes the
+// latest (a slot for all of them would be contended by 16384 waves).
 constexpr int kEndStamps = 512;
 struct DeviceStamps {
   unsigned long long run[7];       // dc, lf, blocks, guide, epf, dots, final

@@ -350,7 +350,7 @@ __global__ void __launch_bounds__(256)
   int16_t q[3][4];
   QuantizeTile(P, B, coef, itable, gsf, ac, (tile % tiles_x) * 4,
                (tile / tiles_x) * 4, s_val, &sh, q);
-  if (B.stamps) StampEnd(B.stamps->end[2], blockIdx.x, gridDim.x);
+  if (B.stamps) StampEnd(B.stamps->end[2], blockIdx.x);
 }
 
 // A step's quantization and forward model in one (KEncQuant, KAdjForward

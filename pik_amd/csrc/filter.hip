@@ -1309,7 +1309,7 @@ __device__ __forceinline__ void KFinalBody(
       }
     }
   }
-  if (B.stamps) StampEnd(B.stamps->end[0], vb.x, vb.nx);
+  if (B.stamps) StampEnd(B.stamps->end[0], vb.x);
 }
 __global__ void __launch_bounds__(256)
     KFinal(FrameParams P, FrameBuffers B, const DeviceConsts* K, int rows) {

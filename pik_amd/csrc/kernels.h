@@ -182,13 +182,16 @@ __device__ inline float DequantPasses(const FrameParams& P,
   return acc;
 }
 
-// Thread 0 of workgroup wg of n: the launch's start, its end.
+// The launch's start (by thread 0 of its first workgroup) and its end: every
+// wave's, into the latest of its workgroup's slot. What a slot holds of
+// earlier launches is older, so no launch clears it.
 __device__ inline void StampStart(unsigned long long* at, int wg) {
   if (wg == 0 && threadIdx.x == 0) *at = wall_clock64();
 }
-__device__ inline void StampEnd(unsigned long long* at, int wg, int n) {
-  if (wg >= n - kEndStamps && threadIdx.x == 0) {
-    at[wg % kEndStamps] = wall_clock64();
+__device__ inline void StampEnd(unsigned long long* at, int wg) {
+  if ((threadIdx.x & 63) == 0) {
+    atomicMax(at + wg % kEndStamps,
+              static_cast<unsigned long long>(wall_clock64()));
   }
 }
 
