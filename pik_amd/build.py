@@ -23,7 +23,7 @@ SOURCES = ["recon_lf.hip", "recon_blocks.hip", "filter.hip", "adjoint.hip",
            "host_tables.cpp", "quant_tables.cpp", "entropy.cpp", "dc_groups.cpp",
            "frame_parse.cpp"]
 HEADERS = ["common.h", "device.h", "kernels.h", "xform.h", "dct1d.h",
-           "dct_consts.h", "host_api.h", "entropy.h"]
+           "dct_consts.h", "host_api.h", "entropy.h", "srgb.h"]
 HOST_OUT = os.path.join(HERE, "libpikgpu_host.so")
 HOST_SOURCES = ["host_check.cpp", "host_tables.cpp", "entropy.cpp",
                 "dc_groups.cpp"]

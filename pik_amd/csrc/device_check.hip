@@ -7,6 +7,7 @@
 
 #include "device.h"
 #include "kernels.h"
+#include "srgb.h"
 
 #define HAPI extern "C" __attribute__((visibility("default")))
 
@@ -33,7 +34,65 @@ __global__ void __launch_bounds__(256)
   pikgpu::StampEnd(S->end[0], blockIdx.x);
 }
 
+// Every float pattern, 256 of them per thread: how many bytes Srgb8x3 gets
+// other than Srgb8Scaled's (of any of its three samples), how many the fast
+// value alone would, and the largest difference of the two values.
+struct SrgbCheck {
+  unsigned long long wrong, fast_wrong;
+  float largest;
+};
+__global__ void __launch_bounds__(256) KSrgbCheck(SrgbCheck* out) {
+  const uint32_t first = (blockIdx.x * 256 + threadIdx.x) * 256;
+  unsigned wrong = 0, fast_wrong = 0;
+  float largest = 0.0f;
+  for (uint32_t i = 0; i < 256; ++i) {
+    const float v = __uint_as_float(first + i);
+    const float exact = pikgpu::Srgb8Scaled(v), fast = pikgpu::Srgb8Fast(v);
+    // one sample beside two that no edge is near
+    const float r[3] = {v, 100.0f, 100.0f}, g[3] = {100.0f, v, 100.0f},
+                b[3] = {100.0f, 100.0f, v};
+    const uint32_t byte = uint32_t(exact);
+    const uint32_t rest = uint32_t(pikgpu::Srgb8Scaled(100.0f));
+    wrong += pikgpu::Srgb8x3(r) != (byte | rest << 8 | rest << 16);
+    wrong += pikgpu::Srgb8x3(g) != (rest | byte << 8 | rest << 16);
+    wrong += pikgpu::Srgb8x3(b) != (rest | rest << 8 | byte << 16);
+    fast_wrong += uint32_t(fast) != byte;
+    largest = fmaxf(largest, fabsf(fast - exact));
+  }
+  for (int m = 32; m >= 1; m >>= 1) {
+    wrong += __shfl_xor(wrong, m, 64);
+    fast_wrong += __shfl_xor(fast_wrong, m, 64);
+    largest = fmaxf(largest, __shfl_xor(largest, m, 64));
+  }
+  if (threadIdx.x % 64 == 0) {
+    if (wrong) atomicAdd(&out->wrong, wrong);
+    if (fast_wrong) atomicAdd(&out->fast_wrong, fast_wrong);
+    // (floats of one sign order as integers)
+    atomicMax(reinterpret_cast<int*>(&out->largest),
+              __float_as_int(largest));
+  }
+}
+
 }  // namespace
+
+HAPI int pikgpu_check_srgb(unsigned long long* wrong,
+                           unsigned long long* fast_wrong, float* largest) {
+  SrgbCheck* d = nullptr;
+  SrgbCheck h = {};
+  hipError_t e = hipMalloc(&d, sizeof h);
+  if (e != hipSuccess) return e;
+  if ((e = hipMemcpy(d, &h, sizeof h, hipMemcpyHostToDevice)) == hipSuccess) {
+    KSrgbCheck<<<65536, 256>>>(d);
+    if ((e = hipGetLastError()) == hipSuccess) {
+      e = hipMemcpy(&h, d, sizeof h, hipMemcpyDeviceToHost);
+    }
+  }
+  (void)hipFree(d);
+  *wrong = h.wrong;
+  *fast_wrong = h.fast_wrong;
+  *largest = h.largest;
+  return e;
+}
 
 // A launch of `groups` workgroups whose wave `slow` ends last: the latest
 // clock before a stamp, and the latest stamp of the slots. HIP's error code.
