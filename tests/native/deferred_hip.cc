@@ -6,9 +6,9 @@
 //
 // Every copy remembers what its source held when it was queued; a source that
 // holds something else, or is no longer mapped, when the copy is carried out
-// is counted by deferred_hip_changed(). A copy with one end in a range known
-// to the runtime (hipHostMalloc, or declared by deferred_hip_range) that does
-// not lie inside that range is refused, as the runtime refuses it.
+// is counted by deferred_hip_changed(). A copy that reaches into or out of a
+// range known to the runtime (hipHostMalloc, or declared by
+// deferred_hip_range) is refused.
 #include <stdint.h>
 #include <stdlib.h>
 #include <string.h>
@@ -35,7 +35,7 @@ struct Copy {
 std::vector<Copy> queue;   // waiting
 std::vector<size_t> sizes; // bytes of every copy queued so far
 size_t done = 0;           // copies carried out
-int changed = 0;
+int changed = 0, refused = 0;
 std::map<uintptr_t, size_t> ranges;
 
 bool Read(const void* from, void* to, size_t n) {
@@ -53,17 +53,22 @@ bool RangeOf(const void* p, uintptr_t* base, size_t* size) {
   return reinterpret_cast<uintptr_t>(p) < *base + *size;
 }
 bool Fits(const void* p, size_t n) {
+  const uintptr_t a = reinterpret_cast<uintptr_t>(p);
   uintptr_t base;
   size_t size;
-  return !RangeOf(p, &base, &size) ||
-         reinterpret_cast<uintptr_t>(p) + n <= base + size;
+  if (RangeOf(p, &base, &size)) return a + n <= base + size;
+  const auto next = ranges.upper_bound(a);
+  return next == ranges.end() || a + n <= next->first;
 }
 
 int Queue(void* dst, size_t dpitch, const void* src, size_t spitch, size_t row,
           size_t rows, int kind) {
   const size_t reach_s = rows ? (rows - 1) * spitch + row : 0;
   const size_t reach_d = rows ? (rows - 1) * dpitch + row : 0;
-  if (!Fits(src, reach_s) || !Fits(dst, reach_d)) return kInvalidValue;
+  if (!Fits(src, reach_s) || !Fits(dst, reach_d)) {
+    refused += 1;
+    return kInvalidValue;
+  }
   Copy c = {static_cast<uint8_t*>(dst), static_cast<const uint8_t*>(src),
             dpitch, spitch, row, rows, {}};
   if (kind == kHostToDevice) {
@@ -103,6 +108,7 @@ int Alloc(void** p, size_t n) {
 }  // namespace
 
 API int deferred_hip_changed() { return changed; }
+API int deferred_hip_refused() { return refused; }
 API int deferred_hip_waiting() { return int(queue.size()); }
 API int deferred_hip_copies() { return int(sizes.size()); }
 API size_t deferred_hip_bytes(int i) { return sizes[i]; }

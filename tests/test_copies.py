@@ -44,6 +44,23 @@ def test_sources_live_until_the_copies_are_done(runtime, w, h, table_mb, dots,
     in_child(runtime, "upload", w, h, table_mb, dots, pad)
 
 
+# Memory that the runtime knows, as (first plane, planes) of five planes one
+# behind the other, of which the library is given 1 to 3; the copies that it
+# may take for them.
+KNOWN = {"ordinary": (), "one": ((1, 3),), "inside": ((0, 5),),
+         "apart": ((1, 1), (2, 1), (3, 1)), "first": ((1, 1), (2, 2)),
+         "last": ((1, 2), (3, 1)), "behind": ((2, 2),)}
+COPIES = {"ordinary": 1, "one": 1, "inside": 1, "apart": 3, "first": 3,
+          "last": 3, "behind": 3}
+
+
+@pytest.mark.parametrize("known", sorted(KNOWN))
+def test_touching_planes(runtime, known):
+    """Planes that touch go in one copy where they are one allocation, or none
+    that the runtime knows, and else in a copy each."""
+    in_child(runtime, "planes", sorted(KNOWN).index(known))
+
+
 # --- in the child -----------------------------------------------------------
 
 def large_table(fr, mb):
@@ -83,6 +100,58 @@ def child_upload(hip, w, h, table_mb, dots, pad):
             assert hip.deferred_hip_waiting() == 0
             assert hip.deferred_hip_changed() == 0
     assert hip.deferred_hip_copies() > 0
+
+
+def child_planes(hip, which):
+    import numpy as np
+    from pik_amd import abi, synth
+    from pik_amd.runtime import Reconstructor
+    known = sorted(KNOWN)[which]
+    hip.deferred_hip_bytes.restype = ctypes.c_size_t
+    hip.deferred_hip_range.argtypes = [ctypes.c_void_p, ctypes.c_size_t]
+    hip.deferred_hip_forget.argtypes = [ctypes.c_void_p]
+
+    def copies(call, at, plane):
+        """Sizes in planes of the copies of `call` that are planes'."""
+        for first, n in KNOWN[known]:
+            hip.deferred_hip_range(at + first * plane, n * plane)
+        k = hip.deferred_hip_copies()
+        call()
+        for first, n in KNOWN[known]:
+            hip.deferred_hip_forget(at + first * plane)
+        return [hip.deferred_hip_bytes(i) // plane
+                for i in range(k, hip.deferred_hip_copies())
+                if hip.deferred_hip_bytes(i) % plane == 0]
+
+    want = [3] if COPIES[known] == 1 else [1, 1, 1]
+    fr = synth.make_frame(520, 264, seed=1)  # AC above 256 KB: copies of it
+    ac = np.zeros((5,) + fr.ac.shape[1:], np.int16)
+    ac[1:4] = fr.ac
+    fr.ac = ac[1:4]
+    fc, keep = fr.to_c()
+    with Reconstructor(0) as rec:
+        def upload():
+            rec._check(rec._lib.pikgpu_frame_upload(rec._ctx,
+                                                    ctypes.byref(fc)))
+        assert copies(upload, ac.ctypes.data, ac[0].nbytes) == want
+        planes = (ctypes.c_void_p * 3)(*[a.ctypes.data for a in ac[1:4]])
+
+        def add_pass():
+            rec._check(rec._lib.pikgpu_frame_add_pass(
+                rec._ctx, planes, ac.shape[2]))
+        assert copies(add_pass, ac.ctypes.data, ac[0].nbytes) == want
+        rec._check(rec._lib.pikgpu_run(rec._ctx, 0))
+        out = np.full((5, 264, 520), 7, np.float32)
+        to = (abi.c_float_p * 3)(
+            *[a.ctypes.data_as(abi.c_float_p) for a in out[1:4]])
+
+        def download():
+            rec._check(rec._lib.pikgpu_download(rec._ctx, to, 520 * 4))
+        assert copies(download, out.ctypes.data, out[0].nbytes) == want
+        assert np.all(out[1:4] == 0) and np.all(out[::4] == 7)
+    # only ordinary memory with an allocation behind it is tried and refused
+    assert hip.deferred_hip_refused() == (3 if known == "behind" else 0)
+    assert hip.deferred_hip_changed() == 0
 
 
 if __name__ == "__main__":
