@@ -10,28 +10,8 @@
 
 namespace pikgpu {
 
-// 3x3 symmetric convolution of one plane at (x, y) with mirrored borders,
-// in the operation order of strategy::Symmetric3 (pik/convolve.h:605-621).
-__device__ inline float Symmetric3(const float* in, int pitch, int W, int H,
-                                   int x, int y, float w0, float w1,
-                                   float w2) {
-  const int xm = Mirror(x - 1, W), xp = Mirror(x + 1, W);
-  const int ym = Mirror(y - 1, H), yp = Mirror(y + 1, H);
-  const float* rt = in + ym * pitch;
-  const float* rm = in + y * pitch;
-  const float* rb = in + yp * pitch;
-  const float sum_tb = rt[x] + rb[x];
-  const float mul0 = rm[x] * w0;
-  const float sum_lr = rm[xm] + rm[xp];
-  const float x1 = sum_tb + sum_lr;
-  const float mul1 = x1 * w1 + mul0;
-  const float sum_t2 = rt[xm] + rt[xp];
-  const float sum_b2 = rb[xm] + rb[xp];
-  const float x2 = sum_t2 + sum_b2;
-  return x2 * w2 + mul1;
-}
-
-// The same at p of an array whose neighbours all lie inside it.
+// 3x3 symmetric convolution at p of an array that holds all its neighbours, in
+// the operation order of strategy::Symmetric3 (pik/convolve.h:605-621).
 __device__ inline float Conv3(const float* p, int pitch, const float (&w)[3]) {
   const float* t = p - pitch;
   const float* b = p + pitch;
@@ -88,24 +68,6 @@ struct BlockDq {
   float cc;
 };
 
-__device__ inline BlockDq MakeBlockDq(const FrameParams& P,
-                                      const FrameBuffers& B, int c, int row,
-                                      int bxa) {
-  const int blk = row * P.bx + bxa;
-  const uint8_t a = B.acs[blk];
-  const int raw = a >> 4, idx = a & 15;
-  const int qf = B.qf[blk];
-  const int tile = (row >> 3) * P.tx + (bxa >> 3);
-  const int qt = B.dqmap[B.dcf[tile] * 256 + qf - 1];
-  BlockDq d;
-  d.m = B.table + B.offsets[(qt * kNumQuantKinds + AcsQuantKind(raw)) * 3 + c] +
-        idx * 64;
-  d.scaled = qf == 0 ? 1E10f : P.inv_global_scale / float(qf);
-  d.cc = c == 0 ? float(B.ytox[tile] - 128) * 0.00390625f
-                : (c == 2 ? float(B.ytob[tile]) * 0.0078125f : 0.0f);
-  return d;
-}
-
 // Writes block i's two dequantisation descriptors (FrameBuffers::desc), so
 // the block kernels reach the dequant matrices with one dependent load
 // instead of the chain strategy -> quant field -> control field -> table
@@ -133,21 +95,7 @@ __device__ inline void WriteBlockDesc(const FrameParams& P,
       __float_as_uint(P.inv_global_scale / float(qfo)));
 }
 
-// MakeBlockDq's values from the block's descriptor (KDcDequant).
-__device__ inline BlockDq DescBlockDq(const FrameParams& P,
-                                      const FrameBuffers& B, int c, int row,
-                                      int bxa) {
-  const uint4 d = B.desc[2 * (row * P.bx + bxa)];
-  const int tile = (row >> 3) * P.tx + (bxa >> 3);
-  BlockDq q;
-  q.m = B.table + (c == 0 ? d.x : (c == 1 ? d.y : d.z));
-  q.scaled = __uint_as_float(d.w);
-  q.cc = c == 0 ? float(B.ytox[tile] - 128) * 0.00390625f
-                : (c == 2 ? float(B.ytob[tile]) * 0.0078125f : 0.0f);
-  return q;
-}
-
-// Coefficient k of a block from its quantized value q, in DequantCoef's
+// Coefficient k of a block from its quantized value q, in Dequant::DoAC's
 // operation order.
 __device__ inline float DequantWith(const BlockDq& d, int c, int16_t q, int k,
                                     float yval) {
@@ -162,24 +110,6 @@ __device__ inline const int16_t* AcPlane(const FrameParams& P,
   const size_t plane = size_t(P.by) * P.bx * 64;
   return p == 0 ? B.ac + c * plane
                 : B.ac_extra + (size_t(p - 1) * 3 + c) * plane;
-}
-
-// DequantWith summed over the frame's passes: the first pass's value, then
-// each later pass's own value (its colour correlation from its own Y) plus
-// the sum so far (Dequant<false>::DoAC, pik/compressed_image.cc:695-703).
-// `at` indexes the coefficient within a plane; dy is read only for c != 1.
-__device__ inline float DequantPasses(const FrameParams& P,
-                                      const FrameBuffers& B, const BlockDq& d,
-                                      const BlockDq& dy, int c, size_t at,
-                                      int k) {
-  float acc = 0.0f;
-  for (int p = 0; p < P.num_passes; ++p) {
-    float yv = 0.0f;
-    if (c != 1) yv = DequantWith(dy, 1, AcPlane(P, B, p, 1)[at], k, 0.0f);
-    const float v = DequantWith(d, c, AcPlane(P, B, p, c)[at], k, yv);
-    acc = p == 0 ? v : v + acc;
-  }
-  return acc;
 }
 
 // The launch's start (by thread 0 of its first workgroup) and its end: every
@@ -790,26 +720,6 @@ __device__ inline void Idct2x2(float a00, float a01, float a10, float a11,
 template <int N>
 constexpr int ScaleIdx() {
   return N == 2 ? 0 : (N == 4 ? 1 : (N == 8 ? 2 : (N == 16 ? 3 : 4)));
-}
-
-// ReinterpretingDCT<DCTN, N, N> (pik/ac_strategy.cc:272-293), N >= 4:
-// N x N input at `in` (pitch ip) -> N x N output at `out` (pitch op); in and
-// out may alias.
-template <int DCTN, int N>
-__device__ inline void ReinterpDct(const DeviceConsts* K, const float* in,
-                                   int ip, float* out, int op) {
-  float blk[N * N], coef[N * N];
-  for (int y = 0; y < N; ++y) {
-    for (int x = 0; x < N; ++x) blk[y * N + x] = in[y * ip + x];
-  }
-  dct1d::Dct2D<N>(blk, N, coef, N);
-  constexpr int ti = ScaleIdx<N>(), ai = ScaleIdx<DCTN>();
-  for (int y = 0; y < N; ++y) {
-    for (int x = 0; x < N; ++x) {
-      const float v = coef[y * N + x] * K->tscale[ti][y][x];
-      out[y * op + x] = v * K->ascale[ai][y][x];
-    }
-  }
 }
 
 // ReinterpretingIDCT<DCTN, LF, N> (pik/ac_strategy.cc:296-315), N >= 4:

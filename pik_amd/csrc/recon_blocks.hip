@@ -54,7 +54,7 @@ __device__ __forceinline__ void KBlocksBody(
   // Every global load that depends only on the tile's position is issued
   // before the first wait: the strategy bytes, the pred2x2 window, the
   // block's dequantisation descriptor (matrix slots and inv_global_scale /
-  // qf, MakeBlockDq's values), its quantized coefficients and CfL factors.
+  // qf: WriteBlockDesc), its quantized coefficients and CfL factors.
   uint8_t a_own = 0xFF;
   if (tid < 16) {
     const int bxa = tbx + (tid & 3), bya = tby + (tid >> 2);

@@ -277,8 +277,8 @@ __device__ inline void LlfUnit(const LfUnit& f, bool lf, LfShared* s) {
   }
 }
 
-// LowFrequenciesFromDC2x2 of a unit, in place: ReinterpDct<8S, 2S> as a
-// column pass, the transpose and a row pass.
+// LowFrequenciesFromDC2x2 of a unit, in place: ReinterpretingDCT<8S, 2S, 2S>
+// (pik/ac_strategy.cc:272-293) as a column pass, the transpose and a row pass.
 template <int S>
 __device__ inline void LfCoefUnit(const LfUnit& f, LfShared* s) {
   constexpr int N = 2 * S;
