@@ -1427,8 +1427,9 @@ int pikgpu_quantize(pikgpu_ctx* ctx, const float* const opsin[3],
                                              corner);
     if (P.predict_hf) {
       // the encoder's pred2x2: the ring as the decoder forms it (KLf), or
-      // without LF prediction its own; the transforms from KEncLf's corners
-      // (positions no block writes were zeroed at upload)
+      // without LF prediction its own; the transforms from KEncLf's corners.
+      // Ring and blocks are all written here; the positions past them are
+      // undefined and reach no pixel that a transform reads.
       if (!P.predict_lf) {
         const int cache_pos = (kGroupDimBlocks + 2) * (kGroupDimBlocks + 2);
         KEncPred2x2Border<<<dim3(DivCeil(cache_pos, 256), P.gx * P.gy, 3), 256,

@@ -357,7 +357,7 @@ __global__ void __launch_bounds__(256)
 // without predictions): the tile's quantized values go from registers through
 // the dequantisation of the decoder (the descriptors of the current field)
 // and the inverse transforms to the IDCT image. Bound by the dither
-// chains' latency (as KEncQuant); on a 1024x1024 image 33 us, 21 + 18 us as two
+// chains' latency (as KEncQuant); on a 1024x1024 image 31 us, 21 + 18 us as two
 // kernels with the values through memory.
 __global__ void __launch_bounds__(256, 4)
     KSearchForward(FrameParams P, FrameBuffers B, const float* coef,

@@ -23,9 +23,9 @@ namespace pikgpu {
 // DC EPF's guide has no Gaborish and its padding repeats pixels of the
 // image, so its range is the image's). At most kDcGroups workgroups, each
 // walking the blocks with a stride, so that every workgroup of the DC EPF
-// can reduce the partials itself: as two kernels of their own the min/max
-// and its reduction took 7 + 4 us of a 4096x4096 frame and 4 + 3 us and two
-// launches of any small one.
+// can reduce the partials itself. With a thread per block and the min/max and
+// its reduction in two kernels of their own a 4096x4096 frame took 8 + 7 + 4
+// us, 14 us so; a small one 4 + 3 us and two launches more.
 __device__ __forceinline__ void KDcDequantBody(
     const FrameParams& P, const FrameBuffers& B, const VBlock& vb) {
   __shared__ float s_mm[8];
@@ -561,12 +561,14 @@ __global__ void __launch_bounds__(kLfThreads)
 // DCT32 and the DCT16 transforms, which wait for their loads at the same time
 // instead of one after the other -- each for all three planes: X and B take
 // the dequantised Y of their colour correlation from the same thread.
-// Bound by the scattered corners' memory sectors (97 MB of a 4096x4096
-// frame). One thread per block and plane, from a list of the blocks by class
-// that the host built at every upload (0.4 ms at that size), took 40 us;
-// inside KLf, whose large workgroups wait for these loads together, 70 us; in
-// one workgroup for the three kinds of a strip 40 us;
-// 37 us so.
+// Bound by the scattered corners' memory sectors: for some 20 MB of corners
+// of a 4096x4096 frame the L2 fetches 80 MB (twice that by a streaming copy's
+// scale) and 21 MB are written. One thread per block and plane, from a list of
+// the blocks by class that the host built at every upload (0.4 ms at that
+// size), took 40 us; inside KLf, whose large workgroups wait for these loads
+// together, 70 us; in one workgroup for the three kinds of a strip 40 us; 37 us
+// so. (Another frame of that size: 46 us from the list, 45 us so.)
+
 // The three planes' corner value of F-matrix row i, column j of the transform
 // of S x S blocks at frame block (bxa, bya), group block (bxg, byg).
 template <int S, bool kEnc>

@@ -85,7 +85,7 @@ __global__ void __launch_bounds__(256)
 // workgroups sum the partials of the evaluation before. An update, a
 // rounding and two sums of their own took 20 us in four launches, this 7 us
 // (1024x1024 image); a step with the distortion in KAdjBackward and the
-// forward model in KSearchForward 69 us instead of 98.
+// forward model in KSearchForward 64 us (31 + 26 + 7) instead of 98.
 __global__ void __launch_bounds__(256)
     KSearchStep(FrameParams P, FrameBuffers B, SearchArgs S, int t,
                 const float* dist, const float* u0, SearchState from,
