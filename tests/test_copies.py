@@ -44,6 +44,11 @@ def test_sources_live_until_the_copies_are_done(runtime, w, h, table_mb, dots,
     in_child(runtime, "upload", w, h, table_mb, dots, pad)
 
 
+@pytest.mark.parametrize("w,h", [(72, 40), (520, 264)])
+def test_sources_of_the_encoder_calls(runtime, w, h):
+    in_child(runtime, "encoder", w, h)
+
+
 # Memory that the runtime knows, as (first plane, planes) of five planes one
 # behind the other, of which the library is given 1 to 3; the copies that it
 # may take for them.
@@ -100,6 +105,29 @@ def child_upload(hip, w, h, table_mb, dots, pad):
             assert hip.deferred_hip_waiting() == 0
             assert hip.deferred_hip_changed() == 0
     assert hip.deferred_hip_copies() > 0
+
+
+def child_encoder(hip, w, h):
+    """Quantizer, adjoint with host pointers and search: nothing waits when
+    they return, and no source changed while it waited."""
+    import numpy as np
+    from pik_amd import synth
+    from pik_amd.runtime import Reconstructor
+    fr, op = synth.make_opsin_frame(w, h, seed=2, predict=False)
+    target = np.zeros((3, h, w), np.float32)
+    weight = np.ones(fr.quant_field.shape, np.float32)
+    with Reconstructor(0) as rec:
+        rec.upload(fr)
+        for call in (lambda: rec.quantize(op),
+                     lambda: rec.fwd_adj(fr.quant_field.astype(np.float32),
+                                         target=target),
+                     lambda: rec.search_quant_field(op, target, steps=2,
+                                                    weight=weight)):
+            before = hip.deferred_hip_copies()
+            call()
+            assert hip.deferred_hip_copies() > before
+            assert hip.deferred_hip_waiting() == 0
+            assert hip.deferred_hip_changed() == 0
 
 
 def child_planes(hip, which):
